@@ -3,6 +3,7 @@
 // parameter).  Arithmetic is plain float32, left to right, never contracted into fused
 // multiply-adds, so the second pass reproduces the first one bit for bit.
 #include "common.cuh"
+#include "raise_max.cuh"
 
 #include <type_traits>
 
@@ -286,9 +287,11 @@ __global__ __launch_bounds__(kAdamThreads) void fused_amax_kernel(msamp_adamw_te
     const uint32_t b = block_max_u32(__float_as_uint(mxm), red);
     const uint32_t c = block_max_u32(__float_as_uint(mxv), red);
     if (threadIdx.x == 0) {
-        if (a) atomicMax(&d.acc[0], a);
-        if (b) atomicMax(&d.acc[1], b);
-        if (c) atomicMax(&d.acc[2], c);
+        // (this pass stores nothing: the words can be looked at now, the three loads together)
+        const uint32_t sa = seen_word(&d.acc[0]), sb = seen_word(&d.acc[1]), sc = seen_word(&d.acc[2]);
+        raise_max(&d.acc[0], a, sa);
+        raise_max(&d.acc[1], b, sb);
+        raise_max(&d.acc[2], c, sc);
     }
 }
 
@@ -842,7 +845,8 @@ __global__ __launch_bounds__(kAdamThreads) void fused_spec_kernel(msamp_adamw_te
     const float inv_m = 1.0f / ms, inv_v = 1.0f / vs;
     uint32_t mxp = 0;
     float mxm = 0.0f, mxv = 0.0f;
-    float floor_p = __uint_as_float(__hip_atomic_load(&d.acc[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const uint32_t seen_p = seen_word(&d.acc[0]), seen_m = seen_word(&d.acc[1]), seen_v = seen_word(&d.acc[2]);
+    float floor_p = __uint_as_float(seen_p);
     if (!(floor_p >= 0.0f)) floor_p = 0.0f;
     if (base + MSAMP_ADAMW_CHUNK <= n) {
         // the folded, clamp-free form of the step where the tensor's factors allow it (see spec_group)
@@ -891,9 +895,9 @@ __global__ __launch_bounds__(kAdamThreads) void fused_spec_kernel(msamp_adamw_te
     const uint32_t b = block_max_u32(__float_as_uint(mxm), red);
     const uint32_t c = block_max_u32(__float_as_uint(mxv), red);
     if (threadIdx.x == 0) {
-        if (a) atomicMax(&d.acc[0], a);
-        if (b) atomicMax(&d.acc[1], b);
-        if (c) atomicMax(&d.acc[2], c);
+        raise_max(&d.acc[0], a, seen_p);
+        raise_max(&d.acc[1], b, seen_m);
+        raise_max(&d.acc[2], c, seen_v);
     }
 }
 
@@ -1438,6 +1442,7 @@ __global__ __launch_bounds__(kAdamThreads) void plain_amax_kernel(msamp_adamw_te
     PT* param = static_cast<PT*>(d.weight);
     const GT* grad = reinterpret_cast<const GT*>(d.grad);
     const float inv_m = 1.0f / *d.m_scale, inv_v = 1.0f / *d.v_scale;
+    const uint32_t seen_m = seen_word(&d.acc[1]), seen_v = seen_word(&d.acc[2]);
     float mxm = 0.0f, mxv = 0.0f;
     for (size_t i = first + threadIdx.x * 4; i < last; i += kAdamThreads * 4) {
         if (i + 4 <= last) {
@@ -1463,8 +1468,8 @@ __global__ __launch_bounds__(kAdamThreads) void plain_amax_kernel(msamp_adamw_te
     const uint32_t a = block_max_u32(__float_as_uint(mxm), red);
     const uint32_t b = block_max_u32(__float_as_uint(mxv), red);
     if (threadIdx.x == 0) {
-        atomicMax(&d.acc[1], a);
-        atomicMax(&d.acc[2], b);
+        raise_max(&d.acc[1], a, seen_m);
+        raise_max(&d.acc[2], b, seen_v);
     }
 }
 

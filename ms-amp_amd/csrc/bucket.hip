@@ -3,6 +3,9 @@
 // all-reduce.  One workgroup handles one 16384-element chunk of one tensor; a device table describes the
 // tensors and a block map assigns the chunks, as in the fused AdamW step.
 #include "common.cuh"
+#include "raise_max.cuh"
+
+#include <algorithm>
 
 namespace msamp {
 
@@ -23,6 +26,7 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_amax_kernel(msamp_bucke
     const IT* x = static_cast<const IT*>(d.src);
     const size_t n = d.numel, base = static_cast<size_t>(chunk) * MSAMP_BUCKET_CHUNK;
     uint32_t m = 0;
+    const uint32_t seen = seen_word(&d.acc);
     uint8_t* out = d.dst;
     const float s = FMT != 0 ? *d.scale : 1.0f;
     const bool vec_out = FMT == 0 || (reinterpret_cast<uintptr_t>(out) & (EPT - 1)) == 0;
@@ -60,7 +64,7 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_amax_kernel(msamp_bucke
         }
     }
     m = block_max_u32(m, red);
-    if (threadIdx.x == 0 && m) atomicMax(&d.acc, m);
+    if (threadIdx.x == 0) raise_max(&d.acc, m, seen);
 }
 
 // amax[0] of every tensor from the accumulated pattern (NaN and +Inf become +Inf when asked: the all-reduce that
@@ -139,14 +143,13 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_cast_kernel(const msamp
 // summed in float32 first): the dequantization factor
 // is constant per tensor and is applied once at the end, so a tensor is read at one byte per element and never
 // expanded to float32 in memory.
+// A workgroup takes a run of `run` consecutive chunks of the block map and adds to a tensor's accumulator once per tensor
+// it meets: additions to one address are served one at a time (about 12 ns each), and with one per chunk the 1 024
+// chunks of a 16.8 M-element tensor queued for longer (12 us) than their 16 MB take to read.
 template <int FMT, int KIND>    // KIND: 1, 2, or 0 for the maximum
 __global__ __launch_bounds__(kBucketThreads) void fp8_norm_kernel(msamp_norm_item* __restrict__ items,
-                                                                   const int32_t* __restrict__ block_map) {
+                                                                   const int32_t* __restrict__ block_map, int n_blocks, int run) {
     __shared__ double red[kBucketThreads / kWave];
-    const int t = block_map[2 * blockIdx.x], chunk = block_map[2 * blockIdx.x + 1];
-    msamp_norm_item& d = items[t];
-    const uint8_t* q = d.q;
-    const size_t n = d.numel, base = static_cast<size_t>(chunk) * MSAMP_BUCKET_CHUNK;
     double acc = 0.0;
     auto take = [&](float v) {
         const double a = fabs(static_cast<double>(v));
@@ -158,62 +161,79 @@ __global__ __launch_bounds__(kBucketThreads) void fp8_norm_kernel(msamp_norm_ite
             acc = fma(a, a, acc);
         }
     };
-    if (base + MSAMP_BUCKET_CHUNK <= n && (reinterpret_cast<uintptr_t>(q) & 15) == 0) {
-        constexpr int kVecs = MSAMP_BUCKET_CHUNK / (kBucketThreads * 16);    // 4
-        uint4 w[kVecs];
+    // the workgroup's total (maximum) -- lanes, then wavefronts -- into tensor t's accumulator
+    auto flush = [&](int t) {
 #pragma unroll
-        for (int u = 0; u < kVecs; ++u)
-            w[u] = *reinterpret_cast<const uint4*>(q + base + (static_cast<size_t>(u) * kBucketThreads + threadIdx.x) * 16);
-#pragma unroll
-        for (int u = 0; u < kVecs; ++u) {
-            const uint32_t words[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float a, b, c, e;
-                dequant4<FMT>(words[j], a, b, c, e);
+        for (int o = 32; o; o >>= 1) {
+            const double other = __shfl_xor(acc, o);
+            if constexpr (KIND == 0) {
+                acc = (other != other || acc != acc) ? (other != other ? other : acc) : (other > acc ? other : acc);
+            } else {
+                acc += other;
+            }
+        }
+        __syncthreads();    // (the words below may still be read for the tensor before)
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            msamp_norm_item& d = items[t];
+            double total = red[0];
+            for (int w = 1; w < kBucketThreads / kWave; ++w) {
                 if constexpr (KIND == 0) {
-                    take(a), take(b), take(c), take(e);
-                } else if constexpr (KIND == 1) {
-                    // four values at a time in float32 (three roundings of 2^-24 each), then into the double sum: a
-                    // double conversion and addition per element kept the vector units busier than the memory
-                    acc += static_cast<double>((fabsf(a) + fabsf(b)) + (fabsf(c) + fabsf(e)));
+                    total = (red[w] != red[w] || total != total) ? (red[w] != red[w] ? red[w] : total) : (red[w] > total ? red[w] : total);
                 } else {
-                    // the square of an FP8 value is exact in float32
-                    acc += static_cast<double>(fmaf(a, a, b * b) + fmaf(c, c, e * e));
+                    total += red[w];
                 }
             }
-        }
-    } else {
-        for (size_t i = base + threadIdx.x; i < n && i < base + MSAMP_BUCKET_CHUNK; i += kBucketThreads) take(dequant1<FMT>(q[i]));
-    }
-    // workgroup total (maximum): lanes, then wavefronts
-#pragma unroll
-    for (int o = 32; o; o >>= 1) {
-        const double other = __shfl_xor(acc, o);
-        if constexpr (KIND == 0) {
-            acc = (other != other || acc != acc) ? (other != other ? other : acc) : (other > acc ? other : acc);
-        } else {
-            acc += other;
-        }
-    }
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double total = red[0];
-        for (int w = 1; w < kBucketThreads / kWave; ++w) {
             if constexpr (KIND == 0) {
-                total = (red[w] != red[w] || total != total) ? (red[w] != red[w] ? red[w] : total) : (red[w] > total ? red[w] : total);
+                // bit patterns of non-negative doubles order like the values, NaN patterns above all of them
+                atomicMax(reinterpret_cast<unsigned long long*>(&d.acc), static_cast<unsigned long long>(__double_as_longlong(total)));
             } else {
-                total += red[w];
+                atomicAdd(&d.acc, total);
             }
         }
-        if constexpr (KIND == 0) {
-            // bit patterns of non-negative doubles order like the values, NaN patterns above all of them
-            atomicMax(reinterpret_cast<unsigned long long*>(&d.acc), static_cast<unsigned long long>(__double_as_longlong(total)));
+        acc = 0.0;
+    };
+    const int first = blockIdx.x * run, last = first + run < n_blocks ? first + run : n_blocks;
+    int current = block_map[2 * first];
+    for (int e = first; e < last; ++e) {
+        const int t = block_map[2 * e], chunk = block_map[2 * e + 1];
+        if (t != current) {
+            flush(current);
+            current = t;
+        }
+        const uint8_t* q = items[t].q;
+        const size_t n = items[t].numel, base = static_cast<size_t>(chunk) * MSAMP_BUCKET_CHUNK;
+        if (base + MSAMP_BUCKET_CHUNK <= n && (reinterpret_cast<uintptr_t>(q) & 15) == 0) {
+            constexpr int kVecs = MSAMP_BUCKET_CHUNK / (kBucketThreads * 16);    // 4
+            uint4 w[kVecs];
+#pragma unroll
+            for (int u = 0; u < kVecs; ++u)
+                w[u] = *reinterpret_cast<const uint4*>(q + base + (static_cast<size_t>(u) * kBucketThreads + threadIdx.x) * 16);
+#pragma unroll
+            for (int u = 0; u < kVecs; ++u) {
+                const uint32_t words[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float a, b, c, f;
+                    dequant4<FMT>(words[j], a, b, c, f);
+                    if constexpr (KIND == 0) {
+                        take(a), take(b), take(c), take(f);
+                    } else if constexpr (KIND == 1) {
+                        // four values at a time in float32 (three roundings of 2^-24 each), then into the double sum: a
+                        // double conversion and addition per element kept the vector units busier than the memory
+                        acc += static_cast<double>((fabsf(a) + fabsf(b)) + (fabsf(c) + fabsf(f)));
+                    } else {
+                        // the square of an FP8 value is exact in float32
+                        acc += static_cast<double>(fmaf(a, a, b * b) + fmaf(c, c, f * f));
+                    }
+                }
+            }
         } else {
-            atomicAdd(&d.acc, total);
+            for (size_t i = base + threadIdx.x; i < n && i < base + MSAMP_BUCKET_CHUNK; i += kBucketThreads) take(dequant1<FMT>(q[i]));
         }
     }
+    flush(current);
 }
 
 // out[i] = |scale_inv| * acc^(1/p) (the maximum itself for KIND 0), rounded to float once; the accumulator goes back to zero
@@ -322,14 +342,17 @@ int msamp_fp8_norms(msamp_norm_item* items, int n_items, const int32_t* block_ma
     MSAMP_REQUIRE(items != nullptr && (n_blocks == 0 || block_map != nullptr), MSAMP_ERR_NULL, "msamp_fp8_norms: null pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (n_blocks > 0) {
+        // eight workgroups per compute unit keep enough loads in flight; beyond that longer runs instead of more workgroups
+        const int run = std::max(1, n_blocks / (cu_count() * 8));
+        const int grid = (n_blocks + run - 1) / run;
 #define NORM_LAUNCH(FMT)                                                                                                \
     do {                                                                                                              \
         if (norm_kind == 0)                                                                                           \
-            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 0>), dim3(n_blocks), dim3(kBucketThreads), 0, st, items, block_map); \
+            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 0>), dim3(grid), dim3(kBucketThreads), 0, st, items, block_map, n_blocks, run); \
         else if (norm_kind == 1)                                                                                      \
-            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 1>), dim3(n_blocks), dim3(kBucketThreads), 0, st, items, block_map); \
+            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 1>), dim3(grid), dim3(kBucketThreads), 0, st, items, block_map, n_blocks, run); \
         else                                                                                                          \
-            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 2>), dim3(n_blocks), dim3(kBucketThreads), 0, st, items, block_map); \
+            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 2>), dim3(grid), dim3(kBucketThreads), 0, st, items, block_map, n_blocks, run); \
     } while (0)
         if (fp8_type == MSAMP_DT_E4M3) NORM_LAUNCH(MSAMP_DT_E4M3); else NORM_LAUNCH(MSAMP_DT_E5M2);
 #undef NORM_LAUNCH

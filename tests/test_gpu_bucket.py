@@ -200,6 +200,31 @@ def test_fp8_norms_against_float64(fp8_dt, fmt, norm_type):
             assert got[k].item() == pytest.approx(ref32.item(), rel=1e-4)
 
 
+@pytest.mark.parametrize('norm_type', [1.0, 2.0, float('inf')])
+def test_fp8_norms_over_runs_of_chunks(norm_type):
+    """More chunks than eight per compute unit: a workgroup then takes several chunks in a row, which cross from one
+    tensor into the next, end in a partial chunk, and end the table.  The two large tensors hold one code, so their
+    norms are exact numbers; the small ones between them are compared with float64 (one float32 rounding: 2^-24)."""
+    from msamp import _backend
+    chunk = 16384
+    big = chunk * 2600 + 5
+    g = torch.Generator().manual_seed(11)
+    small = [torch.randint(0, 0x7B, (n, ), generator=g, dtype=torch.uint8) for n in (1, chunk, chunk + 1, 3 * chunk - 1)]
+    ones = torch.full((big, ), 0x38, dtype=torch.uint8, device='cuda')
+    vals = [ones] + [v.cuda() for v in small] + [ones[:big - chunk]]
+    si = [torch.tensor(1.0, device='cuda')] * len(vals)
+    for _ in range(2):
+        got = _backend.fp8_norms(vals, si, 5, norm_type).cpu().double()
+        for k, v in enumerate(vals):
+            if k in (0, len(vals) - 1):
+                n = float(v.numel())
+                want = 1.0 if norm_type == float('inf') else n ** (1.0 / norm_type)
+            else:
+                x = fp8.decode(v.cpu(), fp8.E4M3).double().abs()
+                want = (x.max() if norm_type == float('inf') else x.pow(norm_type).sum().pow(1.0 / norm_type)).item()
+            assert got[k].item() == pytest.approx(want, rel=2e-7), (k, norm_type)
+
+
 def test_fp8_norms_nan_empty_and_repeat():
     """A NaN code makes that tensor's norm NaN (as torch.norm would) and only that one; an empty tensor has norm 0;
     calling twice gives the same numbers (the scratch accumulators are left clean)."""
