@@ -260,8 +260,8 @@ int msamp_fp8_gemm(const uint8_t* a, int a_type, const float* a_scale_inv, const
  * (nn/functional.py:84-111 of the reference) then read W, x and dy as they are, and the explicit FP8
  * transposes (transformer_engine_wrapper.py:165-176) are not needed.  Results are bit-identical to
  * msamp_fp8_gemm on transposed copies (every kernel behind these entry points adds up the same 128-byte blocks of K
- * in ascending order).  Supported: a K-major alone, or both; k a multiple of 128 and at least 256, and the row
- * count of every K-major operand (m, and n if b_kmajor) a multiple of 256; otherwise MSAMP_ERR_SHAPE. */
+ * in ascending order).  Supported: a K-major alone, or both; k more than 128, and the leading dimension of every
+ * operand (m, n where K-major, k where row-major) a multiple of 16; otherwise MSAMP_ERR_SHAPE. */
 int msamp_fp8_gemm_kmajor(const uint8_t* a, int a_type, const float* a_scale_inv, int a_kmajor, const uint8_t* b,
                           int b_type, const float* b_scale_inv, int b_kmajor, void* d, int d_dtype, int m, int n, int k,
                           int accumulate, const void* bias, int bias_dtype, msamp_stream_t stream);

@@ -19,10 +19,10 @@ static int dispatch_pair(int x_type, int y_type, const GemmCall& c) {
     return run_gemm_pair<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(c);
 }
 
-// K-major operands: only the direct-to-LDS kernel reads them, so the shape must suit it
+// K-major operands: only the direct-to-LDS kernels read them, so the shape must suit them: two slices of K, rows that are
+// read 16 bytes at a time (a K-major operand's row count and a row-major one's K are its leading dimension)
 static bool kmajor_shape_ok(int NR, int NC, int K, bool xt, bool yt) {
-    const bool fits32 = static_cast<unsigned long long>(NR) * K < (1ull << 32) && static_cast<unsigned long long>(NC) * K < (1ull << 32);
-    return K % kBK == 0 && K >= 2 * kBK && fits32 && (!xt || NR % kDmaTile == 0) && (!yt || NC % kDmaTile == 0);
+    return K > kBK && fits_offsets(NR, NC, K) && (xt ? NR % 16 == 0 : K % 16 == 0) && (yt ? NC % 16 == 0 : K % 16 == 0);
 }
 
 // tile walks registered per problem (kernel-side naming: NR x NC output, K, which operands are K-major)
@@ -192,7 +192,7 @@ extern "C" int msamp_fp8_gemm_kmajor(const uint8_t* a, int a_type, const float* 
     MSAMP_REQUIRE(bias == nullptr || is_hp(bias_dtype), MSAMP_ERR_DTYPE, "msamp_fp8_gemm_kmajor: bias dtype %d", bias_dtype);
     MSAMP_REQUIRE(a_kmajor, MSAMP_ERR_SHAPE, "msamp_fp8_gemm_kmajor: b may be K-major only together with a");
     MSAMP_REQUIRE(m > 0 && n > 0 && k > 0 && kmajor_shape_ok(n, m, k, b_kmajor != 0, true), MSAMP_ERR_SHAPE,
-                  "msamp_fp8_gemm_kmajor: m=%d n=%d k=%d (k must be a multiple of 128 and at least 256, the K-major operands' rows multiples of 256)", m, n, k);
+                  "msamp_fp8_gemm_kmajor: m=%d n=%d k=%d (k must be more than 128, leading dimensions multiples of 16)", m, n, k);
     MSAMP_REQUIRE(a && b && d && a_scale_inv && b_scale_inv, MSAMP_ERR_NULL, "msamp_fp8_gemm_kmajor: null pointer");
     MSAMP_REQUIRE(aligned(a, 16) && aligned(b, 16), MSAMP_ERR_ALIGNMENT, "msamp_fp8_gemm_kmajor: operands must be 16-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);

@@ -46,9 +46,14 @@ struct GemmCall {
 
 template <int XF, int YF>
 int run_gemm_pair(const GemmCall& c);
-// The split-wait instantiations of the 256 x 256-tile kernel for one pair of formats (row-major operands, all three
-// output types, both parities of the slice count).  They live in translation units of their own (gemm_inst.hip built
-// with -DMSAMP_GEMM_SPLIT_UNIT) so that they compile beside the others instead of after them.
+// The other half of a pair's instantiations lives in a translation unit of its own (gemm_inst.hip built with
+// -DMSAMP_GEMM_SPLIT_UNIT), so that they compile side by side: the 256 x 256-tile kernel for a ragged last slice of K, the
+// 128 x 128-tile kernel (all layouts and output types), and the split-wait form (row-major operands, all three output
+// types, both parities of the slice count).
+template <int XF, int YF>
+int run_gemm_ragged(const GemmCall& c);
+template <int XF, int YF>
+int run_gemm_small(const GemmCall& c);
 template <int XF, int YF>
 int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int NR, int NC, int K, const float* xs,
                    const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st);
@@ -60,13 +65,18 @@ int small_tile_limit();
 // the grouped dimension x 8 of the walked one).  Any walk gives the same output bits: it only decides which workgroup
 // takes which tile.  Bit 2 (row-major operands only): the tile loads awaited in two parts, see the kernel.
 int registered_walk(int NR, int NC, int K, bool XT, bool YT);
-// ... which is this rule: K in whole slices, at least four of them; up to half the limit always (one small tile per
+// ... which is this rule: at least four slices of K; up to half the limit always (one small tile per
 // compute unit with the default limit), up to the limit where K is long enough for the second round of small tiles to
 // pay (measured: 128 large tiles level at K = 2048, 15 % ahead at 4096).
 inline bool takes_small_tiles(int NR, int NC, int K) {
     const long big_tiles = static_cast<long>((NR + kDmaTile - 1) / kDmaTile) * ((NC + kDmaTile - 1) / kDmaTile);
     const int limit = small_tile_limit();
-    return K % kBK == 0 && K >= 4 * kBK && (big_tiles <= limit / 2 || (big_tiles <= limit && K >= 3072));
+    return K > 3 * kBK && (big_tiles <= limit / 2 || (big_tiles <= limit && K >= 3072));
+}
+
+// row offsets of the direct-to-LDS kernels are 32 bits
+inline bool fits_offsets(int NR, int NC, int K) {
+    return static_cast<unsigned long long>(NR) * K < (1ull << 32) && static_cast<unsigned long long>(NC) * K < (1ull << 32);
 }
 
 // Implemented with the cast kernels: q = FP8(d * *scale) over n elements, unless *redo is zero (then nothing is done).
@@ -77,6 +87,14 @@ extern template int run_gemm_pair<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&)
 extern template int run_gemm_pair<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_pair<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);
 extern template int run_gemm_pair<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
+extern template int run_gemm_ragged<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&);
+extern template int run_gemm_small<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&);
+extern template int run_gemm_ragged<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
+extern template int run_gemm_small<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
+extern template int run_gemm_ragged<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);
+extern template int run_gemm_small<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);
+extern template int run_gemm_ragged<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
+extern template int run_gemm_small<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
 #define MSAMP_SPLIT_ARGS const uint8_t*, const uint8_t*, void*, int, int, int, int, const float*, const float*, int, const void*, int, hipStream_t
 extern template int run_gemm_split<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(MSAMP_SPLIT_ARGS);
 extern template int run_gemm_split<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(MSAMP_SPLIT_ARGS);

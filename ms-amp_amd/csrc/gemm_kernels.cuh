@@ -382,6 +382,26 @@ __device__ __forceinline__ void acc_clear() {
     });
     asm volatile("s_nop 4" : : : MSAMP_ALL_AGPRS);
 }
+// Fragment registers that vector instructions have just written: an MFMA may read them two wait states later, which the
+// compiler cannot know of an MFMA in assembly.
+__device__ __forceinline__ void settle16(int* f) {
+    asm volatile("s_nop 1"
+                 : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]), "+v"(f[7]), "+v"(f[8]), "+v"(f[9]),
+                   "+v"(f[10]), "+v"(f[11]), "+v"(f[12]), "+v"(f[13]), "+v"(f[14]), "+v"(f[15]));
+}
+// 32 fragment registers (four blocks of eight dwords) of the last, ragged K slice: the bytes past its `rem` K bytes become
+// zero.  Dword w of a block holds the four K bytes from (lane / 16) * 32 + 4w.
+__device__ __forceinline__ void mask_fragments(int* f, int g4, int rem) {
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+        const int bytes = rem - (g4 * 32 + w * 4);
+        const int m = bytes >= 4 ? -1 : bytes <= 0 ? 0 : (1 << (bytes * 8)) - 1;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) f[b * 8 + w] &= m;
+    }
+    settle16(f);
+    settle16(f + 16);
+}
 // After the last MFMA: waits out the MFMA pipe (a 16-pass MFMA's result may be read 18 wait states later) and hands out
 // the token that ties the reads below to this point of the program.
 __device__ __forceinline__ uint32_t acc_fence() {
@@ -407,7 +427,7 @@ __device__ __forceinline__ v4f acc_quad(uint32_t token) {
 }
 
 template <int XF, int YF, typename OT, bool XT = false, bool YT = false, int QF = 0, bool ODD_NK = false, bool QSPEC = false,
-          bool SPLIT = false>
+          bool KTAIL = false, bool SPLIT = false>
 __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_t* __restrict__ X,
                                                                      const uint8_t* __restrict__ Y, OT* __restrict__ D,
                                                                      int NR, int NC, int K,
@@ -460,6 +480,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // of 4096 .. 11008: the second barrier), hence the host's rule K >= 12288.  (A flag read at run time instead of a
     // second instantiation cost the plain form 3 to 7 %: the selects between the two orders sat in the K loop.)
     static_assert(!SPLIT || (!XT && !YT && QF == 0 && !QSPEC), "split waits: plain row-major form only");
+    static_assert(!KTAIL || (!SPLIT && QF == 0), "a ragged last slice: plain and speculative forms only");
     // a walk registered for this problem (timed on this machine) overrides the rules
     if (qa.walk_plus_one > 0) by_columns = (qa.walk_plus_one - 1) & 1, wide = ((qa.walk_plus_one - 1) >> 1) & 1;
     tile_of_id(blockIdx.x, tiles_r, tiles_c, by_columns, wide, tr, tc);
@@ -486,6 +507,10 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // K-major operand: one wave instruction fills 4 k-rows of 256 bytes; lane l lands in k-row l/16,
     // position l%16, and fetches the logical chunk position ^ (k-row % 8)
     const int chunk_t = (lane & 15) ^ ((wave & 1) * 4 + (lane >> 4));
+    // K-major operand, last tile: 16-byte chunks past the end of a k-row are fetched from the tile's first chunk instead
+    // (rows of D that do not exist; the row count is a multiple of 16, so a chunk is in or out as a whole)
+    const int xcol = row0 + chunk_t * 16 < NR ? row0 + chunk_t * 16 : row0;
+    const int ycol = col0 + chunk_t * 16 < NC ? col0 + chunk_t * 16 : col0;
     uint32_t xoff[8], yoff[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -494,20 +519,35 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
         gx = gx < NR ? gx : NR - 1;
         gy = gy < NC ? gy : NC - 1;
         const int krow = (i * 4 + wave) * 4 + (lane >> 4);
-        xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NR) + row0 + chunk_t * 16
+        xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NR) + xcol
                      : static_cast<uint32_t>(gx) * static_cast<uint32_t>(K) + chunk * 16;
-        yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NC) + col0 + chunk_t * 16
+        yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NC) + ycol
                      : static_cast<uint32_t>(gy) * static_cast<uint32_t>(K) + chunk * 16;
     }
+    // KTAIL: K is no multiple of 128 and the last slice holds `rem` bytes of K only.  Its loads stay inside the operand (a
+    // lane whose chunk or k-row lies past the end fetches the slice's first one instead) and its fragments are masked
+    // byte by byte between LDS and MFMA, in both operands (what lies past the end may hold NaN codes): zeros, as
+    // the generic kernel has them there, and the same bits out.  The last slice is straight-line code at the end, so
+    // the K loop is the one of the plain form.
+    const int nk = KTAIL ? (K + kBK - 1) / kBK : K / kBK;
+    const int rem = K - (nk - 1) * kBK;
+    const uint32_t tail_back = KTAIL && chunk * 16 >= rem ? chunk * 16 : 0;
     // one of the 16 loads of a slice (0..7: X rows, 8..15: Y rows), so they can be spread between MFMAs
-    auto dma = [&](int kt, int stage, int i) __attribute__((always_inline)) {
+    auto dma = [&](int kt, int stage, int i, bool last = false) __attribute__((always_inline)) {
         // the i-th load of a slice is load i, or in the split form the i-th in order of need
         constexpr int by_need[16] = {0, 1, 4, 5, 8, 9, 12, 13, 10, 11, 14, 15, 2, 3, 6, 7};
         const int which = SPLIT ? by_need[i] : i;
         const bool is_x = which < 8;
         const size_t slice = static_cast<size_t>(kt) * kBK;
         const uint8_t* src = is_x ? X + (XT ? slice * NR : slice) : Y + (YT ? slice * NC : slice);
-        const uint32_t off = which < 8 ? xoff[which] : yoff[which - 8];
+        uint32_t off = which < 8 ? xoff[which] : yoff[which - 8];
+        if (KTAIL && last) {
+            if (is_x ? XT : YT) {
+                if (((which & 7) * 4 + wave) * 4 + (lane >> 4) >= rem) off = is_x ? xcol : ycol;
+            } else {
+                off -= tail_back;
+            }
+        }
         // (wave-uniform by construction; the readfirstlane keeps it in a scalar register whatever the compiler makes of it)
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + stage * kDmaStage + (which < 8 ? 0 : kDmaTile * kBK) +
                                                             ((which & 7) * 4 + wave) * 1024);
@@ -556,7 +596,6 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // accumulator block (i, j): D rows i * 16 + lane % 16, D columns j * 16 + (lane / 16) * 4 .. + 3 of the quadrant
     acc_clear();
 
-    const int nk = K / kBK;
     int fx[2][32], fy[2][32];
 
     // One quarter of a slice: the 16 MFMAs of X half hx against Y half hy, with the reads of one fragment half
@@ -565,7 +604,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // srcA = Y rows (columns of D), srcB = X rows (rows of D): a lane then holds, for D row lane % 16 of a block, four
     // consecutive D columns -- the layout the epilogue wants.
     auto quarter = [&](auto hxc, auto hyc, int* rd_dst, int rd_stage, bool rd_x, int rd_half, bool do_read, int ld_kt,
-                       int ld_stage, int ld_first, bool do_load) __attribute__((always_inline)) {
+                       int ld_stage, int ld_first, bool do_load, bool ld_last = false) __attribute__((always_inline)) {
         constexpr int cb = (YF == MSAMP_DT_E4M3) ? 0 : 1;
         constexpr int bl = (XF == MSAMP_DT_E4M3) ? 0 : 1;
         const int np = rd_x ? kPX : kPY;
@@ -586,7 +625,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                 if constexpr (SPLIT) {    // four loads per quarter, all four quarters
                     if (do_load && (n & 3) == 3) dma(ld_kt, ld_stage, ld_first + (n >> 2));
                 } else {    // eight per quarter in the second half of the step
-                    if (do_load && (n & 1)) dma(ld_kt, ld_stage, ld_first + (n >> 1));
+                    if (do_load && (n & 1)) dma(ld_kt, ld_stage, ld_first + (n >> 1), ld_last);
                 }
                 // Nothing moves across: one MFMA, then the reads and the load that go with it, so that the LDS reads and
                 // the tile loads stay spread evenly between the MFMAs as written.
@@ -602,16 +641,21 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // Split form: at the start of the step the second part of slice kt's loads has landed (behind it in the queue, if the
     // step before issued loads -- prev_loaded --, the sixteen of slice kt + 1) and everybody is past the reads of the
     // step before; the first part of slice kt + 2 then goes out during quarters 1 and 2, into the rows of blocks 0..3.
-    auto slice = [&](int st, bool has_next, int ld_kt, bool do_load, bool prev_loaded = true) __attribute__((always_inline)) {
+    // KTAIL: ld_last, the slice being loaded is the last one; masked, the slice being computed is.
+    auto slice = [&](int st, bool has_next, int ld_kt, bool do_load, bool prev_loaded = true, bool ld_last = false,
+                     bool masked = false) __attribute__((always_inline)) {
         constexpr std::integral_constant<int, 0> c0{};
         constexpr std::integral_constant<int, 1> c1{};
+        if (KTAIL && masked) mask_fragments(fx[0], g4, rem), mask_fragments(fy[0], g4, rem);
         if constexpr (SPLIT) {
             if (prev_loaded) wait_vmcnt<16>();
             else wait_vmcnt<0>();
             __syncthreads();
         }
         quarter(c0, c0, fy[1], st, false, 1, true, ld_kt, st, 0, SPLIT && do_load);
+        if (KTAIL && masked) mask_fragments(fy[1], g4, rem);
         quarter(c0, c1, fx[1], st, true, 1, true, ld_kt, st, 4, SPLIT && do_load);
+        if (KTAIL && masked) mask_fragments(fx[1], g4, rem);
         if (SPLIT && has_next) {
             // the first part of slice kt + 1; behind it its second part and, if this step loads, the first of slice kt + 2
             if (do_load) wait_vmcnt<16>();
@@ -620,8 +664,8 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
             wait_vmcnt<0>();
         }
         __syncthreads();
-        quarter(c1, c0, fx[0], st ^ 1, true, 0, has_next, ld_kt, st, SPLIT ? 8 : 0, do_load);
-        quarter(c1, c1, fy[0], st ^ 1, false, 0, has_next, ld_kt, st, SPLIT ? 12 : 8, do_load);
+        quarter(c1, c0, fx[0], st ^ 1, true, 0, has_next, ld_kt, st, SPLIT ? 8 : 0, do_load, ld_last);
+        quarter(c1, c1, fy[0], st ^ 1, false, 0, has_next, ld_kt, st, SPLIT ? 12 : 8, do_load, ld_last);
     };
 
     // prologue: slices 0 and 1 (the host sends no problem with fewer than two slices here); wait for slice 0; read
@@ -629,7 +673,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
 #pragma unroll
     for (int w = 0; w < 16; ++w) dma(0, 0, w);
 #pragma unroll
-    for (int w = 0; w < 16; ++w) dma(1, 1, w);
+    for (int w = 0; w < 16; ++w) dma(1, 1, w, nk == 2);
     wait_vmcnt<16>();
     __syncthreads();
 #pragma unroll
@@ -640,11 +684,26 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // even, three when it is odd (ODD_NK, chosen by the host) -- follows as straight-line code: the last slices load
     // nothing and the last one reads no fragments for a successor, which the compiler then knows.
     int kt = 0;
-    for (; kt + 3 < nk; kt += 2) {
+    // (KTAIL: the load of the last slice is not part of the loop, and both parities are in one kernel)
+    for (; kt + (KTAIL ? 4 : 3) < nk; kt += 2) {
         slice(0, true, kt + 2, true);
         slice(1, true, kt + 3, true);
     }
-    if constexpr (ODD_NK) {
+    if constexpr (KTAIL) {
+        // two slices left with everything loaded (nk = 2), three with the last one still to load, or four with two to load
+        if (nk - kt == 3) {
+            slice(0, true, kt + 2, true, true, true);
+            slice(1, true, 0, false);
+            slice(0, false, 0, false, false, false, true);
+        } else {
+            if (nk - kt == 4) {
+                slice(0, true, kt + 2, true);
+                slice(1, true, kt + 3, true, true, true);
+            }
+            slice(0, true, 0, false);
+            slice(1, false, 0, false, false, false, true);
+        }
+    } else if constexpr (ODD_NK) {
         slice(0, true, kt + 2, true);
         slice(1, true, 0, false);
         slice(0, false, 0, false, false);
@@ -662,13 +721,14 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
             int ntr, ntc;
             tile_of_id(nid, tiles_r, tiles_c, by_columns, wide, ntr, ntc);
             const int nr0 = ntr * kDmaTile, nc0 = ntc * kDmaTile;
-            // line L of an operand's 512: row-major, half L % 2 of row L / 2 (clamped like the tile loads); K-major (whole
-            // tiles only), half L % 2 of the tile's 256 bytes in k-row L / 2 (K >= 256 here)
+            // line L of an operand's 512: row-major, half L % 2 of row L / 2; K-major, half L % 2 of the tile's 256 bytes in
+            // k-row L / 2; clamped like the tile loads (K > 128 here)
             auto line = [&](int L, bool is_x) __attribute__((always_inline)) -> const uint8_t* {
                 const int r = L >> 1, hf = (L & 1) * 128;
                 const uint8_t* base = is_x ? X : Y;
                 const int n = is_x ? NR : NC, first = is_x ? nr0 : nc0;
-                if (is_x ? XT : YT) return base + static_cast<size_t>(r) * n + first + hf;
+                if (is_x ? XT : YT)
+                    return base + static_cast<size_t>(!KTAIL || r < K ? r : K - 1) * n + (first + hf < n ? first + hf : first);
                 const int row = first + r < n ? first + r : n - 1;
                 return base + static_cast<size_t>(row) * K + hf;
             };
@@ -1107,12 +1167,12 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
 
 // The kernel is built once for an even and once for an odd number of K slices (its last slices are straight-line
 // code); ODD picks the one that fits K.
-template <int XF, int YF, typename OT, bool XT, bool YT, bool ODD, bool SPLIT = false>
+template <int XF, int YF, typename OT, bool XT, bool YT, bool ODD, bool KTAIL = false, bool SPLIT = false>
 static int launch_gemm_dma_parity(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
                                   const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
     constexpr int smem = 2 * kDmaStage;
     static std::atomic<bool> configured{false};    // setting the attribute twice is harmless
-    auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, 0, ODD, false, SPLIT>;
+    auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, 0, ODD, false, KTAIL, SPLIT>;
     if (!configured.load(std::memory_order_acquire)) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(fp8_gemm_dma_kernel)");
@@ -1237,18 +1297,11 @@ static int launch_gemm(const uint8_t* X, const uint8_t* Y, void* D, int NR, int 
 #include "gemm_small_tile.cuh"
 namespace msamp {
 
-// few 256 x 256 tiles leave most compute units idle: 128 x 128 tiles then (takes_small_tiles(), gemm_small_tile.cuh)
-
+// (problems for the 128 x 128 tiles and those with a ragged last slice of K have gone their way in run_gemm_pair)
 template <int XF, int YF, typename OT>
 static int pick_tile(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
                      const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
-    // the direct-to-LDS kernel needs whole 128-byte K slices, at least two of them, and 32-bit row offsets; where it can run it is the
-    // faster one at every size (measured 2.2x from a single 256 x 256 tile up to 121 tiles).  Everything else takes
-    // the generic register-staged kernel with 128 x 128 tiles.
-    const bool fits32 = static_cast<unsigned long long>(NR) * K < (1ull << 32) && static_cast<unsigned long long>(NC) * K < (1ull << 32);
-    if (fits32 && takes_small_tiles(NR, NC, K))
-        return launch_gemm_dma128<XF, YF, OT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
-    if (K % kBK == 0 && K >= 2 * kBK && fits32)
+    if (K % kBK == 0 && K >= 2 * kBK && fits_offsets(NR, NC, K))
         return launch_gemm_dma<XF, YF, OT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
     return launch_gemm<128, 128, XF, YF, OT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
 }
@@ -1266,25 +1319,16 @@ static int pick_out(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, in
     }
 }
 
-template <int XF, int YF, typename OT, bool XT, bool YT>
-static int pick_tile_kmajor(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs, const float* ys,
-                            int accumulate, const void* bias, int bias_dt, hipStream_t st) {
-    // (the entry point has checked the shape: whole 256-row tiles of every K-major operand, 32-bit offsets)
-    if (takes_small_tiles(NR, NC, K))
-        return launch_gemm_dma128<XF, YF, OT, XT, YT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
-    return launch_gemm_dma<XF, YF, OT, XT, YT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
-}
-
 template <int XF, int YF, bool XT, bool YT>
 static int pick_out_kmajor(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int NR, int NC, int K, const float* xs,
                            const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
     switch (d_dtype) {
         case MSAMP_DT_F32:
-            return pick_tile_kmajor<XF, YF, float, XT, YT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
+            return launch_gemm_dma<XF, YF, float, XT, YT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
         case MSAMP_DT_F16:
-            return pick_tile_kmajor<XF, YF, f16_t, XT, YT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
+            return launch_gemm_dma<XF, YF, f16_t, XT, YT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
         default:
-            return pick_tile_kmajor<XF, YF, bf16_t, XT, YT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
+            return launch_gemm_dma<XF, YF, bf16_t, XT, YT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
     }
 }
 
@@ -1322,8 +1366,8 @@ int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int
                    const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
     const bool odd = (K / kBK) & 1;
 #define MSAMP_SPLIT_LAUNCH(OT)                                                                                                         \
-    return odd ? launch_gemm_dma_parity<XF, YF, OT, false, false, true, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st) \
-               : launch_gemm_dma_parity<XF, YF, OT, false, false, false, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st)
+    return odd ? launch_gemm_dma_parity<XF, YF, OT, false, false, true, false, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st) \
+               : launch_gemm_dma_parity<XF, YF, OT, false, false, false, false, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st)
     switch (d_dtype) {
         case MSAMP_DT_F32: MSAMP_SPLIT_LAUNCH(float);
         case MSAMP_DT_F16: MSAMP_SPLIT_LAUNCH(f16_t);
@@ -1331,12 +1375,50 @@ int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int
     }
 #undef MSAMP_SPLIT_LAUNCH
 }
+
+// output type and operand layout of a call -> one instantiation of LAUNCH<XF, YF, output type, XT, YT>
+#define MSAMP_LAYOUT_LAUNCH(LAUNCH, OT)                                                                                              \
+    do {                                                                                                                             \
+        if (c.xt && c.yt) return LAUNCH<XF, YF, OT, true, true>(MSAMP_CALL_ARGS);                                                     \
+        if (c.yt) return LAUNCH<XF, YF, OT, false, true>(MSAMP_CALL_ARGS);                                                            \
+        return LAUNCH<XF, YF, OT, false, false>(MSAMP_CALL_ARGS);                                                                     \
+    } while (0)
+#define MSAMP_CALL_ARGS c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, c.accumulate, c.bias, c.bias_dt, c.st
+#define MSAMP_TYPE_LAUNCH(LAUNCH)                                   \
+    switch (c.d_dtype) {                                            \
+        case MSAMP_DT_F32: MSAMP_LAYOUT_LAUNCH(LAUNCH, float);      \
+        case MSAMP_DT_F16: MSAMP_LAYOUT_LAUNCH(LAUNCH, f16_t);      \
+        default: MSAMP_LAYOUT_LAUNCH(LAUNCH, bf16_t);               \
+    }
+
+template <int XF, int YF, typename OT, bool XT, bool YT>
+static int launch_gemm_ragged(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
+                              const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
+    return launch_gemm_dma_parity<XF, YF, OT, XT, YT, false, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
+}
+template <int XF, int YF>
+int run_gemm_ragged(const GemmCall& c) {
+    MSAMP_TYPE_LAUNCH(launch_gemm_ragged)
+}
+template <int XF, int YF>
+int run_gemm_small(const GemmCall& c) {
+    MSAMP_TYPE_LAUNCH(launch_gemm_dma128)
+}
 #endif
 
 // Everything behind the C entry points for one pair of operand formats.  gemm_inst.hip instantiates it once per
 // pair (four translation units, so that they compile side by side).
+//
+// Which kernel: few 256 x 256 tiles leave most compute units idle and take 128 x 128 tiles (takes_small_tiles()).  The
+// direct-to-LDS kernels need at least two 128-byte slices of K and 32-bit row offsets; where they can run they are the
+// faster ones at every size (256 x 256 x 4096: 35 against 80 us with the generic kernel), also with a ragged last slice
+// (12605 x 4304 x 1200: see the table of the measured cases).  Everything else takes the generic register-staged kernel.
 template <int XF, int YF>
 int run_gemm_pair(const GemmCall& c) {
+    if (c.qa == nullptr && fits_offsets(c.NR, c.NC, c.K)) {
+        if (takes_small_tiles(c.NR, c.NC, c.K)) return run_gemm_small<XF, YF>(c);
+        if (c.K > kBK && c.K % kBK) return run_gemm_ragged<XF, YF>(c);
+    }
     if (c.qa != nullptr && c.qspec) {
         if (c.xt) return pick_out_spec<XF, YF, true>(c.X, c.Y, c.D, c.d_dtype, c.NR, c.NC, c.K, c.xs, c.ys, c.accumulate, *c.qa, c.st);
         return pick_out_spec<XF, YF, false>(c.X, c.Y, c.D, c.d_dtype, c.NR, c.NC, c.K, c.xs, c.ys, c.accumulate, *c.qa, c.st);

@@ -1,6 +1,6 @@
 // The direct-to-LDS FP8 GEMM with 128 x 128 output tiles, for problems that leave most compute units idle with
-// 256 x 256 tiles (a 2048 x 2048 output is 64 of those, a quarter of the chip, and 256 of these).  K a multiple of 128
-// and at least 512; operands row-major (K-contiguous) or, with XT / YT, K-major ([K][rows], rows a multiple of 128):
+// 256 x 256 tiles (a 2048 x 2048 output is 64 of those, a quarter of the chip, and 256 of these).  At least four
+// 128-byte slices of K (the last one may be ragged: KTAIL); operands row-major (K-contiguous) or, with XT / YT, K-major ([K][rows], rows a multiple of 16):
 // the slice then lies in LDS as 128 k-rows of 128 bytes, the 16-byte position XOR-ed with k % 8, and the fragments
 // come from the transposing LDS read, as in the large tile.
 //
@@ -29,12 +29,11 @@ constexpr int kSmallTile = 128;
 constexpr int kSmallStage = 2 * kSmallTile * kBK;    // 32 KiB
 constexpr int kSmallStages = 5;    // all 160 KiB of the LDS
 
-template <int XF, int YF, typename OT, bool XT = false, bool YT = false>
-__global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uint8_t* __restrict__ X, const uint8_t* __restrict__ Y,
-                                                                        OT* __restrict__ D, int NR, int NC, int K,
-                                                                        const float* __restrict__ x_scale_inv,
-                                                                        const float* __restrict__ y_scale_inv, int accumulate,
-                                                                        const void* __restrict__ bias, int bias_dt) {
+template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL>
+__device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const uint8_t* __restrict__ Y, OT* __restrict__ D, int NR,
+                                            int NC, int K, const float* __restrict__ x_scale_inv,
+                                            const float* __restrict__ y_scale_inv, int accumulate, const void* __restrict__ bias,
+                                            int bias_dt) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     const int tiles_r = (NR + kSmallTile - 1) / kSmallTile, tiles_c = (NC + kSmallTile - 1) / kSmallTile;
     int tr, tc;
@@ -53,6 +52,9 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uin
     const int chunk_t = (lane & 7) ^ (lane >> 3);
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
         static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem)));
+    // K-major operand, last tile: chunks past the end of a k-row are fetched from the tile's first chunk instead
+    const int xcol = row0 + chunk_t * 16 < NR ? row0 + chunk_t * 16 : row0;
+    const int ycol = col0 + chunk_t * 16 < NC ? col0 + chunk_t * 16 : col0;
     uint32_t xoff[4], yoff[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -61,24 +63,36 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uin
         gx = gx < NR ? gx : NR - 1;
         gy = gy < NC ? gy : NC - 1;
         const int krow = (i * 4 + wave) * 8 + (lane >> 3);
-        xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NR) + row0 + chunk_t * 16
+        xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NR) + xcol
                      : static_cast<uint32_t>(gx) * static_cast<uint32_t>(K) + chunk * 16;
-        yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NC) + col0 + chunk_t * 16
+        yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NC) + ycol
                      : static_cast<uint32_t>(gy) * static_cast<uint32_t>(K) + chunk * 16;
     }
+    // KTAIL: a ragged last slice of `rem` K bytes, handled as in the large tile (loads kept inside the operand, fragments
+    // masked)
+    const int nk = KTAIL ? (K + kBK - 1) / kBK : K / kBK;    // at least 4 (the host sees to that)
+    const int rem = K - (nk - 1) * kBK;
+    const uint32_t tail_back = KTAIL && chunk * 16 >= rem ? chunk * 16 : 0;
     // one of the 8 loads of a slice (0..3: X rows, 4..7: Y rows); assembly for the reason given at the large tile
-    auto dma = [&](int kt, int which) __attribute__((always_inline)) {
+    auto dma = [&](int kt, int which, bool last = false) __attribute__((always_inline)) {
         const bool is_x = which < 4;
         const size_t slice = static_cast<size_t>(kt) * kBK;
         const uint8_t* src = is_x ? X + (XT ? slice * NR : slice) : Y + (YT ? slice * NC : slice);
-        const uint32_t off = is_x ? xoff[which] : yoff[which - 4];
+        uint32_t off = is_x ? xoff[which] : yoff[which - 4];
+        if (KTAIL && last) {
+            if (is_x ? XT : YT) {
+                if (((which & 3) * 4 + wave) * 8 + (lane >> 3) >= rem) off = is_x ? xcol : ycol;
+            } else {
+                off -= tail_back;
+            }
+        }
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + (kt % kSmallStages) * kSmallStage +
                                                             (is_x ? 0 : kSmallTile * kBK) + ((which & 3) * 4 + wave) * 1024);
         asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(off), "s"(src) : "memory", "m0");
     };
-    auto dma_slice = [&](int kt) __attribute__((always_inline)) {
+    auto dma_slice = [&](int kt, bool last = false) __attribute__((always_inline)) {
 #pragma unroll
-        for (int w = 0; w < 8; ++w) dma(kt, w);
+        for (int w = 0; w < 8; ++w) dma(kt, w, last);
     };
 
     // ---- LDS -> fragments: for row lane % 16 of a 16-row block a lane holds the K-bytes (lane / 16) * 32 .. + 31 of the
@@ -118,8 +132,10 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uin
     // the 16 MFMAs of the slice held in fragment set `cur`, with the 16 fragment reads of slice rd_kt (into the other
     // set) between them.  srcA = Y rows, srcB = X rows: a lane then holds, for D row lane % 16 of a block, four
     // consecutive D columns.
-    auto step = [&](auto curc, int rd_kt, bool do_read, int ld_kt, bool do_load) __attribute__((always_inline)) {
+    auto step = [&](auto curc, int rd_kt, bool do_read, int ld_kt, bool do_load, bool ld_last = false,
+                    bool masked = false) __attribute__((always_inline)) {
         constexpr int cur = decltype(curc)::value;
+        if (KTAIL && masked) mask_fragments(fx[cur], g4, rem), mask_fragments(fy[cur], g4, rem);
         constexpr int cb = (YF == MSAMP_DT_E4M3) ? 0 : 1;
         constexpr int bl = (XF == MSAMP_DT_E4M3) ? 0 : 1;
         static_for<4>([&](auto jc) {
@@ -139,7 +155,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uin
                 }
                 // the eight tile loads of slice ld_kt, one every other MFMA: issued in one go they hold the wave, and with
                 // it its MFMAs, for as long as the memory pipe takes to accept them
-                if (do_load && (n & 1)) dma(ld_kt, n >> 1);
+                if (do_load && (n & 1)) dma(ld_kt, n >> 1, ld_last);
                 __builtin_amdgcn_sched_barrier(0);
             });
         });
@@ -147,11 +163,10 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uin
     constexpr std::integral_constant<int, 0> c0{};
     constexpr std::integral_constant<int, 1> c1{};
 
-    const int nk = K / kBK;    // at least 4 (the host sees to that)
     dma_slice(0);
     dma_slice(1);
     dma_slice(2);
-    dma_slice(3);
+    dma_slice(3, nk == 4);
     wait_vmcnt<24>();
     __syncthreads();
 #pragma unroll
@@ -160,13 +175,13 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uin
     // Before the step of slice kt: slices kt + 1 .. kt + 3 are on their way (24 loads of this wave), slice kt is in
     // registers.  Wait for slice kt + 1, meet (it has landed in every wave's part of the stage, and nobody reads the
     // stage of slice kt - 1 any more), compute slice kt while reading kt + 1 and sending for slice kt + 4 into that stage.
-    auto turn = [&](auto curc, int kt) __attribute__((always_inline)) {
+    auto turn = [&](auto curc, int kt, bool ld_last = false) __attribute__((always_inline)) {
         wait_vmcnt<16>();
         __syncthreads();
-        step(curc, kt + 1, true, kt + 4, true);
+        step(curc, kt + 1, true, kt + 4, true, ld_last);
     };
     int kt = 0;
-    for (; kt + 5 < nk; kt += 2) {
+    for (; kt + (KTAIL ? 6 : 5) < nk; kt += 2) {    // (KTAIL: the load of the last slice is not part of the loop)
         turn(c0, kt);
         turn(c1, kt + 1);
     }
@@ -181,12 +196,17 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uin
         wait_vmcnt<0>();
         __syncthreads();
         step(ac, k0 + 3, true, 0, false);
-        step(bc, 0, false, 0, false);
+        step(bc, 0, false, 0, false, false, true);
     };
     if (kt + 5 == nk) {
-        turn(c0, kt);
+        turn(c0, kt, true);
         tail4(c1, c0, kt + 1);
     } else {
+        if (KTAIL && kt + 6 == nk) {
+            turn(c0, kt);
+            turn(c1, kt + 1, true);
+            kt += 2;
+        }
         tail4(c0, c1, kt);
     }
     const uint32_t acc_token = acc_fence();
@@ -276,11 +296,29 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uin
 }
 
 template <int XF, int YF, typename OT, bool XT = false, bool YT = false>
-static int launch_gemm_dma128(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs, const float* ys,
+__global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma128_kernel(const uint8_t* __restrict__ X, const uint8_t* __restrict__ Y,
+                                                                        OT* __restrict__ D, int NR, int NC, int K,
+                                                                        const float* __restrict__ x_scale_inv,
+                                                                        const float* __restrict__ y_scale_inv, int accumulate,
+                                                                        const void* __restrict__ bias, int bias_dt) {
+    gemm_dma128<XF, YF, OT, XT, YT, false>(X, Y, D, NR, NC, K, x_scale_inv, y_scale_inv, accumulate, bias, bias_dt);
+}
+// the same for a ragged last slice of K
+template <int XF, int YF, typename OT, bool XT = false, bool YT = false>
+__global__ __launch_bounds__(kGemmThreads) void fp8_gemm_ragged128_kernel(const uint8_t* __restrict__ X, const uint8_t* __restrict__ Y,
+                                                                           OT* __restrict__ D, int NR, int NC, int K,
+                                                                           const float* __restrict__ x_scale_inv,
+                                                                           const float* __restrict__ y_scale_inv, int accumulate,
+                                                                           const void* __restrict__ bias, int bias_dt) {
+    gemm_dma128<XF, YF, OT, XT, YT, true>(X, Y, D, NR, NC, K, x_scale_inv, y_scale_inv, accumulate, bias, bias_dt);
+}
+
+template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL>
+static int launch_gemm_dma128_tail(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs, const float* ys,
                               int accumulate, const void* bias, int bias_dt, hipStream_t st) {
     constexpr int smem = kSmallStages * kSmallStage;
     static std::atomic<bool> configured{false};    // setting the attribute twice is harmless
-    auto kern = fp8_gemm_dma128_kernel<XF, YF, OT, XT, YT>;
+    auto kern = KTAIL ? fp8_gemm_ragged128_kernel<XF, YF, OT, XT, YT> : fp8_gemm_dma128_kernel<XF, YF, OT, XT, YT>;
     if (!configured.load(std::memory_order_acquire)) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(fp8_gemm_dma128_kernel)");
@@ -291,6 +329,13 @@ static int launch_gemm_dma128(const uint8_t* X, const uint8_t* Y, void* D, int N
                        bias, bias_dt);
     MSAMP_CHECK_LAUNCH("fp8_gemm_dma128_kernel");
     return MSAMP_OK;
+}
+
+template <int XF, int YF, typename OT, bool XT = false, bool YT = false>
+static int launch_gemm_dma128(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs, const float* ys,
+                              int accumulate, const void* bias, int bias_dt, hipStream_t st) {
+    if (K % kBK) return launch_gemm_dma128_tail<XF, YF, OT, XT, YT, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
+    return launch_gemm_dma128_tail<XF, YF, OT, XT, YT, false>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
 }
 
 }    // namespace msamp

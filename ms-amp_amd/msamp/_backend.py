@@ -487,8 +487,7 @@ def gemm_kmajor_supported(m, n, k, a_kmajor, b_kmajor):
     """Shapes the kernel reads K-major operands for (see msamp_fp8_gemm_kmajor)."""
     if b_kmajor and not a_kmajor:
         return False
-    return k % 128 == 0 and k >= 256 and (not a_kmajor or m % 256 == 0) and (not b_kmajor or n % 256 == 0) and \
-        m * k < 2**32 and n * k < 2**32
+    return k > 128 and (m if a_kmajor else k) % 16 == 0 and (n if b_kmajor else k) % 16 == 0 and m * k < 2**32 and n * k < 2**32
 
 
 # ---- tile walks of the large GEMM, timed at first use ---------------------------------------------------------------
@@ -597,6 +596,8 @@ def fp8_gemm_cast(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, hp_dtype, q_dt, sc
         raise ValueError(f'shape mismatch: a {tuple(a.shape)}, b {tuple(b.shape)}')
     if hp_dtype not in _TORCH_TO_DT:
         raise TypeError(f'unsupported intermediate dtype {hp_dtype}')
+    if m % 256 or n % 256 or k % 128:
+        return None    # (as the library would answer, before anything is allocated for it)
     if accumulate and hp_out is None:
         raise ValueError('accumulate needs hp_out')
     if hp_out is not None and (hp_out.dtype != hp_dtype or tuple(hp_out.shape) != (n, m) or not hp_out.is_contiguous()):

@@ -156,6 +156,72 @@ def test_kmajor_operands_match_transposed_copies(be, a_dt, b_dt, m, n, k, out_dt
         assert same(got2, want2)
 
 
+@pytest.mark.parametrize('small_tiles', [True, False])
+@pytest.mark.parametrize('a_dt,b_dt', [(5, 5), (5, 6)])
+@pytest.mark.parametrize('m,n,k', [
+    (256, 256, 144),      # two slices, the second of 16 bytes
+    (272, 304, 272),      # three slices, one 16-byte chunk past two; tiles that end one chunk into the next
+    (16, 48, 400),        # four slices: the shortest the 128 x 128 tiles take; less than a tile each way
+    (512, 272, 624),      # five slices, 112 bytes in the last
+    (144, 528, 752),      # six slices
+    (304, 16, 1136),      # nine slices
+])
+@pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16])
+def test_ragged_k_and_rows_in_every_layout(be, small_tiles, a_dt, b_dt, m, n, k, out_dtype):
+    """K that ends inside a 128-byte slice, and K-major operands whose rows end inside a tile: the same bits as the same
+    operands padded with zeros to whole slices (row-major, whole slices: the form the other tests tie to the oracle), for
+    every layout and both tile sizes, with bias and accumulation.  Both operands hold a NaN code in one row: whatever lies
+    past the end of K in memory (the next row, which for one row is the NaN) must not reach any other output."""
+    a = _rand_fp8((m, k), a_dt, 7 * m + k).cuda()
+    b = _rand_fp8((n, k), b_dt, 5 * n + k, spread=0.5).cuda()
+    a[m // 2, :24] = 0x7F
+    b[n // 2, :24] = 0x7F
+    sa, sb = torch.tensor(0.25, device='cuda'), torch.tensor(2.0, device='cuda')
+    pad = -k % 128
+    a_pad, b_pad = torch.nn.functional.pad(a, (0, pad)), torch.nn.functional.pad(b, (0, pad))
+    a_t, b_t = a.t().contiguous(), b.t().contiguous()
+    bias = torch.randn(m, device='cuda').to(out_dtype)
+    base = torch.randn(n, m, device='cuda').to(out_dtype)
+    finite = torch.ones(n, m, dtype=torch.bool, device='cuda')
+    finite[n // 2], finite[:, m // 2] = False, False
+    if not small_tiles:
+        be.set_small_tile_limit(0)
+    try:
+        want = be.fp8_gemm(a_pad, a_dt, sa, b_pad, b_dt, sb, torch.empty(n, m, dtype=out_dtype, device='cuda'))
+        want2 = be.fp8_gemm(a_pad, a_dt, sa, b_pad, b_dt, sb, base.clone(), accumulate=True, bias=bias)
+        assert torch.equal(torch.isfinite(want), finite)
+        for layout in (dict(), dict(a_kmajor=True), dict(a_kmajor=True, b_kmajor=True)):
+            x, y = a_t if layout.get('a_kmajor') else a, b_t if layout.get('b_kmajor') else b
+            got = be.fp8_gemm(x, a_dt, sa, y, b_dt, sb, torch.empty(n, m, dtype=out_dtype, device='cuda'), **layout)
+            assert torch.equal(torch.isfinite(got), finite), layout
+            assert torch.equal(got[finite], want[finite]), layout
+            got2 = be.fp8_gemm(x, a_dt, sa, y, b_dt, sb, base.clone(), accumulate=True, bias=bias, **layout)
+            assert torch.equal(got2[finite], want2[finite]), layout
+    finally:
+        be.set_small_tile_limit(128)
+
+
+@pytest.mark.parametrize('k', [129, 191, 257, 383, 385, 511, 1030])
+def test_any_k_when_both_operands_are_kmajor(be, k):
+    """Both operands [K, rows]: K is a number of rows then and need not be a multiple of anything (the token count of a
+    weight gradient).  Same bits as with zero rows up to a whole slice."""
+    m, n = 272, 336
+    a_t, b_t = _rand_fp8((k, m), 5, k).cuda(), _rand_fp8((k, n), 6, k + 1).cuda()
+    one = torch.ones((), device='cuda')
+    pad = (0, 0, 0, -k % 128)
+    a_pad, b_pad = torch.nn.functional.pad(a_t, pad), torch.nn.functional.pad(b_t, pad)
+    for limit in (128, 0):
+        be.set_small_tile_limit(limit)
+        try:
+            want = be.fp8_gemm(a_pad.t().contiguous(), 5, one, b_pad.t().contiguous(), 6, one,
+                               torch.empty(n, m, dtype=torch.bfloat16, device='cuda'))
+            got = be.fp8_gemm(a_t, 5, one, b_t, 6, one, torch.empty(n, m, dtype=torch.bfloat16, device='cuda'), a_kmajor=True,
+                              b_kmajor=True)
+        finally:
+            be.set_small_tile_limit(128)
+        assert torch.equal(got, want)
+
+
 def test_kmajor_rejects_unsupported_shapes(be):
     a = _rand_fp8((128, 100), 5, 1).cuda()    # [K=128, M=100]: M is not a multiple of 256
     b = _rand_fp8((64, 128), 5, 2).cuda()
