@@ -104,6 +104,14 @@ int msamp_cast_to_fp8_intime(const void* x, int in_dtype, size_t n, float* scale
                              uint8_t* out, int fp8_type, int margin, int flags, void* workspace,
                              msamp_stream_t stream);
 
+/* msamp_cast_to_fp8_intime for a meta that does not exist yet (tensor.cast(qtype), msamp/common/tensor/tensor.py:668-690
+ * of the reference, which makes one from four fills first): the meta's words are written, not read -- scale = the scale
+ * rule of max|x| with a fallback of 1, its reciprocal, amax = max|x|, and *counter = 0 if given.  Same payload and meta
+ * as msamp_cast_to_fp8_intime leaves on a scale of 1 and an amax of 0. */
+int msamp_cast_to_fp8_fresh(const void* x, int in_dtype, size_t n, float* scale, float* amax, float* scale_inv,
+                            int32_t* counter, uint8_t* out, int fp8_type, int margin, int flags, void* workspace,
+                            msamp_stream_t stream);
+
 /* msamp_cast_to_fp8_intime without the workspace argument, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): it has no counterpart in
  * the reference.  The MSAMP_WORKSPACE_BYTES of scratch live in a static device array inside the library (each GPU

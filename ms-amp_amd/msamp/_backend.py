@@ -38,6 +38,7 @@ _SIGNATURES = {
     'msamp_compute_scaling_factor': ([_vp, _vp, _i, _vp, _i, _f, _i, _vp], _i),
     'msamp_cast_to_fp8': ([_vp, _i, _sz, _vp, _vp, _vp, _vp, _i, _vp], _i),
     'msamp_cast_to_fp8_intime': ([_vp, _i, _sz, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp], _i),
+    'msamp_cast_to_fp8_fresh': ([_vp, _i, _sz, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp], _i),
     'msamp_cast_to_fp8_intime_static': ([_vp, _i, _sz, _vp, _vp, _vp, _vp, _i, _i, _i, _vp], _i),
     'msamp_cast_scaled_to_fp8': ([_vp, _i, _sz, _vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _vp], _i),
     'msamp_add_to_fp8': ([_vp, _i, _sz, _vp, _vp, _vp, _vp, _i, _vp, _vp], _i),
@@ -341,6 +342,23 @@ def cast_to_fp8_intime(x, scale, amax_cell, scale_inv, fp8_dt, margin=0, nan_to_
             _ptr(workspace(x.device)),
             _stream()
         ), 'msamp_cast_to_fp8_intime'
+    )
+    return out
+
+
+def cast_to_fp8_fresh(x, scale, amax_cell, scale_inv, counter, fp8_dt, nan_to_inf=False, two_pass=False, speculate=True):
+    """cast_to_fp8_intime for a meta that does not exist yet: its words are written (the update count with 0), nothing is
+    read from them."""
+    lib = load()
+    _gpu(x, 'input')
+    out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
+    _check(
+        lib.msamp_cast_to_fp8_fresh(
+            _ptr(x), _dt(x), x.numel(), _ptr(scale), _ptr(amax_cell), _ptr(scale_inv), _ptr(counter), _ptr(out), fp8_dt, 0,
+            (FLAG_NAN_TO_INF if nan_to_inf else 0) | (FLAG_TWO_PASS if two_pass or _two_pass_only() else 0) |
+            (0 if speculate else FLAG_NO_SPECULATION),
+            _ptr(workspace(x.device)), _stream()
+        ), 'msamp_cast_to_fp8_fresh'
     )
     return out
 

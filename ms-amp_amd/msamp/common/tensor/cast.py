@@ -5,6 +5,9 @@ import torch.distributed as dist
 
 from msamp import _backend
 from msamp.common.dtype import Dtypes, Floating
+from msamp.common.tensor.meta import ScalingMeta
+
+_CAST_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 
 def _world_size():
@@ -21,6 +24,12 @@ class TypeCast:
             dist.all_reduce(meta.amax[0], op=dist.ReduceOp.MAX, group=meta.group)
             return meta.amax[0].clone()
         return None
+
+    @staticmethod
+    def takes_fresh_meta(input, sync):
+        """True if cast_to_fp8(input, ScalingMeta(qtype), sync) is one in-time cast on this GPU."""
+        return ScalingMeta.in_time_scaling and input.is_cuda and input.dtype in _CAST_DTYPES and input.numel() > 0 and \
+            not (sync and _world_size() > 1)
 
     @staticmethod
     def cast_to_fp8(input, meta, sync=False, fuse_transpose=False):

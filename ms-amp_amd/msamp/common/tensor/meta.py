@@ -31,8 +31,8 @@ class ScalingMeta:
 
     @classmethod
     def _uninitialized(cls, qtype, window_size, device, group=None):
-        """A meta whose four tensors are views of one uninitialised buffer, for callers whose kernel
-        writes every field (scale, scale_inv, counter, amax window) itself."""
+        """A meta whose four tensors are views of one uninitialised buffer {scale, scale_inv, counter, amax window}, for
+        callers whose kernel writes every field itself."""
         self = cls.__new__(cls)
         slab = torch.empty(3 + window_size, dtype=torch.float32, device=device)
         self.qtype = qtype
@@ -41,6 +41,20 @@ class ScalingMeta:
         self.amax = slab[3:]
         self.window_size = window_size
         self.group = group
+        self.locked = False
+        return self
+
+    @classmethod
+    def _unwritten(cls, qtype, device):
+        """A meta with a window of 1 whose tensors hold nothing yet, for a cast that writes them all.  (The float words
+        share one allocation, the counter has its own: torch.save refuses one storage seen as two types.)"""
+        self = cls.__new__(cls)
+        words = torch.empty(3, dtype=torch.float32, device=device)
+        self.qtype = qtype
+        self.scale, self.scale_inv, self.amax = words[0], words[1], words[2:]
+        self.amax_counter = torch.empty((), dtype=torch.int32, device=device)
+        self.window_size = 1
+        self.group = None
         self.locked = False
         return self
 

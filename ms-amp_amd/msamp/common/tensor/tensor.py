@@ -349,6 +349,12 @@ class TorchOverider:
         """tensor.cast(qtype, meta=None, sync=False) -> ScalingTensor (new window-1 meta by default)."""
         src = self.contiguous()
         if meta is None:
+            if Dtypes.is_fp8_qtype(qtype) and TypeCast.takes_fresh_meta(src, sync):
+                # the meta comes out of the cast's own kernel instead of four fills before it
+                meta = ScalingMeta._unwritten(qtype, src.device)
+                value = _backend.cast_to_fp8_fresh(src, meta.scale, meta.amax, meta.scale_inv, meta.amax_counter, int(qtype),
+                                                   nan_to_inf=sync)
+                return ScalingTensor(value, meta=meta)
             meta = ScalingMeta(qtype, device=src.device)
         if Dtypes.is_fp8_qtype(qtype):
             return ScalingTensor(TypeCast.cast_to_fp8(src, meta, sync=sync), meta=meta)

@@ -516,3 +516,57 @@ def test_speculative_in_time_cast_beyond_the_one_pass_limit(be, dtype, n):
         assert am[0].item() == src.float().abs().max().item()
         want = fp8.encode(src[:head].float().cpu() * s.cpu(), fp8.E4M3)
         assert torch.equal(q[:head].cpu(), want)
+
+
+def _fresh(be, x, fp8_dt, **kw):
+    words = torch.full((3, ), float('nan'), device='cuda')    # what the call must not read
+    count = torch.full((), -7, dtype=torch.int32, device='cuda')
+    q = be.cast_to_fp8_fresh(x, words[0], words[2:], words[1], count, fp8_dt, **kw)
+    return q, words[0], words[1], count, words[2:]
+
+
+@pytest.mark.parametrize('two_pass', [False, True])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('n', [1, 5, 4096, 8192 * 5 + 3, 1 << 20])
+def test_fresh_meta_cast_equals_the_cast_on_a_new_meta(be, dtype, n, two_pass):
+    """The cast that writes its meta itself against the in-time cast on {1, 1, 0}: payload, scale, scale_inv and amax bit for
+    bit, the update count zero; ordinary values, all zeros, NaN and Inf."""
+    g = torch.Generator(device='cuda').manual_seed(n)
+    x0 = torch.randn(n, device='cuda', generator=g).to(dtype)
+    for fp8_dt in (5, 6):
+        for special in (None, 0.0, float('nan'), float('inf')):
+            x = x0.clone()
+            if special == 0.0:
+                x.zero_()
+            elif special is not None:
+                x[n // 2] = special
+            s, si, am = make_meta()
+            want = be.cast_to_fp8_intime(x, s, am[0:1], si, fp8_dt, nan_to_inf=True, two_pass=True, speculate=False)
+            got, fs, fsi, count, fam = _fresh(be, x, fp8_dt, nan_to_inf=True, two_pass=two_pass)
+            assert torch.equal(got, want) and same_float(fs, s) and same_float(fsi, si) and same_float(fam, am)
+            assert count.item() == 0
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('what', ['sample tells', 'sample misses the maximum', 'sample misses everything', 'nan', 'inf'])
+def test_fresh_meta_cast_guesses_from_a_sample(be, dtype, what):
+    """Beyond the one-pass limit the scale is guessed from a sample of 512 pieces of 16 KiB, spread evenly; whatever the
+    sample says, the result is the one of the two plain passes."""
+    esz = torch.finfo(dtype).bits // 8
+    n = (96 << 20) // esz + 1021
+    piece = 16384 // esz
+    x = torch.full((n, ), 0.5, device='cuda').to(dtype)
+    pieces = n // piece
+    taken = {pieces * b // 512 for b in range(512)}
+    free = next(p for p in range(pieces) if p not in taken) * piece
+    if what == 'sample misses the maximum':
+        x[free + 3] = 300.0
+    elif what == 'sample misses everything':
+        x.zero_()
+        x[free + 3] = 2.0
+    elif what != 'sample tells':
+        x[free + 3] = float(what)
+    s, si, am = make_meta()
+    want = be.cast_to_fp8_intime(x, s, am[0:1], si, 5, two_pass=True, speculate=False)
+    got, fs, fsi, count, fam = _fresh(be, x, 5)
+    assert torch.equal(got, want) and same_float(fs, s) and same_float(fsi, si) and same_float(fam, am) and count.item() == 0
