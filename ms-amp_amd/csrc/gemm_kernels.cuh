@@ -489,6 +489,17 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     const int wr = wave >> 1, wc = wave & 1;
     // the output factor is fetched now: left to the epilogue, the two scalar loads sit on its critical path
     float alpha_early = (*x_scale_inv) * (*y_scale_inv);
+    // and so are the bias values of two of this wave's 128 columns per lane (-0 without a bias: fma(x, y, -0) is x * y to
+    // the bit, signed zeros included)
+    float bias_early[2] = {-0.0f, -0.0f};
+    if constexpr (QF == 0 && !QSPEC) {
+        if (bias != nullptr) {
+            const int c = col0 + wc * 128 + lane * 2;
+            bias_early[0] = c < NC ? load_bias(bias, bias_dt, c) : 0.0f;
+            bias_early[1] = c + 1 < NC ? load_bias(bias, bias_dt, c + 1) : 0.0f;
+        }
+        asm volatile("" : "+v"(bias_early[0]), "+v"(bias_early[1]));
+    }
     asm volatile("" : "+v"(alpha_early));
     // QSPEC: the scale the codes are written with, as the meta holds it now (the last workgroup rewrites the meta)
     float guess = 1.0f;
@@ -879,7 +890,6 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     uint8_t* patch = smem + wave * (32 * kPitch);
     const float alpha = alpha_early;
     const bool vec_ok = (NC % (16 / kEsz) == 0) && ((reinterpret_cast<uintptr_t>(D) & 15) == 0);
-    const bool plain = !accumulate && bias == nullptr;    // (rows that 16-byte stores do not fit go out element by element)
     const bool pairs_ok = (NC % 2 == 0) && ((reinterpret_cast<uintptr_t>(D) & 3) == 0);
     constexpr int kChunksPerRow = 128 * kEsz / 16;      // 16 (2-byte) or 32 (float)
     constexpr int kRowsPerPass = 64 / kChunksPerRow;    // 4 or 2
@@ -899,7 +909,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
         }
     };
     auto emit_fused_rows = [&]() __attribute__((always_inline)) {
-        // ---- bias and / or accumulation with 16-byte row accesses: the raw float32 accumulators of a 32-row unit go
+        // ---- accumulation (and bias) with 16-byte row accesses: the raw float32 accumulators of a 32-row unit go
         // through a per-wave float32 patch, each lane picks up one 16-byte segment of an output row, reads the old
         // output there if it is to be added, and stores fma(acc, alpha, bias) (+ old) rounded once -- the expression of
         // the element-wise path below and of the generic kernel.  A lane's columns are the same in every pass, so
@@ -998,11 +1008,11 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
             });
         });
     };
-    if (!QSPEC && !plain && vec_ok) {
+    if (!QSPEC && accumulate && vec_ok) {
         emit_fused_rows();
         return;
     }
-    if (!QSPEC && !plain) {
+    if (!QSPEC && accumulate) {
         static_for<8>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
             static_for<8>([&](auto jc) {
@@ -1018,12 +1028,29 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // whole tile with 16-byte row stores (no bounds checks; the address is a scalar row base plus one per-lane offset),
     // 16-byte row stores with bounds checks (tiles on the right or bottom edge), and rows that 16-byte stores do not fit.
     // (With the choice made per store, every store dragged three variants and their branches along.)
+    // A bias is added here as well, as fma(acc, alpha, bias): a lane's accumulators lie in 32 columns, whose values it
+    // takes from the wave's patch, where the lanes put the two each of them fetched at the start.  (Through the float32
+    // patch of the accumulating form, with the bias fetched after the K loop, a tile took about 8 us longer: 8192 x 8192
+    // x 2048 with a bias 142 us, now 114; 12605 x 4304 x 1200 into float16 116 us, now 93.)
     auto emit_plain = [&](auto vec_c, auto inside_c) __attribute__((always_inline)) {
         constexpr bool kVec = decltype(vec_c)::value, kInside = decltype(inside_c)::value;
         const int pc = lane % kChunksPerRow, prl = lane / kChunksPerRow;
         const int gcol = col0 + wc * 128 + pc * kElemsPerChunk;
         // whole tile: byte offset of this lane's segment from the first element of its pass's first row
         const uint32_t lane_off = (static_cast<uint32_t>(prl) * static_cast<uint32_t>(NC) + static_cast<uint32_t>(pc * kElemsPerChunk)) * kEsz;
+        float bq[32];
+        if constexpr (!QSPEC) {
+            *reinterpret_cast<uint2*>(patch + lane * 8) = make_uint2(__float_as_uint(bias_early[0]), __float_as_uint(bias_early[1]));
+            asm volatile("" : : : "memory");
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint4 b = *reinterpret_cast<const uint4*>(patch + (j * 16 + g4 * 4) * 4);
+                bq[4 * j] = __uint_as_float(b.x), bq[4 * j + 1] = __uint_as_float(b.y);
+                bq[4 * j + 2] = __uint_as_float(b.z), bq[4 * j + 3] = __uint_as_float(b.w);
+            }
+            asm volatile("" : : : "memory");
+        }
+        auto scaled = [&](float x, int c) __attribute__((always_inline)) { return QSPEC ? x * alpha : fmaf(x, alpha, bq[c]); };
         static_for<4>([&](auto uc) {
             constexpr int u = decltype(uc)::value;
             static_for<2>([&](auto hc) {
@@ -1034,7 +1061,8 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                     // 8-byte writes of 16 rows at a time: rows r and r + 8 are 8 * (pitch mod 128 bytes) = 128 bytes apart in
                     // bank terms, the same 8-byte slot; the upper eight rows swap each pair of slots (undone when read back)
                     uint8_t* dst = patch + (h * 16 + l16) * kPitch + (((j * 16 + g4 * 4) * kEsz) ^ (kEsz == 2 ? ((l16 >> 3) & 1) << 3 : 0));
-                    const float v0 = a[0] * alpha, v1 = a[1] * alpha, v2 = a[2] * alpha, v3 = a[3] * alpha;
+                    const float v0 = scaled(a[0], 4 * j), v1 = scaled(a[1], 4 * j + 1), v2 = scaled(a[2], 4 * j + 2),
+                                v3 = scaled(a[3], 4 * j + 3);
                     float r0 = v0, r1 = v1, r2 = v2, r3 = v3;    // QSPEC: the outputs as OT holds them
                     if constexpr (kEsz == 4) {
                         *reinterpret_cast<float4*>(dst) = make_float4(v0, v1, v2, v3);

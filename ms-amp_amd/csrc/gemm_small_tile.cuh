@@ -41,7 +41,22 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     const int row0 = tr * kSmallTile, col0 = tc * kSmallTile;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = wave >> 1, wc = wave & 1;
+    // the output factor and this lane's bias values are fetched now: in the epilogue they would sit on its critical path
+    constexpr int kEsz = static_cast<int>(sizeof(OT));
+    constexpr int kElems = 16 / kEsz;              // outputs per 16-byte segment: 8 or 4
+    constexpr int kSegs = 64 / kElems;             // segments per 64-column row: 8 or 16
+    const int seg = lane % kSegs;
+    const int gcol = col0 + wc * 64 + seg * kElems;
     float alpha = (*x_scale_inv) * (*y_scale_inv);
+    float bv[kElems];
+#pragma unroll
+    for (int e = 0; e < kElems; ++e) bv[e] = 0.0f;
+    if (bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < kElems; ++e) bv[e] = gcol + e < NC ? load_bias(bias, bias_dt, gcol + e) : 0.0f;
+#pragma unroll
+        for (int e = 0; e < kElems; ++e) asm volatile("" : "+v"(bv[e]));
+    }
     asm volatile("" : "+v"(alpha));
 
     // ---- global -> LDS: one wave instruction fills 8 rows of 128 bytes (lane l: row l / 8, 16-byte position l % 8,
@@ -214,19 +229,12 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
 
     // ---- epilogue: the raw accumulators of a 16-row block go through a per-wave float32 patch; each lane then picks up
     // one 16-byte segment of an output row and applies the factor (bias, old output) with one rounding
-    constexpr int kEsz = static_cast<int>(sizeof(OT));
-    constexpr int kElems = 16 / kEsz;              // outputs per 16-byte segment: 8 or 4
-    constexpr int kSegs = 64 / kElems;             // segments per 64-column row: 8 or 16
     constexpr int kRowsPerPass = 64 / kSegs;       // 8 or 4
     constexpr int kFPitch = 64 * 4 + 16;           // bytes per patch row
     uint8_t* patch = smem + wave * (16 * kFPitch);
     const bool vec_ok = (NC % kElems == 0) && ((reinterpret_cast<uintptr_t>(D) & 15) == 0);
     const bool plain = !accumulate && bias == nullptr;
-    const int seg = lane % kSegs, prl = lane / kSegs;
-    const int gcol = col0 + wc * 64 + seg * kElems;
-    float bv[kElems];
-#pragma unroll
-    for (int e = 0; e < kElems; ++e) bv[e] = (bias != nullptr && gcol + e < NC) ? load_bias(bias, bias_dt, gcol + e) : 0.0f;
+    const int prl = lane / kSegs;
     static_for<4>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         static_for<4>([&](auto jc) {
