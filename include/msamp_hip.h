@@ -255,6 +255,24 @@ typedef struct msamp_norm_item {
 int msamp_fp8_norms(msamp_norm_item* items, int n_items, const int32_t* block_map, int n_blocks, int fp8_type,
                     int norm_kind, msamp_stream_t stream);
 
+/* The total norm of a list of gradients of any types and the factor that clips them to max_norm (nn/clip_grad.py:29-88),
+ * without the host waiting for either.  `grads`: HOST array, read during the call; contiguous tensors of F32 / F16 / BF16
+ * (scale_inv null), or E4M3 / E5M2 codes with their scale_inv.  norms[i] = norm of tensor i, *total = norm of the norms,
+ * *coef = min(1, max_norm / (total + 1e-6)) (NaN stays NaN); sums in double, each result rounded to float once.  norm_kind
+ * as above.  `partials`: scratch for n + MSAMP_GRAD_BLOCKS doubles. */
+#define MSAMP_GRAD_BLOCKS 2048
+typedef struct msamp_grad {
+    const void* data;
+    const float* scale_inv;
+    uint64_t numel;
+    int64_t dtype;
+} msamp_grad;
+int msamp_grad_norms(const msamp_grad* grads, int n, int norm_kind, float max_norm, double* partials, float* norms, float* total,
+                     float* coef, msamp_stream_t stream);
+/* Multiplies every tensor of the list by *coef (device) if that is below 1: an FP8 tensor through its scale_inv, a
+ * 16-bit one with the factor rounded to its type.  No tensor may appear twice. */
+int msamp_grad_clip(const msamp_grad* grads, int n, const float* coef, msamp_stream_t stream);
+
 /* tex.te_gemm as Gemm.fp8_gemm calls it (gemm.py:121-144; transa=True, transb=False):
  * D[N][M] = (B[N][K] . A[M][K]^T) * *a_scale_inv * *b_scale_inv (+ bias[M]) (+ D if accumulate).
  * A, B: FP8 bytes, row-major, K contiguous, K % 16 == 0, 16-byte aligned.  d_dtype: F32/F16/BF16.

@@ -143,6 +143,49 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_cast_kernel(const msamp
 // summed in float32 first): the dequantization factor
 // is constant per tensor and is applied once at the end, so a tensor is read at one byte per element and never
 // expanded to float32 in memory.
+// (one chunk, into `acc`)
+template <int FMT, int KIND>    // KIND: 1, 2, or 0 for the maximum
+__device__ __forceinline__ void fp8_norm_chunk(const uint8_t* q, size_t base, size_t n, double& acc) {
+    auto take = [&](float v) {
+        const double a = fabs(static_cast<double>(v));
+        if constexpr (KIND == 0) {
+            acc = (a != a || acc != acc) ? (a != a ? a : acc) : (a > acc ? a : acc);    // NaN wins
+        } else if constexpr (KIND == 1) {
+            acc += a;
+        } else {
+            acc = fma(a, a, acc);
+        }
+    };
+    if (base + MSAMP_BUCKET_CHUNK <= n && (reinterpret_cast<uintptr_t>(q) & 15) == 0) {
+        constexpr int kVecs = MSAMP_BUCKET_CHUNK / (kBucketThreads * 16);    // 4
+        uint4 w[kVecs];
+#pragma unroll
+        for (int u = 0; u < kVecs; ++u)
+            w[u] = *reinterpret_cast<const uint4*>(q + base + (static_cast<size_t>(u) * kBucketThreads + threadIdx.x) * 16);
+#pragma unroll
+        for (int u = 0; u < kVecs; ++u) {
+            const uint32_t words[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float a, b, c, f;
+                dequant4<FMT>(words[j], a, b, c, f);
+                if constexpr (KIND == 0) {
+                    take(a), take(b), take(c), take(f);
+                } else if constexpr (KIND == 1) {
+                    // four values at a time in float32 (three roundings of 2^-24 each), then into the double sum: a
+                    // double conversion and addition per element kept the vector units busier than the memory
+                    acc += static_cast<double>((fabsf(a) + fabsf(b)) + (fabsf(c) + fabsf(f)));
+                } else {
+                    // the square of an FP8 value is exact in float32
+                    acc += static_cast<double>(fmaf(a, a, b * b) + fmaf(c, c, f * f));
+                }
+            }
+        }
+    } else {
+        for (size_t i = base + threadIdx.x; i < n && i < base + MSAMP_BUCKET_CHUNK; i += kBucketThreads) take(dequant1<FMT>(q[i]));
+    }
+}
+
 // A workgroup takes a run of `run` consecutive chunks of the block map and adds to a tensor's accumulator once per tensor
 // it meets: additions to one address are served one at a time (about 12 ns each), and with one per chunk the 1 024
 // chunks of a 16.8 M-element tensor queued for longer (12 us) than their 16 MB take to read.
@@ -151,16 +194,6 @@ __global__ __launch_bounds__(kBucketThreads) void fp8_norm_kernel(msamp_norm_ite
                                                                    const int32_t* __restrict__ block_map, int n_blocks, int run) {
     __shared__ double red[kBucketThreads / kWave];
     double acc = 0.0;
-    auto take = [&](float v) {
-        const double a = fabs(static_cast<double>(v));
-        if constexpr (KIND == 0) {
-            acc = (a != a || acc != acc) ? (a != a ? a : acc) : (a > acc ? a : acc);    // NaN stays
-        } else if constexpr (KIND == 1) {
-            acc += a;
-        } else {
-            acc = fma(a, a, acc);
-        }
-    };
     // the workgroup's total (maximum) -- lanes, then wavefronts -- into tensor t's accumulator
     auto flush = [&](int t) {
 #pragma unroll
@@ -204,34 +237,7 @@ __global__ __launch_bounds__(kBucketThreads) void fp8_norm_kernel(msamp_norm_ite
         }
         const uint8_t* q = items[t].q;
         const size_t n = items[t].numel, base = static_cast<size_t>(chunk) * MSAMP_BUCKET_CHUNK;
-        if (base + MSAMP_BUCKET_CHUNK <= n && (reinterpret_cast<uintptr_t>(q) & 15) == 0) {
-            constexpr int kVecs = MSAMP_BUCKET_CHUNK / (kBucketThreads * 16);    // 4
-            uint4 w[kVecs];
-#pragma unroll
-            for (int u = 0; u < kVecs; ++u)
-                w[u] = *reinterpret_cast<const uint4*>(q + base + (static_cast<size_t>(u) * kBucketThreads + threadIdx.x) * 16);
-#pragma unroll
-            for (int u = 0; u < kVecs; ++u) {
-                const uint32_t words[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float a, b, c, f;
-                    dequant4<FMT>(words[j], a, b, c, f);
-                    if constexpr (KIND == 0) {
-                        take(a), take(b), take(c), take(f);
-                    } else if constexpr (KIND == 1) {
-                        // four values at a time in float32 (three roundings of 2^-24 each), then into the double sum: a
-                        // double conversion and addition per element kept the vector units busier than the memory
-                        acc += static_cast<double>((fabsf(a) + fabsf(b)) + (fabsf(c) + fabsf(f)));
-                    } else {
-                        // the square of an FP8 value is exact in float32
-                        acc += static_cast<double>(fmaf(a, a, b * b) + fmaf(c, c, f * f));
-                    }
-                }
-            }
-        } else {
-            for (size_t i = base + threadIdx.x; i < n && i < base + MSAMP_BUCKET_CHUNK; i += kBucketThreads) take(dequant1<FMT>(q[i]));
-        }
+        fp8_norm_chunk<FMT, KIND>(q, base, n, acc);
     }
     flush(current);
 }
@@ -245,6 +251,216 @@ __global__ void fp8_norm_finish_kernel(msamp_norm_item* items, int n_items, int 
     d.acc = 0.0;
     const double root = kind == 2 ? sqrt(acc) : acc;
     *d.out = static_cast<float>(fabs(static_cast<double>(*d.scale_inv)) * root);
+}
+
+// ---- clipping a list of gradients (clip_grad_norm_) ----------------------------------------------------------------
+// The norms of all gradients of a model, whatever their types (FP8 codes with a scale_inv, or plain float32 / 16-bit
+// tensors), their total and the clipping factor in two launches per 64 tensors, and the clipping itself in one, which
+// looks at the factor on the device.  Per tensor this was a conversion to float32 with torch.norm or a multiplication
+// (two to four launches of 1.3 to 4 us and 6 to 9 us of host time each), and the host waited for the factor.
+// The descriptors travel as kernel arguments: no table in memory, no copy, nothing kept between calls.
+// 32 FP8 gradients of 4 M codes, quantized as a bucket and clipped: 365 us in all with the calls per tensor, of which the
+// GPU worked 150; 117 us now (norms 24 us, finish 5, clipping 4).  A small model's 13 parameters: 0.2 ms a step less.
+constexpr int kGradTable = 64;         // 64 descriptors are 1.9 KB of the 4 KB that kernel arguments may take
+constexpr int kGradBlocks = MSAMP_GRAD_BLOCKS;    // eight workgroups per compute unit; beyond that each takes a run of chunks
+struct GradTable {
+    const void* data[kGradTable];
+    const float* scale_inv[kGradTable];    // nullptr: a plain tensor
+    uint64_t numel[kGradTable];
+    int32_t first[kGradTable + 1];         // tensor t has the workgroups first[t] .. first[t + 1] - 1
+    uint8_t dtype[kGradTable];
+    int32_t n;
+};
+
+__device__ __forceinline__ int tensor_of_block(const GradTable& g, int block) {
+    int lo = 0, hi = g.n;    // first[lo] <= block < first[hi]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (g.first[mid] <= block) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+template <int KIND>
+__device__ __forceinline__ double norm_join(double a, double b) {
+    if constexpr (KIND == 0) return a != a ? a : (b != b || b > a ? b : a);    // (NaN wins)
+    else return a + b;
+}
+
+// elements base .. base + MSAMP_BUCKET_CHUNK - 1 of a plain tensor, in double: no square or sum is rounded to float32
+template <typename IT, int KIND>
+__device__ __forceinline__ void norm_chunk(const IT* x, size_t base, size_t n, double& acc) {
+    constexpr int EPT = In16<IT>::EPT;
+    auto take = [&](float v) {
+        const double a = fabs(static_cast<double>(v));
+        if constexpr (KIND == 2) acc = fma(a, a, acc);
+        else acc = norm_join<KIND>(acc, a);
+    };
+    if (base + MSAMP_BUCKET_CHUNK <= n && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+        constexpr int kVecs = MSAMP_BUCKET_CHUNK / (kBucketThreads * EPT);    // 16 (float32) or 8
+#pragma unroll 2
+        for (int v = 0; v < kVecs; v += 4) {
+            uint4 w[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                w[u] = *reinterpret_cast<const uint4*>(x + base + (static_cast<size_t>(v + u) * kBucketThreads + threadIdx.x) * EPT);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                float f[EPT];
+                In16<IT>::decode(w[u], f);
+#pragma unroll
+                for (int e = 0; e < EPT; ++e) take(f[e]);
+            }
+        }
+    } else {
+        for (size_t i = base + threadIdx.x; i < n && i < base + MSAMP_BUCKET_CHUNK; i += kBucketThreads) take(Elem<IT>::load(x + i));
+    }
+}
+
+// partial[block]: sum of |x|^p (maximum for KIND 0) over the workgroup's run of chunks of its tensor
+template <int KIND>
+__global__ __launch_bounds__(kBucketThreads) void grad_norm_kernel(GradTable g, double* __restrict__ partial) {
+    __shared__ double red[kBucketThreads / kWave];
+    const int t = tensor_of_block(g, blockIdx.x);
+    const size_t n = g.numel[t], chunks = (n + MSAMP_BUCKET_CHUNK - 1) / MSAMP_BUCKET_CHUNK;
+    const size_t blocks = g.first[t + 1] - g.first[t], run = (chunks + blocks - 1) / blocks;
+    const size_t from = (blockIdx.x - g.first[t]) * run, to = from + run < chunks ? from + run : chunks;
+    const void* x = g.data[t];
+    const int dt = g.dtype[t];
+    double acc = 0.0;
+    for (size_t c = from; c < to; ++c) {
+        const size_t base = c * MSAMP_BUCKET_CHUNK;
+        if (dt == MSAMP_DT_E4M3) fp8_norm_chunk<MSAMP_DT_E4M3, KIND>(static_cast<const uint8_t*>(x), base, n, acc);
+        else if (dt == MSAMP_DT_E5M2) fp8_norm_chunk<MSAMP_DT_E5M2, KIND>(static_cast<const uint8_t*>(x), base, n, acc);
+        else if (dt == MSAMP_DT_F32) norm_chunk<float, KIND>(static_cast<const float*>(x), base, n, acc);
+        else if (dt == MSAMP_DT_F16) norm_chunk<f16_t, KIND>(static_cast<const f16_t*>(x), base, n, acc);
+        else norm_chunk<bf16_t, KIND>(static_cast<const bf16_t*>(x), base, n, acc);
+    }
+#pragma unroll
+    for (int o = 32; o; o >>= 1) acc = norm_join<KIND>(acc, __shfl_xor(acc, o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBucketThreads / kWave; ++w) acc = norm_join<KIND>(acc, red[w]);
+        partial[blockIdx.x] = acc;
+    }
+}
+
+// One workgroup: norms[base + t] of the table's tensors, a wavefront each; with `total` also the norm of all norms[0 ..
+// base + g.n - 1] and min(1, max_norm / (total + 1e-6)), evaluated as torch does (a reciprocal and a product).
+constexpr int kNormFinishThreads = 1024;
+template <int KIND>
+__global__ __launch_bounds__(kNormFinishThreads) void grad_norm_finish_kernel(GradTable g, const double* __restrict__ partial,
+                                                                              float* norms, int base, float* total, float* coef,
+                                                                              float max_norm) {
+    __shared__ double red[kNormFinishThreads / kWave];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int t = wave; t < g.n; t += kNormFinishThreads / kWave) {
+        double acc = 0.0;
+        for (int b = g.first[t] + lane; b < g.first[t + 1]; b += 64) acc = norm_join<KIND>(acc, partial[b]);
+#pragma unroll
+        for (int o = 32; o; o >>= 1) acc = norm_join<KIND>(acc, __shfl_xor(acc, o));
+        if (lane == 0) {
+            const double root = KIND == 2 ? sqrt(acc) : acc;
+            const double si = g.scale_inv[t] != nullptr ? fabs(static_cast<double>(*g.scale_inv[t])) : 1.0;
+            norms[base + t] = static_cast<float>(si * root);
+        }
+    }
+    if (total == nullptr) return;
+    __syncthreads();
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < base + g.n; i += kNormFinishThreads) {
+        const double v = norms[i];
+        acc = KIND == 2 ? fma(v, v, acc) : norm_join<KIND>(acc, v);
+    }
+#pragma unroll
+    for (int o = 32; o; o >>= 1) acc = norm_join<KIND>(acc, __shfl_xor(acc, o));
+    if (lane == 0) red[wave] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kNormFinishThreads / kWave; ++w) acc = norm_join<KIND>(acc, red[w]);
+        const float norm = static_cast<float>(KIND == 2 ? sqrt(acc) : acc);
+        const float recip = 1.0f / (norm + 1e-6f);
+        const float c = recip * max_norm;
+        *total = norm;
+        *coef = c > 1.0f ? 1.0f : c;    // (NaN stays)
+    }
+}
+
+template <typename IT>
+__device__ __forceinline__ void scale_run(IT* x, size_t from, size_t to, float factor) {
+    constexpr int EPT = In16<IT>::EPT;
+    size_t i = from + static_cast<size_t>(threadIdx.x) * EPT;
+    if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {    // (`from` is a multiple of the chunk)
+        for (; i + EPT <= to; i += kBucketThreads * EPT) {
+            float f[EPT];
+            In16<IT>::load(x + i, f);
+            IT o[EPT];
+#pragma unroll
+            for (int e = 0; e < EPT; ++e) Elem<IT>::store(o + e, f[e] * factor);
+            uint4 w;
+            __builtin_memcpy(&w, o, 16);
+            *reinterpret_cast<uint4*>(x + i) = w;
+        }
+        if (i < to)
+            for (size_t j = i; j < to; ++j) Elem<IT>::store(x + j, Elem<IT>::load(x + j) * factor);
+    } else {
+        for (size_t j = from + threadIdx.x; j < to; j += kBucketThreads) Elem<IT>::store(x + j, Elem<IT>::load(x + j) * factor);
+    }
+}
+
+// x *= coef where coef < 1; of an FP8 tensor only its scale_inv.  A 16-bit tensor takes the factor in its own type, as
+// torch's product with a zero-dimensional float32 tensor does.
+__global__ __launch_bounds__(kBucketThreads) void grad_clip_kernel(GradTable g, const float* __restrict__ coef) {
+    const float c = *coef;
+    if (!(c < 1.0f)) return;
+    const int t = tensor_of_block(g, blockIdx.x);
+    if (g.scale_inv[t] != nullptr) {
+        if (threadIdx.x == 0) {
+            float* si = const_cast<float*>(g.scale_inv[t]);
+            *si *= c;
+        }
+        return;
+    }
+    const size_t n = g.numel[t], chunks = (n + MSAMP_BUCKET_CHUNK - 1) / MSAMP_BUCKET_CHUNK;
+    const size_t blocks = g.first[t + 1] - g.first[t], run = (chunks + blocks - 1) / blocks * MSAMP_BUCKET_CHUNK;
+    const size_t from = (blockIdx.x - g.first[t]) * run, to = from + run < n ? from + run : n;
+    void* x = const_cast<void*>(g.data[t]);
+    const int dt = g.dtype[t];
+    if (dt == MSAMP_DT_F32) scale_run(static_cast<float*>(x), from, to, c);
+    else if (dt == MSAMP_DT_F16) scale_run(static_cast<f16_t*>(x), from, to, f16_bits_to_float(float_to_f16_bits(c)));
+    else scale_run(static_cast<bf16_t*>(x), from, to, bf16_bits_to_float(float_to_bf16_bits(c)));
+}
+
+static int check_grads(const char* who, const msamp_grad* grads, int n) {
+    MSAMP_REQUIRE(n >= 0, MSAMP_ERR_SHAPE, "%s: n=%d", who, n);
+    MSAMP_REQUIRE(n == 0 || grads != nullptr, MSAMP_ERR_NULL, "%s: null table", who);
+    for (int i = 0; i < n; ++i) {
+        MSAMP_REQUIRE(is_hp(grads[i].dtype) || is_fp8(grads[i].dtype), MSAMP_ERR_DTYPE, "%s: tensor %d: dtype %d", who, i, grads[i].dtype);
+        MSAMP_REQUIRE(grads[i].data != nullptr || grads[i].numel == 0, MSAMP_ERR_NULL, "%s: tensor %d: null data", who, i);
+        MSAMP_REQUIRE((grads[i].scale_inv != nullptr) == is_fp8(grads[i].dtype), MSAMP_ERR_NULL,
+                      "%s: tensor %d: FP8 codes come with a scale_inv, plain tensors without", who, i);
+        MSAMP_REQUIRE(aligned(grads[i].data, is_fp8(grads[i].dtype) ? 1 : hp_size(grads[i].dtype)), MSAMP_ERR_SHAPE, "%s: tensor %d: misaligned", who, i);
+    }
+    return MSAMP_OK;
+}
+// tensors from .. from + (at most) kGradTable - 1; `run`: chunks per workgroup; scales_only: one workgroup per FP8 tensor
+static GradTable grad_table(const msamp_grad* grads, int from, int n, size_t run, bool scales_only) {
+    GradTable g = {};
+    g.n = std::min(kGradTable, n - from);
+    for (int i = 0; i < g.n; ++i) {
+        const msamp_grad& e = grads[from + i];
+        const size_t chunks = (e.numel + MSAMP_BUCKET_CHUNK - 1) / MSAMP_BUCKET_CHUNK;
+        const size_t blocks = scales_only && e.scale_inv != nullptr ? 1 : std::max<size_t>(1, (chunks + run - 1) / run);
+        g.data[i] = e.data, g.scale_inv[i] = e.scale_inv, g.numel[i] = e.numel, g.dtype[i] = static_cast<uint8_t>(e.dtype);
+        g.first[i + 1] = g.first[i] + static_cast<int32_t>(blocks);
+    }
+    return g;
+}
+static size_t grad_run(const msamp_grad* grads, int n) {
+    size_t chunks = 0;
+    for (int i = 0; i < n; ++i) chunks += (grads[i].numel + MSAMP_BUCKET_CHUNK - 1) / MSAMP_BUCKET_CHUNK;
+    return std::max<size_t>(1, (chunks + kGradBlocks - 1) / kGradBlocks);
 }
 
 static int check_bucket_args(const char* who, const msamp_bucket_item* items, int n_items, const int32_t* block_map,
@@ -360,6 +576,45 @@ int msamp_fp8_norms(msamp_norm_item* items, int n_items, const int32_t* block_ma
     }
     hipLaunchKernelGGL(fp8_norm_finish_kernel, dim3((n_items + 63) / 64), dim3(64), 0, st, items, n_items, norm_kind);
     MSAMP_CHECK_LAUNCH("fp8_norm_finish_kernel");
+    return MSAMP_OK;
+}
+
+int msamp_grad_norms(const msamp_grad* grads, int n, int norm_kind, float max_norm, double* partials, float* norms, float* total,
+                     float* coef, msamp_stream_t stream) {
+    const int rc = check_grads("msamp_grad_norms", grads, n);
+    if (rc != MSAMP_OK) return rc;
+    MSAMP_REQUIRE(norm_kind >= 0 && norm_kind <= 2, MSAMP_ERR_SHAPE, "msamp_grad_norms: norm_kind %d (1, 2, or 0 for the maximum)",
+                  norm_kind);
+    MSAMP_REQUIRE(n > 0 && partials && norms && total && coef, MSAMP_ERR_NULL, "msamp_grad_norms: nothing to do or null pointer");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const size_t run = grad_run(grads, n);
+    for (int from = 0; from < n; from += kGradTable) {
+        const GradTable g = grad_table(grads, from, n, run, false);
+        const bool last = from + g.n == n;
+        float* total_out = last ? total : nullptr;
+#define NORM_LAUNCH(KIND)                                                                                                 \
+    do {                                                                                                                \
+        hipLaunchKernelGGL((grad_norm_kernel<KIND>), dim3(g.first[g.n]), dim3(kBucketThreads), 0, st, g, partials);        \
+        MSAMP_CHECK_LAUNCH("grad_norm_kernel");                                                                         \
+        hipLaunchKernelGGL((grad_norm_finish_kernel<KIND>), dim3(1), dim3(kNormFinishThreads), 0, st, g, partials, norms, from, total_out, coef, max_norm); \
+        MSAMP_CHECK_LAUNCH("grad_norm_finish_kernel");                                                                  \
+    } while (0)
+        if (norm_kind == 0) NORM_LAUNCH(0); else if (norm_kind == 1) NORM_LAUNCH(1); else NORM_LAUNCH(2);
+#undef NORM_LAUNCH
+    }
+    return MSAMP_OK;
+}
+
+int msamp_grad_clip(const msamp_grad* grads, int n, const float* coef, msamp_stream_t stream) {
+    const int rc = check_grads("msamp_grad_clip", grads, n);
+    if (rc != MSAMP_OK || n == 0) return rc;
+    MSAMP_REQUIRE(coef != nullptr, MSAMP_ERR_NULL, "msamp_grad_clip: null factor");
+    const size_t run = grad_run(grads, n);
+    for (int from = 0; from < n; from += kGradTable) {
+        const GradTable g = grad_table(grads, from, n, run, true);
+        hipLaunchKernelGGL(grad_clip_kernel, dim3(g.first[g.n]), dim3(kBucketThreads), 0, static_cast<hipStream_t>(stream), g, coef);
+        MSAMP_CHECK_LAUNCH("grad_clip_kernel");
+    }
     return MSAMP_OK;
 }
 

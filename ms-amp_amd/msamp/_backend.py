@@ -56,6 +56,8 @@ _SIGNATURES = {
     'msamp_mfma_probe': ([_vp, _vp, _i, _i, _i, _vp, _vp], _i),
     'msamp_set_small_tile_limit': ([_i], None),
     'msamp_scale_update_groups': ([_vp, _i, _i, _vp], _i),
+    'msamp_grad_norms': ([_vp, _i, _i, _f, _vp, _vp, _vp, _vp, _vp], _i),
+    'msamp_grad_clip': ([_vp, _i, _vp, _vp], _i),
     'msamp_fp8_norms': ([_vp, _i, _vp, _i, _i, _i, _vp], _i),
     'msamp_bucket_amax': ([_vp, _i, _vp, _i, _i, _i, _vp], _i),
     'msamp_bucket_amax_speculative': ([_vp, _i, _vp, _i, _i, _i, _i, _vp], _i),
@@ -758,6 +760,33 @@ def fp8_norms(values, scale_invs, fp8_dt, norm_type):
         'msamp_fp8_norms'
     )
     return result.clone()
+
+
+GRAD_BLOCKS = 2048    # MSAMP_GRAD_BLOCKS
+
+
+def grad_table(entries):
+    """Host table (msamp_grad) of (data pointer, scale_inv pointer or 0, numel, library dtype) tuples."""
+    flat = [word for e in entries for word in e]
+    return (ctypes.c_longlong * len(flat))(*flat)
+
+
+def grad_norms(table, n, norm_type, max_norm, device):
+    """(per-tensor norms, total norm, clipping factor) of the table's tensors, all on the GPU."""
+    kind = {1.0: 1, 2.0: 2, float('inf'): 0}[float(norm_type)]
+    norms = torch.empty(n + 1, dtype=torch.float32, device=device)    # the factor is the last word
+    total = torch.empty((), dtype=torch.float32, device=device)
+    partials = torch.empty(n + GRAD_BLOCKS, dtype=torch.float64, device=device)
+    _check(
+        load().msamp_grad_norms(table, n, kind, max_norm, _ptr(partials), _ptr(norms), _ptr(total), _ptr(norms) + 4 * n,
+                                _stream()), 'msamp_grad_norms'
+    )
+    return norms[:n], total, norms[n]
+
+
+def grad_clip(table, n, factor):
+    """Multiplies the table's tensors (FP8 ones through their scale_inv) by factor where that is below 1."""
+    _check(load().msamp_grad_clip(table, n, _ptr(factor), _stream()), 'msamp_grad_clip')
 
 
 # ---- AdamW --------------------------------------------------------------------------------------

@@ -7,34 +7,44 @@ from msamp.common.dtype import Dtypes
 from msamp.common.tensor import ScalingTensor
 
 
-def _fused_fp8_norms(grads, norm_type):
-    """Norms of the FP8 ScalingTensor gradients among `grads`, straight from their codes (one pass at a byte per
-    element instead of dequantizing each to float32 first); None for the others."""
-    norms = [None] * len(grads)
-    if norm_type not in (1.0, 2.0, float('inf')):
-        return norms
-    by_qtype = {}
-    for i, g in enumerate(grads):
-        if isinstance(g, ScalingTensor) and Dtypes.is_fp8_qtype(g.qtype) and g.is_cuda and g.value.is_contiguous():
-            by_qtype.setdefault(g.qtype, []).append(i)
-    for qtype, idx in by_qtype.items():
-        out = _backend.fp8_norms([grads[i].value for i in idx], [grads[i].meta.scale_inv for i in idx], int(qtype), norm_type)
-        for k, i in enumerate(idx):
-            norms[i] = out[k]
-    return norms
+_KINDS = (1.0, 2.0, float('inf'))
+_PLAIN = (torch.float32, torch.float16, torch.bfloat16)
 
 
-def _compute_total_norm(parameters, norm_type=2.0):
-    grads = [p.grad for p in parameters if p.grad is not None]
-    if not grads:
-        return torch.tensor(0.)
+def _table(grads, norm_type):
+    """Descriptors of the gradients for the kernels that take the whole list at once, or None if one of them is not a
+    contiguous FP8 ScalingTensor or plain tensor on the current GPU, or shares memory with another."""
+    if norm_type not in _KINDS or not grads:
+        return None
+    entries, seen, device = [], set(), None
+    for g in grads:
+        if type(g) is ScalingTensor:
+            value, si = g.value, g.meta.scale_inv
+            if not Dtypes.is_fp8_qtype(g.qtype) or si.dtype != torch.float32 or si.numel() != 1 or si.device != value.device:
+                return None
+            dtype, si, at = int(g.qtype), si.data_ptr(), si.data_ptr()
+        else:
+            value, si = g, 0
+            if type(g) not in (torch.Tensor, torch.nn.Parameter) or g.layout != torch.strided or g.dtype not in _PLAIN or \
+                    g.requires_grad:
+                return None
+            dtype, at = _backend.hp_dt(g), g.data_ptr()
+        if device is None:
+            device = value.device
+        n = value.numel()
+        if n == 0 or not value.is_cuda or value.device != device or not value.is_contiguous() or at in seen:
+            return None
+        seen.add(at)
+        entries.append((value.data_ptr(), si, n, dtype))
+    return _backend.grad_table(entries) if device.index == torch.cuda.current_device() else None
+
+
+def _compute_total_norm(grads, norm_type):
     device = grads[0].device
-    norm_type = float(norm_type)
-    norms = _fused_fp8_norms(grads, norm_type)
-    for i, g in enumerate(grads):
-        if norms[i] is None:
-            g32 = g.to(torch.float32).detach()
-            norms[i] = (g32.abs().max() if norm_type == float('inf') else torch.norm(g32, norm_type)).to(device)
+    norms = []
+    for g in grads:
+        g32 = g.to(torch.float32).detach()
+        norms.append((g32.abs().max() if norm_type == float('inf') else torch.norm(g32, norm_type)).to(device))
     if norm_type == float('inf'):
         return norms[0] if len(norms) == 1 else torch.max(torch.stack(norms))
     return torch.norm(torch.stack(norms), norm_type)
@@ -47,18 +57,28 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
         parameters = [parameters]
     else:
         parameters = list(parameters)
-    total_norm = _compute_total_norm(parameters, norm_type=norm_type)
+    grads = [p.grad for p in parameters if p.grad is not None]
+    norm_type, max_norm = float(norm_type), float(max_norm)
+    table = _table(grads, norm_type)
+    if table is not None:
+        # norms, factor and clipping without the host waiting for any of them
+        _, total_norm, factor = _backend.grad_norms(table, len(grads), norm_type, max_norm, grads[0].device)
+    else:
+        total_norm = _compute_total_norm(grads, norm_type) if grads else torch.tensor(0.)
     if error_if_nonfinite and torch.logical_or(total_norm.isnan(), total_norm.isinf()):
         raise RuntimeError(
             f'The total norm of order {norm_type} for gradients from `parameters` is non-finite, so it cannot be '
             'clipped. To disable this error and scale the gradients by the non-finite norm anyway, set '
             '`error_if_nonfinite=False`'
         )
-    max_norm = float(max_norm)
-    if max_norm > 0:
+    if max_norm > 0 and table is not None:
+        _backend.grad_clip(table, len(grads), factor)
+        # (what autograd saved of them, if anything, has changed)
+        changed = [g.meta.scale_inv if type(g) is ScalingTensor else g for g in grads]
+        torch.autograd.graph.increment_version([t for t in changed if not t.is_inference()])
+    elif max_norm > 0:
         coef = torch.clamp(max_norm / (total_norm + 1e-6), max=1.0)
         if coef.item() < 1.0:
-            for p in parameters:
-                if p.grad is not None:
-                    p.grad.detach().mul_(coef)
+            for g in grads:
+                g.detach().mul_(coef)
     return total_norm

@@ -284,3 +284,70 @@ def test_bucket_larger_than_the_caches_equals_its_tensors_one_by_one(speculate):
             for name in ('scale', 'scale_inv'):
                 assert same_float(getattr(out.meta, name), getattr(out_big[i].meta, name)), (rnd, i, name)
             assert same_float(out.meta.amax[0], out_big[i].meta.amax[0])
+
+
+def _clip_case(count):
+    """Plain and FP8 gradients of all types; sizes around a chunk (16384), one element off 16-byte alignment."""
+    from msamp.common.dtype import Dtypes
+    g = torch.Generator().manual_seed(count)
+    sizes = [1, 7, 16383, 16384, 16384 * 3 + 11, 300001]
+    grads = []
+    for i in range(count):
+        n = sizes[i % len(sizes)] if count < 20 else 1 + 37 * i
+        x = (torch.randn(n + 1, generator=g) * 10.0 ** (i % 3 - 2)).cuda()
+        kind = i % 5
+        if kind < 3:
+            x = x.to((torch.float32, torch.float16, torch.bfloat16)[kind])
+            grads.append(x[1:] if i % 2 else x[:n].clone())
+        else:
+            grads.append(x[:n].clone().cast((Dtypes.kfloat8_e4m3, Dtypes.kfloat8_e5m2)[kind - 3]))
+    return grads
+
+
+class _Owner:
+    def __init__(self, grad):
+        self.grad = grad
+
+
+@pytest.mark.parametrize('count', [1, 6, 17, 64, 65, 131])
+@pytest.mark.parametrize('norm_type', [1.0, 2.0, float('inf')])
+def test_clip_over_a_list_of_all_types(count, norm_type):
+    """One total over every type (sums in double: one float32 rounding per tensor and one of the total, 2 * 2^-24), and
+    every gradient multiplied as torch multiplies it by that factor, bit for bit; tables of 64 tensors and their edges."""
+    import msamp
+    grads = _clip_case(count)
+    owners = [_Owner(g) for g in grads]
+    wide = torch.cat([g.float().double().flatten() for g in grads])
+    want = wide.abs().max() if norm_type == float('inf') else wide.abs().pow(norm_type).sum().pow(1 / norm_type)
+    plain = [None if hasattr(g, 'meta') else g.clone() for g in grads]
+    scales = [g.meta.scale_inv.clone() if hasattr(g, 'meta') else None for g in grads]
+    versions = [g._version if p is not None else 0 for g, p in zip(grads, plain)]
+    total = msamp.clip_grad_norm_(owners, want.item() * 2, norm_type=norm_type)    # nothing to clip
+    assert total.item() == pytest.approx(want.item(), rel=2.5e-7)
+    for g, p, si in zip(grads, plain, scales):
+        assert torch.equal(g, p) if p is not None else torch.equal(g.meta.scale_inv, si)
+    total = msamp.clip_grad_norm_(owners, want.item() / 3, norm_type=norm_type)
+    coef = torch.clamp((want.item() / 3) / (total + 1e-6), max=1.0)
+    for g, p, si, v in zip(grads, plain, scales, versions):
+        if p is None:
+            assert torch.equal(g.meta.scale_inv, si * coef)
+        else:
+            assert torch.equal(g, p.mul_(coef)) and g._version > v
+
+
+def test_clip_with_a_nan_and_with_a_shared_gradient():
+    """A NaN total clips nothing; a gradient that two parameters share is clipped once for each, as before."""
+    import msamp
+    grads = _clip_case(5)
+    grads[2][3] = float('nan')
+    before = [g.value.clone() if hasattr(g, 'meta') else g.clone() for g in grads]
+    scales = [g.meta.scale_inv.clone() if hasattr(g, 'meta') else None for g in grads]
+    assert math.isnan(msamp.clip_grad_norm_([_Owner(g) for g in grads], 1e-3).item())
+    for g, b, si in zip(grads, before, scales):
+        assert torch.equal(getattr(g, 'value', g).view(torch.uint8), b.view(torch.uint8))
+        assert si is None or torch.equal(si, g.meta.scale_inv)
+    with pytest.raises(RuntimeError):
+        msamp.clip_grad_norm_([_Owner(g) for g in grads], 1.0, error_if_nonfinite=True)
+    x = torch.full((4, ), 3.0, device='cuda')
+    total = msamp.clip_grad_norm_([_Owner(x), _Owner(x)], 1.0)
+    assert total.item() == pytest.approx(math.sqrt(72.0)) and torch.allclose(x, torch.full_like(x, 3.0 / 72.0))
