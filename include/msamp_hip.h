@@ -465,6 +465,31 @@ int msamp_adamw_f32(float* param, const void* grad, int grad_dtype, size_t n, fl
                     double beta1, double beta2, double eps, double weight_decay, int step, int bias_correction, int adam_mode,
                     int maximize, msamp_stream_t stream);
 
+/* The same step for a list of parameters, a launch (two with scaled weights) per 32 of them.  `list`: HOST array, read during
+ * the call.  param: F32 / F16 / BF16 (scale null), or a scaled F16 weight with its meta's scale, scale_inv and amax[0] (all
+ * rewritten: rule(max|p'|, old scale), 1 / scale, max|p'|; payload F16(p' * scale)).  grad: F32 / F16 / BF16, or E4M3 / E5M2 with
+ * grad_scale_inv.  exp_avg, exp_avg_sq: F32.  The entry's own `scratch` is ignored.
+ * scratch: float32, 16-byte aligned, room for the largest scaled weight rounded up to four elements (with room for several
+ * they share launches); words: MSAMP_F32_WORDS 32-bit words of scratch. */
+#define MSAMP_F32_BLOCKS 4096
+#define MSAMP_F32_WORDS (MSAMP_F32_BLOCKS + 64)
+typedef struct msamp_f32_param {
+    void* param;
+    float* scale;
+    float* scale_inv;
+    float* amax;
+    const void* grad;
+    const float* grad_scale_inv;
+    float* exp_avg;
+    float* exp_avg_sq;
+    float* scratch;
+    uint64_t numel;
+    int32_t param_dtype, grad_dtype;
+} msamp_f32_param;
+int msamp_adamw_f32_list(const msamp_f32_param* list, int n, float* scratch, size_t scratch_elems, uint32_t* words, double lr,
+                         double beta1, double beta2, double eps, double weight_decay, int step, int bias_correction, int adam_mode,
+                         int maximize, msamp_stream_t stream);
+
 /* The same step (adamw.py:148-199: stage 1, the scale rule on the two amaxs, stage 2) for parameters kept in high
  * precision -- biases, norm weights, embeddings: a plain F32 / F16 / BF16 parameter and gradient, exp_avg in E4M3, exp_avg_sq
  * in scaled F16 -- for n_tensors of them at once, with nothing read back by the host (the reference takes a dozen launches

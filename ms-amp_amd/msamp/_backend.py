@@ -69,6 +69,7 @@ _SIGNATURES = {
     'msamp_fp8_gemm_get_walk': ([_i, _i, _i, _i, _i], _i),
     'msamp_fp8_gemm_tune': ([_vp, _i, _vp, _i, _vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _vp, _i, _vp, _vp], _i),
     'msamp_adamw_f32': ([_vp, _vp, _i, _sz, _vp, _vp, _d, _d, _d, _d, _d, _i, _i, _i, _i, _vp], _i),
+    'msamp_adamw_f32_list': ([_vp, _i, _vp, _sz, _vp, _d, _d, _d, _d, _d, _i, _i, _i, _i, _vp], _i),
     'msamp_adamw_plain_fused': ([_vp, _i, _vp, _i, _i, _i, _d, _d, _d, _d, _d, _i, _i, _i, _i, _i, _vp], _i),
     'msamp_adamw_fp8_fused_shift': ([_vp, _vp, _vp, _i, _vp, _i, ctypes.c_longlong, _i, _i, _d, _d, _d, _d, _d, _i, _i, _i, _i, _i, _vp, _vp], _i),
     'msamp_adamw_fp8_fused_speculative': ([_vp, _vp, _vp, _i, _vp, _i, _i, _i, _d, _d, _d, _d, _d, _i, _i, _i, _i, _i, _vp], _i),
@@ -873,6 +874,27 @@ def adamw_f32(param, grad, exp_avg, exp_avg_sq, lr, beta1, beta2, eps, weight_de
             _ptr(param), _ptr(grad), _dt(grad), param.numel(), _ptr(exp_avg), _ptr(exp_avg_sq), lr, beta1, beta2, eps,
             weight_decay, step, 1 if bias_correction else 0, 1 if adam_mode else 0, 1 if maximize else 0, _stream()
         ), 'msamp_adamw_f32'
+    )
+
+
+F32_WORDS = 4096 + 64    # MSAMP_F32_WORDS
+F32_SCRATCH = 64 << 20    # float32 elements of scratch in one launch: what the memory-side cache holds
+
+
+def adamw_f32_list(rows, scaled_numels, device, lr, beta1, beta2, eps, weight_decay, step, bias_correction, adam_mode, maximize):
+    """One AdamW / Adam step of a list of parameters with float32 moments.  `rows`: msamp_f32_param as tuples of eleven
+    words; `scaled_numels`: sizes of the scaled weights among them (they share float32 scratch)."""
+    flat = [word for row in rows for word in row]
+    table = (ctypes.c_longlong * len(flat))(*flat)
+    padded = [(n + 3) // 4 * 4 for n in scaled_numels]
+    room = max(max(padded), min(sum(padded), F32_SCRATCH)) if padded else 0
+    words = torch.empty(F32_WORDS, dtype=torch.int32, device=device)
+    scratch = torch.empty(room, dtype=torch.float32, device=device) if room else None
+    _check(
+        load().msamp_adamw_f32_list(
+            table, len(rows), _ptr(scratch), room, _ptr(words), lr, beta1, beta2, eps, weight_decay, step,
+            1 if bias_correction else 0, 1 if adam_mode else 0, 1 if maximize else 0, _stream()
+        ), 'msamp_adamw_f32_list'
     )
 
 

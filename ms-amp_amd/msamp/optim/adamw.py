@@ -397,12 +397,17 @@ class LBAdamW(LBAdamWBase):
 
     # ---- float32 moments ---------------------------------------------------------------------
     def _f32_step(self, p, g, exp_avg, exp_avg_sq, step, *, beta1, beta2, lr, weight_decay, eps, maximize):
-        """The chain of element-wise calls of the reference's float32 branch (msamp/optim/adamw.py:200-232) as one kernel,
-        same bits; False where the kernel does not apply (the chain below then runs as written)."""
+        """The chain of element-wise calls of the reference's float32 branch (msamp/optim/adamw.py:200-232), same bits, in
+        kernels of the library; False where they do not apply (the chain below then runs as written).  Most parameters
+        are put on a list for `_f32_flush`, which steps all of them at once; the others are stepped here."""
         moments = (exp_avg, exp_avg_sq)
         if any(isinstance(t, ScalingTensor) or t.dtype != torch.float32 or not t.is_cuda or not t.is_contiguous()
                for t in moments):
             return False
+        row = self._f32_row(p, g, exp_avg, exp_avg_sq)
+        if row is not None:
+            self._f32_pending.append((step, row, p, g))
+            return True
         param = p.float()
         grad = g.float() if isinstance(g, ScalingTensor) or g.dtype not in self._PLAIN_DTYPES else g
         if not (param.is_cuda and grad.is_cuda) or any(t.numel() != param.numel() for t in (grad, ) + moments):
@@ -415,6 +420,59 @@ class LBAdamW(LBAdamWBase):
         elif param.data_ptr() != p.data_ptr():
             p.copy_(param)
         return True
+
+    @classmethod
+    def _f32_row(cls, p, g, exp_avg, exp_avg_sq):
+        """The parameter's entry of the list kernels, or None: they take contiguous plain tensors, float16 weights whose scale
+        follows from the new maximum (window 1, in-time scaling), and plain or FP8 gradients, all on the current GPU."""
+        n = p.numel()
+        if isinstance(p, ScalingTensor):
+            meta = p.meta
+            if meta.qtype != Dtypes.kfloat16 or meta.window_size != 1 or not ScalingMeta.in_time_scaling or not meta.is_cuda:
+                return None
+            value, p_dt = p.value, _backend.DT_F16
+            meta_ptrs = (meta.scale.data_ptr(), meta.scale_inv.data_ptr(), meta.amax.data_ptr())
+        else:
+            if p.dtype not in cls._PLAIN_DTYPES:
+                return None
+            value, p_dt, meta_ptrs = p, _backend.hp_dt(p), (0, 0, 0)
+        if isinstance(g, ScalingTensor):
+            if not Dtypes.is_fp8_qtype(g.qtype) or not g.meta.scale_inv.is_cuda:
+                return None
+            g_value, g_dt, g_si = g.value, int(g.qtype), g.meta.scale_inv.data_ptr()
+        else:
+            if g.dtype not in cls._PLAIN_DTYPES or g.layout != torch.strided:
+                return None
+            g_value, g_dt, g_si = g, _backend.hp_dt(g), 0
+        if n == 0 or g_value.numel() != n or exp_avg.numel() != n or exp_avg_sq.numel() != n or value.layout != torch.strided or \
+                not (value.is_cuda and g_value.is_cuda and value.is_contiguous() and g_value.is_contiguous()):
+            return None
+        if value.device.index != torch.cuda.current_device() or \
+                any(t.device != value.device for t in (g_value, exp_avg, exp_avg_sq)):
+            return None
+        return (value.data_ptr(), ) + meta_ptrs + (g_value.data_ptr(), g_si, exp_avg.data_ptr(), exp_avg_sq.data_ptr(), 0, n,
+                                                   p_dt | g_dt << 32)
+
+    def _f32_flush(self, *, beta1, beta2, lr, weight_decay, eps, maximize):
+        pending, self._f32_pending = self._f32_pending, []
+        by_step = {}
+        for step, row, p, g in pending:
+            group = by_step.setdefault(step, ([], [], set()))
+            if row[0] in group[2]:    # (a payload that is on the list already: its second step comes after the first)
+                self._f32_launch(step, group, beta1, beta2, lr, weight_decay, eps, maximize)
+                group = by_step[step] = ([], [], set())
+            group[0].append(row)
+            group[2].add(row[0])
+            if row[1]:
+                group[1].append(row[9])
+        for step, group in by_step.items():
+            self._f32_launch(step, group, beta1, beta2, lr, weight_decay, eps, maximize)
+        written = [p.value if isinstance(p, ScalingTensor) else p for _, _, p, _ in pending]
+        torch.autograd.graph.increment_version([t for t in written if t.dtype != torch.float32 and not t.is_inference()])
+
+    def _f32_launch(self, step, group, beta1, beta2, lr, weight_decay, eps, maximize):
+        _backend.adamw_f32_list(group[0], group[1], torch.device('cuda', torch.cuda.current_device()), lr, beta1, beta2, eps,
+                                weight_decay, step, self.bias_correction, self.use_adam, maximize)
 
     # ---- per-tensor path (reference recipe) -----------------------------------------------
     def _staged_step(self, idx, params, grads, exp_avgs, exp_avg_sqs, state_steps, *, beta1, beta2, lr, weight_decay,
@@ -499,6 +557,7 @@ class LBAdamW(LBAdamWBase):
             self._staged_step(staged, params, grads, exp_avgs, exp_avg_sqs, state_steps, **hyper)
             return
         # float32 moments: whole-tensor float32 update, then requantize the parameter if it is low-bit
+        self._f32_pending = []
         for i, p in enumerate(params):
             if self._f32_step(p, grads[i], exp_avgs[i], exp_avg_sqs[i], state_steps[i], beta1=beta1, beta2=beta2, lr=lr,
                               weight_decay=weight_decay, eps=eps, maximize=maximize):
@@ -521,3 +580,4 @@ class LBAdamW(LBAdamWBase):
                 p.copy_(param.cast(p.qtype, meta=p.meta))
             elif param.data_ptr() != p.data_ptr():
                 p.copy_(param)
+        self._f32_flush(beta1=beta1, beta2=beta2, lr=lr, weight_decay=weight_decay, eps=eps, maximize=maximize)

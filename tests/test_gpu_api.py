@@ -883,3 +883,52 @@ def test_float32_moment_step_in_one_kernel_has_the_bits_of_the_chain(monkeypatch
         for t, (x, y) in enumerate(zip(a, b)):
             for which, (u, v) in enumerate(zip(x, y)):
                 assert same_float(u, v), (step, t, which, (u.float() - v.float()).abs().max().item())
+
+
+@pytest.mark.parametrize('kw', [dict(weight_decay=0.1), dict(weight_decay=0.0, maximize=True)])
+def test_float32_moment_step_over_a_list_has_the_bits_of_one_parameter_at_a_time(monkeypatch, kw):
+    """Seventy parameters (more than two tables of 32): plain and scaled-float16 ones, FP8 and plain gradients, sizes
+    around a workgroup's 1024 elements and with remainders modulo 4, a NaN, a weight of zeros (its scale stays), a view off
+    a 16-byte boundary, scratch for part of the weights only.  Parameters, metas and moments agree bit for bit with the
+    step taken for one parameter at a time."""
+    sizes = (1, 3, 5, 1023, 1024, 1025, 4099, 20001)
+    runs = []
+    for listed in (True, False):
+        gen = torch.Generator(device='cuda').manual_seed(5)
+        params = []
+        for i in range(70):
+            n = sizes[i % len(sizes)]
+            x = torch.randn(n, device='cuda', generator=gen) * 0.1
+            if i == 11:
+                x.zero_()
+            if i % 3 == 0:
+                params.append(torch.nn.Parameter(x.to((torch.float32, torch.bfloat16, torch.float16)[i // 3 % 3])))
+            else:
+                params.append(ScalingParameter(x.cast(Dtypes.kfloat16)))
+        params.append(torch.nn.Parameter(torch.randn(4098, device='cuda', generator=gen)[1:]))
+        opt = LBAdamW(params, lr=2e-3, exp_avg_dtype=torch.float32, exp_avg_sq_dtype=torch.float32, **kw)
+        if listed:
+            monkeypatch.setattr('msamp._backend.F32_SCRATCH', 30000)
+        else:
+            monkeypatch.setattr(LBAdamW, '_f32_row', classmethod(lambda cls, *a: None))
+        for step in range(3):
+            for i, p in enumerate(params):
+                g = torch.randn(p.shape, device='cuda', generator=gen) * 10.0 ** (step - 1)
+                if i == 11:
+                    g.zero_()
+                if i == 14 and step == 2:
+                    g[0] = float('nan')
+                if isinstance(p, ScalingParameter):
+                    p.grad = g.cast((Dtypes.kfloat8_e4m3, Dtypes.kfloat8_e5m2)[i % 2]) if i % 4 else g.half()
+                else:
+                    p.grad = g.to(p.dtype)
+            opt.step()
+        monkeypatch.undo()
+        out = []
+        for p in params:
+            out += [p.value, p.meta.scale, p.meta.scale_inv, p.meta.amax] if isinstance(p, ScalingParameter) else [p.detach()]
+            out += [opt.state[p]['exp_avg'], opt.state[p]['exp_avg_sq']]
+        runs.append(out)
+    for k, (a, b) in enumerate(zip(*runs)):
+        assert same_float(a, b), k
+
