@@ -140,6 +140,15 @@ int msamp_cast_to_fp8_gated(const void* x, int in_dtype, size_t n, float* scale,
                             uint8_t* out, int fp8_type, int margin, int flags, const int32_t* warmup_counter, int window,
                             void* workspace, msamp_stream_t stream);
 
+/* msamp_cast_to_fp8_gated of a 2-D x[rows][cols] that also forms its column sums, as the backward of a linear layer needs
+ * them for the bias: sum[c] = T(sum over r of x[r][c]) converted to sum_dtype, T = x's type, the sum taken in float32 in a
+ * fixed order.  (The reference leaves them to autograd, msamp/nn/functional.py:184-185.)  `scratch`: as many floats as
+ * msamp_cast_colsum_scratch says. */
+int msamp_cast_colsum_scratch(int rows, int cols, int in_dtype, size_t* n_floats);
+int msamp_cast_to_fp8_colsum_gated(const void* x, int in_dtype, int rows, int cols, float* scale, float* amax, float* scale_inv,
+                                   uint8_t* out, int fp8_type, void* sum, int sum_dtype, float* scratch, int margin, int flags,
+                                   const int32_t* warmup_counter, int window, void* workspace, msamp_stream_t stream);
+
 /* Arithmetic.add_to_fp8 (msamp/operators/arithmetic/arithmetic.py:15-35, vectorized_pointwise.h:184-301): in place,
  * q <- in-time cast of (T(dequant(q)) + other), T = other's dtype, the sum rounded to T as torch adds two T tensors;
  * amax[0] = max|sum|, *scale by the rule (fallback the old *scale), *scale_inv = 1 / *scale.  Equal, bit for bit, to

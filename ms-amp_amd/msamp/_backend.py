@@ -49,6 +49,8 @@ _SIGNATURES = {
     'msamp_scale_cast': ([_vp, _i, _sz, _vp, _vp, _i, _vp], _i),
     'msamp_scale_update': ([_vp, _vp, _vp, _vp, _i, _i, _f, _i, _vp], _i),
     'msamp_cast_to_fp8_gated': ([_vp, _i, _sz, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp], _i),
+    'msamp_cast_colsum_scratch': ([_i, _i, _i, _vp], _i),
+    'msamp_cast_to_fp8_colsum_gated': ([_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _vp, _i, _i, _vp, _i, _vp, _vp], _i),
     'msamp_cast_transpose_gated': ([_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp], _i),
     'msamp_fp8_gemm': ([_vp, _i, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp, _i, _vp], _i),
     'msamp_fp8_gemm_kmajor': ([_vp, _i, _vp, _i, _vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _i, _vp, _i, _vp], _i),
@@ -401,6 +403,26 @@ def cast_to_fp8_gated(x, scale, amax_cell, scale_inv, fp8_dt, counter, window, m
         ), 'msamp_cast_to_fp8_gated'
     )
     return out
+
+
+def cast_to_fp8_gated_colsum(x, scale, amax_cell, scale_inv, fp8_dt, counter, window, sum_dtype):
+    """cast_to_fp8_gated of a non-empty 2-D x, and x.sum(0).to(sum_dtype) from the same pass."""
+    lib = load()
+    _gpu(x, 'input')
+    _gpu(counter, 'warm-up counter')
+    rows, cols = x.shape
+    out = torch.empty((rows, cols), dtype=torch.uint8, device=x.device)
+    sums = torch.empty((cols, ), dtype=sum_dtype, device=x.device)
+    words = ctypes.c_size_t()
+    _check(lib.msamp_cast_colsum_scratch(rows, cols, _dt(x), ctypes.addressof(words)), 'msamp_cast_colsum_scratch')
+    scratch = torch.empty((words.value, ), dtype=torch.float32, device=x.device)
+    _check(
+        lib.msamp_cast_to_fp8_colsum_gated(
+            _ptr(x), _dt(x), rows, cols, _ptr(scale), _ptr(amax_cell), _ptr(scale_inv), _ptr(out), fp8_dt, _ptr(sums), _dt(sums),
+            _ptr(scratch), 0, FLAG_TWO_PASS if _two_pass_only() else 0, _ptr(counter), window, _ptr(workspace(x.device)), _stream()
+        ), 'msamp_cast_to_fp8_colsum_gated'
+    )
+    return out, sums
 
 
 def cast_scaled_to_fp8(x, amax, old_scale_inv, scale, scale_inv, fp8_dt, margin=0, amax_out=None, counter_out=None):

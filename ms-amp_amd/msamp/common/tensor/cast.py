@@ -87,6 +87,20 @@ class TypeCast:
         return out
 
     @staticmethod
+    def takes_column_sums(input, meta, sum_dtype):
+        """True if cast_to_fp8_with_column_sums does what cast_to_fp8(input, meta) and input.sum(0).to(sum_dtype) do."""
+        return meta.scaling_mode() == 'gated' and input.dim() == 2 and input.numel() > 0 and input.is_cuda and \
+            input.is_contiguous() and input.dtype in _CAST_DTYPES and sum_dtype in _CAST_DTYPES and meta.scale.is_cuda and \
+            not (torch.is_grad_enabled() and input.requires_grad)
+
+    @staticmethod
+    def cast_to_fp8_with_column_sums(input, meta, sum_dtype):
+        """(payload, column sums): the cast of a bias's output gradient and the bias gradient in one pass over it."""
+        return _backend.cast_to_fp8_gated_colsum(
+            input, meta.scale, meta.amax[0:1], meta.scale_inv, int(meta.qtype), meta.amax_counter, meta.window_size, sum_dtype
+        )
+
+    @staticmethod
     def cast_to_fp16(input, meta, sync=False):
         """Scaled 16-bit (or 32-bit) payload: (input * scale).to(dtype of meta.qtype)."""
         in_time = meta.is_in_time_scaling()

@@ -4,7 +4,7 @@ import torch
 import torch.nn.functional as F
 
 from msamp.common.dtype import Dtypes
-from msamp.common.tensor import ScalingTensor
+from msamp.common.tensor import ScalingTensor, TypeCast
 from msamp.operators.gemm import Gemm
 from msamp.nn.state import model_state
 
@@ -47,7 +47,11 @@ class _FP8GemmFunction(torch.autograd.Function):
         # the shapes allow, dy is only cast and W, x, dy go to the GEMMs as they are (same results).
         in_place = (not need_dgrad or Gemm.kmajor_supported(d_in, tokens, d_out, True, False)) and \
             (not need_wgrad or Gemm.kmajor_supported(d_in, d_out, tokens, True, True))
-        if in_place:
+        bias_grad = None
+        if in_place and ctx.need_bias_grad and TypeCast.takes_column_sums(output_grad, metas['ograd'], ctx.bias_dtype):
+            payload, bias_grad = TypeCast.cast_to_fp8_with_column_sums(output_grad, metas['ograd'], ctx.bias_dtype)
+            ograd_fp8, ograd_fp8_t = ScalingTensor(payload, metas['ograd']), None
+        elif in_place:
             ograd_fp8 = output_grad.cast(Dtypes.kfloat8_e5m2, meta=metas['ograd'])
             ograd_fp8_t = None
         else:
@@ -92,7 +96,8 @@ class _FP8GemmFunction(torch.autograd.Function):
             del old_wgrad
             ctx.weight.backward_grad_update(wgrad)
 
-        bias_grad = output_grad.sum(0).to(ctx.bias_dtype) if ctx.need_bias_grad else None
+        if ctx.need_bias_grad and bias_grad is None:
+            bias_grad = output_grad.sum(0).to(ctx.bias_dtype)
         return input_grad, None, None, None, bias_grad
 
 

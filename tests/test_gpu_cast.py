@@ -570,3 +570,31 @@ def test_fresh_meta_cast_guesses_from_a_sample(be, dtype, what):
     want = be.cast_to_fp8_intime(x, s, am[0:1], si, 5, two_pass=True, speculate=False)
     got, fs, fsi, count, fam = _fresh(be, x, 5)
     assert torch.equal(got, want) and same_float(fs, s) and same_float(fsi, si) and same_float(fam, am) and count.item() == 0
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('rows,cols', [(1, 1), (3, 8), (16, 512), (17, 520), (96, 1001), (1000, 260), (4099, 384), (33, 4304)])
+def test_cast_with_column_sums(be, dtype, rows, cols):
+    """Codes and meta of the gated cast, on both sides of the gate, and the columns' sums: float32 sums of at most `chain`
+    terms in a row (2^-24 each of the sum of magnitudes), rounded to the input's type; a view that 16-byte loads do not fit."""
+    g = torch.Generator().manual_seed(rows + cols)
+    flat = torch.randn(rows * cols + 3, generator=g).to(dtype).cuda()
+    for x in (flat[:rows * cols].view(rows, cols), flat[3:].view(rows, cols)):
+        for counter, sum_dtype in ((0, torch.float32), (16, dtype)):
+            cnt = torch.full((), counter, dtype=torch.int32, device='cuda')
+            s, si, am = make_meta(window=16, scale=4.0)
+            s2, si2, am2 = make_meta(window=16, scale=4.0)
+            q, sums = be.cast_to_fp8_gated_colsum(x, s, am[0:1], si, 6, cnt, 16, sum_dtype)
+            want = be.cast_to_fp8_gated(x, s2, am2[0:1], si2, 6, cnt, 16)
+            assert torch.equal(q, want) and same_float(am, am2) and same_float(s, s2) and same_float(si, si2)
+            exact, size = x.double().sum(0), x.double().abs().sum(0)
+            chain = 3 * 16 + rows / 4    # a slab's quarter, the sixteenth of the slabs, the runs
+            rounding = {torch.float32: 2.0**-24, torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}[dtype]
+            tiny = 2.0**-25 if dtype == torch.float16 else 0.0
+            bound = size * min(chain, rows) * 2.0**-24 + exact.abs() * rounding * 1.01 + tiny
+            assert sums.dtype == sum_dtype and ((sums.double() - exact).abs() <= bound).all()
+    x = torch.full((5, 16), 2.0, dtype=dtype, device='cuda')
+    x[1, 3], x[2, 4] = float('nan'), float('inf')
+    s, si, am = make_meta(window=16)
+    _, sums = be.cast_to_fp8_gated_colsum(x, s, am[0:1], si, 6, torch.full((), 16, dtype=torch.int32, device='cuda'), 16, dtype)
+    assert torch.equal(torch.nan_to_num(sums, nan=-1.0), torch.nan_to_num(x.sum(0), nan=-1.0))
