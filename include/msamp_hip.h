@@ -301,6 +301,15 @@ int msamp_fp8_gemm_kmajor(const uint8_t* a, int a_type, const float* a_scale_inv
                           int b_type, const float* b_scale_inv, int b_kmajor, void* d, int d_dtype, int m, int n, int k,
                           int accumulate, const void* bias, int bias_dtype, msamp_stream_t stream);
 
+/* msamp_fp8_gemm_kmajor with both operands K-major and no bias (a weight gradient, K = tokens), in parts of K where the
+ * output is too few tiles to fill the device: float32 partial sums in `scratch`, added up in a fixed order and scaled by a
+ * second kernel (another order of the same float32 sum).  msamp_fp8_gemm_ksplit_scratch says how many floats that takes,
+ * 0 where the product is better taken whole; only problems for which it is not 0 are accepted. */
+int msamp_fp8_gemm_ksplit_scratch(int m, int n, int k, size_t* n_floats);
+int msamp_fp8_gemm_ksplit(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type,
+                          const float* b_scale_inv, void* d, int d_dtype, int m, int n, int k, int accumulate,
+                          float* scratch, size_t n_floats, msamp_stream_t stream);
+
 /* The weight-gradient GEMM of a linear layer followed by its cast to FP8 (nn/functional.py:100-111 followed by
  * :121-123 of the reference: `wgrad = Gemm.fp8_gemm(...)`, then `wgrad.cast(Dtypes.kfloat8_e4m3, meta=..., sync=True)`)
  * without the second trip over the product: q = FP8 codes of round_to_d_dtype(D) * scale, with

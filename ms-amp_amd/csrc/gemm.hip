@@ -25,6 +25,76 @@ static bool kmajor_shape_ok(int NR, int NC, int K, bool xt, bool yt) {
     return K > kBK && fits_offsets(NR, NC, K) && (xt ? NR % 16 == 0 : K % 16 == 0) && (yt ? NC % 16 == 0 : K % 16 == 0);
 }
 
+static int dispatch_parts(int x_type, int y_type, const GemmCall& c, const KSplit& s) {
+    if (x_type == MSAMP_DT_E4M3 && y_type == MSAMP_DT_E4M3) return run_gemm_parts<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(c, s);
+    if (x_type == MSAMP_DT_E4M3) return run_gemm_parts<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(c, s);
+    if (y_type == MSAMP_DT_E4M3) return run_gemm_parts<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(c, s);
+    return run_gemm_parts<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(c, s);
+}
+
+// Weight gradients (both operands K-major, K = tokens) whose output is a few tiles leave compute units idle, or run a second
+// round of 128 x 128 tiles that is nearly empty; K is long there, so the chip is filled with parts of K.  What a form takes is
+// estimated, in microseconds, as rounds of tiles times what a tile costs (a 128-byte slice 0.6 with small and 1.65 with large
+// tiles, both with every compute unit busy; 5 and 9 around the K loop) plus, if split, the second launch and the way of the
+// partial sums to memory and back.  The split must promise 15 % less, so that it is not taken where the estimate
+// is near even.  Only problems of the 128 x 128 tiles are looked at: the others have tiles enough.  Whole against split, m x n
+// x k in us: 1200 x 4304 x 12605 128.9 -> 83.0 (three parts of large tiles; 340 small tiles on 256 compute units before),
+// 128 x 512 x 16000 54.9 -> 15.2, 256 x 1024 x 8192 29.9 -> 15.6, 1024 x 1024 x 16384 57.6 -> 33.4, 16 x 8192 x 8192 30.3 -> 19.7,
+// 2048 x 1024 x 8192 32.8 -> 27.4, 512 x 512 x 2500 12.7 -> 11.4.  FP8Linear 12605 x 1200 -> 4304, forward and backward: 335 -> 292.
+static KSplit ksplit_rule(int NR, int NC, int K) {
+    KSplit best = {true, 1};
+    if (!takes_small_tiles(NR, NC, K) || !kmajor_shape_ok(NR, NC, K, true, true)) return best;
+    const int nk = (K + kBK - 1) / kBK, cus = cu_count();
+    auto tiles = [&](int edge) { return ((NR + edge - 1) / edge) * ((NC + edge - 1) / edge); };
+    const int small = tiles(kDmaTile / 2), large = tiles(kDmaTile);
+    const double out = static_cast<double>(NR) * NC;
+    auto estimate = [&](int n, int parts, double slice, double around) {
+        const double rounds = (n * parts + cus - 1) / cus;
+        return rounds * ((nk + parts - 1) / parts * slice + around) + (parts > 1 ? 4.0 + out * (8.0 * parts + 2.0) / 5e6 : 0.0);
+    };
+    double least = 0.85 * estimate(small, 1, 0.6, 5.0);
+    // (at least four slices to a part, which is also what the small tile needs)
+    for (int parts = 2; parts <= 32 && nk / parts >= 4; ++parts) {
+        if (static_cast<long>(small) * parts <= 4L * cus) {
+            const double t = estimate(small, parts, 0.6, 5.0);
+            if (t < least) least = t, best = {true, parts};
+        }
+        if (static_cast<long>(large) * parts <= 4L * cus) {
+            const double t = estimate(large, parts, 1.65, 9.0);
+            if (t < least) least = t, best = {false, parts};
+        }
+    }
+    return best;
+}
+
+// D = (sum of the parts, in their order) * alpha (+ D), the expressions of the GEMM's own epilogue, one rounding.  Bound by
+// the read of the parts; four elements a lane.
+template <typename OT>
+__global__ __launch_bounds__(256) void ksplit_finish_kernel(const float* __restrict__ part, OT* __restrict__ D, size_t n, int parts,
+                                                            const float* __restrict__ xs, const float* __restrict__ ys, int accumulate) {
+    const size_t i = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+    if (i >= n) return;    // (n is a multiple of 4)
+    const float alpha = (*xs) * (*ys);
+    float4 s = *reinterpret_cast<const float4*>(part + i);
+#pragma unroll 4
+    for (int p = 1; p < parts; ++p) {
+        const float4 v = *reinterpret_cast<const float4*>(part + static_cast<size_t>(p) * n + i);
+        s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+    }
+    const float r[4] = {s.x, s.y, s.z, s.w};
+    struct __attribute__((aligned(4 * sizeof(OT)))) Four { OT v[4]; };
+    Four o;
+    if (accumulate) {
+        const Four old = *reinterpret_cast<const Four*>(D + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Elem<OT>::store(&o.v[e], fmaf(r[e], alpha, 0.0f) + Elem<OT>::load(&old.v[e]));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Elem<OT>::store(&o.v[e], r[e] * alpha);
+    }
+    *reinterpret_cast<Four*>(D + i) = o;
+}
+
 // tile walks registered per problem (kernel-side naming: NR x NC output, K, which operands are K-major)
 static std::mutex g_walk_mutex;
 static std::map<std::tuple<int, int, int, int>, int> g_walks;
@@ -199,6 +269,43 @@ extern "C" int msamp_fp8_gemm_kmajor(const uint8_t* a, int a_type, const float* 
     // X = b (rows of D), Y = a (columns of D)
     const GemmCall c = {b, a, d, d_dtype, n, m, k, b_scale_inv, a_scale_inv, accumulate, bias, bias_dtype, b_kmajor != 0, true, nullptr, st};
     return dispatch_pair(b_type, a_type, c);
+}
+
+extern "C" int msamp_fp8_gemm_ksplit_scratch(int m, int n, int k, size_t* n_floats) {
+    MSAMP_REQUIRE(m > 0 && n > 0 && k > 0, MSAMP_ERR_SHAPE, "msamp_fp8_gemm_ksplit_scratch: m=%d n=%d k=%d", m, n, k);
+    MSAMP_REQUIRE(n_floats != nullptr, MSAMP_ERR_NULL, "msamp_fp8_gemm_ksplit_scratch: null pointer");
+    const KSplit split = ksplit_rule(n, m, k);
+    *n_floats = split.parts > 1 ? static_cast<size_t>(split.parts) * n * m : 0;
+    return MSAMP_OK;
+}
+
+extern "C" int msamp_fp8_gemm_ksplit(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type,
+                                     const float* b_scale_inv, void* d, int d_dtype, int m, int n, int k, int accumulate,
+                                     float* scratch, size_t n_floats, msamp_stream_t stream) {
+    MSAMP_REQUIRE(is_fp8(a_type) && is_fp8(b_type), MSAMP_ERR_DTYPE, "msamp_fp8_gemm_ksplit: operand types %d, %d", a_type, b_type);
+    MSAMP_REQUIRE(is_hp(d_dtype), MSAMP_ERR_DTYPE, "msamp_fp8_gemm_ksplit: output dtype %d", d_dtype);
+    MSAMP_REQUIRE(m > 0 && n > 0 && k > 0, MSAMP_ERR_SHAPE, "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d", m, n, k);
+    MSAMP_REQUIRE(a && b && d && a_scale_inv && b_scale_inv && scratch, MSAMP_ERR_NULL, "msamp_fp8_gemm_ksplit: null pointer");
+    MSAMP_REQUIRE(aligned(a, 16) && aligned(b, 16) && aligned(d, 16) && aligned(scratch, 16), MSAMP_ERR_ALIGNMENT,
+                  "msamp_fp8_gemm_ksplit: operands, output and scratch must be 16-byte aligned");
+    // X = b (rows of D), Y = a (columns of D)
+    const KSplit split = ksplit_rule(n, m, k);
+    const size_t count = static_cast<size_t>(n) * m;
+    MSAMP_REQUIRE(split.parts > 1 && n_floats >= split.parts * count, MSAMP_ERR_SHAPE,
+                  "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d is not split, or needs more scratch than %zu floats", m, n, k, n_floats);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const GemmCall c = {b, a, scratch, MSAMP_DT_F32, n, m, k, b_scale_inv, a_scale_inv, 0, nullptr, 0, true, true, nullptr, st};
+    const int rc = dispatch_parts(b_type, a_type, c, split);
+    if (rc != MSAMP_OK) return rc;
+    const dim3 grid(static_cast<unsigned>((count / 4 + 255) / 256));
+#define FINISH(OT) \
+    hipLaunchKernelGGL((ksplit_finish_kernel<OT>), grid, dim3(256), 0, st, static_cast<const float*>(scratch), static_cast<OT*>(d), count, split.parts, b_scale_inv, a_scale_inv, accumulate)
+    if (d_dtype == MSAMP_DT_F32) FINISH(float);
+    else if (d_dtype == MSAMP_DT_F16) FINISH(f16_t);
+    else FINISH(bf16_t);
+#undef FINISH
+    MSAMP_CHECK_LAUNCH("ksplit_finish_kernel");
+    return MSAMP_OK;
 }
 
 extern "C" int msamp_fp8_gemm(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type,

@@ -54,6 +54,14 @@ template <int XF, int YF>
 int run_gemm_ragged(const GemmCall& c);
 template <int XF, int YF>
 int run_gemm_small(const GemmCall& c);
+// A product in parts of K: which tile, and how many parts (1: not split).
+struct KSplit {
+    bool small_tiles;
+    int parts;
+};
+// Both operands K-major; c.D is the float32 scratch of `parts` arrays that receives the parts' unscaled sums.
+template <int XF, int YF>
+int run_gemm_parts(const GemmCall& c, const KSplit& split);
 template <int XF, int YF>
 int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int NR, int NC, int K, const float* xs,
                    const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st);
@@ -89,12 +97,16 @@ extern template int run_gemm_pair<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&)
 extern template int run_gemm_pair<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_ragged<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&);
 extern template int run_gemm_small<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&);
+extern template int run_gemm_parts<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&, const KSplit&);
 extern template int run_gemm_ragged<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_small<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
+extern template int run_gemm_parts<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&, const KSplit&);
 extern template int run_gemm_ragged<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);
 extern template int run_gemm_small<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);
+extern template int run_gemm_parts<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&, const KSplit&);
 extern template int run_gemm_ragged<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_small<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
+extern template int run_gemm_parts<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&, const KSplit&);
 #define MSAMP_SPLIT_ARGS const uint8_t*, const uint8_t*, void*, int, int, int, int, const float*, const float*, int, const void*, int, hipStream_t
 extern template int run_gemm_split<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(MSAMP_SPLIT_ARGS);
 extern template int run_gemm_split<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(MSAMP_SPLIT_ARGS);

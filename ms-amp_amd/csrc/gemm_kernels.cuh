@@ -426,6 +426,23 @@ __device__ __forceinline__ v4f acc_quad(uint32_t token) {
     return r;
 }
 
+// A product in gridDim.y parts of K (both operands K-major, so that a part is only another pointer and another K): this
+// workgroup's part.  Its unscaled float32 sum goes to the y-th of gridDim.y arrays of NR x NC; ksplit_finish_kernel adds
+// them up.  Every part but the last is whole slices.
+template <typename OT, bool XT, bool YT>
+constexpr bool kTakesKParts = XT && YT && std::is_same<OT, float>::value;
+template <typename In, typename Out>
+__device__ __forceinline__ void k_part(In& X, In& Y, Out& D, int NR, int NC, int& K) {
+    if (gridDim.y == 1) return;
+    const int nk = (K + kBK - 1) / kBK, parts = gridDim.y, y = blockIdx.y;
+    const int first = static_cast<int>(static_cast<long long>(nk) * y / parts) * kBK;
+    const int end = y + 1 == parts ? K : static_cast<int>(static_cast<long long>(nk) * (y + 1) / parts) * kBK;
+    X += static_cast<size_t>(first) * NR;
+    Y += static_cast<size_t>(first) * NC;
+    D += static_cast<size_t>(y) * NR * NC;
+    K = end - first;
+}
+
 template <int XF, int YF, typename OT, bool XT = false, bool YT = false, int QF = 0, bool ODD_NK = false, bool QSPEC = false,
           bool KTAIL = false, bool SPLIT = false>
 __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_t* __restrict__ X,
@@ -436,6 +453,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                                                                      const void* __restrict__ bias, int bias_dt,
                                                                      QuantArgs qa) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    if constexpr (KTAIL && kTakesKParts<OT, XT, YT>) k_part(X, Y, D, NR, NC, K);
     const int tiles_r = (NR + kDmaTile - 1) / kDmaTile, tiles_c = (NC + kDmaTile - 1) / kDmaTile;
     bool by_columns = walk_by_columns(tiles_r, tiles_c, K);
     int tr, tc;
@@ -489,6 +507,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     const int wr = wave >> 1, wc = wave & 1;
     // the output factor is fetched now: left to the epilogue, the two scalar loads sit on its critical path
     float alpha_early = (*x_scale_inv) * (*y_scale_inv);
+    if constexpr (KTAIL && kTakesKParts<OT, XT, YT>) alpha_early = gridDim.y > 1 ? 1.0f : alpha_early;
     // and so are the bias values of two of this wave's 128 columns per lane (-0 without a bias: fma(x, y, -0) is x * y to
     // the bit, signed zeros included)
     float bias_early[2] = {-0.0f, -0.0f};
@@ -1197,7 +1216,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
 // code); ODD picks the one that fits K.
 template <int XF, int YF, typename OT, bool XT, bool YT, bool ODD, bool KTAIL = false, bool SPLIT = false>
 static int launch_gemm_dma_parity(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
-                                  const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
+                                  const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st, int parts = 1) {
     constexpr int smem = 2 * kDmaStage;
     static std::atomic<bool> configured{false};    // setting the attribute twice is harmless
     auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, 0, ODD, false, KTAIL, SPLIT>;
@@ -1209,7 +1228,7 @@ static int launch_gemm_dma_parity(const uint8_t* X, const uint8_t* Y, void* D, i
     const int tiles = ((NR + kDmaTile - 1) / kDmaTile) * ((NC + kDmaTile - 1) / kDmaTile);
     QuantArgs qa = {};
     qa.walk_plus_one = registered_walk(NR, NC, K, XT, YT) + 1;
-    hipLaunchKernelGGL(kern, dim3(tiles), dim3(kGemmThreads), smem, st, X, Y, static_cast<OT*>(D), NR, NC, K, xs, ys,
+    hipLaunchKernelGGL(kern, dim3(tiles, parts), dim3(kGemmThreads), smem, st, X, Y, static_cast<OT*>(D), NR, NC, K, xs, ys,
                        accumulate, bias, bias_dt, qa);
     MSAMP_CHECK_LAUNCH("fp8_gemm_dma_kernel");
     return MSAMP_OK;
@@ -1431,6 +1450,12 @@ int run_gemm_ragged(const GemmCall& c) {
 template <int XF, int YF>
 int run_gemm_small(const GemmCall& c) {
     MSAMP_TYPE_LAUNCH(launch_gemm_dma128)
+}
+template <int XF, int YF>
+int run_gemm_parts(const GemmCall& c, const KSplit& split) {
+    if (split.small_tiles)
+        return launch_gemm_dma128_tail<XF, YF, float, true, true, true>(c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, 0, nullptr, 0, c.st, split.parts);
+    return launch_gemm_dma_parity<XF, YF, float, true, true, false, true>(c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, 0, nullptr, 0, c.st, split.parts);
 }
 #endif
 

@@ -35,6 +35,7 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
                                             const float* __restrict__ y_scale_inv, int accumulate, const void* __restrict__ bias,
                                             int bias_dt) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    if constexpr (KTAIL && kTakesKParts<OT, XT, YT>) k_part(X, Y, D, NR, NC, K);
     const int tiles_r = (NR + kSmallTile - 1) / kSmallTile, tiles_c = (NC + kSmallTile - 1) / kSmallTile;
     int tr, tc;
     tile_of_id(blockIdx.x, tiles_r, tiles_c, false, false, tr, tc);
@@ -48,6 +49,7 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     const int seg = lane % kSegs;
     const int gcol = col0 + wc * 64 + seg * kElems;
     float alpha = (*x_scale_inv) * (*y_scale_inv);
+    if constexpr (KTAIL && kTakesKParts<OT, XT, YT>) alpha = gridDim.y > 1 ? 1.0f : alpha;
     float bv[kElems];
 #pragma unroll
     for (int e = 0; e < kElems; ++e) bv[e] = 0.0f;
@@ -323,7 +325,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_ragged128_kernel(const 
 
 template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL>
 static int launch_gemm_dma128_tail(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs, const float* ys,
-                              int accumulate, const void* bias, int bias_dt, hipStream_t st) {
+                              int accumulate, const void* bias, int bias_dt, hipStream_t st, int parts = 1) {
     constexpr int smem = kSmallStages * kSmallStage;
     static std::atomic<bool> configured{false};    // setting the attribute twice is harmless
     auto kern = KTAIL ? fp8_gemm_ragged128_kernel<XF, YF, OT, XT, YT> : fp8_gemm_dma128_kernel<XF, YF, OT, XT, YT>;
@@ -333,7 +335,7 @@ static int launch_gemm_dma128_tail(const uint8_t* X, const uint8_t* Y, void* D, 
         configured.store(true, std::memory_order_release);
     }
     const int tiles = ((NR + kSmallTile - 1) / kSmallTile) * ((NC + kSmallTile - 1) / kSmallTile);
-    hipLaunchKernelGGL(kern, dim3(tiles), dim3(kGemmThreads), smem, st, X, Y, static_cast<OT*>(D), NR, NC, K, xs, ys, accumulate,
+    hipLaunchKernelGGL(kern, dim3(tiles, parts), dim3(kGemmThreads), smem, st, X, Y, static_cast<OT*>(D), NR, NC, K, xs, ys, accumulate,
                        bias, bias_dt);
     MSAMP_CHECK_LAUNCH("fp8_gemm_dma128_kernel");
     return MSAMP_OK;

@@ -54,6 +54,8 @@ _SIGNATURES = {
     'msamp_cast_transpose_gated': ([_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp], _i),
     'msamp_fp8_gemm': ([_vp, _i, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp, _i, _vp], _i),
     'msamp_fp8_gemm_kmajor': ([_vp, _i, _vp, _i, _vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _i, _vp, _i, _vp], _i),
+    'msamp_fp8_gemm_ksplit_scratch': ([_i, _i, _i, _vp], _i),
+    'msamp_fp8_gemm_ksplit': ([_vp, _i, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp, _sz, _vp], _i),
     'msamp_fp8_gemm_cast': ([_vp, _i, _vp, _i, _vp, _i, _vp, _i, _vp, _i, _i, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp], _i),
     'msamp_mfma_probe': ([_vp, _vp, _i, _i, _i, _vp, _vp], _i),
     'msamp_set_small_tile_limit': ([_i], None),
@@ -616,6 +618,30 @@ def fp8_gemm(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, out, accumulate=False, 
         ), 'msamp_fp8_gemm'
     )
     return out
+
+
+def fp8_gemm_ksplit(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, out, accumulate=False):
+    """fp8_gemm(..., a_kmajor=True, b_kmajor=True) in parts of K that fill the device, for outputs of a few tiles: the same
+    float32 sum in another, fixed order.  False (and nothing done) where the product is better taken whole."""
+    lib = load()
+    k, m = a.shape
+    kb, n = b.shape
+    if kb != k or tuple(out.shape) != (n, m):
+        raise ValueError(f'shape mismatch: a {tuple(a.shape)}, b {tuple(b.shape)}, out {tuple(out.shape)}')
+    words = ctypes.c_size_t()
+    _check(lib.msamp_fp8_gemm_ksplit_scratch(m, n, k, ctypes.addressof(words)), 'msamp_fp8_gemm_ksplit_scratch')
+    if words.value == 0 or _ptr(out) % 16:
+        return False
+    _gpu(a, 'mat_a')
+    _gpu(b, 'mat_b')
+    scratch = torch.empty((words.value, ), dtype=torch.float32, device=a.device)
+    _check(
+        lib.msamp_fp8_gemm_ksplit(
+            _ptr(a), a_dt, _ptr(a_scale_inv), _ptr(b), b_dt, _ptr(b_scale_inv), _ptr(out), _dt(out), m, n, k,
+            1 if accumulate else 0, _ptr(scratch), words.value, _stream()
+        ), 'msamp_fp8_gemm_ksplit'
+    )
+    return True
 
 
 NOT_FUSED = 1

@@ -89,10 +89,12 @@ class Gemm:
                     out = torch.empty(N, M, dtype=out_dtype, device=mat_a.device)
                 else:
                     assert out.is_cuda and out.is_contiguous() and out.dtype == out_dtype
-                _backend.fp8_gemm(
+                operands = (
                     cls._aligned(mat_a.value), int(mat_a.qtype), mat_a.meta.scale_inv, cls._aligned(mat_b.value),
-                    int(mat_b.qtype), mat_b.meta.scale_inv, out, accumulate, bias, a_kmajor=a_kmajor, b_kmajor=b_kmajor
+                    int(mat_b.qtype), mat_b.meta.scale_inv, out, accumulate
                 )
+                if not (a_kmajor and b_kmajor and bias is None and _backend.fp8_gemm_ksplit(*operands)):
+                    _backend.fp8_gemm(*operands, bias, a_kmajor=a_kmajor, b_kmajor=b_kmajor)
                 return out
             if a_kmajor:
                 mat_a = mat_a.fp8_transpose()

@@ -222,6 +222,55 @@ def test_any_k_when_both_operands_are_kmajor(be, k):
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize('a_dt,b_dt', [(5, 6), (6, 5), (5, 5)])
+@pytest.mark.parametrize('m,n,k', [
+    (16, 48, 2600),         # less than a tile; parts of five and four slices, the last one ragged
+    (272, 336, 4097),       # one byte in the last slice, tiles that end one chunk into the next
+    (1024, 1024, 8192),     # whole tiles, whole slices
+    (1200, 4304, 12605),    # more small tiles than compute units: the large tile in parts
+    (128, 256, 16384),      # few tiles, many parts
+])
+@pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16, torch.float16])
+def test_weight_gradient_in_parts_of_k(be, a_dt, b_dt, m, n, k, out_dtype):
+    """A product taken in parts of K.  Operands of whole numbers up to 2: every product and every sum is a whole number below
+    2**24 (4 * K), exact in float32 in any order, so the result is the exact one rounded once, to the bit, and the same as of
+    the product taken whole; with accumulation as well.  What lies behind the operands is NaN codes."""
+    g = torch.Generator(device='cuda').manual_seed(m + n + k)
+
+    def operand(rows, dt):
+        values = torch.randint(-2, 3, (k, rows), device='cuda', generator=g)
+        codes = torch.tensor([{5: 0xC0, 6: 0xC0}[dt], {5: 0xB8, 6: 0xBC}[dt], 0, {5: 0x38, 6: 0x3C}[dt], 0x40], device='cuda',
+                             dtype=torch.uint8)
+        behind = torch.full((k * rows + 128 * rows, ), 0x7F, dtype=torch.uint8, device='cuda')
+        behind[:k * rows] = codes[values + 2].view(-1)
+        return behind[:k * rows].view(k, rows), values.double()
+
+    a, av = operand(m, a_dt)
+    b, bv = operand(n, b_dt)
+    sa, sb = torch.tensor(0.25, device='cuda'), torch.tensor(2.0, device='cuda')
+    exact = 0.5 * (bv.t().contiguous() @ av)
+    out = torch.empty(n, m, dtype=out_dtype, device='cuda')
+    assert be.fp8_gemm_ksplit(a, a_dt, sa, b, b_dt, sb, out) is True
+    assert torch.equal(out, exact.to(out_dtype))
+    whole = be.fp8_gemm(a, a_dt, sa, b, b_dt, sb, torch.empty_like(out), a_kmajor=True, b_kmajor=True)
+    assert torch.equal(out, whole)
+    base = torch.randint(-64, 65, (n, m), device='cuda', generator=g).to(out_dtype)
+    out = base.clone()
+    assert be.fp8_gemm_ksplit(a, a_dt, sa, b, b_dt, sb, out, accumulate=True) is True
+    assert torch.equal(out, (exact + base.double()).to(out_dtype))
+
+
+def test_weight_gradient_taken_whole(be):
+    """Outputs of many tiles, short K and an output that 16-byte accesses do not fit are left to the product as a whole."""
+    one = torch.ones((), device='cuda')
+    for m, n, k in [(4096, 4096, 4096), (256, 256, 512), (48, 16, 130), (24, 256, 8192)]:
+        a, b = torch.zeros(k, m, dtype=torch.uint8, device='cuda'), torch.zeros(k, n, dtype=torch.uint8, device='cuda')
+        assert be.fp8_gemm_ksplit(a, 5, one, b, 6, one, torch.empty(n, m, dtype=torch.bfloat16, device='cuda')) is False
+    a, b = torch.zeros(8192, 128, dtype=torch.uint8, device='cuda'), torch.zeros(8192, 128, dtype=torch.uint8, device='cuda')
+    out = torch.empty(128 * 128 + 1, dtype=torch.bfloat16, device='cuda')[1:].view(128, 128)
+    assert be.fp8_gemm_ksplit(a, 5, one, b, 6, one, out) is False
+
+
 def test_kmajor_rejects_unsupported_shapes(be):
     a = _rand_fp8((128, 100), 5, 1).cuda()    # [K=128, M=100]: M is not a multiple of 256
     b = _rand_fp8((64, 128), 5, 2).cuda()
