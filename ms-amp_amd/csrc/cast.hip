@@ -183,7 +183,9 @@ __global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restri
 // fixed order, and the sums of the slabs are added by colsum_finish_kernel, 16 runs of slabs at a time: the same bits on
 // every run, and no chain longer than a slab's quarter, a sixteenth of the slabs, or 16.
 // Slabs: about 2048 workgroups (eight a CU), so that the partial sums stay a hundredth of the tensor, and at least 16
-// rows.  12605 x 4304 float16: 26 us for the cast and 48 us for the sum (two clears and a reduction) before; FP8Linear
+// rows.  The workgroups' maxima go to memory and are folded into the amax by the second kernel: an atomic each, on a
+// cell that the window update has just cleared, held the cast of 8192 x 2048 bfloat16 at 40.8 us instead of 12.3.
+// 12605 x 4304 float16: 26 us for the cast and 48 us for the sum (two clears and a reduction) before; FP8Linear
 // 12605 x 1200 -> 4304 forward and backward 387 -> 339 us, a training step of two 2048-wide blocks at 8192 tokens
 // 2840 -> 2711 us.  Taken at every size: at 96 x 512 it is the same two launches less.
 constexpr int kColsumThreads = 256;
@@ -192,8 +194,9 @@ constexpr int kColsumRows = 16;
 template <typename IT, int FMT, bool VEC>
 __global__ __launch_bounds__(kColsumThreads) void cast_colsum_kernel(const IT* __restrict__ x, uint8_t* __restrict__ out,
                                                                      int rows, int cols, int rows_per_slab,
-                                                                     const float* __restrict__ scale_p, float* amax,
-                                                                     float* scale_inv, float* __restrict__ partial, int stream) {
+                                                                     const float* __restrict__ scale_p, float* scale_inv,
+                                                                     float* __restrict__ partial, float* __restrict__ tops,
+                                                                     int stream) {
     constexpr int EPT = In16<IT>::EPT;
     constexpr int W = kWave * EPT, NW = kColsumThreads / kWave, U = 4;
     static_assert(NW * U == kColsumRows, "one round of loads per kColsumRows rows");
@@ -269,17 +272,25 @@ __global__ __launch_bounds__(kColsumThreads) void cast_colsum_kernel(const IT* _
         }
     }
     if (threadIdx.x == 0) {
-        amax_publish(amax, __uint_as_float(m));
+        tops[static_cast<size_t>(blockIdx.y) * gridDim.x + blockIdx.x] = __uint_as_float(m);
         if (blockIdx.x == 0 && blockIdx.y == 0) *scale_inv = 1.0f / s;
     }
 }
 
-// adds the slabs' sums up, rounds to the input's type (as a sum in that type ends) and on to the type asked for
+// adds the slabs' sums up, rounds to the input's type (as a sum in that type ends) and on to the type asked for; workgroup 0
+// also folds the `n_tops` maxima of the cast's workgroups into *amax
 template <typename IT, typename OT>
 __global__ __launch_bounds__(1024) void colsum_finish_kernel(const float* __restrict__ partial, OT* __restrict__ sum, int slabs,
-                                                             int cols) {
+                                                             int cols, const float* __restrict__ tops, int n_tops, float* amax) {
     __shared__ float part[16][kWave];
+    __shared__ uint32_t red[16];
     const int lane = threadIdx.x & 63, run = threadIdx.x >> 6;
+    if (blockIdx.x == 0) {
+        float top = 0.0f;
+        for (int i = threadIdx.x; i < n_tops; i += 1024) top = fmaxf(top, tops[i]);
+        const uint32_t m = block_max_u32(__float_as_uint(top), red);
+        if (threadIdx.x == 0) amax_publish(amax, __uint_as_float(m));
+    }
     const int c = blockIdx.x * kWave + lane;
     float t = 0.0f;
     if (c < cols) {
@@ -1433,10 +1444,11 @@ static int launch_colsum(const IT* x, int dtype, int rows, int cols, const float
     int per = 0;
     const int slabs = colsum_slabs(rows, cols, dtype, &per);
     const dim3 grid((cols + kWave * EPT - 1) / (kWave * EPT), slabs);
+    float* tops = partial + static_cast<size_t>(slabs) * cols;
     const bool vec = cols % EPT == 0 && aligned(x, 16) && aligned(out, EPT);
     const int stream = static_cast<size_t>(rows) * cols * sizeof(IT) >= kStreamBytes;
 #define LAUNCH(FMT, VEC) \
-    hipLaunchKernelGGL((cast_colsum_kernel<IT, FMT, VEC>), grid, dim3(kColsumThreads), 0, st, x, out, rows, cols, per, scale, amax, scale_inv, partial, stream)
+    hipLaunchKernelGGL((cast_colsum_kernel<IT, FMT, VEC>), grid, dim3(kColsumThreads), 0, st, x, out, rows, cols, per, scale, scale_inv, partial, tops, stream)
     if (fp8_type == MSAMP_DT_E4M3) {
         if (vec) LAUNCH(MSAMP_DT_E4M3, true); else LAUNCH(MSAMP_DT_E4M3, false);
     } else {
@@ -1445,7 +1457,7 @@ static int launch_colsum(const IT* x, int dtype, int rows, int cols, const float
 #undef LAUNCH
     MSAMP_CHECK_LAUNCH("cast_colsum_kernel");
 #define FINISH(OT) \
-    hipLaunchKernelGGL((colsum_finish_kernel<IT, OT>), dim3((cols + kWave - 1) / kWave), dim3(1024), 0, st, static_cast<const float*>(partial), static_cast<OT*>(sum), slabs, cols)
+    hipLaunchKernelGGL((colsum_finish_kernel<IT, OT>), dim3((cols + kWave - 1) / kWave), dim3(1024), 0, st, static_cast<const float*>(partial), static_cast<OT*>(sum), slabs, cols, static_cast<const float*>(tops), static_cast<int>(grid.x * grid.y), amax)
     if (sum_dtype == MSAMP_DT_F32) FINISH(float);
     else if (sum_dtype == MSAMP_DT_F16) FINISH(f16_t);
     else FINISH(bf16_t);
@@ -1856,7 +1868,9 @@ int msamp_cast_colsum_scratch(int rows, int cols, int in_dtype, size_t* n_floats
     MSAMP_REQUIRE(rows > 0 && cols > 0, MSAMP_ERR_SHAPE, "msamp_cast_colsum_scratch: shape %d x %d", rows, cols);
     MSAMP_REQUIRE(n_floats != nullptr, MSAMP_ERR_NULL, "msamp_cast_colsum_scratch: null pointer");
     int per = 0;
-    *n_floats = static_cast<size_t>(colsum_slabs(rows, cols, in_dtype, &per)) * cols;
+    const int w = kWave * 16 / hp_size(in_dtype);
+    // (the sums of the slabs, and a maximum per workgroup)
+    *n_floats = static_cast<size_t>(colsum_slabs(rows, cols, in_dtype, &per)) * (static_cast<size_t>(cols) + (cols + w - 1) / w);
     return MSAMP_OK;
 }
 
