@@ -11,32 +11,49 @@ _KINDS = (1.0, 2.0, float('inf'))
 _PLAIN = (torch.float32, torch.float16, torch.bfloat16)
 
 
+def _entry(g):
+    """Descriptor of a gradient for the kernels that take a whole list at once, or None if it is not a contiguous FP8
+    ScalingTensor or plain tensor on the current GPU."""
+    if type(g) is ScalingTensor:
+        value, si = g.value, g.meta.scale_inv
+        if not Dtypes.is_fp8_qtype(g.qtype) or si.dtype != torch.float32 or si.numel() != 1 or si.device != value.device:
+            return None
+        dtype, si = int(g.qtype), si.data_ptr()
+    else:
+        value, si = g, 0
+        if type(g) not in (torch.Tensor, torch.nn.Parameter) or g.layout != torch.strided or g.dtype not in _PLAIN or \
+                g.requires_grad:
+            return None
+        dtype = _backend.hp_dt(g)
+    if value.numel() == 0 or not value.is_cuda or value.device.index != torch.cuda.current_device() or \
+            not value.is_contiguous():
+        return None
+    return value.data_ptr(), si, value.numel(), dtype
+
+
+def _rounds(entries):
+    """The entries in as few lists as it takes so that clipping those of one list writes no word twice (an FP8 gradient's
+    scale_inv, a plain one's values): what a launch scales at the same time must not overlap."""
+    rounds, ends = [], []
+    for lo, hi, e in sorted(((e[1], e[1] + 4, e) if e[1] else (e[0], e[0] + e[2] * (4 if e[3] == _backend.DT_F32 else 2), e)
+                             for e in entries)):
+        at = next((i for i, end in enumerate(ends) if end <= lo), len(ends))
+        if at == len(ends):
+            rounds.append([])
+            ends.append(hi)
+        ends[at] = hi
+        rounds[at].append(e)
+    return rounds
+
+
 def _table(grads, norm_type):
-    """Descriptors of the gradients for the kernels that take the whole list at once, or None if one of them is not a
-    contiguous FP8 ScalingTensor or plain tensor on the current GPU, or shares memory with another."""
+    """Descriptors of the gradients, or None if one of them has none or shares memory with another."""
     if norm_type not in _KINDS or not grads:
         return None
-    entries, seen, device = [], set(), None
-    for g in grads:
-        if type(g) is ScalingTensor:
-            value, si = g.value, g.meta.scale_inv
-            if not Dtypes.is_fp8_qtype(g.qtype) or si.dtype != torch.float32 or si.numel() != 1 or si.device != value.device:
-                return None
-            dtype, si, at = int(g.qtype), si.data_ptr(), si.data_ptr()
-        else:
-            value, si = g, 0
-            if type(g) not in (torch.Tensor, torch.nn.Parameter) or g.layout != torch.strided or g.dtype not in _PLAIN or \
-                    g.requires_grad:
-                return None
-            dtype, at = _backend.hp_dt(g), g.data_ptr()
-        if device is None:
-            device = value.device
-        n = value.numel()
-        if n == 0 or not value.is_cuda or value.device != device or not value.is_contiguous() or at in seen:
-            return None
-        seen.add(at)
-        entries.append((value.data_ptr(), si, n, dtype))
-    return _backend.grad_table(entries) if device.index == torch.cuda.current_device() else None
+    entries = [_entry(g) for g in grads]
+    if None in entries or len(_rounds(entries)) > 1:
+        return None
+    return _backend.grad_table(entries)
 
 
 def _compute_total_norm(grads, norm_type):

@@ -351,3 +351,19 @@ def test_clip_with_a_nan_and_with_a_shared_gradient():
     x = torch.full((4, ), 3.0, device='cuda')
     total = msamp.clip_grad_norm_([_Owner(x), _Owner(x)], 1.0)
     assert total.item() == pytest.approx(math.sqrt(72.0)) and torch.allclose(x, torch.full_like(x, 3.0 / 72.0))
+
+
+def test_clip_of_gradients_that_overlap():
+    """Views of one buffer that start at different places: an element that two of them hold is clipped twice, one gradient
+    after the other, as torch does it."""
+    import msamp
+    flat = torch.arange(1.0, 70001.0, device='cuda')
+    want = flat.clone()
+    views = [flat[:60000], flat[17:50017], flat[50020:], flat[60000:60003]]
+    wide = torch.cat(views).double()
+    total = msamp.clip_grad_norm_([_Owner(v) for v in views], 2.0)
+    assert total.item() == pytest.approx(wide.norm().item(), rel=1e-6)
+    coef = torch.clamp(2.0 / (total + 1e-6), max=1.0)
+    for v in (want[:60000], want[17:50017], want[50020:], want[60000:60003]):
+        v.mul_(coef)
+    assert torch.equal(flat, want)

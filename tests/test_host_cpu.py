@@ -5,6 +5,7 @@ import ctypes
 import itertools
 import json
 import os
+import random
 import re
 
 import pytest
@@ -340,6 +341,30 @@ def test_entry_points_refuse_bad_arguments_before_touching_a_gpu():
     assert lib.msamp_adamw_plain_fused(None, 3, None, 0, _backend.DT_F32, _backend.DT_F32, *hyper, 1, None) == -3
     assert lib.msamp_adamw_plain_fused(p, 3, None, 0, _backend.DT_E5M2, _backend.DT_F32, *hyper, 1, None) == -1
     assert lib.msamp_adamw_plain_fused(p, -1, None, 0, _backend.DT_F32, _backend.DT_F32, *hyper, 1, None) == -2
+
+
+def test_gradients_clipped_in_one_launch_share_no_memory():
+    """Gradients whose values (FP8: whose scale_inv) overlap anywhere, not only where they start, go to different launches;
+    no more launches than gradients lie over one byte, and each gradient in exactly one."""
+    from msamp.nn.clip_grad import _rounds
+    flat = 1 << 20
+    views = [(flat, 0, 6, _backend.DT_F32), (flat + 8, 0, 6, _backend.DT_F32), (flat + 24, 0, 2, _backend.DT_BF16)]
+    assert [len(r) for r in _rounds(views[:2])] == [1, 1] and len(_rounds([views[0], views[2]])) == 1
+    gen = random.Random(3)
+    for _ in range(200):
+        entries = []
+        for _ in range(gen.randint(1, 12)):
+            at, n = 2 * gen.randint(0, 60), gen.randint(1, 12)
+            entries.append((at, 0, n, gen.choice((_backend.DT_F32, _backend.DT_F16))) if gen.random() < 0.7 else
+                           (7, at + 4, n, _backend.DT_E4M3))
+        words = [set(range(si, si + 4)) if si else set(range(at, at + n * (4 if dt == _backend.DT_F32 else 2)))
+                 for at, si, n, dt in entries]
+        rounds = _rounds(entries)
+        assert sorted(e for r in rounds for e in r) == sorted(entries)
+        assert len(rounds) == max(sum(b in w for w in words) for b in set.union(*words))
+        for r in rounds:
+            spans = [words[entries.index(e)] for e in r]
+            assert sum(map(len, spans)) == len(set.union(*spans))
 
 
 def test_every_tile_walk_is_a_bijection(tmp_path):
