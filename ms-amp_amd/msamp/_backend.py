@@ -901,6 +901,11 @@ def adamw_fused(desc, n_tensors, block_map, n_blocks, weight_dt, grad_dt, lr, be
     )
 
 
+def dt_size(dt):
+    """Bytes of an element of a library type code."""
+    return 4 if dt == DT_F32 else 1 if dt in (DT_E4M3, DT_E5M2) else 2
+
+
 def hp_dt(tensor):
     """Library code of a float32 / float16 / bfloat16 tensor's element type."""
     return _dt(tensor)

@@ -35,7 +35,7 @@ def _rounds(entries):
     """The entries in as few lists as it takes so that clipping those of one list writes no word twice (an FP8 gradient's
     scale_inv, a plain one's values): what a launch scales at the same time must not overlap."""
     rounds, ends = [], []
-    for lo, hi, e in sorted(((e[1], e[1] + 4, e) if e[1] else (e[0], e[0] + e[2] * (4 if e[3] == _backend.DT_F32 else 2), e)
+    for lo, hi, e in sorted(((e[1], e[1] + 4, e) if e[1] else (e[0], e[0] + e[2] * _backend.dt_size(e[3]), e)
                              for e in entries)):
         at = next((i for i, end in enumerate(ends) if end <= lo), len(ends))
         if at == len(ends):

@@ -19,6 +19,25 @@ from msamp.optim.adamw_base import LBAdamWBase
 _FUSED_WEIGHT_QTYPES = (Dtypes.kfloat8_e4m3, Dtypes.kfloat8_e5m2, Dtypes.kfloat16)
 
 
+def _collide(spans):
+    """True if one of the (start, end, written) spans is written and another one overlaps it."""
+    end_any = end_written = 0
+    for start, end, written in sorted(spans):
+        if start < end_written or (written and start < end_any):
+            return True
+        end_any = max(end_any, end)
+        if written:
+            end_written = max(end_written, end)
+    return False
+
+
+def _storages(t):
+    """Spans of whatever memory a step of the tensor may touch: the storages of its payload and meta."""
+    tensors = (t.value, t.meta.scale, t.meta.scale_inv, t.meta.amax) if isinstance(t, ScalingTensor) else (t, )
+    storages = [x.untyped_storage() for x in tensors if x.layout == torch.strided]
+    return [(s.data_ptr(), s.data_ptr() + s.nbytes(), True) for s in storages]
+
+
 class _FusedPlan:
     """What one group of fusable parameters needs from step to step: the device tables of the fused kernels and, for
     the one-pass forms, where the payloads live."""
@@ -401,13 +420,17 @@ class LBAdamW(LBAdamWBase):
         kernels of the library; False where they do not apply (the chain below then runs as written).  Most parameters
         are put on a list for `_f32_flush`, which steps all of them at once; the others are stepped here."""
         moments = (exp_avg, exp_avg_sq)
-        if any(isinstance(t, ScalingTensor) or t.dtype != torch.float32 or not t.is_cuda or not t.is_contiguous()
-               for t in moments):
-            return False
-        row = self._f32_row(p, g, exp_avg, exp_avg_sq)
+        plain = all(not isinstance(t, ScalingTensor) and t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() for t in moments)
+        row = self._f32_row(p, g, exp_avg, exp_avg_sq) if plain else None
         if row is not None:
             self._f32_pending.append((step, row, p, g))
             return True
+        # stepped now, so what it shares memory with on the list comes first
+        if self._f32_pending and _collide([s for _, r, _, _ in self._f32_pending for s in self._f32_spans(r)] +
+                                          [s for t in (p, g) + moments for s in _storages(t)]):
+            self._f32_flush(beta1=beta1, beta2=beta2, lr=lr, weight_decay=weight_decay, eps=eps, maximize=maximize)
+        if not plain:
+            return False
         param = p.float()
         grad = g.float() if isinstance(g, ScalingTensor) or g.dtype not in self._PLAIN_DTYPES else g
         if not (param.is_cuda and grad.is_cuda) or any(t.numel() != param.numel() for t in (grad, ) + moments):
@@ -453,26 +476,40 @@ class LBAdamW(LBAdamWBase):
         return (value.data_ptr(), ) + meta_ptrs + (g_value.data_ptr(), g_si, exp_avg.data_ptr(), exp_avg_sq.data_ptr(), 0, n,
                                                    p_dt | g_dt << 32)
 
+    @staticmethod
+    def _f32_spans(row):
+        """(start, end, written) of the memory that a row stands for."""
+        param, scale, scale_inv, amax, grad, grad_si, exp_avg, exp_avg_sq, _, n, dts = row
+        spans = [(param, param + n * _backend.dt_size(dts & 0xffffffff), True), (exp_avg, exp_avg + 4 * n, True),
+                 (exp_avg_sq, exp_avg_sq + 4 * n, True), (grad, grad + n * _backend.dt_size(dts >> 32), False)]
+        if scale:
+            spans += [(scale, scale + 4, True), (scale_inv, scale_inv + 4, True), (amax, amax + 4, True)]
+        return spans + [(grad_si, grad_si + 4, False)] if grad_si else spans
+
     def _f32_flush(self, *, beta1, beta2, lr, weight_decay, eps, maximize):
         pending, self._f32_pending = self._f32_pending, []
-        by_step = {}
-        for step, row, p, g in pending:
-            group = by_step.setdefault(step, ([], [], set()))
-            if row[0] in group[2]:    # (a payload that is on the list already: its second step comes after the first)
-                self._f32_launch(step, group, beta1, beta2, lr, weight_decay, eps, maximize)
-                group = by_step[step] = ([], [], set())
-            group[0].append(row)
-            group[2].add(row[0])
-            if row[1]:
-                group[1].append(row[9])
-        for step, group in by_step.items():
-            self._f32_launch(step, group, beta1, beta2, lr, weight_decay, eps, maximize)
+        # parameters that share memory are stepped one after the other, as everywhere else: a launch holds none of them together
+        batches, spans = [pending], [self._f32_spans(row) for _, row, _, _ in pending]
+        if _collide([s for row_spans in spans for s in row_spans]):
+            batches, held = [], []
+            for entry, row_spans in zip(pending, spans):
+                if not batches or _collide(held + row_spans):
+                    batches.append([])
+                    held = []
+                batches[-1].append(entry)
+                held += row_spans
+        for batch in batches:
+            by_step = {}
+            for step, row, p, g in batch:
+                rows, scaled = by_step.setdefault(step, ([], []))
+                rows.append(row)
+                if row[1]:
+                    scaled.append(row[9])
+            for step, (rows, scaled) in by_step.items():
+                _backend.adamw_f32_list(rows, scaled, torch.device('cuda', torch.cuda.current_device()), lr, beta1, beta2, eps,
+                                        weight_decay, step, self.bias_correction, self.use_adam, maximize)
         written = [p.value if isinstance(p, ScalingTensor) else p for _, _, p, _ in pending]
         torch.autograd.graph.increment_version([t for t in written if t.dtype != torch.float32 and not t.is_inference()])
-
-    def _f32_launch(self, step, group, beta1, beta2, lr, weight_decay, eps, maximize):
-        _backend.adamw_f32_list(group[0], group[1], torch.device('cuda', torch.cuda.current_device()), lr, beta1, beta2, eps,
-                                weight_decay, step, self.bias_correction, self.use_adam, maximize)
 
     # ---- per-tensor path (reference recipe) -----------------------------------------------
     def _staged_step(self, idx, params, grads, exp_avgs, exp_avg_sqs, state_steps, *, beta1, beta2, lr, weight_decay,
@@ -558,6 +595,13 @@ class LBAdamW(LBAdamWBase):
             return
         # float32 moments: whole-tensor float32 update, then requantize the parameter if it is low-bit
         self._f32_pending = []
+        try:
+            self._f32_steps(params, grads, exp_avgs, exp_avg_sqs, state_steps, beta1=beta1, beta2=beta2, lr=lr,
+                            weight_decay=weight_decay, eps=eps, maximize=maximize)
+        finally:    # (also where one of them fails: those before it are stepped)
+            self._f32_flush(beta1=beta1, beta2=beta2, lr=lr, weight_decay=weight_decay, eps=eps, maximize=maximize)
+
+    def _f32_steps(self, params, grads, exp_avgs, exp_avg_sqs, state_steps, *, beta1, beta2, lr, weight_decay, eps, maximize):
         for i, p in enumerate(params):
             if self._f32_step(p, grads[i], exp_avgs[i], exp_avg_sqs[i], state_steps[i], beta1=beta1, beta2=beta2, lr=lr,
                               weight_decay=weight_decay, eps=eps, maximize=maximize):
@@ -580,4 +624,3 @@ class LBAdamW(LBAdamWBase):
                 p.copy_(param.cast(p.qtype, meta=p.meta))
             elif param.data_ptr() != p.data_ptr():
                 p.copy_(param)
-        self._f32_flush(beta1=beta1, beta2=beta2, lr=lr, weight_decay=weight_decay, eps=eps, maximize=maximize)

@@ -367,6 +367,19 @@ def test_gradients_clipped_in_one_launch_share_no_memory():
             assert sum(map(len, spans)) == len(set.union(*spans))
 
 
+def test_spans_that_collide():
+    """Spans of memory of which one is written and another overlaps it, against a look at every pair."""
+    from msamp.optim.adamw import _collide
+    gen = random.Random(8)
+    for _ in range(2000):
+        spans = []
+        for _ in range(gen.randint(1, 6)):
+            start = gen.randint(0, 30)
+            spans.append((start, start + gen.randint(1, 6), gen.random() < 0.5))
+        want = any((a[2] or b[2]) and a[0] < b[1] and b[0] < a[1] for a, b in itertools.combinations(spans, 2))
+        assert _collide(spans) == want, spans
+
+
 def test_every_tile_walk_is_a_bijection(tmp_path):
     """The function that maps a workgroup id to its output tile, taken as it stands in the kernel header and compiled for
     the host: for every grid of 1..140 x 1..140 tiles and each of the four walks (groups of rows or of columns, the
