@@ -129,6 +129,8 @@ __global__ __launch_bounds__(kAdamThreads) void stage2_kernel(const float* __res
 
 // ---- fused multi-tensor step -------------------------------------------------------------------
 constexpr int kEPT = 16;                                   // elements per thread per step
+// tensors of more chunks than these look at their maxima's words before they raise them (raise_max.cuh)
+constexpr size_t kAmaxLookChunks = 448, kSpecLookChunks = 384;
 constexpr int kSteps = MSAMP_ADAMW_CHUNK / (kAdamThreads * kEPT);    // 4
 
 template <int WDT>
@@ -286,13 +288,7 @@ __global__ __launch_bounds__(kAdamThreads) void fused_amax_kernel(msamp_adamw_te
     const uint32_t a = block_max_u32(mxp, red);
     const uint32_t b = block_max_u32(__float_as_uint(mxm), red);
     const uint32_t c = block_max_u32(__float_as_uint(mxv), red);
-    if (threadIdx.x == 0) {
-        // (this pass stores nothing: the words can be looked at now, the three loads together)
-        const uint32_t sa = seen_word(&d.acc[0]), sb = seen_word(&d.acc[1]), sc = seen_word(&d.acc[2]);
-        raise_max(&d.acc[0], a, sa);
-        raise_max(&d.acc[1], b, sb);
-        raise_max(&d.acc[2], c, sc);
-    }
+    if (threadIdx.x == 0) raise_max3(d.acc, a, b, c, n > kAmaxLookChunks * MSAMP_ADAMW_CHUNK);
 }
 
 __global__ void fused_scales_kernel(msamp_adamw_tensor* tensors, int n_tensors, float w_fp_max, int tensor_scale,
@@ -845,8 +841,7 @@ __global__ __launch_bounds__(kAdamThreads) void fused_spec_kernel(msamp_adamw_te
     const float inv_m = 1.0f / ms, inv_v = 1.0f / vs;
     uint32_t mxp = 0;
     float mxm = 0.0f, mxv = 0.0f;
-    const uint32_t seen_p = seen_word(&d.acc[0]), seen_m = seen_word(&d.acc[1]), seen_v = seen_word(&d.acc[2]);
-    float floor_p = __uint_as_float(seen_p);
+    float floor_p = __uint_as_float(seen_word(&d.acc[0]));
     if (!(floor_p >= 0.0f)) floor_p = 0.0f;
     if (base + MSAMP_ADAMW_CHUNK <= n) {
         // the folded, clamp-free form of the step where the tensor's factors allow it (see spec_group)
@@ -894,11 +889,7 @@ __global__ __launch_bounds__(kAdamThreads) void fused_spec_kernel(msamp_adamw_te
     const uint32_t a = block_max_u32(mxp, red);
     const uint32_t b = block_max_u32(__float_as_uint(mxm), red);
     const uint32_t c = block_max_u32(__float_as_uint(mxv), red);
-    if (threadIdx.x == 0) {
-        raise_max(&d.acc[0], a, seen_p);
-        raise_max(&d.acc[1], b, seen_m);
-        raise_max(&d.acc[2], c, seen_v);
-    }
+    if (threadIdx.x == 0) raise_max3(d.acc, a, b, c, n > kSpecLookChunks * MSAMP_ADAMW_CHUNK);
 }
 
 // ---- the one-pass step inside shifting arenas -------------------------------------------------------------
@@ -1442,7 +1433,6 @@ __global__ __launch_bounds__(kAdamThreads) void plain_amax_kernel(msamp_adamw_te
     PT* param = static_cast<PT*>(d.weight);
     const GT* grad = reinterpret_cast<const GT*>(d.grad);
     const float inv_m = 1.0f / *d.m_scale, inv_v = 1.0f / *d.v_scale;
-    const uint32_t seen_m = seen_word(&d.acc[1]), seen_v = seen_word(&d.acc[2]);
     float mxm = 0.0f, mxv = 0.0f;
     for (size_t i = first + threadIdx.x * 4; i < last; i += kAdamThreads * 4) {
         if (i + 4 <= last) {
@@ -1468,8 +1458,8 @@ __global__ __launch_bounds__(kAdamThreads) void plain_amax_kernel(msamp_adamw_te
     const uint32_t a = block_max_u32(__float_as_uint(mxm), red);
     const uint32_t b = block_max_u32(__float_as_uint(mxv), red);
     if (threadIdx.x == 0) {
-        raise_max(&d.acc[1], a, seen_m);
-        raise_max(&d.acc[2], b, seen_v);
+        raise_max(&d.acc[1], a);
+        raise_max(&d.acc[2], b);
     }
 }
 

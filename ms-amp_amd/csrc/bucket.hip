@@ -26,7 +26,6 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_amax_kernel(msamp_bucke
     const IT* x = static_cast<const IT*>(d.src);
     const size_t n = d.numel, base = static_cast<size_t>(chunk) * MSAMP_BUCKET_CHUNK;
     uint32_t m = 0;
-    const uint32_t seen = seen_word(&d.acc);
     uint8_t* out = d.dst;
     const float s = FMT != 0 ? *d.scale : 1.0f;
     const bool vec_out = FMT == 0 || (reinterpret_cast<uintptr_t>(out) & (EPT - 1)) == 0;
@@ -64,7 +63,7 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_amax_kernel(msamp_bucke
         }
     }
     m = block_max_u32(m, red);
-    if (threadIdx.x == 0) raise_max(&d.acc, m, seen);
+    if (threadIdx.x == 0) raise_max(&d.acc, m);
 }
 
 // amax[0] of every tensor from the accumulated pattern (NaN and +Inf become +Inf when asked: the all-reduce that

@@ -216,6 +216,25 @@ def test_fused_step_sparse_gradient_and_zero_state(be):
         _check(dev[0], t, fp8.E4M3, fp8.E5M2, step, **kw)
 
 
+@pytest.mark.parametrize('chunks', [384, 448])
+def test_maxima_of_tensors_around_the_looking_lines(be, chunks):
+    """Tensors of as many chunks as the first passes raise their maxima without a look at the words for, and one element
+    more: repetitions of a small tensor, so every one of them has the small one's maxima, scales and codes, in place and in
+    one pass."""
+    base = _inputs(2 * 16384, 61, fp8.E4M3, fp8.E5M2)
+    tensors = [base]
+    for n in (chunks * 16384, chunks * 16384 + 1):
+        tensors.append({k: v.repeat(-(-n // v.numel()))[:n] if isinstance(v, torch.Tensor) else v for k, v in base.items()})
+    for kw in (dict(), dict(speculative=True)):
+        first, *rest = _fused(be, tensors, 5, 6, 2, **kw)
+        _check(first, base, fp8.E4M3, fp8.E5M2, 2)
+        for d in rest:
+            n = d['w'].numel()
+            for k in ('w', 'm', 'v'):
+                assert torch.equal(d[k], first[k].repeat(-(-n // first[k].numel()))[:n]), (n, k)
+            assert all(same_float(x, y) for k in ('wm', 'mm', 'vm') for x, y in zip(d[k], first[k])), n
+
+
 def _same_state(a, b):
     bits = lambda t: t.view(torch.int32) if t.dtype == torch.float32 else (t.view(torch.int16) if t.dtype == torch.float16 else t)
     return all(torch.equal(bits(x), bits(y)) for x, y in zip([a['w'], a['m'], a['v']] + a['wm'] + a['mm'] + a['vm'],
