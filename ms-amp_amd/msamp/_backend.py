@@ -665,12 +665,12 @@ def fp8_gemm_cast(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, hp_dtype, q_dt, sc
         raise ValueError(f'shape mismatch: a {tuple(a.shape)}, b {tuple(b.shape)}')
     if hp_dtype not in _TORCH_TO_DT:
         raise TypeError(f'unsupported intermediate dtype {hp_dtype}')
-    if m % 256 or n % 256 or k % 128:
-        return None    # (as the library would answer, before anything is allocated for it)
     if accumulate and hp_out is None:
         raise ValueError('accumulate needs hp_out')
     if hp_out is not None and (hp_out.dtype != hp_dtype or tuple(hp_out.shape) != (n, m) or not hp_out.is_contiguous()):
         raise ValueError(f'hp_out must be a contiguous {hp_dtype} tensor of shape {(n, m)}')
+    if (m % 256 or n % 256 or k % 128) and min(m, n, k) > 0 and all(dt in (DT_E4M3, DT_E5M2) for dt in (a_dt, b_dt, q_dt)):
+        return None    # (as the library would answer, before anything is allocated for it)
     if hp_out is None and speculate and m % 256 == 0 and n % 256 == 0 and (n // 256) * (m // 256) > 0:
         hp_out = torch.empty(n, m, dtype=hp_dtype, device=a.device)
     if _tune_walks and (a_kmajor or not b_kmajor):

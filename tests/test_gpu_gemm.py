@@ -271,6 +271,21 @@ def test_weight_gradient_taken_whole(be):
     assert be.fp8_gemm_ksplit(a, 5, one, b, 6, one, out) is False
 
 
+def test_gemm_cast_refuses_bad_arguments_for_every_shape(be):
+    """Also for a problem that neither fused form takes (100 x 64 x 128)."""
+    a, b = _rand_fp8((100, 128), 5, 1).cuda(), _rand_fp8((64, 128), 5, 2).cuda()
+    one = torch.ones((), device='cuda')
+    s, si, am = torch.ones((), device='cuda'), torch.ones((), device='cuda'), torch.zeros(1, device='cuda')
+    call = lambda hp=torch.bfloat16, q_dt=5, **kw: be.fp8_gemm_cast(a, 5, one, b, 5, one, hp, q_dt, s, am, si, **kw)
+    assert call() is None
+    with pytest.raises(ValueError):
+        call(accumulate=True)
+    with pytest.raises(ValueError):
+        call(hp_out=torch.empty(64, 99, dtype=torch.bfloat16, device='cuda'))
+    with pytest.raises(RuntimeError):
+        call(q_dt=3)
+
+
 def test_kmajor_rejects_unsupported_shapes(be):
     a = _rand_fp8((128, 100), 5, 1).cuda()    # [K=128, M=100]: M is not a multiple of 256
     b = _rand_fp8((64, 128), 5, 2).cuda()
