@@ -820,9 +820,10 @@ def grad_table(entries):
     return (ctypes.c_longlong * len(flat))(*flat)
 
 
-def grad_norms(table, n, norm_type, max_norm, device):
-    """(per-tensor norms, total norm, clipping factor) of the table's tensors, all on the GPU."""
+def grad_norms(table, n, norm_type, max_norm):
+    """(per-tensor norms, total norm, clipping factor) of the table's tensors, all on the current GPU."""
     kind = {1.0: 1, 2.0: 2, float('inf'): 0}[float(norm_type)]
+    device = torch.device('cuda', torch.cuda.current_device())
     norms = torch.empty(n + 1, dtype=torch.float32, device=device)    # the factor is the last word
     total = torch.empty((), dtype=torch.float32, device=device)
     partials = torch.empty(n + GRAD_BLOCKS, dtype=torch.float64, device=device)
@@ -835,6 +836,7 @@ def grad_norms(table, n, norm_type, max_norm, device):
 
 def grad_clip(table, n, factor):
     """Multiplies the table's tensors (FP8 ones through their scale_inv) by factor where that is below 1."""
+    factor = factor.to(torch.device('cuda', torch.cuda.current_device()))    # (the total may be on another GPU, as its first gradient)
     _check(load().msamp_grad_clip(table, n, _ptr(factor), _stream()), 'msamp_grad_clip')
 
 

@@ -46,22 +46,12 @@ def _rounds(entries):
     return rounds
 
 
-def _table(grads, norm_type):
-    """Descriptors of the gradients, or None if one of them has none or shares memory with another."""
-    if norm_type not in _KINDS or not grads:
-        return None
-    entries = [_entry(g) for g in grads]
-    if None in entries or len(_rounds(entries)) > 1:
-        return None
-    return _backend.grad_table(entries)
+def _norm(g, norm_type):
+    g32 = g.to(torch.float32).detach()
+    return g32.abs().max() if norm_type == float('inf') else torch.norm(g32, norm_type)
 
 
-def _compute_total_norm(grads, norm_type):
-    device = grads[0].device
-    norms = []
-    for g in grads:
-        g32 = g.to(torch.float32).detach()
-        norms.append((g32.abs().max() if norm_type == float('inf') else torch.norm(g32, norm_type)).to(device))
+def _join(norms, norm_type):
     if norm_type == float('inf'):
         return norms[0] if len(norms) == 1 else torch.max(torch.stack(norms))
     return torch.norm(torch.stack(norms), norm_type)
@@ -76,26 +66,36 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
         parameters = list(parameters)
     grads = [p.grad for p in parameters if p.grad is not None]
     norm_type, max_norm = float(norm_type), float(max_norm)
-    table = _table(grads, norm_type)
-    if table is not None:
+    # contiguous FP8 and plain gradients on this GPU go through the kernels that take them all at once, the others one by one
+    entries = [_entry(g) if norm_type in _KINDS else None for g in grads]
+    listed = [e for e in entries if e is not None]
+    total_norm = torch.tensor(0.)
+    if listed:
         # norms, factor and clipping without the host waiting for any of them
-        _, total_norm, factor = _backend.grad_norms(table, len(grads), norm_type, max_norm, grads[0].device)
-    else:
-        total_norm = _compute_total_norm(grads, norm_type) if grads else torch.tensor(0.)
+        norms, total_norm, coef = _backend.grad_norms(_backend.grad_table(listed), len(listed), norm_type, max_norm)
+    if len(listed) < len(grads):
+        listed_norms = iter(norms.unbind()) if listed else None
+        total_norm = _join([(_norm(g, norm_type) if e is None else next(listed_norms)).to(grads[0].device)
+                            for g, e in zip(grads, entries)], norm_type)
     if error_if_nonfinite and torch.logical_or(total_norm.isnan(), total_norm.isinf()):
         raise RuntimeError(
             f'The total norm of order {norm_type} for gradients from `parameters` is non-finite, so it cannot be '
             'clipped. To disable this error and scale the gradients by the non-finite norm anyway, set '
             '`error_if_nonfinite=False`'
         )
-    if max_norm > 0 and table is not None:
-        _backend.grad_clip(table, len(grads), factor)
-        # (what autograd saved of them, if anything, has changed)
-        changed = [g.meta.scale_inv if type(g) is ScalingTensor else g for g in grads]
-        torch.autograd.graph.increment_version([t for t in changed if not t.is_inference()])
-    elif max_norm > 0:
+    if not max_norm > 0 or not grads:
+        return total_norm
+    if len(listed) < len(grads):
         coef = torch.clamp(max_norm / (total_norm + 1e-6), max=1.0)
-        if coef.item() < 1.0:
-            for g in grads:
+        if not coef.item() < 1.0:
+            return total_norm
+        for g, e in zip(grads, entries):
+            if e is None:
                 g.detach().mul_(coef)
+    if listed:
+        for part in _rounds(listed):
+            _backend.grad_clip(_backend.grad_table(part), len(part), coef)
+        # (what autograd saved of them, if anything, has changed)
+        changed = [g.meta.scale_inv if type(g) is ScalingTensor else g for g, e in zip(grads, entries) if e is not None]
+        torch.autograd.graph.increment_version([t for t in changed if not t.is_inference()])
     return total_norm

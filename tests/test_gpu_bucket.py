@@ -367,3 +367,45 @@ def test_clip_of_gradients_that_overlap():
     for v in (want[:60000], want[17:50017], want[50020:], want[60000:60003]):
         v.mul_(coef)
     assert torch.equal(flat, want)
+
+
+@pytest.mark.parametrize('norm_type,odd', [(n, o) for n in (1.0, 2.0, float('inf'), 3.0)
+                                           for o in ('channels-last', 'float64', 'scaled float16', 'empty')
+                                           if (n, o) != (float('inf'), 'empty')])    # (torch has no maximum of nothing)
+def test_clip_of_a_list_with_one_gradient_the_kernels_do_not_take(monkeypatch, norm_type, odd):
+    """The others still go through the kernels (FP8 ones are not expanded to float32), with one total over all of them, and
+    every gradient is multiplied by its factor: bit for bit what torch makes of it."""
+    import msamp
+    from msamp import _backend
+    from msamp.common.dtype import Dtypes
+    from msamp.common.tensor import ScalingTensor
+    grads = _clip_case(6)
+    x = torch.randn(3, 5, 4, 6, device='cuda', generator=torch.Generator(device='cuda').manual_seed(1))
+    extra = {'channels-last': x.to(memory_format=torch.channels_last), 'float64': x.double(), 'empty': x[:0],
+             'scaled float16': x.cast(Dtypes.kfloat16)}[odd]
+    grads.insert(2, extra)
+    grads.append(grads[4])    # an FP8 gradient of two parameters
+    assert isinstance(grads[4], ScalingTensor)
+    taken = []
+    norms = _backend.grad_norms
+    monkeypatch.setattr(_backend, 'grad_norms', lambda table, n, *a: (taken.append(n), norms(table, n, *a))[1])
+    wide = torch.cat([g.float().double().flatten() for g in grads])
+    want = wide.abs().max().item() if norm_type == float('inf') else wide.abs().pow(norm_type).sum().pow(1 / norm_type).item()
+    before = [g.float().clone() for g in grads]
+    values = [g.value.clone() if isinstance(g, ScalingTensor) else g.clone() for g in grads]
+    scales = [g.meta.scale_inv.clone() if isinstance(g, ScalingTensor) else None for g in grads]
+    # (torch's float32 sums, of at most 300001 terms: some 19 levels of 2**-24 and the powers' few)
+    close = pytest.approx(want, rel=30 * 2.0**-24)
+    assert msamp.clip_grad_norm_([_Owner(g) for g in grads], 2 * want, norm_type=norm_type).item() == close
+    assert all(torch.equal(g.float(), b) for g, b in zip(grads, before))
+    total = msamp.clip_grad_norm_([_Owner(g) for g in grads], want / 3, norm_type=norm_type)
+    assert taken == ([] if norm_type == 3.0 else [len(grads) - 1] * 2)
+    coef = torch.clamp((want / 3) / (total + 1e-6), max=1.0)
+    for i, (g, v, si) in enumerate(zip(grads, values, scales)):
+        if si is not None:
+            times = 2 if g is grads[-1] else 1
+            for _ in range(times):
+                si = si * coef
+            assert torch.equal(g.meta.scale_inv, si) and torch.equal(g.value, v), i
+        else:
+            assert torch.equal(g, v.mul_(coef)), i
