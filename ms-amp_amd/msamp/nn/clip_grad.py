@@ -57,6 +57,16 @@ def _join(norms, norm_type):
     return torch.norm(torch.stack(norms), norm_type)
 
 
+def _held_elsewhere(p):
+    """True if a graph may have saved the gradient of p: something holds it beside its owner and Python, or holds a view of it."""
+    g = p.grad
+    if type(g) is ScalingTensor:
+        return g.meta.scale_inv._use_count() > 1
+    # (the storage: the gradient, and the handle it is asked through)
+    return g._use_count() > (2 if isinstance(p, torch.Tensor) else 1) or \
+        torch._C._storage_Use_Count(g.untyped_storage()._cdata) > 2
+
+
 def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=False):
     """Clip the global gradient norm in place and return it.  ScalingTensor gradients are dequantized
     for the norm and clipped by scaling their scale_inv (no pass over the payload)."""
@@ -64,7 +74,8 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
         parameters = [parameters]
     else:
         parameters = list(parameters)
-    grads = [p.grad for p in parameters if p.grad is not None]
+    parameters = [p for p in parameters if p.grad is not None]
+    grads = [p.grad for p in parameters]
     norm_type, max_norm = float(norm_type), float(max_norm)
     # contiguous FP8 and plain gradients on this GPU go through the kernels that take them all at once, the others one by one
     entries = [_entry(g) if norm_type in _KINDS else None for g in grads]
@@ -92,10 +103,13 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
         for g, e in zip(grads, entries):
             if e is None:
                 g.detach().mul_(coef)
+    elif max_norm == float('inf') or (any(map(_held_elsewhere, parameters)) and
+                                      not torch.cuda.is_current_stream_capturing() and not coef.item() < 1.0):
+        # nothing to clip; what a graph has saved must then not count as changed, so the host waits to know, but only for those
+        return total_norm
     if listed:
         for part in _rounds(listed):
             _backend.grad_clip(_backend.grad_table(part), len(part), coef)
-        # (what autograd saved of them, if anything, has changed)
         changed = [g.meta.scale_inv if type(g) is ScalingTensor else g for g, e in zip(grads, entries) if e is not None]
         torch.autograd.graph.increment_version([t for t in changed if not t.is_inference()])
     return total_norm

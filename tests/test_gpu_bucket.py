@@ -409,3 +409,38 @@ def test_clip_of_a_list_with_one_gradient_the_kernels_do_not_take(monkeypatch, n
             assert torch.equal(g.meta.scale_inv, si) and torch.equal(g.value, v), i
         else:
             assert torch.equal(g, v.mul_(coef)), i
+
+
+@pytest.mark.parametrize('saved', ['gradient', 'view', 'detached', 'scale_inv'])
+@pytest.mark.parametrize('owner', ['parameter', 'other'])
+def test_clip_counts_as_a_change_only_where_it_clips(saved, owner):
+    """A graph that saved a gradient (a view of it, the scale_inv of an FP8 one) can be run backward after a clip that had
+    nothing to clip, and is refused after one that had.  No gradient is held so in a plain training step, which then does not
+    wait for the factor."""
+    import msamp
+    from msamp.common.dtype import Dtypes
+    for clips in (False, True):
+        model = torch.nn.Linear(16, 8).cuda()
+        model(torch.ones(4, 16, device='cuda')).sum().backward()
+        owners = list(model.parameters()) + [_Owner(torch.ones(20, device='cuda').cast(Dtypes.kfloat8_e4m3))]
+        if owner == 'other':
+            owners = [_Owner(p.grad.clone()) for p in owners[:2]] + owners[2:]
+        torch.cuda.set_sync_debug_mode('error')
+        try:
+            msamp.clip_grad_norm_(owners, 1e9)
+            msamp.clip_grad_norm_(owners, float('inf'))
+        finally:
+            torch.cuda.set_sync_debug_mode('default')
+        g = owners[0].grad
+        keep = {'gradient': g, 'view': g[2:5], 'detached': g.detach(), 'scale_inv': owners[2].grad.meta.scale_inv}[saved]
+        w = torch.ones_like(keep, requires_grad=True)
+        loss = (w * keep).sum()
+        want = keep.clone()
+        del g, keep
+        msamp.clip_grad_norm_(owners, 1e-3 if clips else 1e9)
+        if clips:
+            with pytest.raises(RuntimeError, match='inplace operation'):
+                loss.backward()
+        else:
+            loss.backward()
+            assert torch.equal(w.grad, want)
