@@ -185,73 +185,6 @@ __device__ __forceinline__ void fp8_norm_chunk(const uint8_t* q, size_t base, si
     }
 }
 
-// A workgroup takes a run of `run` consecutive chunks of the block map and adds to a tensor's accumulator once per tensor
-// it meets: additions to one address are served one at a time (about 12 ns each), and with one per chunk the 1 024
-// chunks of a 16.8 M-element tensor queued for longer (12 us) than their 16 MB take to read.
-template <int FMT, int KIND>    // KIND: 1, 2, or 0 for the maximum
-__global__ __launch_bounds__(kBucketThreads) void fp8_norm_kernel(msamp_norm_item* __restrict__ items,
-                                                                   const int32_t* __restrict__ block_map, int n_blocks, int run) {
-    __shared__ double red[kBucketThreads / kWave];
-    double acc = 0.0;
-    // the workgroup's total (maximum) -- lanes, then wavefronts -- into tensor t's accumulator
-    auto flush = [&](int t) {
-#pragma unroll
-        for (int o = 32; o; o >>= 1) {
-            const double other = __shfl_xor(acc, o);
-            if constexpr (KIND == 0) {
-                acc = (other != other || acc != acc) ? (other != other ? other : acc) : (other > acc ? other : acc);
-            } else {
-                acc += other;
-            }
-        }
-        __syncthreads();    // (the words below may still be read for the tensor before)
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            msamp_norm_item& d = items[t];
-            double total = red[0];
-            for (int w = 1; w < kBucketThreads / kWave; ++w) {
-                if constexpr (KIND == 0) {
-                    total = (red[w] != red[w] || total != total) ? (red[w] != red[w] ? red[w] : total) : (red[w] > total ? red[w] : total);
-                } else {
-                    total += red[w];
-                }
-            }
-            if constexpr (KIND == 0) {
-                // bit patterns of non-negative doubles order like the values, NaN patterns above all of them
-                atomicMax(reinterpret_cast<unsigned long long*>(&d.acc), static_cast<unsigned long long>(__double_as_longlong(total)));
-            } else {
-                atomicAdd(&d.acc, total);
-            }
-        }
-        acc = 0.0;
-    };
-    const int first = blockIdx.x * run, last = first + run < n_blocks ? first + run : n_blocks;
-    int current = block_map[2 * first];
-    for (int e = first; e < last; ++e) {
-        const int t = block_map[2 * e], chunk = block_map[2 * e + 1];
-        if (t != current) {
-            flush(current);
-            current = t;
-        }
-        const uint8_t* q = items[t].q;
-        const size_t n = items[t].numel, base = static_cast<size_t>(chunk) * MSAMP_BUCKET_CHUNK;
-        fp8_norm_chunk<FMT, KIND>(q, base, n, acc);
-    }
-    flush(current);
-}
-
-// out[i] = |scale_inv| * acc^(1/p) (the maximum itself for KIND 0), rounded to float once; the accumulator goes back to zero
-__global__ void fp8_norm_finish_kernel(msamp_norm_item* items, int n_items, int kind) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n_items) return;
-    msamp_norm_item& d = items[t];
-    const double acc = d.acc;
-    d.acc = 0.0;
-    const double root = kind == 2 ? sqrt(acc) : acc;
-    *d.out = static_cast<float>(fabs(static_cast<double>(*d.scale_inv)) * root);
-}
-
 // ---- clipping a list of gradients (clip_grad_norm_) ----------------------------------------------------------------
 // The norms of all gradients of a model, whatever their types (FP8 codes with a scale_inv, or plain float32 / 16-bit
 // tensors), their total and the clipping factor in two launches per 64 tensors, and the clipping itself in one, which
@@ -544,37 +477,6 @@ int msamp_bucket_cast(msamp_bucket_item* items, int n_items, const int32_t* bloc
     else BUCKET_CAST(bf16_t);
 #undef BUCKET_CAST
     MSAMP_CHECK_LAUNCH("bucket_cast_kernel");
-    return MSAMP_OK;
-}
-
-int msamp_fp8_norms(msamp_norm_item* items, int n_items, const int32_t* block_map, int n_blocks, int fp8_type, int norm_kind,
-                    msamp_stream_t stream) {
-    MSAMP_REQUIRE(n_items >= 0 && n_blocks >= 0, MSAMP_ERR_SHAPE, "msamp_fp8_norms: n_items=%d n_blocks=%d", n_items, n_blocks);
-    MSAMP_REQUIRE(is_fp8(fp8_type), MSAMP_ERR_DTYPE, "msamp_fp8_norms: fp8_type %d", fp8_type);
-    MSAMP_REQUIRE(norm_kind >= 0 && norm_kind <= 2, MSAMP_ERR_SHAPE, "msamp_fp8_norms: norm_kind %d (1, 2, or 0 for the maximum)",
-                  norm_kind);
-    if (n_items == 0) return MSAMP_OK;
-    MSAMP_REQUIRE(items != nullptr && (n_blocks == 0 || block_map != nullptr), MSAMP_ERR_NULL, "msamp_fp8_norms: null pointer");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (n_blocks > 0) {
-        // eight workgroups per compute unit keep enough loads in flight; beyond that longer runs instead of more workgroups
-        const int run = std::max(1, n_blocks / (cu_count() * 8));
-        const int grid = (n_blocks + run - 1) / run;
-#define NORM_LAUNCH(FMT)                                                                                                \
-    do {                                                                                                              \
-        if (norm_kind == 0)                                                                                           \
-            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 0>), dim3(grid), dim3(kBucketThreads), 0, st, items, block_map, n_blocks, run); \
-        else if (norm_kind == 1)                                                                                      \
-            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 1>), dim3(grid), dim3(kBucketThreads), 0, st, items, block_map, n_blocks, run); \
-        else                                                                                                          \
-            hipLaunchKernelGGL((fp8_norm_kernel<FMT, 2>), dim3(grid), dim3(kBucketThreads), 0, st, items, block_map, n_blocks, run); \
-    } while (0)
-        if (fp8_type == MSAMP_DT_E4M3) NORM_LAUNCH(MSAMP_DT_E4M3); else NORM_LAUNCH(MSAMP_DT_E5M2);
-#undef NORM_LAUNCH
-        MSAMP_CHECK_LAUNCH("fp8_norm_kernel");
-    }
-    hipLaunchKernelGGL(fp8_norm_finish_kernel, dim3((n_items + 63) / 64), dim3(64), 0, st, items, n_items, norm_kind);
-    MSAMP_CHECK_LAUNCH("fp8_norm_finish_kernel");
     return MSAMP_OK;
 }
 

@@ -62,7 +62,6 @@ _SIGNATURES = {
     'msamp_scale_update_groups': ([_vp, _i, _i, _vp], _i),
     'msamp_grad_norms': ([_vp, _i, _i, _f, _vp, _vp, _vp, _vp, _vp], _i),
     'msamp_grad_clip': ([_vp, _i, _vp, _vp], _i),
-    'msamp_fp8_norms': ([_vp, _i, _vp, _i, _i, _i, _vp], _i),
     'msamp_bucket_amax': ([_vp, _i, _vp, _i, _i, _i, _vp], _i),
     'msamp_bucket_amax_speculative': ([_vp, _i, _vp, _i, _i, _i, _i, _vp], _i),
     'msamp_bucket_cast': ([_vp, _i, _vp, _i, _i, _i, _f, _f, _i, _vp], _i),
@@ -775,42 +774,6 @@ def bucket_cast(items, block_map, in_dt, fp8_dt, pre_scale, scale_inv_div=1.0, m
     )
 
 
-NORM_ITEM_WORDS = 5    # int64 words per msamp_norm_item (40 bytes)
-
-
-_NORM_TABLES = {}
-
-
-def fp8_norms(values, scale_invs, fp8_dt, norm_type):
-    """Per-tensor p-norms (p = 1, 2 or inf) of FP8 payloads times their scale_inv, as one float32 vector.  The
-    descriptor table is kept per set of payload and scale_inv addresses (a training loop asks for the same gradients'
-    norms every step), the result is a fresh tensor every time."""
-    import numpy as np
-    kind = {1.0: 1, 2.0: 2, float('inf'): 0}[float(norm_type)]
-    lib = load()
-    sig = (tuple(v.data_ptr() for v in values), tuple(si.data_ptr() for si in scale_invs), tuple(v.numel() for v in values))
-    cached = _NORM_TABLES.get(sig)
-    if cached is None:
-        for v in values:
-            _gpu(v, 'fp8 tensor')
-            if not v.is_contiguous():
-                raise ValueError('fp8 tensors must be contiguous')
-        device = values[0].device
-        result = torch.empty(len(values), dtype=torch.float32, device=device)
-        rows = [(v.data_ptr(), si.data_ptr(), result.data_ptr() + 4 * i, v.numel(), 0) for i, (v, si) in enumerate(zip(values, scale_invs))]
-        items = torch.from_numpy(np.asarray(rows, dtype=np.int64).reshape(len(rows), NORM_ITEM_WORDS)).to(device)
-        cached = (items, chunk_map(sig[2], device), result)
-        if len(_NORM_TABLES) >= 8:
-            _NORM_TABLES.pop(next(iter(_NORM_TABLES)))
-        _NORM_TABLES[sig] = cached
-    items, block_map, result = cached
-    _check(
-        lib.msamp_fp8_norms(_ptr(items), len(values), _ptr(block_map), block_map.shape[0], fp8_dt, kind, _stream()),
-        'msamp_fp8_norms'
-    )
-    return result.clone()
-
-
 GRAD_BLOCKS = 2048    # MSAMP_GRAD_BLOCKS
 
 
@@ -832,6 +795,16 @@ def grad_norms(table, n, norm_type, max_norm):
                                 _stream()), 'msamp_grad_norms'
     )
     return norms[:n], total, norms[n]
+
+
+def fp8_norms(values, scale_invs, fp8_dt, norm_type):
+    """Per-tensor p-norms (p = 1, 2 or inf) of FP8 payloads times their scale_inv, as one float32 vector."""
+    for v in values:
+        _gpu(v, 'fp8 tensor')
+        if not v.is_contiguous():
+            raise ValueError('fp8 tensors must be contiguous')
+    table = grad_table((_ptr(v), _ptr(si), v.numel(), fp8_dt) for v, si in zip(values, scale_invs))
+    return grad_norms(table, len(values), norm_type, float('inf'))[0]
 
 
 def grad_clip(table, n, factor):

@@ -202,8 +202,8 @@ def test_fp8_norms_against_float64(fp8_dt, fmt, norm_type):
 
 @pytest.mark.parametrize('norm_type', [1.0, 2.0, float('inf')])
 def test_fp8_norms_over_runs_of_chunks(norm_type):
-    """More chunks than eight per compute unit: a workgroup then takes several chunks in a row, which cross from one
-    tensor into the next, end in a partial chunk, and end the table.  The two large tensors hold one code, so their
+    """More chunks than eight per compute unit: a workgroup then takes several chunks of a tensor in a row, the last of them
+    fewer, and ends in a partial chunk.  The two large tensors hold one code, so their
     norms are exact numbers; the small ones between them are compared with float64 (one float32 rounding: 2^-24)."""
     from msamp import _backend
     chunk = 16384
