@@ -621,7 +621,8 @@ def fp8_gemm(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, out, accumulate=False, 
 
 def fp8_gemm_ksplit(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, out, accumulate=False):
     """fp8_gemm(..., a_kmajor=True, b_kmajor=True) in parts of K that fill the device, for outputs of a few tiles: the same
-    float32 sum in another, fixed order.  False (and nothing done) where the product is better taken whole."""
+    float32 sum in another, fixed order.  False (and nothing done) where the product is better taken whole, or there is no
+    memory for the partial sums (up to 256 MiB), which the whole product does without."""
     lib = load()
     k, m = a.shape
     kb, n = b.shape
@@ -633,7 +634,10 @@ def fp8_gemm_ksplit(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, out, accumulate=
         return False
     _gpu(a, 'mat_a')
     _gpu(b, 'mat_b')
-    scratch = torch.empty((words.value, ), dtype=torch.float32, device=a.device)
+    try:
+        scratch = torch.empty((words.value, ), dtype=torch.float32, device=a.device)
+    except torch.OutOfMemoryError:
+        return False
     _check(
         lib.msamp_fp8_gemm_ksplit(
             _ptr(a), a_dt, _ptr(a_scale_inv), _ptr(b), b_dt, _ptr(b_scale_inv), _ptr(out), _dt(out), m, n, k,
@@ -911,13 +915,20 @@ F32_SCRATCH = 64 << 20    # float32 elements of scratch in one launch: what the 
 
 def adamw_f32_list(rows, scaled_numels, device, lr, beta1, beta2, eps, weight_decay, step, bias_correction, adam_mode, maximize):
     """One AdamW / Adam step of a list of parameters with float32 moments.  `rows`: msamp_f32_param as tuples of eleven
-    words; `scaled_numels`: sizes of the scaled weights among them (they share float32 scratch)."""
+    words; `scaled_numels`: sizes of the scaled weights among them (they share float32 scratch, that of the largest one if there
+    is no memory for more)."""
     flat = [word for row in rows for word in row]
     table = (ctypes.c_longlong * len(flat))(*flat)
     padded = [(n + 3) // 4 * 4 for n in scaled_numels]
     room = max(max(padded), min(sum(padded), F32_SCRATCH)) if padded else 0
     words = torch.empty(F32_WORDS, dtype=torch.int32, device=device)
-    scratch = torch.empty(room, dtype=torch.float32, device=device) if room else None
+    scratch = None
+    if room:
+        try:
+            scratch = torch.empty(room, dtype=torch.float32, device=device)
+        except torch.OutOfMemoryError:
+            room = max(padded)
+            scratch = torch.empty(room, dtype=torch.float32, device=device)
     _check(
         load().msamp_adamw_f32_list(
             table, len(rows), _ptr(scratch), room, _ptr(words), lr, beta1, beta2, eps, weight_decay, step,

@@ -956,3 +956,40 @@ def test_float32_moment_step_of_parameters_that_share_memory(monkeypatch):
         runs.append([flat, other] + [opt.state[p][k] for p in params for k in ('exp_avg', 'exp_avg_sq')])
     for k, (a, b) in enumerate(zip(*runs)):
         assert torch.equal(a, b), k
+
+
+def test_scratch_that_cannot_be_had_costs_launches_only(monkeypatch):
+    """Where there is no memory for optional scratch the results are the same: a weight gradient is taken whole (codes of whole
+    numbers, exact in any order), and the scaled weights of a step share what the largest of them needs."""
+    from msamp import _backend
+    empty, refused = torch.empty, []
+
+    def scarce(*size, **kw):
+        n = torch.Size(size[0] if isinstance(size[0], (tuple, list)) else size).numel()
+        if kw.get('dtype') == torch.float32 and n > limit:
+            refused.append(n)
+            raise torch.OutOfMemoryError('no memory')
+        return empty(*size, **kw)
+
+    one = torch.ones((), device='cuda')
+    a = torch.randint(0, 2, (8192, 128), device='cuda', dtype=torch.uint8) * 0x38
+    b = torch.randint(0, 2, (8192, 256), device='cuda', dtype=torch.uint8) * 0x38
+    out = torch.full((256, 128), -1.0, device='cuda')
+    limit = 256 * 128
+    monkeypatch.setattr(torch, 'empty', scarce)
+    assert _backend.fp8_gemm_ksplit(a, 5, one, b, 5, one, out) is False and len(refused) == 1 and (out == -1.0).all()
+    monkeypatch.undo()
+    runs = []
+    for limit in (1 << 60, 5000):
+        gen = torch.Generator(device='cuda').manual_seed(2)
+        params = [ScalingParameter(torch.randn(n, device='cuda', generator=gen).cast(Dtypes.kfloat16)) for n in (4000, 5000, 3001)]
+        opt = LBAdamW(params, lr=1e-2, exp_avg_dtype=torch.float32, exp_avg_sq_dtype=torch.float32)
+        for p in params:
+            p.grad = torch.randn(p.shape, device='cuda', generator=gen).cast(Dtypes.kfloat8_e4m3)
+        refused.clear()
+        monkeypatch.setattr(torch, 'empty', scarce)
+        opt.step()
+        monkeypatch.undo()
+        assert len(refused) == (limit == 5000)
+        runs.append([t for p in params for t in (p.value, p.meta.scale, p.meta.scale_inv, p.meta.amax)])
+    assert all(same_float(x, y) for x, y in zip(*runs))
