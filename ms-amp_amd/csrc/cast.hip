@@ -27,11 +27,14 @@ __device__ __forceinline__ void amax_publish(float* amax, float v) {
 // (float bit patterns of |x|, NaN patterns included).
 constexpr int kWsPartials = 16;
 constexpr int kMaxPartials = 1024;
-// word kWsSpecDone: non-zero when the first pass of an in-time cast also wrote the output, quantized with the scale
-// in force before the call (word 0); the second pass then only has to run when the rule gives another scale
+// word kWsSpecDone: non-zero when the first pass of an in-time cast also wrote the output, quantized with a guessed scale
+// (word kWsGuess, as a bit pattern: the one in force before the call, or one from a sample); the second pass then only has to
+// run when the rule gives another scale
 constexpr int kWsSpecDone = 9;
-// word kWsGuess: the scale that pass wrote the output with (bit pattern)
 constexpr int kWsGuess = 13;
+// word kWsMissed: non-zero when that pass met a value too large for its guess and wrote no further output
+constexpr int kWsMissed = 14;
+static_assert(kWsMissed < kWsPartials, "the words in front of the partial maxima");
 // a sample of partial maxima from which a fresh meta's scale is guessed: kSampleBlocks words behind the meeting slots
 constexpr int kWsSampleBytes = 12544;
 constexpr int kSampleBlocks = 512;
@@ -111,8 +114,8 @@ __global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restri
     float s;
     if constexpr (INTIME == kInTime) {
         s = resolve_in_time_scale(it, red, scale_inv);
-        // the first pass quantized with the scale it found in the meta, and the rule confirms that scale: done
-        if (it.speculative && it.ws[kWsSpecDone] != 0u && __float_as_uint(s) == it.ws[kWsGuess]) return;
+        // the first pass quantized all of x with its guess, and the rule confirms that scale: done
+        if (it.speculative && it.ws[kWsSpecDone] != 0u && it.ws[kWsMissed] == 0u && __float_as_uint(s) == it.ws[kWsGuess]) return;
     } else if constexpr (INTIME == kRescale) {
         const float s_new = scale_rule(*it.known_amax, 1.0f, it.fp_max, it.margin);
         s = s_new * *it.old_scale_inv;
@@ -410,9 +413,10 @@ __global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __
 
 // First pass of the in-time cast of a tensor too large for the one-pass kernel, with the output written on
 // speculation: max|x| per workgroup as above, and every element quantized with a guessed scale: the one the meta holds
-// before the call, or, for a meta that has never been used, the one a sample of x suggests.  A power-of-two scale rarely changes between two calls on the same meta; when the second pass finds that
-// the rule confirms it, it returns at once and x has been read once (sizeof(in) + 1 bytes per element instead of
-// 2 * sizeof(in) + 1).  Otherwise the second pass quantizes again with the new scale: the same bytes as without
+// before the call, or, for a meta that has never been used, the one a sample of x suggests.  A power-of-two scale rarely
+// changes between two calls on the same meta; when the second pass finds that the rule confirms it, it returns at once and
+// x has been read once (sizeof(in) + 1 bytes per element instead of 2 * sizeof(in) + 1).  Otherwise the second pass
+// quantizes again with the new scale: the same bytes as without
 // speculation, since the output is not an input.
 //
 // The sample (cast_sample_kernel) is the maxima of 512 pieces of 16 KiB spread evenly over x, 8 MiB in all.  The maximum of
@@ -421,9 +425,13 @@ __global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __
 // extrapolated: the square of the maximum of N values grows about linearly in log N (exactly so for normal tails), and
 // its growth from a piece (m0, the mean of the 512 maxima) to 64 pieces (m1, the mean over the eight wavefronts'
 // 64-piece maxima) is continued to the size of x.  What counts is only whether guess and maximum lie in the same binade of
-// fp_max / amax.  235 M bfloat16 elements with a fresh meta: 203 us in two passes (maxima, then the cast), 122 us when the
-// guess holds, 257 us when it does not (10 of 10 normal and uniform tensors guessed right, 19 of 20 with rare outliers, 3 of 10
-// with exponential tails, each over a full binade of maxima).
+// fp_max / amax.  235 M bfloat16 elements with a fresh meta: 203 us in two passes (maxima, then the cast; 213 with the fills
+// that made the meta), 122 us when the guess holds, and 257 us when it does not, if all of x is quantized with it all the
+// same.  So a wavefront that meets a value beyond what the guess can stand for raises kWsMissed, and from where a workgroup
+// learns of it, it only takes maxima: 221 to 254 us, the later the few values beyond the guess lie in x (a guess too small a
+// scale is not found out: 257).  Over eight scales in an octave, us on average with the guess, and in two passes with the
+// fills: normal values 138, 213; with rare outliers 123, 216; exponential tails 169, 214; Cauchy 122, 214; log-normal 217,
+// 213 (seven of eight missed; 241 before the pass looked at what it met).
 // A meta that was used before but holds amax 0 and scale 1 is not speculated on: the pass then only takes the maxima.
 constexpr int kSpecThreads = 512;
 
@@ -460,7 +468,8 @@ __device__ __forceinline__ float scale_from_sample(uint32_t mine, float growth, 
 }
 
 template <typename IT>
-__global__ __launch_bounds__(kCastThreads) void cast_sample_kernel(const IT* __restrict__ x, size_t n, uint32_t* sample) {
+__global__ __launch_bounds__(kCastThreads) void cast_sample_kernel(const IT* __restrict__ x, size_t n, uint32_t* sample,
+                                                                   uint32_t* missed) {
     constexpr int EPT = 16 / sizeof(IT);
     constexpr size_t kPiece = static_cast<size_t>(kCastThreads) * EPT * 4;
     __shared__ uint32_t red[kCastThreads / kWave];
@@ -484,6 +493,7 @@ __global__ __launch_bounds__(kCastThreads) void cast_sample_kernel(const IT* __r
     if (threadIdx.x == 0) {
         if constexpr (sizeof(IT) == 2 && !__is_same(IT, bf16_t)) m = __float_as_uint(f16_bits_to_float(m >> 16));
         sample[blockIdx.x] = m;
+        if (blockIdx.x == 0) *missed = 0u;
     }
 }
 
@@ -497,18 +507,22 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
     constexpr int EPT = In16<IT>::EPT;
     constexpr size_t TILE = static_cast<size_t>(kSpecThreads) * EPT * kCastUnroll;
     __shared__ uint32_t red[kSpecThreads / kWave];
+    __shared__ uint32_t s_missed;    // (raised by any wavefront at any time, read whenever it suits: no barrier in the loop)
     const int tid = threadIdx.x;
     float guess = 1.0f, in_force = 1.0f;
     bool spec = false;
     if (sample != nullptr) {
         static_assert(kSampleBlocks == kSpecThreads, "one word of the sample per lane");
+        if (tid == 0) s_missed = 0u;
         guess = scale_from_sample(sample[tid], growth, fp_max, margin, red);
         spec = guess > 0.0f && guess < __uint_as_float(0x7f800000u);
     } else if (scale != nullptr) {
         guess = in_force = *scale;
         spec = !(*amax == 0.0f && guess == 1.0f);
     }
-    uint32_t m = 0;
+    const bool guessed = spec;
+    const float limit = fp_max / guess;    // of a value that the guess can stand for
+    uint32_t m = 0, turn = 0;
     const size_t ntiles = (n + TILE - 1) / TILE;
     for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const size_t base = t * TILE;
@@ -517,6 +531,13 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
 #pragma unroll
             for (int u = 0; u < kCastUnroll; ++u)
                 raw[u] = ld16(x + base + (static_cast<size_t>(u) * kSpecThreads + tid) * EPT, (vec_ok & 2) != 0);
+            // One wavefront looks whether another workgroup has found the guess too small, every fourth tile and behind the
+            // tile's loads: the look takes longer than they do (in front of them, every tile: 122 -> 127 us when the guess holds).
+            uint32_t elsewhere = 0;
+            if (spec && sample != nullptr) {
+                if (tid < kWave && (++turn & 3) == 0) elsewhere = __hip_atomic_load(ws + kWsMissed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                spec = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&s_missed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) == 0u;
+            }
 #pragma unroll
             for (int u = 0; u < kCastUnroll; ++u) {
                 const uint32_t w[4] = {raw[u].x, raw[u].y, raw[u].z, raw[u].w};
@@ -537,6 +558,12 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
                     else *reinterpret_cast<uint2*>(o) = make_uint2(q[0], q[1]);
                 }
             }
+            if (spec && sample != nullptr) {
+                const float top = sizeof(IT) == 2 && !__is_same(IT, bf16_t) ? f16_bits_to_float(m >> 16) : __uint_as_float(m);
+                const bool here = !(top <= limit);
+                if (here) __hip_atomic_store(ws + kWsMissed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (here || elsewhere != 0u) __hip_atomic_store(&s_missed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
         } else {
             const size_t end = (base + TILE < n) ? base + TILE : n;
             for (size_t i = base + tid; i < end; i += kSpecThreads) {
@@ -556,8 +583,9 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
         if (blockIdx.x == 0) {
             ws[0] = __float_as_uint(in_force);
             ws[1] = gridDim.x;
-            ws[kWsSpecDone] = spec ? 1u : 0u;
+            ws[kWsSpecDone] = guessed ? 1u : 0u;
             ws[kWsGuess] = __float_as_uint(guess);
+            if (sample == nullptr) ws[kWsMissed] = 0u;
         }
     }
 }
@@ -1377,7 +1405,7 @@ static int launch_speculative(const IT* x, size_t n, const float* scale, const f
     uint32_t* sample = nullptr;
     if (scale == nullptr && aligned(x, 16) && n * sizeof(IT) >= static_cast<size_t>(kSampleBlocks) * kCastThreads * 16 * 4 * 4) {
         sample = ws + kWsSampleBytes / 4;
-        hipLaunchKernelGGL((cast_sample_kernel<IT>), dim3(kSampleBlocks), dim3(kCastThreads), 0, st, x, n, sample);
+        hipLaunchKernelGGL((cast_sample_kernel<IT>), dim3(kSampleBlocks), dim3(kCastThreads), 0, st, x, n, sample, ws + kWsMissed);
         MSAMP_CHECK_LAUNCH("cast_sample_kernel");
     }
     const float growth = static_cast<float>(log2(static_cast<double>(n) * sizeof(IT) / (64.0 * kCastThreads * 64)) / 6.0);

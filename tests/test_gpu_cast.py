@@ -548,7 +548,8 @@ def test_fresh_meta_cast_equals_the_cast_on_a_new_meta(be, dtype, n, two_pass):
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize('what', ['sample tells', 'sample misses the maximum', 'sample misses everything', 'nan', 'inf'])
+@pytest.mark.parametrize('what', ['sample tells', 'sample misses the maximum', 'sample misses everything', 'nan', 'inf',
+                                  'inf beside a guess of 1', 'misses everywhere'])
 def test_fresh_meta_cast_guesses_from_a_sample(be, dtype, what):
     """Beyond the one-pass limit the scale is guessed from a sample of 512 pieces of 16 KiB, spread evenly; whatever the
     sample says, the result is the one of the two plain passes."""
@@ -564,6 +565,13 @@ def test_fresh_meta_cast_guesses_from_a_sample(be, dtype, what):
     elif what == 'sample misses everything':
         x.zero_()
         x[free + 3] = 2.0
+    elif what == 'inf beside a guess of 1':    # (what the rule falls back to: the guess must not count as confirmed)
+        x.fill_(300.0)
+        x[free + 3] = float('inf')
+    elif what == 'misses everywhere':    # (all of x but the sample is too large for the guess: every workgroup finds that out)
+        x.fill_(32.0)
+        for p in taken:
+            x[p * piece:(p + 1) * piece] = 0.5
     elif what != 'sample tells':
         x[free + 3] = float(what)
     s, si, am = make_meta()
