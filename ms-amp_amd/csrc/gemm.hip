@@ -115,7 +115,7 @@ int small_tile_limit() { return g_small_tile_limit.load(std::memory_order_relaxe
 using namespace msamp;
 
 extern "C" void msamp_set_small_tile_limit(int big_tiles) {
-    msamp::g_small_tile_limit.store(big_tiles < 0 ? 0 : big_tiles, std::memory_order_relaxed);
+    msamp::g_small_tile_limit.store(big_tiles, std::memory_order_relaxed);
 }
 
 extern "C" int msamp_fp8_gemm_set_walk(int m, int n, int k, int a_kmajor, int b_kmajor, int walk) {

@@ -66,7 +66,8 @@ template <int XF, int YF>
 int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int NR, int NC, int K, const float* xs,
                    const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st);
 
-// Problems of at most this many 256 x 256 tiles take the kernel with 128 x 128 tiles (msamp_set_small_tile_limit) ...
+// Problems of at most this many 256 x 256 tiles take the kernel with 128 x 128 tiles (msamp_set_small_tile_limit; negative: the
+// generic kernel for every row-major product, to compare the others with) ...
 int small_tile_limit();
 // The tile walk registered for this problem of the 256 x 256-tile kernel (msamp_fp8_gemm_set_walk / _tune), or -1: bit 0 =
 // groups of tile columns walked row by row instead of groups of tile rows, bit 1 = the XCD's patch of 32 tiles turned (4 of

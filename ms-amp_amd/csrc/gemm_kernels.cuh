@@ -1348,7 +1348,7 @@ namespace msamp {
 template <int XF, int YF, typename OT>
 static int pick_tile(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
                      const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
-    if (K % kBK == 0 && K >= 2 * kBK && fits_offsets(NR, NC, K))
+    if (K % kBK == 0 && K >= 2 * kBK && fits_offsets(NR, NC, K) && small_tile_limit() >= 0)
         return launch_gemm_dma<XF, YF, OT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
     return launch_gemm<128, 128, XF, YF, OT>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
 }
@@ -1470,7 +1470,7 @@ template <int XF, int YF>
 int run_gemm_pair(const GemmCall& c) {
     if (c.qa == nullptr && fits_offsets(c.NR, c.NC, c.K)) {
         if (takes_small_tiles(c.NR, c.NC, c.K)) return run_gemm_small<XF, YF>(c);
-        if (c.K > kBK && c.K % kBK) return run_gemm_ragged<XF, YF>(c);
+        if (c.K > kBK && c.K % kBK && (c.yt || small_tile_limit() >= 0)) return run_gemm_ragged<XF, YF>(c);
     }
     if (c.qa != nullptr && c.qspec) {
         if (c.xt) return pick_out_spec<XF, YF, true>(c.X, c.Y, c.D, c.d_dtype, c.NR, c.NC, c.K, c.xs, c.ys, c.accumulate, *c.qa, c.st);

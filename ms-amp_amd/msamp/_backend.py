@@ -698,7 +698,8 @@ def fp8_gemm_cast(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, hp_dtype, q_dt, sc
 
 
 def set_small_tile_limit(big_tiles):
-    """Row-major GEMMs of at most this many 256 x 256 output tiles run 128 x 128 tiles (default 128, 0 = never)."""
+    """Row-major GEMMs of at most this many 256 x 256 output tiles run 128 x 128 tiles (default 128, 0 = never; negative:
+    row-major ones run the generic kernel)."""
     load().msamp_set_small_tile_limit(int(big_tiles))
 
 

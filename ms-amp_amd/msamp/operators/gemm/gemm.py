@@ -71,7 +71,9 @@ class Gemm:
 
         a_kmajor / b_kmajor (not in the reference): the tensor passed is the transpose of the operand,
         [K, M] / [K, N], as the backward pass of a linear layer has them; the kernel reads it in place
-        when the shape allows, otherwise it is transposed first.  Same result either way.
+        when the shape allows, otherwise it is transposed first.  Same result either way, except that with both
+        K-major and an output of a few tiles the float32 sum may be taken in parts of K (msamp_fp8_gemm_ksplit):
+        another order of the same sum, which depends on the sizes and the device only.
         """
         assert isinstance(mat_a, ScalingTensor)
         assert isinstance(mat_b, ScalingTensor)

@@ -260,6 +260,21 @@ def test_weight_gradient_in_parts_of_k(be, a_dt, b_dt, m, n, k, out_dtype):
     assert torch.equal(out, (exact + base.double()).to(out_dtype))
 
 
+@pytest.mark.parametrize('m,n,k', [(128, 256, 16384), (1024, 1024, 8192), (1200, 4304, 12605), (272, 336, 4097)])
+def test_weight_gradient_in_parts_of_k_is_no_less_exact(be, m, n, k):
+    """Codes of normal values: the sum in parts of K against the product in float64, beside the product taken whole.  A part's
+    sum is shorter and so are its roundings; the parts are added in float32 once more: no further off than the whole."""
+    a, b = _gpu_codes((k, m), 5, m + k), _gpu_codes((k, n), 6, n + k)
+    one = torch.ones((), device='cuda')
+    split, whole = torch.empty(n, m, device='cuda'), torch.empty(n, m, device='cuda')
+    assert be.fp8_gemm_ksplit(a, 5, one, b, 6, one, split) is True
+    be.fp8_gemm(a, 5, one, b, 6, one, whole, a_kmajor=True, b_kmajor=True)
+    wide = lambda t, dt: be.cast_from_fp8(t, one, dt, torch.float32).double()
+    exact = wide(b, 6).t().contiguous() @ wide(a, 5)
+    errors = [((t.double() - exact).norm() / exact.norm()).item() for t in (split, whole)]
+    assert errors[0] <= errors[1] and errors[0] < TOL_F32, errors
+
+
 def test_weight_gradient_taken_whole(be):
     """Outputs of many tiles, short K and an output that 16-byte accesses do not fit are left to the product as a whole."""
     one = torch.ones((), device='cuda')
@@ -287,7 +302,7 @@ def test_gemm_cast_refuses_bad_arguments_for_every_shape(be):
 
 
 def test_kmajor_rejects_unsupported_shapes(be):
-    a = _rand_fp8((128, 100), 5, 1).cuda()    # [K=128, M=100]: M is not a multiple of 256
+    a = _rand_fp8((128, 100), 5, 1).cuda()    # [K=128, M=100]: a single slice of K, and M no multiple of 16
     b = _rand_fp8((64, 128), 5, 2).cuda()
     one = torch.ones((), device='cuda')
     with pytest.raises(RuntimeError):
@@ -740,39 +755,45 @@ def test_gemm_with_fused_cast_many_random_cases(be, large_tiles_only):
     assert cases == 48
 
 
-@pytest.mark.parametrize('m,n,k', [(256, 256, 256), (300, 200, 384), (1024, 768, 1024), (2048, 2048, 4096)])
+@pytest.mark.parametrize('m,n,k', [(256, 256, 256), (300, 200, 384), (1024, 768, 1024), (2048, 2048, 4096), (300, 200, 144),
+                                   (256, 512, 400), (1024, 768, 1040), (2048, 2048, 4080)])
 @pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16])
 def test_generic_and_direct_to_lds_kernels_agree_to_the_bit(be, m, n, k, out_dtype):
-    """K a multiple of 128 goes to the direct-to-LDS kernel; the same operands with 16 zero bytes appended to every row
-    (K + 16) go to the generic kernel.  The zeros add nothing, and both kernels add up the 128-byte blocks of K in
-    ascending order, so the outputs must be equal bit for bit (which makes results independent of the dispatch)."""
+    """The direct-to-LDS kernels (large and small tiles, whole and ragged last slices of K) against the generic,
+    register-staged kernel on the same operands: all of them add up the 128-byte blocks of K in ascending order, so the
+    outputs must be equal bit for bit (which makes results independent of the dispatch)."""
     a, b = _gpu_codes((m, k), 5, 3 * m + k), _gpu_codes((n, k), 6, 7 * n + k)
     sa, sb = torch.tensor(0.5, device='cuda'), torch.tensor(0.25, device='cuda')
-    want = be.fp8_gemm(a, 5, sa, b, 6, sb, torch.empty(n, m, dtype=out_dtype, device='cuda'))
-    a2, b2 = torch.nn.functional.pad(a, (0, 16)).contiguous(), torch.nn.functional.pad(b, (0, 16)).contiguous()
-    got = be.fp8_gemm(a2, 5, sa, b2, 6, sb, torch.empty(n, m, dtype=out_dtype, device='cuda'))
-    assert torch.equal(got, want)
+    outs = []
+    try:
+        for limit in (-1, 0, 1 << 20):
+            be.set_small_tile_limit(limit)
+            outs.append(be.fp8_gemm(a, 5, sa, b, 6, sb, torch.full((n, m), float('nan'), dtype=out_dtype, device='cuda')))
+    finally:
+        be.set_small_tile_limit(128)
+    assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
 
 
-@pytest.mark.parametrize('m,n,k', [(4396, 4616, 384), (4352, 4608, 640), (8192, 4352, 256)])
+@pytest.mark.parametrize('m,n,k', [(4396, 4616, 384), (4352, 4608, 640), (8192, 4352, 256), (4396, 4616, 400), (4352, 4608, 1136)])
 @pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize('mode', ['plain', 'bias_and_sum'])
+@pytest.mark.parametrize('mode', ['plain', 'bias', 'bias_and_sum'])
 def test_several_rounds_of_tiles_agree_with_the_generic_kernel(be, m, n, k, out_dtype, mode):
     """More 256 x 256 tiles than compute units (several rounds of workgroups, whole tiles and tiles on the ragged edges
-    mixed), every output type, with and without bias and sum: the direct-to-LDS kernel compared bit for bit with the
-    generic kernel (the same operands with 16 zero bytes appended to every row)."""
+    mixed), whole and ragged last slices of K, every output type, with and without bias and sum: the direct-to-LDS kernel
+    compared bit for bit with the generic kernel."""
     a, b = _gpu_codes((m, k), 5, 5 * m + k), _gpu_codes((n, k), 6, 11 * n + k)
     sa, sb = torch.tensor(0.5, device='cuda'), torch.tensor(0.125, device='cuda')
-    a2, b2 = torch.nn.functional.pad(a, (0, 16)).contiguous(), torch.nn.functional.pad(b, (0, 16)).contiguous()
     g = torch.Generator(device='cuda').manual_seed(m + n)
-    bias = prev = None
-    if mode == 'bias_and_sum':
-        bias = torch.randn(m, device='cuda', generator=g).to(out_dtype)
-        prev = torch.randn(n, m, device='cuda', generator=g).to(out_dtype)
+    bias = torch.randn(m, device='cuda', generator=g).to(out_dtype) if mode != 'plain' else None
+    prev = torch.randn(n, m, device='cuda', generator=g).to(out_dtype) if mode == 'bias_and_sum' else None
     outs = []
-    for x, y in ((a, b), (a2, b2)):
-        out = prev.clone() if prev is not None else torch.full((n, m), float('nan'), dtype=out_dtype, device='cuda')
-        outs.append(be.fp8_gemm(x, 5, sa, y, 6, sb, out, accumulate=prev is not None, bias=bias))
+    try:
+        for limit in (128, -1):
+            be.set_small_tile_limit(limit)
+            out = prev.clone() if prev is not None else torch.full((n, m), float('nan'), dtype=out_dtype, device='cuda')
+            outs.append(be.fp8_gemm(a, 5, sa, b, 6, sb, out, accumulate=prev is not None, bias=bias))
+    finally:
+        be.set_small_tile_limit(128)
     assert torch.equal(outs[0].view(torch.int32 if out_dtype == torch.float32 else torch.int16),
                        outs[1].view(torch.int32 if out_dtype == torch.float32 else torch.int16))
     assert not bool(outs[0].isnan().any())
@@ -781,7 +802,7 @@ def test_several_rounds_of_tiles_agree_with_the_generic_kernel(be, m, n, k, out_
 @pytest.mark.parametrize('m,n,k', [(2048, 2048, 4096), (4096, 1024, 4096), (1024, 768, 1024), (2056, 1100, 512), (300, 200, 640),
                                    (128, 128, 512), (1031, 1999, 1152), (1, 1, 512), (33, 65, 1024), (7, 513, 768)])
 @pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize('mode', ['plain', 'bias_and_sum'])
+@pytest.mark.parametrize('mode', ['plain', 'bias', 'bias_and_sum'])
 def test_small_and_large_tiles_agree_to_the_bit(be, m, n, k, out_dtype, mode):
     """Problems with few 256 x 256 tiles run 128 x 128 tiles (four stages, fragments read a slice ahead).  The same
     problem through both, the limit set to take the one and then the other: every output equal bit for bit, on whole
@@ -790,10 +811,8 @@ def test_small_and_large_tiles_agree_to_the_bit(be, m, n, k, out_dtype, mode):
         a, b = _gpu_codes((m, k), a_dt, 5 * m + k + a_dt), _gpu_codes((n, k), b_dt, 11 * n + k + b_dt)
         sa, sb = torch.tensor(0.5, device='cuda'), torch.tensor(0.125, device='cuda')
         g = torch.Generator(device='cuda').manual_seed(m + n)
-        bias = prev = None
-        if mode == 'bias_and_sum':
-            bias = torch.randn(m, device='cuda', generator=g).to(out_dtype)
-            prev = torch.randn(n, m, device='cuda', generator=g).to(out_dtype)
+        bias = torch.randn(m, device='cuda', generator=g).to(out_dtype) if mode != 'plain' else None
+        prev = torch.randn(n, m, device='cuda', generator=g).to(out_dtype) if mode == 'bias_and_sum' else None
         outs = []
         try:
             for limit in (1 << 20, 0):
@@ -843,8 +862,9 @@ def test_small_tiles_read_kmajor_operands_like_the_large_tile(be, m, n, k, out_d
 
 
 def test_random_small_ragged_problems_with_bias_and_accumulation(be):
-    """Random shapes up to 700 x 700 with K both a multiple of 128 (direct-to-LDS kernel, whose 256 x 256 tiles are
-    mostly padding here) and not (generic kernel), every output type, with and without bias and accumulation."""
+    """Random shapes up to 700 x 700 with K of several slices, whole and with a ragged last one (direct-to-LDS kernels, whose
+    tiles are mostly padding here), and of one slice at most (generic kernel), every output type, with and without bias
+    and accumulation."""
     import random
     rng = random.Random(4)
     for it in range(32):
@@ -939,9 +959,8 @@ def test_split_waits_change_no_bit(be, large_tiles_only, n, m, k):
         assert torch.equal(plain.view(torch.int16), outs[0][0].view(torch.int16)), walk
         assert torch.equal(summed.view(torch.int16), outs[0][1].view(torch.int16)), walk
     if k <= 4096:
-        # the generic kernel (K made unfit for the direct-to-LDS kernel by 16 columns of zero codes)
-        pad = lambda t: torch.cat([t, torch.zeros(t.shape[0], 16, dtype=torch.uint8, device='cuda')], dim=1)    # noqa: E731
-        generic = be.fp8_gemm(pad(a), 5, a_si, pad(b), 6, b_si, torch.empty(n - 3, m, dtype=torch.bfloat16, device='cuda'))
+        be.set_small_tile_limit(-1)    # (the fixture puts the default back)
+        generic = be.fp8_gemm(a, 5, a_si, b, 6, b_si, torch.empty(n - 3, m, dtype=torch.bfloat16, device='cuda'))
         assert torch.equal(generic.view(torch.int16), outs[0][0].view(torch.int16))
 
 
