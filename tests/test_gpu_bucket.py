@@ -444,3 +444,24 @@ def test_clip_counts_as_a_change_only_where_it_clips(saved, owner):
         else:
             loss.backward()
             assert torch.equal(w.grad, want)
+
+
+@pytest.mark.parametrize('norm_type', [1.0, 2.0, float('inf')])
+def test_clip_where_workgroups_take_runs_of_chunks(norm_type):
+    """More than 2048 chunks of 16384 in all, so that a workgroup takes several: plain and FP8 tensors that end inside a run and
+    inside a chunk, one of them off 16-byte alignment, beside small ones.  Every element is what torch makes of it."""
+    import msamp
+    from msamp.common.dtype import Dtypes
+    gen = torch.Generator(device='cuda').manual_seed(4)
+    chunk = 16384
+    x = lambda n: torch.randn(n, device='cuda', generator=gen)
+    grads = [x(700 * chunk + 5), x(5).half(), x(601 * chunk + 7).bfloat16(), x(401 * chunk + 4).half()[1:],
+             x(902 * chunk + 3).cast(Dtypes.kfloat8_e5m2), x(chunk).bfloat16(), x(2 * chunk + 1).cast(Dtypes.kfloat8_e4m3)]
+    wide = torch.stack([torch.linalg.vector_norm(g.float().double(), norm_type) for g in grads])
+    want = torch.linalg.vector_norm(wide, norm_type).item()
+    plain = [g.meta.scale_inv.clone() if hasattr(g, 'meta') else g.clone() for g in grads]
+    total = msamp.clip_grad_norm_([_Owner(g) for g in grads], want / 7, norm_type=norm_type)
+    assert total.item() == pytest.approx(want, rel=2.5e-7)    # (one float32 rounding per tensor and one of the total)
+    coef = torch.clamp((want / 7) / (total + 1e-6), max=1.0)
+    for g, p in zip(grads, plain):
+        assert torch.equal(g.meta.scale_inv if hasattr(g, 'meta') else g, p.mul_(coef))

@@ -581,7 +581,8 @@ def test_fresh_meta_cast_guesses_from_a_sample(be, dtype, what):
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize('rows,cols', [(1, 1), (3, 8), (16, 512), (17, 520), (96, 1001), (1000, 260), (4099, 384), (33, 4304)])
+@pytest.mark.parametrize('rows,cols', [(1, 1), (3, 8), (16, 512), (17, 520), (96, 1001), (1000, 260), (4099, 384), (33, 4304),
+                                       (12605, 4304), (70001, 264), (40001, 1001)])    # (slabs of several rounds of 16 rows)
 def test_cast_with_column_sums(be, dtype, rows, cols):
     """Codes and meta of the gated cast, on both sides of the gate, and the columns' sums: float32 sums of at most `chain`
     terms in a row (2^-24 each of the sum of magnitudes), rounded to the input's type; a view that 16-byte loads do not fit."""
