@@ -6,6 +6,7 @@ There is no CPU or eager fallback: if the library cannot be loaded, or an operan
 the GPU, the call raises.
 """
 
+import array
 import ctypes
 import os
 
@@ -784,8 +785,7 @@ GRAD_BLOCKS = 2048    # MSAMP_GRAD_BLOCKS
 
 def grad_table(entries):
     """Host table (msamp_grad) of (data pointer, scale_inv pointer or 0, numel, library dtype) tuples."""
-    flat = [word for e in entries for word in e]
-    return (ctypes.c_longlong * len(flat))(*flat)
+    return array.array('q', [word for e in entries for word in e])
 
 
 def grad_norms(table, n, norm_type, max_norm):
@@ -796,7 +796,7 @@ def grad_norms(table, n, norm_type, max_norm):
     total = torch.empty((), dtype=torch.float32, device=device)
     partials = torch.empty(n + GRAD_BLOCKS, dtype=torch.float64, device=device)
     _check(
-        load().msamp_grad_norms(table, n, kind, max_norm, _ptr(partials), _ptr(norms), _ptr(total), _ptr(norms) + 4 * n,
+        load().msamp_grad_norms(table.buffer_info()[0], n, kind, max_norm, _ptr(partials), _ptr(norms), _ptr(total), _ptr(norms) + 4 * n,
                                 _stream()), 'msamp_grad_norms'
     )
     return norms[:n], total, norms[n]
@@ -814,8 +814,7 @@ def fp8_norms(values, scale_invs, fp8_dt, norm_type):
 
 def grad_clip(table, n, factor):
     """Multiplies the table's tensors (FP8 ones through their scale_inv) by factor where that is below 1."""
-    factor = factor.to(torch.device('cuda', torch.cuda.current_device()))    # (the total may be on another GPU, as its first gradient)
-    _check(load().msamp_grad_clip(table, n, _ptr(factor), _stream()), 'msamp_grad_clip')
+    _check(load().msamp_grad_clip(table.buffer_info()[0], n, _ptr(factor), _stream()), 'msamp_grad_clip')
 
 
 # ---- AdamW --------------------------------------------------------------------------------------

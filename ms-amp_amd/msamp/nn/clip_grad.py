@@ -8,35 +8,52 @@ from msamp.common.tensor import ScalingTensor
 
 
 _KINDS = (1.0, 2.0, float('inf'))
-_PLAIN = (torch.float32, torch.float16, torch.bfloat16)
+_PLAIN = {torch.float32: _backend.DT_F32, torch.float16: _backend.DT_F16, torch.bfloat16: _backend.DT_BF16}
 
 
-def _entry(g):
-    """Descriptor of a gradient for the kernels that take a whole list at once, or None if it is not a contiguous FP8
+def _entries(grads):
+    """Per gradient its descriptor for the kernels that take a whole list at once, or None if it is not a contiguous FP8
     ScalingTensor or plain tensor on the current GPU."""
-    if type(g) is ScalingTensor:
-        value, si = g.value, g.meta.scale_inv
-        if not Dtypes.is_fp8_qtype(g.qtype) or si.dtype != torch.float32 or si.numel() != 1 or si.device != value.device:
-            return None
-        dtype, si = int(g.qtype), si.data_ptr()
-    else:
-        value, si = g, 0
-        if type(g) not in (torch.Tensor, torch.nn.Parameter) or g.layout != torch.strided or g.dtype not in _PLAIN or \
-                g.requires_grad:
-            return None
-        dtype = _backend.hp_dt(g)
-    if value.numel() == 0 or not value.is_cuda or value.device.index != torch.cuda.current_device() or \
-            not value.is_contiguous():
-        return None
-    return value.data_ptr(), si, value.numel(), dtype
+    current, entries = None, []
+    for g in grads:
+        kind = type(g)
+        if kind is ScalingTensor:
+            value, si = g.value, g.meta.scale_inv
+            device, word, dtype = value.get_device(), si.data_ptr(), int(g.qtype) if Dtypes.is_fp8_qtype(g.qtype) else 0
+            if si.dtype != torch.float32 or si.numel() != 1 or si.get_device() != device:
+                dtype = 0
+        else:
+            value, word, dtype = g, 0, 0
+            if (kind is torch.Tensor or kind is torch.nn.Parameter) and g.layout == torch.strided and not g.requires_grad:
+                device, dtype = g.get_device(), _PLAIN.get(g.dtype, 0)
+        if dtype and device >= 0:
+            if current is None:
+                current = torch.cuda.current_device()
+            numel = value.numel()
+            if numel and device == current and value.is_contiguous():
+                entries.append((value.data_ptr(), word, numel, dtype))
+                continue
+        entries.append(None)
+    return entries
 
 
 def _rounds(entries):
     """The entries in as few lists as it takes so that clipping those of one list writes no word twice (an FP8 gradient's
     scale_inv, a plain one's values): what a launch scales at the same time must not overlap."""
+    words = {e[1] for e in entries}
+    if 0 not in words and len(words) == len(entries):
+        return [entries]    # (FP8 throughout: words of four bytes, aligned)
+    spans = sorted([(e[1], e[1] + 4, e) if e[1] else (e[0], e[0] + e[2] * _backend.dt_size(e[3]), e) for e in entries])
+    end, apart = 0, True
+    for lo, hi, _ in spans:
+        if lo < end:
+            apart = False
+            break
+        end = hi
+    if apart:
+        return [entries]
     rounds, ends = [], []
-    for lo, hi, e in sorted(((e[1], e[1] + 4, e) if e[1] else (e[0], e[0] + e[2] * _backend.dt_size(e[3]), e)
-                             for e in entries)):
+    for lo, hi, e in spans:
         at = next((i for i, end in enumerate(ends) if end <= lo), len(ends))
         if at == len(ends):
             rounds.append([])
@@ -57,14 +74,16 @@ def _join(norms, norm_type):
     return torch.norm(torch.stack(norms), norm_type)
 
 
-def _held_elsewhere(p):
-    """True if a graph may have saved the gradient of p: something holds it beside its owner and Python, or holds a view of it."""
-    g = p.grad
-    if type(g) is ScalingTensor:
-        return g.meta.scale_inv._use_count() > 1
-    # (the storage: the gradient, and the handle it is asked through)
-    return g._use_count() > (2 if isinstance(p, torch.Tensor) else 1) or \
-        torch._C._storage_Use_Count(g.untyped_storage()._cdata) > 2
+def _held_elsewhere(parameters, grads):
+    """True if a graph may have saved one of the gradients: something holds it beside its owner and Python, or a view of it."""
+    for p, g in zip(parameters, grads):
+        if type(g) is ScalingTensor:
+            if g.meta.scale_inv._use_count() > 1:
+                return True
+        elif g._use_count() > (2 if isinstance(p, torch.Tensor) else 1) or \
+                torch._C._storage_Use_Count(g.untyped_storage()._cdata) > 2:    # (the gradient, and the handle it is asked through)
+            return True
+    return False
 
 
 def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=False):
@@ -78,16 +97,18 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
     grads = [p.grad for p in parameters]
     norm_type, max_norm = float(norm_type), float(max_norm)
     # contiguous FP8 and plain gradients on this GPU go through the kernels that take them all at once, the others one by one
-    entries = [_entry(g) if norm_type in _KINDS else None for g in grads]
-    listed = [e for e in entries if e is not None]
-    total_norm = torch.tensor(0.)
+    entries = _entries(grads) if norm_type in _KINDS else [None] * len(grads)
+    listed = entries if None not in entries else [e for e in entries if e is not None]
     if listed:
         # norms, factor and clipping without the host waiting for any of them
-        norms, total_norm, coef = _backend.grad_norms(_backend.grad_table(listed), len(listed), norm_type, max_norm)
+        table = _backend.grad_table(listed)
+        norms, total_norm, coef = _backend.grad_norms(table, len(listed), norm_type, max_norm)
     if len(listed) < len(grads):
         listed_norms = iter(norms.unbind()) if listed else None
         total_norm = _join([(_norm(g, norm_type) if e is None else next(listed_norms)).to(grads[0].device)
                             for g, e in zip(grads, entries)], norm_type)
+    elif not grads:
+        total_norm = torch.tensor(0.)
     if error_if_nonfinite and torch.logical_or(total_norm.isnan(), total_norm.isinf()):
         raise RuntimeError(
             f'The total norm of order {norm_type} for gradients from `parameters` is non-finite, so it cannot be '
@@ -103,13 +124,15 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
         for g, e in zip(grads, entries):
             if e is None:
                 g.detach().mul_(coef)
-    elif max_norm == float('inf') or (any(map(_held_elsewhere, parameters)) and
+        if listed:
+            coef = coef.to(norms.device)
+    elif max_norm == float('inf') or (_held_elsewhere(parameters, grads) and
                                       not torch.cuda.is_current_stream_capturing() and not coef.item() < 1.0):
         # nothing to clip; what a graph has saved must then not count as changed, so the host waits to know, but only for those
         return total_norm
     if listed:
         for part in _rounds(listed):
-            _backend.grad_clip(_backend.grad_table(part), len(part), coef)
+            _backend.grad_clip(table if part is listed else _backend.grad_table(part), len(part), coef)
         changed = [g.meta.scale_inv if type(g) is ScalingTensor else g for g, e in zip(grads, entries) if e is not None]
         torch.autograd.graph.increment_version([t for t in changed if not t.is_inference()])
     return total_norm
