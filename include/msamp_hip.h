@@ -473,6 +473,8 @@ int msamp_adamw_f32(float* param, const void* grad, int grad_dtype, size_t n, fl
  * the call.  param: F32 / F16 / BF16 (scale null), or a scaled F16 weight with its meta's scale, scale_inv and amax[0] (all
  * rewritten: rule(max|p'|, old scale), 1 / scale, max|p'|; payload F16(p' * scale)).  grad: F32 / F16 / BF16, or E4M3 / E5M2 with
  * grad_scale_inv.  exp_avg, exp_avg_sq: F32.  The entry's own `scratch` is ignored.
+ * Parameters that share memory (payloads, moments, metas, or one's gradient with another's parameter) are stepped in the
+ * list's order: no launch holds two of them.
  * scratch: float32, 16-byte aligned, room for the largest scaled weight rounded up to four elements (with room for several
  * they share launches); words: MSAMP_F32_WORDS 32-bit words of scratch. */
 #define MSAMP_F32_BLOCKS 4096

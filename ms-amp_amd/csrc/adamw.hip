@@ -5,6 +5,7 @@
 #include "common.cuh"
 #include "raise_max.cuh"
 
+#include <algorithm>
 #include <type_traits>
 
 #include <cmath>
@@ -1764,6 +1765,46 @@ __global__ __launch_bounds__(kAdamThreads) void f32_list_requant_kernel(F32Table
     for (size_t i = done + threadIdx.x; i < to; i += kAdamThreads) out[i] = static_cast<uint16_t>(float_to_f16_bits(d.scratch[i] * s));
 }
 
+// How many of the list's first n entries can share a launch: those in front of the first one that another of them meets in
+// memory that either writes (that one is stepped after them, by a later launch).
+struct MemSpan {
+    uintptr_t lo, hi;
+    bool written;
+};
+static bool spans_collide(MemSpan* s, int n) {
+    std::sort(s, s + n, [](const MemSpan& a, const MemSpan& b) { return a.lo < b.lo; });
+    uintptr_t end_any = 0, end_written = 0;
+    for (int i = 0; i < n; ++i) {
+        if (s[i].lo < end_written || (s[i].written && s[i].lo < end_any)) return true;
+        end_any = std::max(end_any, s[i].hi);
+        if (s[i].written) end_written = std::max(end_written, s[i].hi);
+    }
+    return false;
+}
+static bool entries_collide(const msamp_f32_param* list, int n) {
+    MemSpan s[kF32List * 8];
+    int k = 0;
+    auto add = [&](const void* p, size_t bytes, bool written) {
+        const uintptr_t lo = reinterpret_cast<uintptr_t>(p);
+        s[k++] = {lo, lo + bytes, written};
+    };
+    for (int i = 0; i < n; ++i) {
+        const msamp_f32_param& e = list[i];
+        add(e.param, e.numel * hp_size(e.param_dtype), true);
+        add(e.exp_avg, e.numel * 4, true), add(e.exp_avg_sq, e.numel * 4, true);
+        add(e.grad, e.numel * (is_fp8(e.grad_dtype) ? 1 : hp_size(e.grad_dtype)), false);
+        if (e.scale != nullptr) add(e.scale, 4, true), add(e.scale_inv, 4, true), add(e.amax, 4, true);
+        if (e.grad_scale_inv != nullptr) add(e.grad_scale_inv, 4, false);
+    }
+    return spans_collide(s, k);
+}
+static int entries_apart(const msamp_f32_param* list, int n) {
+    if (n < 2 || !entries_collide(list, n)) return n;
+    int k = 1;
+    while (k + 1 <= n && !entries_collide(list, k + 1)) ++k;
+    return k;
+}
+
 }    // namespace msamp
 
 using namespace msamp;
@@ -2004,7 +2045,7 @@ int msamp_adamw_f32_list(const msamp_f32_param* list, int n, float* scratch, siz
         F32Table t = {};
         size_t room = scratch_elems, total = 0;
         bool any_scaled = false;
-        for (; t.n < kF32List && from < n; ++from) {
+        for (const int end = from + entries_apart(list + from, std::min(n - from, kF32List)); from < end; ++from) {
             msamp_f32_param e = list[from];
             if (e.scale != nullptr) {
                 const size_t need = (e.numel + 3) / 4 * 4;

@@ -6,6 +6,7 @@ kept in high precision (biases, norm weights) with quantized moments take one la
 everything else follows the reference's two-stage recipe tensor by tensor.
 """
 
+import itertools
 import math
 
 import numpy as np
@@ -488,26 +489,18 @@ class LBAdamW(LBAdamWBase):
 
     def _f32_flush(self, *, beta1, beta2, lr, weight_decay, eps, maximize):
         pending, self._f32_pending = self._f32_pending, []
-        # parameters that share memory are stepped one after the other, as everywhere else: a launch holds none of them together
-        batches, spans = [pending], [self._f32_spans(row) for _, row, _, _ in pending]
-        if _collide([s for row_spans in spans for s in row_spans]):
-            batches, held = [], []
-            for entry, row_spans in zip(pending, spans):
-                if not batches or _collide(held + row_spans):
-                    batches.append([])
-                    held = []
-                batches[-1].append(entry)
-                held += row_spans
-        for batch in batches:
-            by_step = {}
-            for step, row, p, g in batch:
-                rows, scaled = by_step.setdefault(step, ([], []))
-                rows.append(row)
-                if row[1]:
-                    scaled.append(row[9])
-            for step, (rows, scaled) in by_step.items():
-                _backend.adamw_f32_list(rows, scaled, torch.device('cuda', torch.cuda.current_device()), lr, beta1, beta2, eps,
-                                        weight_decay, step, self.bias_correction, self.use_adam, maximize)
+        runs = {}
+        for step, row, _, _ in pending:
+            runs.setdefault(step, []).append(row)
+        # one call per step count; within a call parameters that share memory are stepped in their order, and where step counts
+        # differ the order across the calls is kept as well
+        if len(runs) > 1 and _collide([s for _, row, _, _ in pending for s in self._f32_spans(row)]):
+            runs = [(step, [row for _, row, _, _ in run]) for step, run in itertools.groupby(pending, lambda entry: entry[0])]
+        else:
+            runs = runs.items()
+        for step, rows in runs:
+            _backend.adamw_f32_list(rows, [row[9] for row in rows if row[1]], torch.device('cuda', torch.cuda.current_device()), lr,
+                                    beta1, beta2, eps, weight_decay, step, self.bias_correction, self.use_adam, maximize)
         written = [p.value if isinstance(p, ScalingTensor) else p for _, _, p, _ in pending]
         torch.autograd.graph.increment_version([t for t in written if t.dtype != torch.float32 and not t.is_inference()])
 

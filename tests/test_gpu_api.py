@@ -933,8 +933,10 @@ def test_float32_moment_step_over_a_list_has_the_bits_of_one_parameter_at_a_time
         assert same_float(a, b), k
 
 
-def test_float32_moment_step_of_parameters_that_share_memory(monkeypatch):
-    """Parameters that overlap are stepped one after the other in their order, whatever path each of them takes: views of one
+@pytest.mark.parametrize('late', [False, True])
+def test_float32_moment_step_of_parameters_that_share_memory(monkeypatch, late):
+    """Parameters that overlap are stepped one after the other in their order, whatever path each of them takes and also where
+    one has come later than the others and counts other steps: views of one
     buffer with different starts, the same view twice, one that is not contiguous (stepped at once, not from the list)
     between two that are, and one whose gradient is another parameter."""
     runs = []
@@ -947,10 +949,12 @@ def test_float32_moment_step_of_parameters_that_share_memory(monkeypatch):
         opt = LBAdamW(params, lr=1e-2, weight_decay=0.1, exp_avg_dtype=torch.float32, exp_avg_sq_dtype=torch.float32)
         if not listed:
             monkeypatch.setattr(LBAdamW, '_f32_row', classmethod(lambda cls, *a: None))
-        for _ in range(3):
+        for step in range(3):
             for p in params[:-1]:
                 p.grad = torch.randn(p.shape, device='cuda', generator=gen)
             params[-1].grad = flat[3000:6000]
+            if late and step == 0:
+                params[1].grad = None
             opt.step()
         monkeypatch.undo()
         runs.append([flat, other] + [opt.state[p][k] for p in params for k in ('exp_avg', 'exp_avg_sq')])
