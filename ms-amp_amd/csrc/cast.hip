@@ -185,8 +185,9 @@ __global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restri
 // float32 sum per column in registers; the four wavefronts of a workgroup take rows in turn and add up through LDS in a
 // fixed order, and the sums of the slabs are added by colsum_finish_kernel, 16 runs of slabs at a time: the same bits on
 // every run, and no chain longer than a slab's quarter, a sixteenth of the slabs, or 16.
-// Slabs: about 2048 workgroups (eight a CU), so that the partial sums stay a hundredth of the tensor, and at least 16
-// rows.  The workgroups' maxima go to memory and are folded into the amax by the second kernel: an atomic each, on a
+// Slabs: about 2048 workgroups (eight a CU), and at least 16 rows.  The partial sums, written once and read once, are 4 / (rows
+// of a slab * bytes of an element) of the tensor and 4 MiB at most: an eighth of 8192 x 2048 bfloat16 (16 rows), a 32nd of
+// 12605 x 4304 float16 (64).  The workgroups' maxima go to memory and are folded into the amax by the second kernel: an atomic each, on a
 // cell that the window update has just cleared, held the cast of 8192 x 2048 bfloat16 at 40.8 us instead of 12.3.
 // 12605 x 4304 float16: 26 us for the cast and 48 us for the sum (two clears and a reduction) before; FP8Linear
 // 12605 x 1200 -> 4304 forward and backward 387 -> 339 us, a training step of two 2048-wide blocks at 8192 tokens
