@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kAdamThreads) void stage2_kernel(const float* __res
 // ---- fused multi-tensor step -------------------------------------------------------------------
 constexpr int kEPT = 16;                                   // elements per thread per step
 // tensors of more chunks than these look at their maxima's words before they raise them (raise_max.cuh)
-constexpr size_t kAmaxLookChunks = 448, kSpecLookChunks = 384;
+constexpr size_t kAmaxLookChunks = 320, kSpecLookChunks = 384;
 constexpr int kSteps = MSAMP_ADAMW_CHUNK / (kAdamThreads * kEPT);    // 4
 
 template <int WDT>

@@ -11,7 +11,8 @@
 //   chunks                                                 256       384       512       768      1024       1536       2048
 //   fused_amax_kernel (stores nothing, three maxima)    675, 730  684, 708  683, 710  716, 700  763, 702   957, 690  1195, 724
 //   fused_spec_kernel (stores, three maxima)            463, 474  464, 463  483, 457  500, 454  566, 454  1000, 445  1295, 471
-// (Four tensors of 512 chunks by themselves take 112 and 104 us in the first of them, hence its line below that.)
+// (Few tensors by themselves gain from smaller sizes on, and so the line of the first lies below its row above: eight of 256
+// chunks 100, 99, of 384 141, 137, of 512 201, 198.)
 // plain_amax_kernel (two maxima, 120 M parameters) is within 1 % either way up to 1536 chunks, and bucket_amax_kernel (one)
 // loses up to there (120 M elements, 256 chunks: 69, 148; 1536: 86, 96): they never look.
 #pragma once

@@ -804,12 +804,12 @@ def grad_norms(table, n, norm_type, max_norm):
 
 def fp8_norms(values, scale_invs, fp8_dt, norm_type):
     """Per-tensor p-norms (p = 1, 2 or inf) of FP8 payloads times their scale_inv, as one float32 vector."""
-    for v in values:
-        _gpu(v, 'fp8 tensor')
-        if not v.is_contiguous():
-            raise ValueError('fp8 tensors must be contiguous')
-    table = grad_table((_ptr(v), _ptr(si), v.numel(), fp8_dt) for v, si in zip(values, scale_invs))
-    return grad_norms(table, len(values), norm_type, float('inf'))[0]
+    words = []
+    for v, si in zip(values, scale_invs):
+        if not (v.is_cuda and v.is_contiguous()):
+            raise ValueError('fp8 tensors must be contiguous, in GPU memory')
+        words += (v.data_ptr(), si.data_ptr(), v.numel(), fp8_dt)
+    return grad_norms(array.array('q', words), len(values), norm_type, float('inf'))[0]
 
 
 def grad_clip(table, n, factor):

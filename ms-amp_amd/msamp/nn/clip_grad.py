@@ -74,9 +74,9 @@ def _join(norms, norm_type):
     return torch.norm(torch.stack(norms), norm_type)
 
 
-def _held_elsewhere(parameters, grads):
+def _held_elsewhere(owners, grads):
     """True if a graph may have saved one of the gradients: something holds it beside its owner and Python, or a view of it."""
-    for p, g in zip(parameters, grads):
+    for p, g in zip(owners, grads):
         if type(g) is ScalingTensor:
             if g.meta.scale_inv._use_count() > 1:
                 return True
@@ -93,8 +93,12 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
         parameters = [parameters]
     else:
         parameters = list(parameters)
-    parameters = [p for p in parameters if p.grad is not None]
-    grads = [p.grad for p in parameters]
+    owners, grads = [], []
+    for p in parameters:
+        g = p.grad
+        if g is not None:
+            owners.append(p)
+            grads.append(g)
     norm_type, max_norm = float(norm_type), float(max_norm)
     # contiguous FP8 and plain gradients on this GPU go through the kernels that take them all at once, the others one by one
     entries = _entries(grads) if norm_type in _KINDS else [None] * len(grads)
@@ -126,7 +130,7 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
                 g.detach().mul_(coef)
         if listed:
             coef = coef.to(norms.device)
-    elif max_norm == float('inf') or (_held_elsewhere(parameters, grads) and
+    elif max_norm == float('inf') or (_held_elsewhere(owners, grads) and
                                       not torch.cuda.is_current_stream_capturing() and not coef.item() < 1.0):
         # nothing to clip; what a graph has saved must then not count as changed, so the host waits to know, but only for those
         return total_norm

@@ -216,7 +216,7 @@ def test_fused_step_sparse_gradient_and_zero_state(be):
         _check(dev[0], t, fp8.E4M3, fp8.E5M2, step, **kw)
 
 
-@pytest.mark.parametrize('chunks', [384, 448])
+@pytest.mark.parametrize('chunks', [320, 384])
 def test_maxima_of_tensors_around_the_looking_lines(be, chunks):
     """Tensors of as many chunks as the first passes raise their maxima without a look at the words for, and one element
     more: repetitions of a small tensor, so every one of them has the small one's maxima, scales and codes, in place and in
