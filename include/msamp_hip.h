@@ -264,7 +264,7 @@ typedef struct msamp_grad {
 int msamp_grad_norms(const msamp_grad* grads, int n, int norm_kind, float max_norm, double* partials, float* norms, float* total,
                      float* coef, msamp_stream_t stream);
 /* Multiplies every tensor of the list by *coef (device) if that is below 1: an FP8 tensor through its scale_inv, a
- * 16-bit one with the factor rounded to its type.  No tensor may appear twice. */
+ * 16-bit one with the factor rounded to its type.  What it writes of two tensors (the values, or the scale_inv) must not overlap. */
 int msamp_grad_clip(const msamp_grad* grads, int n, const float* coef, msamp_stream_t stream);
 
 /* tex.te_gemm as Gemm.fp8_gemm calls it (gemm.py:121-144; transa=True, transb=False):

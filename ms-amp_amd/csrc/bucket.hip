@@ -192,7 +192,7 @@ __device__ __forceinline__ void fp8_norm_chunk(const uint8_t* q, size_t base, si
 // (two to four launches of 1.3 to 4 us and 6 to 9 us of host time each), and the host waited for the factor.
 // The descriptors travel as kernel arguments: no table in memory, no copy, nothing kept between calls.
 // 32 FP8 gradients of 4 M codes, quantized as a bucket and clipped: 365 us in all with the calls per tensor, of which the
-// GPU worked 150; 117 us now (norms 24 us, finish 5, clipping 4).  A small model's 13 parameters: 0.2 ms a step less.
+// GPU worked 150; 110 us now (norms 24 us, finish 5, clipping 4).  A small model's 13 parameters: 0.2 ms a step less.
 constexpr int kGradTable = 64;         // 64 descriptors are 1.9 KB of the 4 KB that kernel arguments may take
 constexpr int kGradBlocks = MSAMP_GRAD_BLOCKS;    // eight workgroups per compute unit; beyond that each takes a run of chunks
 struct GradTable {
