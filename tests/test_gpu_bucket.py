@@ -465,3 +465,25 @@ def test_clip_where_workgroups_take_runs_of_chunks(norm_type):
     coef = torch.clamp((want / 7) / (total + 1e-6), max=1.0)
     for g, p in zip(grads, plain):
         assert torch.equal(g.meta.scale_inv if hasattr(g, 'meta') else g, p.mul_(coef))
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('level', ['O1', 'O2'])
+def test_clip_does_not_wait_in_a_training_step(level, dtype):
+    """Gradients as a step leaves them (FP8 weights, biases beside them, a norm's weights; a first and a later step): nothing
+    else holds them, so clipping synchronizes nothing."""
+    import msamp
+    torch.manual_seed(1)
+    model = torch.nn.Sequential(torch.nn.Linear(64, 64), torch.nn.LayerNorm(64), torch.nn.GELU(), torch.nn.Linear(64, 32)).cuda().to(dtype)
+    model, optimizer = msamp.initialize(model, torch.optim.AdamW(model.parameters()), opt_level=level)
+    x = torch.randn(48, 64, device='cuda').to(dtype)
+    for _ in range(3):
+        optimizer.zero_grad()
+        model(x).float().square().mean().backward()
+        torch.cuda.synchronize()
+        torch.cuda.set_sync_debug_mode('error')
+        try:
+            msamp.clip_grad_norm_(model.parameters(), 1e-3)
+        finally:
+            torch.cuda.set_sync_debug_mode('default')
+        optimizer.step()
