@@ -733,8 +733,8 @@ def test_fp8linear_weight_gradient_uses_the_fused_kernel_and_matches(be, large_t
 
 
 def test_gemm_with_fused_cast_many_random_cases(be, large_tiles_only):
-    """A sweep over seeds, scales, layouts and output types, with few tiles (where the unfused row-major GEMM runs the
-    generic kernel) and many: every case equal to the two steps, to the bit."""
+    """A sweep over seeds, scales, layouts and output types, with few tiles and many: every case equal to the two
+    steps, to the bit."""
     cases = 0
     for it in range(12):
         for (m, n, k), kmajor in (((1024, 768, 384), True), ((256, 256, 1024), False), ((3072, 3072, 256), False),
