@@ -320,6 +320,77 @@ int msamp_fp8_gemm_cast(const uint8_t* a, int a_type, const float* a_scale_inv, 
                         float* scale, float* amax, float* scale_inv, int m, int n, int k, int margin, int flags,
                         void* workspace, msamp_stream_t stream);
 
+/* One direction of an FP8Linear layer as one call (the reference's sequence of calls: msamp/nn/functional.py:20-123): the
+ * entry points named below, one after the other on `stream`, with the arguments a layer in gated scaling gives them.  Every
+ * field is eight bytes wide.  Results, metas and error codes are those of the entry points.
+ *
+ * Forward: msamp_cast_to_fp8_gated (x to E4M3), msamp_cast_scaled_to_fp8 (the scaled 16- or 32-bit weight to E4M3; w_meta
+ * receives {scale, scale_inv, update count, amax window} as four-byte words), msamp_fp8_gemm with the bias.  d_in must be a
+ * multiple of 16. */
+typedef struct msamp_linear_forward_args {
+    const void* x;             /* [tokens][d_in], x_dtype */
+    int64_t x_dtype, tokens, d_in, d_out;
+    float* x_scale;            /* the input meta */
+    float* x_amax;
+    float* x_scale_inv;
+    const int32_t* x_counter;
+    int64_t x_window;
+    uint8_t* x_codes;          /* out: [tokens][d_in] E4M3 */
+    const void* w;             /* [d_out][d_in], w_dtype, the values times their scale */
+    int64_t w_dtype;
+    const float* w_amax;
+    const float* w_scale_inv;
+    int64_t w_window;
+    uint8_t* w_codes;          /* out: [d_out][d_in] E4M3 */
+    float* w_meta;             /* out: 3 + w_window words */
+    void* y;                   /* out: [tokens][d_out], y_dtype */
+    int64_t y_dtype;
+    const void* bias;          /* nullable: [d_out], bias_dtype */
+    int64_t bias_dtype;
+    int64_t flags;             /* MSAMP_FLAG_TWO_PASS */
+    void* workspace;
+} msamp_linear_forward_args;
+int msamp_linear_forward(const msamp_linear_forward_args* args, msamp_stream_t stream);
+
+/* Backward: msamp_cast_to_fp8_gated of dy to E5M2 (msamp_cast_to_fp8_colsum_gated if bias_sum is given); dx with
+ * msamp_fp8_gemm_kmajor if dx is given; and if wq is given the weight gradient, added to the dequantized old one if there is
+ * one: msamp_fp8_gemm_ksplit (if it splits the product and the scratch has room) or msamp_fp8_gemm_kmajor, and
+ * msamp_cast_to_fp8_intime with MSAMP_FLAG_NAN_TO_INF.  (A product that msamp_fp8_gemm_cast takes is better left to that: without
+ * wq the codes of dy are there for it.)  Shapes as msamp_fp8_gemm_kmajor takes them.
+ * msamp_linear_backward_scratch: the bytes of `scratch` (16-byte aligned) to give, and the least that will do. */
+typedef struct msamp_linear_backward_args {
+    const void* dy;            /* [tokens][d_out], dy_dtype */
+    int64_t dy_dtype, tokens, d_in, d_out;
+    float* g_scale;            /* the output gradient's meta */
+    float* g_amax;
+    float* g_scale_inv;
+    const int32_t* g_counter;
+    int64_t g_window;
+    uint8_t* dy_codes;         /* out: [tokens][d_out] E5M2 */
+    const uint8_t* x_codes;    /* from the forward call */
+    const float* x_scale_inv;
+    const uint8_t* w_codes;
+    const float* w_scale_inv;
+    void* dx;                  /* nullable, out: [tokens][d_in], out_dtype */
+    int64_t out_dtype;         /* of dx, and of the weight gradient before its cast */
+    uint8_t* wq;               /* nullable, out: [d_out][d_in] E4M3 */
+    float* q_scale;            /* the weight gradient's meta */
+    float* q_amax;
+    float* q_scale_inv;
+    const uint8_t* old_codes;  /* nullable: the weight gradient to add to, [d_out][d_in], old_type (may share q_scale_inv) */
+    const float* old_scale_inv;
+    int64_t old_type;
+    void* bias_sum;            /* nullable, out: [d_out], bias_sum_dtype */
+    int64_t bias_sum_dtype;
+    int64_t flags;             /* MSAMP_FLAG_TWO_PASS */
+    void* scratch;
+    int64_t scratch_bytes;
+    void* workspace;
+} msamp_linear_backward_args;
+int msamp_linear_backward_scratch(int tokens, int d_in, int d_out, int dy_dtype, int out_dtype, int want_wgrad, int want_bias,
+                                  size_t* bytes, size_t* least);
+int msamp_linear_backward(const msamp_linear_backward_args* args, msamp_stream_t stream);
+
 /* Tile walks of the 256 x 256-tile kernel (no counterpart in the reference, whose GEMM is cuBLASLt behind
  * transformer_engine_wrapper.py:63-103).  Which workgroup takes which output tile decides what the 32 compute units of
  * an XCD share through their L2; the library picks a walk from the shape by rules measured on Llama shapes, and the

@@ -9,6 +9,7 @@ the GPU, the call raises.
 import array
 import ctypes
 import os
+import struct
 
 import torch
 import torch.distributed as _dist
@@ -58,6 +59,9 @@ _SIGNATURES = {
     'msamp_fp8_gemm_ksplit_scratch': ([_i, _i, _i, _vp], _i),
     'msamp_fp8_gemm_ksplit': ([_vp, _i, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp, _sz, _vp], _i),
     'msamp_fp8_gemm_cast': ([_vp, _i, _vp, _i, _vp, _i, _vp, _i, _vp, _i, _i, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp], _i),
+    'msamp_linear_forward': ([ctypes.c_char_p, _vp], _i),
+    'msamp_linear_backward_scratch': ([_i, _i, _i, _i, _i, _i, _i, _vp, _vp], _i),
+    'msamp_linear_backward': ([ctypes.c_char_p, _vp], _i),
     'msamp_mfma_probe': ([_vp, _vp, _i, _i, _i, _vp, _vp], _i),
     'msamp_set_small_tile_limit': ([_i], None),
     'msamp_scale_update_groups': ([_vp, _i, _i, _vp], _i),
@@ -698,9 +702,91 @@ def fp8_gemm_cast(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, hp_dtype, q_dt, sc
     return out
 
 
+# ---- a linear layer's directions, one call each -----------------------------------------------------------------
+_LINEAR_FORWARD = struct.Struct('@24q')     # msamp_linear_forward_args
+_LINEAR_BACKWARD = struct.Struct('@30q')    # msamp_linear_backward_args
+
+
+def gemm_walk_settled(m, n, k, a_kmajor, b_kmajor):
+    """True if fp8_gemm would not time the walks of this problem (see _tune_walk)."""
+    return not _tune_walks or ((n + 255) // 256) * ((m + 255) // 256) < _TUNE_MIN_TILES or k < 512 or k % 128 != 0 or \
+        (m, n, k, a_kmajor, b_kmajor) in _walk_seen
+
+
+_small_tile_limit = 128
+
+
+def gemm_cast_declines(m, n, k):
+    """True if fp8_gemm_cast answers None for this problem whatever the types: shapes it has no form for, and those that are
+    better off with 128 x 128 tiles and a cast (takes_small_tiles() of the library)."""
+    big, limit = ((n + 255) // 256) * ((m + 255) // 256), _small_tile_limit
+    return m % 256 != 0 or n % 256 != 0 or k % 128 != 0 or (k > 384 and (big <= limit // 2 or (big <= limit and k >= 3072)))
+
+
+def linear_forward(x, x_meta, w, w_meta, out_dtype, bias):
+    """y = x . w^T (+ bias) through msamp_linear_forward.  x: contiguous [tokens, d_in], cast with x_meta (gated scaling); w: the
+    contiguous scaled payload [d_out, d_in] of a weight with w_meta.  Returns y, the E4M3 codes of x and of w, and the words
+    {scale, scale_inv, update count, amax window} of the codes of w."""
+    lib = load()
+    (tokens, d_in), d_out, device, window = x.shape, w.shape[0], x.device, w_meta.window_size
+    x_codes = torch.empty((tokens, d_in), dtype=torch.uint8, device=device)
+    w_codes = torch.empty((d_out, d_in), dtype=torch.uint8, device=device)
+    words = torch.empty(3 + window, dtype=torch.float32, device=device)
+    y = torch.empty((tokens, d_out), dtype=out_dtype, device=device)
+    args = _LINEAR_FORWARD.pack(
+        x.data_ptr(), _TORCH_TO_DT[x.dtype], tokens, d_in, d_out, x_meta.scale.data_ptr(), x_meta.amax.data_ptr(),
+        x_meta.scale_inv.data_ptr(), x_meta.amax_counter.data_ptr(), x_meta.window_size, x_codes.data_ptr(), w.data_ptr(),
+        _TORCH_TO_DT[w.dtype], w_meta.amax.data_ptr(), w_meta.scale_inv.data_ptr(), window, w_codes.data_ptr(), words.data_ptr(),
+        y.data_ptr(), _TORCH_TO_DT[out_dtype], 0 if bias is None else bias.data_ptr(),
+        DT_F32 if bias is None else _TORCH_TO_DT[bias.dtype], FLAG_TWO_PASS if _two_pass_only() else 0, workspace(device).data_ptr()
+    )
+    _check(lib.msamp_linear_forward(args, _stream()), 'msamp_linear_forward')
+    return y, x_codes, w_codes, words
+
+
+def linear_backward(dy, g_meta, x_codes, x_scale_inv, w_codes, w_scale_inv_ptr, out_dtype, need_dx, q_meta, old, bias_dtype):
+    """Gradients of linear_forward through msamp_linear_backward: the E5M2 codes of dy, dx in out_dtype (None unless need_dx), the
+    E4M3 codes of the weight gradient (None unless q_meta, its meta, is given; `old`, a ScalingTensor or None, is added to it) and
+    the column sums of dy (None unless bias_dtype is given)."""
+    lib = load()
+    (tokens, d_out), d_in, device = dy.shape, x_codes.shape[1], dy.device
+    dt, out_dt = _TORCH_TO_DT[dy.dtype], _TORCH_TO_DT[out_dtype]
+    codes = torch.empty((tokens, d_out), dtype=torch.uint8, device=device)
+    dx = torch.empty((tokens, d_in), dtype=out_dtype, device=device) if need_dx else None
+    wq = torch.empty((d_out, d_in), dtype=torch.uint8, device=device) if q_meta is not None else None
+    sums = torch.empty((d_out, ), dtype=bias_dtype, device=device) if bias_dtype is not None else None
+    scratch, size = None, 0
+    if wq is not None or sums is not None:
+        sizes = (ctypes.c_size_t * 2)()
+        where = ctypes.addressof(sizes)
+        _check(lib.msamp_linear_backward_scratch(tokens, d_in, d_out, dt, out_dt, wq is not None, sums is not None, where, where + 8),
+               'msamp_linear_backward_scratch')
+        size, least = sizes
+        try:
+            scratch = torch.empty((size, ), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            if size == least:
+                raise
+            size = least    # without the room for a product in parts of K
+            scratch = torch.empty((size, ), dtype=torch.uint8, device=device)
+    args = _LINEAR_BACKWARD.pack(
+        dy.data_ptr(), dt, tokens, d_in, d_out, g_meta.scale.data_ptr(), g_meta.amax.data_ptr(), g_meta.scale_inv.data_ptr(),
+        g_meta.amax_counter.data_ptr(), g_meta.window_size, codes.data_ptr(), x_codes.data_ptr(), x_scale_inv.data_ptr(),
+        w_codes.data_ptr(), w_scale_inv_ptr, 0 if dx is None else dx.data_ptr(), out_dt, *((0, 0, 0, 0) if wq is None else
+        (wq.data_ptr(), q_meta.scale.data_ptr(), q_meta.amax.data_ptr(), q_meta.scale_inv.data_ptr())),
+        *((0, 0, 0) if wq is None or old is None else (old.value.data_ptr(), old.meta.scale_inv.data_ptr(), int(old.meta.qtype))),
+        0 if sums is None else sums.data_ptr(), DT_F32 if sums is None else _TORCH_TO_DT[bias_dtype],
+        FLAG_TWO_PASS if _two_pass_only() else 0, 0 if scratch is None else scratch.data_ptr(), size, workspace(device).data_ptr()
+    )
+    _check(lib.msamp_linear_backward(args, _stream()), 'msamp_linear_backward')
+    return codes, dx, wq, sums
+
+
 def set_small_tile_limit(big_tiles):
     """Row-major GEMMs of at most this many 256 x 256 output tiles run 128 x 128 tiles (default 128, 0 = never; negative:
     row-major ones run the generic kernel)."""
+    global _small_tile_limit
+    _small_tile_limit = int(big_tiles)
     load().msamp_set_small_tile_limit(int(big_tiles))
 
 

@@ -33,13 +33,17 @@ class ScalingMeta:
     def _uninitialized(cls, qtype, window_size, device, group=None):
         """A meta whose four tensors are views of one uninitialised buffer {scale, scale_inv, counter, amax window}, for
         callers whose kernel writes every field itself."""
+        return cls._of_words(qtype, torch.empty(3 + window_size, dtype=torch.float32, device=device), group)
+
+    @classmethod
+    def _of_words(cls, qtype, slab, group=None):
+        """A meta whose four tensors are views of the words {scale, scale_inv, counter, amax window}."""
         self = cls.__new__(cls)
-        slab = torch.empty(3 + window_size, dtype=torch.float32, device=device)
         self.qtype = qtype
         self.scale, self.scale_inv = slab[0], slab[1]
         self.amax_counter = slab[2:3].view(torch.int32).reshape(())
         self.amax = slab[3:]
-        self.window_size = window_size
+        self.window_size = slab.numel() - 3
         self.group = group
         self.locked = False
         return self

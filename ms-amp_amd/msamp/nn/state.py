@@ -93,10 +93,10 @@ class ModelState:
             return
         for key, meta in scaling_metas.items():
             flat = self._flattened_scaling_metas[key]
-            ModelState._check_in_mem(meta.scale, flat['scales'])
-            ModelState._check_in_mem(meta.scale_inv, flat['scales_inv'])
-            ModelState._check_in_mem(meta.amax, flat['amaxs'])
-            ModelState._check_in_mem(meta.amax_counter, flat['amax_counters'])
+            for inner, outer in ((meta.scale, flat['scales']), (meta.scale_inv, flat['scales_inv']), (meta.amax, flat['amaxs']),
+                                 (meta.amax_counter, flat['amax_counters'])):
+                if not 0 <= inner.data_ptr() - outer.data_ptr() <= outer.nbytes - inner.nbytes:
+                    ModelState._check_in_mem(inner, outer)
 
     def register_scaling_metas(self, model, group=None):
         """Collect `scaling_metas` of every module of `model` and (re)flatten all registered ones."""

@@ -997,3 +997,57 @@ def test_scratch_that_cannot_be_had_costs_launches_only(monkeypatch):
         assert len(refused) == (limit == 5000)
         runs.append([t for p in params for t in (p.value, p.meta.scale, p.meta.scale_inv, p.meta.amax)])
     assert all(same_float(x, y) for x, y in zip(*runs))
+
+
+@pytest.mark.parametrize('tokens,d_in,d_out', [(256, 512, 768), (2048, 256, 512), (300, 272, 144), (129, 16, 16), (96, 128, 512),
+                                               (200, 40, 24), (2500, 512, 512)])
+@pytest.mark.parametrize('dtype,bias_dtype', [(torch.bfloat16, None), (torch.float16, torch.float16), (torch.float32, torch.float32),
+                                              (torch.bfloat16, torch.float32)])
+def test_a_linear_layer_by_one_call_each_way_has_the_bits_of_the_single_calls(monkeypatch, tokens, d_in, d_out, dtype, bias_dtype):
+    """Outputs, gradients and metas over warm-up and delayed scaling, with the weight gradient new and added to an old one, against
+    the same layer with every entry point called from Python.  Shapes that only the single calls take are among them."""
+    from msamp import _backend
+    from msamp.nn import functional
+    gen = torch.Generator(device='cuda').manual_seed(tokens + d_in)
+    draw = lambda *shape: torch.randn(shape, device='cuda', generator=gen)
+    w0, b0 = draw(d_out, d_in) * 0.05, draw(d_out)
+    xs = [draw(tokens, d_in).to(dtype) * f for f in (1.0, 3.0, 0.2)]
+    dys = [draw(tokens, d_out).to(dtype) * f for f in (1e-3, 1e-2, 1e-4)]
+    calls = []
+    for name in ('linear_forward', 'linear_backward'):
+        monkeypatch.setattr(_backend, name, lambda *a, real=getattr(_backend, name), name=name: (calls.append(name), real(*a))[1])
+
+    def run():
+        model_state.clear()
+        lin = torch.nn.Linear(d_in, d_out, bias=bias_dtype is not None).cuda().to(bias_dtype or dtype)
+        with torch.no_grad():
+            lin.weight.copy_(w0)
+            if bias_dtype is not None:
+                lin.bias.copy_(b0)
+        model = LinearReplacer.replace(lin, Dtypes.kfloat16)
+        opt = LBAdamW(model.parameters(), lr=0.0)
+        out = []
+        for step in range(18):
+            for micro in range(2):
+                x = xs[(step + micro) % 3].clone().requires_grad_(True)
+                y = model(x)
+                y.backward(dys[(step + 2 * micro) % 3])
+                g = model.weight.grad
+                out += [y.detach(), x.grad, g.value, g.meta.scale_inv.clone()]
+            if bias_dtype is not None:
+                out.append(model.bias.grad.clone())
+                model.bias.grad = None
+            out += [t.clone() for m in model.scaling_metas.values() for t in (m.scale, m.scale_inv, m.amax)]
+            model.weight.grad = None
+            opt.step()
+        return out
+
+    got = run()
+    taken = list(calls)
+    for name in ('_forward_in_one_call', '_backward_in_one_call'):
+        monkeypatch.setattr(functional, name, lambda *a: False)
+    calls.clear()
+    want = run()
+    assert not calls and taken.count('linear_forward') == (36 if d_in % 16 == 0 else 0)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a.view(torch.uint8) if a.dim() else a, b.view(torch.uint8) if b.dim() else b), i

@@ -420,3 +420,17 @@ int main() {
     subprocess.run(['g++', '-O2', '-o', str(exe), str(cpp)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0 and out.stdout.strip() == 'OK 78400', out.stdout[-300:]
+
+
+@pytest.mark.parametrize('name', ['forward', 'backward'])
+def test_argument_blocks_of_the_linear_calls_have_the_fields_of_the_header(name):
+    """The blocks are packed by position: as many eight-byte words as the struct has members, and no member that is not eight
+    bytes wide."""
+    from msamp import _backend
+    header = open(os.path.join(ROOT, 'include', 'msamp_hip.h')).read()
+    body = re.search(r'typedef struct msamp_linear_%s_args \{(.*?)\}' % name, header, re.S).group(1)
+    members = [m.strip() for m in re.sub(r'/\*.*?\*/', '', body, flags=re.S).split(';') if m.strip()]
+    assert all('*' in m or m.startswith('int64_t ') for m in members)
+    fields = sum(len(m.split(',')) for m in members)
+    packer = _backend._LINEAR_FORWARD if name == 'forward' else _backend._LINEAR_BACKWARD
+    assert packer.size == 8 * fields
