@@ -356,7 +356,7 @@ int msamp_linear_forward(const msamp_linear_forward_args* args, msamp_stream_t s
  * msamp_fp8_gemm_kmajor if dx is given; and if wq is given the weight gradient, added to the dequantized old one if there is
  * one: msamp_fp8_gemm_ksplit (if it splits the product and the scratch has room) or msamp_fp8_gemm_kmajor, and
  * msamp_cast_to_fp8_intime with MSAMP_FLAG_NAN_TO_INF.  (A product that msamp_fp8_gemm_cast takes is better left to that: without
- * wq the codes of dy are there for it.)  Shapes as msamp_fp8_gemm_kmajor takes them.
+ * wq the codes of dy are there for it.)  Shapes as msamp_fp8_gemm_kmajor takes them, but for K, which may be a single slice.
  * msamp_linear_backward_scratch: the bytes of `scratch` (16-byte aligned) to give, and the least that will do. */
 typedef struct msamp_linear_backward_args {
     const void* dy;            /* [tokens][d_out], dy_dtype */
@@ -411,12 +411,12 @@ int msamp_fp8_gemm_tune(const uint8_t* a, int a_type, const float* a_scale_inv, 
                         const float* b_scale_inv, int b_kmajor, void* d, int d_dtype, int m, int n, int k, const void* bias,
                         int bias_dtype, int* chosen, msamp_stream_t stream);
 
-/* msamp_fp8_gemm with row-major operands runs 256 x 256 output tiles, one workgroup each; a problem with few of them
- * (a 2048 x 2048 output has 64, a quarter of the compute units) runs 128 x 128 tiles instead when it has at most
- * `big_tiles` of the large ones (at most half that many if K < 3072) and K is more than 384.  Same bits either way.
- * Default 128 (up to two small tiles per compute unit: measured faster up to there); 0 = the large tile always; negative:
- * every row-major product by the generic kernel that K of at most 128 and operands of 4 GiB and more take (for comparisons:
- * slower, same bits).  Process-wide; no counterpart in the reference. */
+/* The GEMM runs 256 x 256 output tiles, one workgroup to a compute unit, where there are enough of them, and 128 x 128 tiles
+ * otherwise: two workgroups to a compute unit if the product has at most two such tiles a unit (at most one if K is more than
+ * 2048), or a single slice of K; one, with the whole LDS, for longer K.  Same bits whichever.  To compare the kernels, any value
+ * but the default, 128, switches the form with two workgroups off: at most `big_tiles` large tiles (at most half that many if K <
+ * 3072) with K of more than 384 then run small ones; 0 = the large tile always; negative: every row-major product by the generic
+ * kernel that operands of 4 GiB and more take.  Process-wide; no counterpart in the reference. */
 void msamp_set_small_tile_limit(int big_tiles);
 
 /* Calibration aid, no counterpart in the reference: `workgroups` workgroups of four wavefronts each issue

@@ -21,9 +21,10 @@ static int dispatch_pair(int x_type, int y_type, const GemmCall& c) {
 
 // K-major operands: only the direct-to-LDS kernels read them, so the shape must suit them: two slices of K, rows that are
 // read 16 bytes at a time (a K-major operand's row count and a row-major one's K are its leading dimension)
-static bool kmajor_shape_ok(int NR, int NC, int K, bool xt, bool yt) {
-    return K > kBK && fits_offsets(NR, NC, K) && (xt ? NR % 16 == 0 : K % 16 == 0) && (yt ? NC % 16 == 0 : K % 16 == 0);
+static bool kmajor_rows_ok(int NR, int NC, int K, bool xt, bool yt) {
+    return fits_offsets(NR, NC, K) && (xt ? NR % 16 == 0 : K % 16 == 0) && (yt ? NC % 16 == 0 : K % 16 == 0);
 }
+static bool kmajor_shape_ok(int NR, int NC, int K, bool xt, bool yt) { return K > kBK && kmajor_rows_ok(NR, NC, K, xt, yt); }
 
 static int dispatch_parts(int x_type, int y_type, const GemmCall& c, const KSplit& s) {
     if (x_type == MSAMP_DT_E4M3 && y_type == MSAMP_DT_E4M3) return run_gemm_parts<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(c, s);
@@ -38,9 +39,10 @@ static int dispatch_parts(int x_type, int y_type, const GemmCall& c, const KSpli
 // tiles, both with every compute unit busy; 5 and 9 around the K loop) plus, if split, the second launch and the way of the
 // partial sums to memory and back.  The split must promise 15 % less, so that it is not taken where the estimate
 // is near even.  Only problems of the 128 x 128 tiles are looked at: the others have tiles enough.  Whole against split, m x n
-// x k in us: 1200 x 4304 x 12605 128.9 -> 83.0 (three parts of large tiles; 340 small tiles on 256 compute units before),
-// 128 x 512 x 16000 54.9 -> 15.2, 256 x 1024 x 8192 29.9 -> 15.6, 1024 x 1024 x 16384 57.6 -> 33.4, 16 x 8192 x 8192 30.3 -> 19.7,
-// 2048 x 1024 x 8192 32.8 -> 27.4, 512 x 512 x 2500 12.7 -> 11.4.  FP8Linear 12605 x 1200 -> 4304, forward and backward: 335 -> 292.
+// x k in us: 1200 x 4304 x 12605 128.9 -> 83.0 (three parts of large tiles; 340 small tiles, one to a compute unit, before; two to
+// a unit 121.3), 128 x 512 x 16000 54.9 -> 15.2, 256 x 1024 x 8192 29.9 -> 15.6, 1024 x 1024 x 16384 57.6 -> 33.4,
+// 16 x 8192 x 8192 30.3 -> 19.7, 2048 x 1024 x 8192 32.8 -> 27.4, 512 x 512 x 2500 12.7 -> 11.4.  FP8Linear 12605 x 1200 -> 4304,
+// forward and backward: 335 -> 292.
 static KSplit ksplit_rule(int NR, int NC, int K) {
     KSplit best = {true, 1};
     if (!takes_small_tiles(NR, NC, K) || !kmajor_shape_ok(NR, NC, K, true, true)) return best;
@@ -107,7 +109,7 @@ int registered_walk(int NR, int NC, int K, bool XT, bool YT) {
     return it == g_walks.end() ? -1 : it->second;
 }
 
-static std::atomic<int> g_small_tile_limit{128};
+static std::atomic<int> g_small_tile_limit{kSmallTileLimit};
 int small_tile_limit() { return g_small_tile_limit.load(std::memory_order_relaxed); }
 
 }    // namespace msamp
@@ -268,6 +270,21 @@ extern "C" int msamp_fp8_gemm_kmajor(const uint8_t* a, int a_type, const float* 
     hipStream_t st = static_cast<hipStream_t>(stream);
     // X = b (rows of D), Y = a (columns of D)
     const GemmCall c = {b, a, d, d_dtype, n, m, k, b_scale_inv, a_scale_inv, accumulate, bias, bias_dtype, b_kmajor != 0, true, nullptr, st};
+    return dispatch_pair(b_type, a_type, c);
+}
+
+int msamp::gemm_kmajor(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv,
+                       int b_kmajor, void* d, int d_dtype, int m, int n, int k, int accumulate, hipStream_t st) {
+    if (k > kBK)
+        return msamp_fp8_gemm_kmajor(a, a_type, a_scale_inv, 1, b, b_type, b_scale_inv, b_kmajor, d, d_dtype, m, n, k, accumulate, nullptr,
+                                     MSAMP_DT_F32, st);
+    MSAMP_REQUIRE(is_fp8(a_type) && is_fp8(b_type) && is_hp(d_dtype), MSAMP_ERR_DTYPE, "gemm_kmajor: types %d, %d -> %d", a_type, b_type,
+                  d_dtype);
+    MSAMP_REQUIRE(m > 0 && n > 0 && k > 0 && kmajor_rows_ok(n, m, k, b_kmajor != 0, true), MSAMP_ERR_SHAPE,
+                  "gemm_kmajor: m=%d n=%d k=%d (leading dimensions must be multiples of 16)", m, n, k);
+    MSAMP_REQUIRE(a && b && d && a_scale_inv && b_scale_inv, MSAMP_ERR_NULL, "gemm_kmajor: null pointer");
+    MSAMP_REQUIRE(aligned(a, 16) && aligned(b, 16), MSAMP_ERR_ALIGNMENT, "gemm_kmajor: operands must be 16-byte aligned");
+    const GemmCall c = {b, a, d, d_dtype, n, m, k, b_scale_inv, a_scale_inv, accumulate, nullptr, MSAMP_DT_F32, b_kmajor != 0, true, nullptr, st};
     return dispatch_pair(b_type, a_type, c);
 }
 

@@ -54,6 +54,8 @@ template <int XF, int YF>
 int run_gemm_ragged(const GemmCall& c);
 template <int XF, int YF>
 int run_gemm_small(const GemmCall& c);
+template <int XF, int YF>
+int run_gemm_pair128(const GemmCall& c);
 // A product in parts of K: which tile, and how many parts (1: not split).
 struct KSplit {
     bool small_tiles;
@@ -66,15 +68,17 @@ template <int XF, int YF>
 int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int NR, int NC, int K, const float* xs,
                    const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st);
 
-// Problems of at most this many 256 x 256 tiles take the kernel with 128 x 128 tiles (msamp_set_small_tile_limit; negative: the
-// generic kernel for every row-major product, to compare the others with) ...
+// The size up to which 128 x 128 tiles are looked at, in 256 x 256 tiles (msamp_set_small_tile_limit).  Any other value than the
+// default serves to compare the kernels: the paired form is off then, and a negative one sends every row-major product to the
+// generic kernel.
+constexpr int kSmallTileLimit = 128;
 int small_tile_limit();
 // The tile walk registered for this problem of the 256 x 256-tile kernel (msamp_fp8_gemm_set_walk / _tune), or -1: bit 0 =
 // groups of tile columns walked row by row instead of groups of tile rows, bit 1 = the XCD's patch of 32 tiles turned (4 of
 // the grouped dimension x 8 of the walked one).  Any walk gives the same output bits: it only decides which workgroup
 // takes which tile.  Bit 2 (row-major operands only): the tile loads awaited in two parts, see the kernel.
 int registered_walk(int NR, int NC, int K, bool XT, bool YT);
-// ... which is this rule: at least four slices of K; up to half the limit always (one small tile per
+// 128 x 128 tiles with the whole LDS to a workgroup: at least four slices of K; up to half the limit always (one small tile per
 // compute unit with the default limit), up to the limit where K is long enough for the second round of small tiles to
 // pay (measured: 128 large tiles level at K = 2048, 15 % ahead at 4096).
 inline bool takes_small_tiles(int NR, int NC, int K) {
@@ -82,6 +86,25 @@ inline bool takes_small_tiles(int NR, int NC, int K) {
     const int limit = small_tile_limit();
     return K > 3 * kBK && (big_tiles <= limit / 2 || (big_tiles <= limit && K >= 3072));
 }
+
+// 128 x 128 tiles with two workgroups to a compute unit, us against the kernel that would take the product otherwise (row-major,
+// both K-major):
+//   K <= 128 (the generic kernel)                        1024 x 1024  13.8 -> 4.6     8192 x 4096  58.5 -> 17.9
+//   one tile a unit or fewer, K = 256 (large tiles)      2048 x 2048   8.4 -> 5.4,     8.7 -> 5.6
+//     K = 1024 (small tiles, one workgroup a unit)       2048 x 2048   7.5 -> 7.0,     8.3 -> 7.3
+//     K = 2048                                           2048 x 2048   9.9 -> 9.5,    11.4 -> 10.2    K = 4096: 18.1 -> 20.8, 20.1 -> 20.6
+//   up to two tiles a unit, K = 1024 (large tiles)       4096 x 2048  13.9 -> 10.4,   14.2 -> 10.9
+//     K = 4096 (small tiles)                             4096 x 2048  35.5 -> 30.4,   41.0 -> 31.9    K = 12288: 89.0 -> 83.2, 104.5 -> 87.6
+//   more (large tiles)                                   3072 x 4096 x 1024  14.8 -> 13.9, 15.1 -> 15.1;   4096 x 4096 x 1024  16.9 -> 17.7, 17.3 -> 18.8
+inline bool takes_paired_tiles(int NR, int NC, int K) {
+    if (small_tile_limit() != kSmallTileLimit) return false;
+    const long tiles = static_cast<long>((NR + kDmaTile / 2 - 1) / (kDmaTile / 2)) * ((NC + kDmaTile / 2 - 1) / (kDmaTile / 2));
+    return K <= kBK || (tiles <= 2L * cu_count() && (tiles > cu_count() || K <= 2048));
+}
+
+// msamp_fp8_gemm_kmajor for any K: a single slice of K is left to the paired tiles.
+int gemm_kmajor(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv,
+                int b_kmajor, void* d, int d_dtype, int m, int n, int k, int accumulate, hipStream_t st);
 
 // row offsets of the direct-to-LDS kernels are 32 bits
 inline bool fits_offsets(int NR, int NC, int K) {
@@ -98,15 +121,19 @@ extern template int run_gemm_pair<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&)
 extern template int run_gemm_pair<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_ragged<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&);
 extern template int run_gemm_small<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&);
+extern template int run_gemm_pair128<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&);
 extern template int run_gemm_parts<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&, const KSplit&);
 extern template int run_gemm_ragged<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_small<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
+extern template int run_gemm_pair128<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_parts<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&, const KSplit&);
 extern template int run_gemm_ragged<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);
 extern template int run_gemm_small<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);
+extern template int run_gemm_pair128<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);
 extern template int run_gemm_parts<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&, const KSplit&);
 extern template int run_gemm_ragged<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_small<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
+extern template int run_gemm_pair128<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_parts<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&, const KSplit&);
 #define MSAMP_SPLIT_ARGS const uint8_t*, const uint8_t*, void*, int, int, int, int, const float*, const float*, int, const void*, int, hipStream_t
 extern template int run_gemm_split<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(MSAMP_SPLIT_ARGS);

@@ -8,6 +8,7 @@ namespace msamp {
 template int run_gemm_split<MSAMP_XF, MSAMP_YF>(MSAMP_SPLIT_ARGS);
 template int run_gemm_ragged<MSAMP_XF, MSAMP_YF>(const GemmCall&);
 template int run_gemm_small<MSAMP_XF, MSAMP_YF>(const GemmCall&);
+template int run_gemm_pair128<MSAMP_XF, MSAMP_YF>(const GemmCall&);
 template int run_gemm_parts<MSAMP_XF, MSAMP_YF>(const GemmCall&, const KSplit&);
 #else
 template int run_gemm_pair<MSAMP_XF, MSAMP_YF>(const GemmCall&);

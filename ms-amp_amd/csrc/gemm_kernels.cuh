@@ -1452,6 +1452,10 @@ int run_gemm_small(const GemmCall& c) {
     MSAMP_TYPE_LAUNCH(launch_gemm_dma128)
 }
 template <int XF, int YF>
+int run_gemm_pair128(const GemmCall& c) {
+    MSAMP_TYPE_LAUNCH(launch_gemm_pair128)
+}
+template <int XF, int YF>
 int run_gemm_parts(const GemmCall& c, const KSplit& split) {
     if (split.small_tiles)
         return launch_gemm_dma128_tail<XF, YF, float, true, true, true>(c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, 0, nullptr, 0, c.st, split.parts);
@@ -1462,14 +1466,15 @@ int run_gemm_parts(const GemmCall& c, const KSplit& split) {
 // Everything behind the C entry points for one pair of operand formats.  gemm_inst.hip instantiates it once per
 // pair (four translation units, so that they compile side by side).
 //
-// Which kernel: few 256 x 256 tiles leave most compute units idle and take 128 x 128 tiles (takes_small_tiles()).  The
-// direct-to-LDS kernels need at least two 128-byte slices of K and 32-bit row offsets; where they can run they are the
-// faster ones at every size (256 x 256 x 4096: 14 against 80 us with the generic kernel, 8192 x 4096 x 4096: 100 against
-// 555), also with a ragged last slice (12605 x 4304 x 1200 into float16: 94 against 153, 8192 x 4096 x 4080: 121 against
-// 195).  Everything else takes the generic register-staged kernel.
+// Which kernel: few 256 x 256 tiles leave most compute units idle and take 128 x 128 tiles, two workgroups to a compute unit
+// (takes_paired_tiles()) or one (takes_small_tiles()).  The direct-to-LDS kernels need 32-bit row offsets and, but for the paired
+// form, more than one 128-byte slice of K; where they can run they are the faster ones at every size (256 x 256 x 4096: 14 against
+// 80 us with the generic kernel, 8192 x 4096 x 4096: 100 against 555), also with a ragged last slice (12605 x 4304 x 1200 into
+// float16: 94 against 153, 8192 x 4096 x 4080: 121 against 195).  Everything else takes the generic register-staged kernel.
 template <int XF, int YF>
 int run_gemm_pair(const GemmCall& c) {
     if (c.qa == nullptr && fits_offsets(c.NR, c.NC, c.K)) {
+        if (takes_paired_tiles(c.NR, c.NC, c.K) || (c.yt && c.K <= kBK)) return run_gemm_pair128<XF, YF>(c);
         if (takes_small_tiles(c.NR, c.NC, c.K)) return run_gemm_small<XF, YF>(c);
         if (c.K > kBK && c.K % kBK && (c.yt || small_tile_limit() >= 0)) return run_gemm_ragged<XF, YF>(c);
     }

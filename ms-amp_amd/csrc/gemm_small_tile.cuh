@@ -19,8 +19,17 @@
 // MFMAs and 15.5 us without them (an ablation), 95 GB/s per compute unit where a bare loop of such loads reaches 121.
 // It is the faster kernel only while the large tile leaves compute units idle, and the host picks it only then.
 //
+// PAIR: two workgroups to a compute unit, so that one's launch, prologue and epilogue run under the other's products, and up to
+// two tiles a unit go side by side instead of one after the other (which products: takes_paired_tiles()).  80 KiB of LDS each:
+// a ring of five units of 16 KiB, one operand's part of a slice, with a slice being read and one and a half on their way; any
+// number of slices.  Two waves to a SIMD leave each 256 registers: the X fragments are not doubled (a block of the next slice is
+// read behind the last product of the present one), and the accumulators are v192 .. v255, which the compiler is kept from by
+// amdgpu_num_vgpr (half of 192: the unit of the attribute is a pair here).  With AGPRs in use it would halve the 256 instead, and
+// 128 do not hold the fragments.  Bound by the LDS: 96 KiB through it per slice and tile, 768 of its cycles beside 512 of the
+// matrix pipes; hence the larger tiles where there are enough of them.
+//
 // Every output element is accumulated over the 128-byte blocks of K in ascending order, one MFMA per block, and
-// scaled, biased, summed and rounded with the expressions of the large tile: the two kernels agree to the bit.
+// scaled, biased, summed and rounded with the expressions of the large tile: the kernels agree to the bit.
 #pragma once
 
 namespace msamp {
@@ -28,14 +37,57 @@ namespace msamp {
 constexpr int kSmallTile = 128;
 constexpr int kSmallStage = 2 * kSmallTile * kBK;    // 32 KiB
 constexpr int kSmallStages = 5;    // all 160 KiB of the LDS
+constexpr int kPairUnit = kSmallTile * kBK;    // PAIR: one operand's part of a slice, 16 KiB
+constexpr int kPairUnits = 5;                  // 80 KiB, half of the LDS
 
-template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL>
+// The accumulators of the PAIR form, block n in v[192 + 4n .. 195 + 4n], handled as those in AGPRs are (gemm_kernels.cuh).
+#define MSAMP_VACC                                                                                                      \
+    "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199", "v200", "v201", "v202", "v203", "v204", "v205", "v206", \
+        "v207", "v208", "v209", "v210", "v211", "v212", "v213", "v214", "v215", "v216", "v217", "v218", "v219", "v220",     \
+        "v221", "v222", "v223", "v224", "v225", "v226", "v227", "v228", "v229", "v230", "v231", "v232", "v233", "v234",     \
+        "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "v245", "v246", "v247", "v248",     \
+        "v249", "v250", "v251", "v252", "v253", "v254", "v255"
+constexpr int kVacc = 192;
+template <int N, int CB, int BL>
+__device__ __forceinline__ void vmfma_fixed(const v8i& a, const v8i& b) {
+    asm volatile("v_mfma_f32_16x16x128_f8f6f4 v[%2:%3], %0, %1, v[%2:%3] cbsz:%4 blgp:%5"
+                 :
+                 : "v"(a), "v"(b), "n"(kVacc + N * 4), "n"(kVacc + N * 4 + 3), "n"(CB), "n"(BL));
+}
+__device__ __forceinline__ void vacc_clear() {
+    static_for<16>([&](auto nc) {
+        constexpr int n = decltype(nc)::value;
+        asm volatile("v_mov_b32 v[%0], 0\n\tv_mov_b32 v[%1], 0\n\tv_mov_b32 v[%2], 0\n\tv_mov_b32 v[%3], 0"
+                     :
+                     : "n"(kVacc + n * 4), "n"(kVacc + n * 4 + 1), "n"(kVacc + n * 4 + 2), "n"(kVacc + n * 4 + 3));
+    });
+    asm volatile("s_nop 4" : : : MSAMP_VACC);
+}
+__device__ __forceinline__ uint32_t vacc_fence() {
+    uint32_t token;
+    asm volatile("s_nop 15\n\ts_nop 7\n\tv_mov_b32 %0, 0" : "=v"(token) : : MSAMP_VACC);
+    return token;
+}
+template <int N>
+__device__ __forceinline__ v4f vacc_quad(uint32_t token) {
+    v4f r;
+    float x, y, z, w;
+    asm("v_mov_b32 %0, v[%1]" : "=v"(x) : "n"(kVacc + N * 4), "v"(token));
+    asm("v_mov_b32 %0, v[%1]" : "=v"(y) : "n"(kVacc + N * 4 + 1), "v"(token));
+    asm("v_mov_b32 %0, v[%1]" : "=v"(z) : "n"(kVacc + N * 4 + 2), "v"(token));
+    asm("v_mov_b32 %0, v[%1]" : "=v"(w) : "n"(kVacc + N * 4 + 3), "v"(token));
+    r[0] = x, r[1] = y, r[2] = z, r[3] = w;
+    return r;
+}
+
+template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL, bool PAIR = false>
 __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const uint8_t* __restrict__ Y, OT* __restrict__ D, int NR,
                                             int NC, int K, const float* __restrict__ x_scale_inv,
                                             const float* __restrict__ y_scale_inv, int accumulate, const void* __restrict__ bias,
                                             int bias_dt) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    if constexpr (KTAIL && kTakesKParts<OT, XT, YT>) k_part(X, Y, D, NR, NC, K);
+    constexpr bool kParts = KTAIL && !PAIR && kTakesKParts<OT, XT, YT>;
+    if constexpr (kParts) k_part(X, Y, D, NR, NC, K);
     const int tiles_r = (NR + kSmallTile - 1) / kSmallTile, tiles_c = (NC + kSmallTile - 1) / kSmallTile;
     int tr, tc;
     tile_of_id(blockIdx.x, tiles_r, tiles_c, false, false, tr, tc);
@@ -49,16 +101,18 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     const int seg = lane % kSegs;
     const int gcol = col0 + wc * 64 + seg * kElems;
     float alpha = (*x_scale_inv) * (*y_scale_inv);
-    if constexpr (KTAIL && kTakesKParts<OT, XT, YT>) alpha = gridDim.y > 1 ? 1.0f : alpha;
+    if constexpr (kParts) alpha = gridDim.y > 1 ? 1.0f : alpha;
     float bv[kElems];
 #pragma unroll
     for (int e = 0; e < kElems; ++e) bv[e] = 0.0f;
-    if (bias != nullptr) {
+    auto fetch_bias = [&]() __attribute__((always_inline)) {
+        if (bias == nullptr) return;
 #pragma unroll
         for (int e = 0; e < kElems; ++e) bv[e] = gcol + e < NC ? load_bias(bias, bias_dt, gcol + e) : 0.0f;
 #pragma unroll
         for (int e = 0; e < kElems; ++e) asm volatile("" : "+v"(bv[e]));
-    }
+    };
+    if constexpr (!PAIR) fetch_bias();
     asm volatile("" : "+v"(alpha));
 
     // ---- global -> LDS: one wave instruction fills 8 rows of 128 bytes (lane l: row l / 8, 16-byte position l % 8,
@@ -87,9 +141,14 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     }
     // KTAIL: a ragged last slice of `rem` K bytes, handled as in the large tile (loads kept inside the operand, fragments
     // masked)
-    const int nk = KTAIL ? (K + kBK - 1) / kBK : K / kBK;    // at least 4 (the host sees to that)
+    const int nk = KTAIL ? (K + kBK - 1) / kBK : K / kBK;    // at least 4, PAIR: 1 (the host sees to that)
     const int rem = K - (nk - 1) * kBK;
     const uint32_t tail_back = KTAIL && chunk * 16 >= rem ? chunk * 16 : 0;
+    // where the X or Y half of slice kt lies in the LDS
+    auto place = [&](int kt, bool is_x) __attribute__((always_inline)) {
+        return PAIR ? (2 * kt + (is_x ? 0 : 1)) % kPairUnits * kPairUnit
+                    : kt % kSmallStages * kSmallStage + (is_x ? 0 : kSmallTile * kBK);
+    };
     // one of the 8 loads of a slice (0..3: X rows, 4..7: Y rows); assembly for the reason given at the large tile
     auto dma = [&](int kt, int which, bool last = false) __attribute__((always_inline)) {
         const bool is_x = which < 4;
@@ -103,8 +162,7 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
                 off -= tail_back;
             }
         }
-        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + (kt % kSmallStages) * kSmallStage +
-                                                            (is_x ? 0 : kSmallTile * kBK) + ((which & 3) * 4 + wave) * 1024);
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + place(kt, is_x) + ((which & 3) * 4 + wave) * 1024);
         asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(off), "s"(src) : "memory", "m0");
     };
     auto dma_slice = [&](int kt, bool last = false) __attribute__((always_inline)) {
@@ -118,15 +176,15 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     const int fsw = (lane & 7) ^ ((lane >> 3) & 1);
     const int off_lo = ((2 * g4) ^ fsw) << 4;
     const int xrow = (wr * 64 + l16) * kBK;
-    const int yrow = kSmallTile * kBK + (wc * 64 + l16) * kBK;
+    const int yrow = (wc * 64 + l16) * kBK;
     const int tj = l16 >> 1;
     const int t_lane = (g4 * 32 + tj) * kBK + (l16 & 1) * 8;    // k-row and 8-byte half of this lane's transposing reads
     // A slice's fragments arrive in pieces: two 16-byte reads per 16-row block of a row-major operand (block p / 2, half
     // p % 2), four 8-byte transposing reads per block of a K-major one (block p / 4, eight k each); X pieces first.
     constexpr int kPX = XT ? 16 : 8, kPY = YT ? 16 : 8, kPieces = kPX + kPY;
-    auto read_piece = [&](int* fxd, int* fyd, int kt, int p) __attribute__((always_inline)) {
-        const uint8_t* base = smem + (kt % kSmallStages) * kSmallStage;
+    auto read_piece = [&](int* fxd, int* fyd, int px, int py, int p) __attribute__((always_inline)) {
         const bool is_x = p < kPX;
+        const uint8_t* base = smem + (is_x ? px : py);
         const int q = is_x ? p : p - kPX;
         if ((is_x && !XT) || (!is_x && !YT)) {
             const int b = q >> 1, hf = q & 1;
@@ -136,97 +194,180 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
         } else {
             const int b = q >> 2, qq = q & 3;
             const int wq = is_x ? wr : wc;
-            const int addr = (is_x ? 0 : kSmallTile * kBK) + t_lane + (qq * 8) * kBK + (((wq * 4 + b) ^ tj) << 4);
+            const int addr = t_lane + (qq * 8) * kBK + (((wq * 4 + b) ^ tj) << 4);
             const v2i val = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(base + addr));
             int* d = (is_x ? fxd : fyd) + b * 8 + qq * 2;
             d[0] = val[0], d[1] = val[1];
         }
     };
 
-    acc_clear();
-    int fx[2][32], fy[2][32];
+    if constexpr (PAIR) vacc_clear();
+    else acc_clear();
+    int fx[PAIR ? 1 : 2][32], fy[2][32];
 
     // the 16 MFMAs of the slice held in fragment set `cur`, with the 16 fragment reads of slice rd_kt (into the other
     // set) between them.  srcA = Y rows, srcB = X rows: a lane then holds, for D row lane % 16 of a block, four
     // consecutive D columns.
-    auto step = [&](auto curc, int rd_kt, bool do_read, int ld_kt, bool do_load, bool ld_last = false,
-                    bool masked = false) __attribute__((always_inline)) {
+    // PAIR: `do_load` stands for the Y half of slice ld_kt, `next_x` for the X half of the slice behind it, and `ld_last`
+    // for the last slice of K being the one (if next_x) or the other.
+    auto step = [&](auto curc, int rd_kt, bool do_read, int ld_kt, bool do_load, bool ld_last = false, bool masked = false,
+                    bool next_x = false) __attribute__((always_inline)) {
         constexpr int cur = decltype(curc)::value;
-        if (KTAIL && masked) mask_fragments(fx[cur], g4, rem), mask_fragments(fy[cur], g4, rem);
+        if (KTAIL && masked) mask_fragments(fx[PAIR ? 0 : cur], g4, rem), mask_fragments(fy[cur], g4, rem);
         constexpr int cb = (YF == MSAMP_DT_E4M3) ? 0 : 1;
         constexpr int bl = (XF == MSAMP_DT_E4M3) ? 0 : 1;
-        static_for<4>([&](auto jc) {
-            static_for<4>([&](auto ic) {
-                constexpr int i = decltype(ic)::value, j = decltype(jc)::value;
-                const int* cx = fx[cur] + i * 8;
-                const int* cy = fy[cur] + j * 8;
-                const v8i vx = {cx[0], cx[1], cx[2], cx[3], cx[4], cx[5], cx[6], cx[7]};
-                const v8i vy = {cy[0], cy[1], cy[2], cy[3], cy[4], cy[5], cy[6], cy[7]};
+        int px = place(rd_kt, true), py = place(rd_kt, false);
+        // (opaque: otherwise every read's address is worked out for both turns in front of the loop, in registers that PAIR
+        // does not have)
+        if constexpr (PAIR) asm volatile("" : "+s"(px), "+s"(py));
+        static_for<16>([&](auto nc) {
+            constexpr int n = decltype(nc)::value;
+            constexpr int i = PAIR ? n >> 2 : n & 3, j = PAIR ? n & 3 : n >> 2;
+            const int* cx = fx[PAIR ? 0 : cur] + i * 8;
+            const int* cy = fy[cur] + j * 8;
+            const v8i vx = {cx[0], cx[1], cx[2], cx[3], cx[4], cx[5], cx[6], cx[7]};
+            const v8i vy = {cy[0], cy[1], cy[2], cy[3], cy[4], cy[5], cy[6], cy[7]};
+            if constexpr (PAIR) {
+                vmfma_fixed<i * 4 + j, cb, bl>(vy, vx);
+                // the Y fragments of the next slice with the first eight MFMAs, an X block in place of this slice's behind
+                // its last MFMA
+                if (do_read && n < 8) {
+#pragma unroll
+                    for (int p = n * kPY / 8; p < (n + 1) * kPY / 8; ++p) read_piece(fx[0], fy[cur ^ 1], px, py, kPX + p);
+                }
+                if (do_read && (n & 3) == 3) {
+#pragma unroll
+                    for (int p = i * kPX / 4; p < (i + 1) * kPX / 4; ++p) read_piece(fx[0], fy[cur ^ 1], px, py, p);
+                }
+                if (do_load && (n & 1) && n < 8) dma(ld_kt, 4 + (n >> 1), ld_last && !next_x);
+                if (next_x && (n & 1) && n >= 8) dma(ld_kt + 1, (n >> 1) - 4, ld_last);
+            } else {
                 mfma_fixed<i * 4 + j, cb, bl>(vy, vx);
                 // the fragment reads go with the first eight MFMAs (two to four each) and have come back by the barrier that
                 // follows the last one; nothing moves across, so they stay spread as written
-                constexpr int n = j * 4 + i;
                 if (do_read && n < 8) {
 #pragma unroll
-                    for (int p = n * kPieces / 8; p < (n + 1) * kPieces / 8; ++p) read_piece(fx[cur ^ 1], fy[cur ^ 1], rd_kt, p);
+                    for (int p = n * kPieces / 8; p < (n + 1) * kPieces / 8; ++p) read_piece(fx[cur ^ 1], fy[cur ^ 1], px, py, p);
                 }
                 // the eight tile loads of slice ld_kt, one every other MFMA: issued in one go they hold the wave, and with
                 // it its MFMAs, for as long as the memory pipe takes to accept them
                 if (do_load && (n & 1)) dma(ld_kt, n >> 1, ld_last);
-                __builtin_amdgcn_sched_barrier(0);
-            });
+            }
+            __builtin_amdgcn_sched_barrier(0);
         });
     };
     constexpr std::integral_constant<int, 0> c0{};
     constexpr std::integral_constant<int, 1> c1{};
 
-    dma_slice(0);
-    dma_slice(1);
-    dma_slice(2);
-    dma_slice(3, nk == 4);
-    wait_vmcnt<24>();
-    __syncthreads();
+    if constexpr (PAIR) {
+        auto half = [&](int kt, int first, bool last = false) __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 0; p < kPieces; ++p) read_piece(fx[0], fy[0], 0, p);
+            for (int w = 0; w < 4; ++w) dma(kt, first + w, last);
+        };
+        dma_slice(0, nk == 1);
+        if (nk > 1) dma_slice(1, nk == 2);
+        if (nk > 2) {
+            half(2, 0, nk == 3);
+            wait_vmcnt<12>();
+        } else if (nk == 2) {
+            wait_vmcnt<8>();
+        } else {
+            wait_vmcnt<0>();
+        }
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) read_piece(fx[0], fy[0], place(0, true), place(0, false), p);
 
-    // Before the step of slice kt: slices kt + 1 .. kt + 3 are on their way (24 loads of this wave), slice kt is in
-    // registers.  Wait for slice kt + 1, meet (it has landed in every wave's part of the stage, and nobody reads the
-    // stage of slice kt - 1 any more), compute slice kt while reading kt + 1 and sending for slice kt + 4 into that stage.
-    auto turn = [&](auto curc, int kt, bool ld_last = false) __attribute__((always_inline)) {
-        wait_vmcnt<16>();
-        __syncthreads();
-        step(curc, kt + 1, true, kt + 4, true, ld_last);
-    };
-    int kt = 0;
-    for (; kt + (KTAIL ? 6 : 5) < nk; kt += 2) {    // (KTAIL: the load of the last slice is not part of the loop)
-        turn(c0, kt);
-        turn(c1, kt + 1);
-    }
-    // four or five slices are left; the last four load nothing
-    auto tail4 = [&](auto ac, auto bc, int k0) __attribute__((always_inline)) {
-        wait_vmcnt<16>();
-        __syncthreads();
-        step(ac, k0 + 1, true, 0, false);
-        wait_vmcnt<8>();
-        __syncthreads();
-        step(bc, k0 + 2, true, 0, false);
-        wait_vmcnt<0>();
-        __syncthreads();
-        step(ac, k0 + 3, true, 0, false);
-        step(bc, 0, false, 0, false, false, true);
-    };
-    if (kt + 5 == nk) {
-        turn(c0, kt, true);
-        tail4(c1, c0, kt + 1);
-    } else {
-        if (KTAIL && kt + 6 == nk) {
+        // Before the step of slice kt: slice kt is in registers, slice kt + 1 and the X half of kt + 2 are on their way.  Wait
+        // for slice kt + 1, meet (it has landed, and the two units of slice kt are free), compute slice kt while reading
+        // kt + 1 and sending for the Y half of kt + 2 and the X half of kt + 3.
+        auto turn = [&](auto curc, int kt, bool ld_last = false) __attribute__((always_inline)) {
+            wait_vmcnt<4>();
+            __syncthreads();
+            step(curc, kt + 1, true, kt + 2, true, ld_last, false, true);
+        };
+        auto tail2 = [&](auto ac, auto bc, int k0) __attribute__((always_inline)) {
+            wait_vmcnt<0>();
+            __syncthreads();
+            step(ac, k0 + 1, true, 0, false);
+            step(bc, 0, false, 0, false, false, true);
+        };
+        auto tail3 = [&](auto ac, auto bc, int k0) __attribute__((always_inline)) {
+            wait_vmcnt<4>();
+            __syncthreads();
+            step(ac, k0 + 1, true, k0 + 2, true, true);
+            tail2(bc, ac, k0 + 1);
+        };
+        int kt = 0;
+        for (; kt + 5 < nk; kt += 2) {
+            turn(c0, kt);
+            turn(c1, kt + 1);
+        }
+        // four or five slices are left, or there are three or fewer in all
+        if (kt + 5 == nk) {
             turn(c0, kt);
             turn(c1, kt + 1, true);
-            kt += 2;
+            tail3(c0, c1, kt + 2);
+        } else if (kt + 4 == nk) {
+            turn(c0, kt, true);
+            tail3(c1, c0, kt + 1);
+        } else if (nk == 3) {
+            tail3(c0, c1, 0);
+        } else if (nk == 2) {
+            tail2(c0, c1, 0);
+        } else {
+            step(c0, 0, false, 0, false, false, true);
         }
-        tail4(c0, c1, kt);
+    } else {
+        dma_slice(0);
+        dma_slice(1);
+        dma_slice(2);
+        dma_slice(3, nk == 4);
+        wait_vmcnt<24>();
+        __syncthreads();
+    #pragma unroll
+        for (int p = 0; p < kPieces; ++p) read_piece(fx[0], fy[0], place(0, true), place(0, false), p);
+
+        // Before the step of slice kt: slices kt + 1 .. kt + 3 are on their way (24 loads of this wave), slice kt is in
+        // registers.  Wait for slice kt + 1, meet (it has landed in every wave's part of the stage, and nobody reads the
+        // stage of slice kt - 1 any more), compute slice kt while reading kt + 1 and sending for slice kt + 4 into that stage.
+        auto turn = [&](auto curc, int kt, bool ld_last = false) __attribute__((always_inline)) {
+            wait_vmcnt<16>();
+            __syncthreads();
+            step(curc, kt + 1, true, kt + 4, true, ld_last);
+        };
+        int kt = 0;
+        for (; kt + (KTAIL ? 6 : 5) < nk; kt += 2) {    // (KTAIL: the load of the last slice is not part of the loop)
+            turn(c0, kt);
+            turn(c1, kt + 1);
+        }
+        // four or five slices are left; the last four load nothing
+        auto tail4 = [&](auto ac, auto bc, int k0) __attribute__((always_inline)) {
+            wait_vmcnt<16>();
+            __syncthreads();
+            step(ac, k0 + 1, true, 0, false);
+            wait_vmcnt<8>();
+            __syncthreads();
+            step(bc, k0 + 2, true, 0, false);
+            wait_vmcnt<0>();
+            __syncthreads();
+            step(ac, k0 + 3, true, 0, false);
+            step(bc, 0, false, 0, false, false, true);
+        };
+        if (kt + 5 == nk) {
+            turn(c0, kt, true);
+            tail4(c1, c0, kt + 1);
+        } else {
+            if (KTAIL && kt + 6 == nk) {
+                turn(c0, kt);
+                turn(c1, kt + 1, true);
+                kt += 2;
+            }
+            tail4(c0, c1, kt);
+        }
     }
-    const uint32_t acc_token = acc_fence();
+    if constexpr (PAIR) fetch_bias();    // (no registers for them before; the other workgroup works meanwhile)
+    const uint32_t acc_token = PAIR ? vacc_fence() : acc_fence();
     __syncthreads();    // every wave is through with the stages, which the patches below reuse
 
     // ---- epilogue: the raw accumulators of a 16-row block go through a per-wave float32 patch; each lane then picks up
@@ -241,7 +382,7 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
         constexpr int i = decltype(ic)::value;
         static_for<4>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
-            const v4f a = acc_quad<i * 4 + j>(acc_token);
+            const v4f a = PAIR ? vacc_quad<i * 4 + j>(acc_token) : acc_quad<i * 4 + j>(acc_token);
             *reinterpret_cast<float4*>(patch + l16 * kFPitch + (j * 16 + g4 * 4) * 4) = make_float4(a[0], a[1], a[2], a[3]);
         });
         // (the patch is private to this wave and the LDS serves one wave's requests in order: no waits needed)
@@ -321,6 +462,40 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_ragged128_kernel(const 
                                                                            const float* __restrict__ y_scale_inv, int accumulate,
                                                                            const void* __restrict__ bias, int bias_dt) {
     gemm_dma128<XF, YF, OT, XT, YT, true>(X, Y, D, NR, NC, K, x_scale_inv, y_scale_inv, accumulate, bias, bias_dt);
+}
+
+template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_num_vgpr(96))) void fp8_gemm_pair128_kernel(const uint8_t* __restrict__ X, const uint8_t* __restrict__ Y,
+                                                                            OT* __restrict__ D, int NR, int NC, int K,
+                                                                            const float* __restrict__ x_scale_inv,
+                                                                            const float* __restrict__ y_scale_inv, int accumulate,
+                                                                            const void* __restrict__ bias, int bias_dt) {
+    gemm_dma128<XF, YF, OT, XT, YT, KTAIL, true>(X, Y, D, NR, NC, K, x_scale_inv, y_scale_inv, accumulate, bias, bias_dt);
+}
+
+template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL>
+static int launch_gemm_pair128_tail(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs, const float* ys,
+                                    int accumulate, const void* bias, int bias_dt, hipStream_t st) {
+    constexpr int smem = kPairUnits * kPairUnit;
+    static std::atomic<bool> configured{false};    // setting the attribute twice is harmless
+    auto kern = fp8_gemm_pair128_kernel<XF, YF, OT, XT, YT, KTAIL>;
+    if (!configured.load(std::memory_order_acquire)) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(fp8_gemm_pair128_kernel)");
+        configured.store(true, std::memory_order_release);
+    }
+    const int tiles = ((NR + kSmallTile - 1) / kSmallTile) * ((NC + kSmallTile - 1) / kSmallTile);
+    hipLaunchKernelGGL(kern, dim3(tiles), dim3(kGemmThreads), smem, st, X, Y, static_cast<OT*>(D), NR, NC, K, xs, ys, accumulate, bias,
+                       bias_dt);
+    MSAMP_CHECK_LAUNCH("fp8_gemm_pair128_kernel");
+    return MSAMP_OK;
+}
+
+template <int XF, int YF, typename OT, bool XT = false, bool YT = false>
+static int launch_gemm_pair128(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs, const float* ys,
+                               int accumulate, const void* bias, int bias_dt, hipStream_t st) {
+    if (K % kBK) return launch_gemm_pair128_tail<XF, YF, OT, XT, YT, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
+    return launch_gemm_pair128_tail<XF, YF, OT, XT, YT, false>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
 }
 
 template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL>

@@ -4,6 +4,8 @@
 // these, the same launches: forward of 16 x 512 -> 512 61 -> 33 us, training step of two 1024-wide blocks over 2048 tokens
 // 1522 -> 1137 us.
 #include "common.cuh"
+#include "gemm_call.h"
+
 
 namespace msamp {
 
@@ -83,6 +85,7 @@ extern "C" int msamp_linear_backward(const msamp_linear_backward_args* a, msamp_
     if (rc != MSAMP_OK) return rc;
     MSAMP_REQUIRE(s.parts == 0 || (a->scratch && aligned(a->scratch, 16) && a->scratch_bytes >= static_cast<int64_t>(s.parts)),
                   MSAMP_ERR_WORKSPACE, "msamp_linear_backward: scratch of %lld bytes", static_cast<long long>(a->scratch_bytes));
+    hipStream_t st = static_cast<hipStream_t>(stream);
     uint8_t* codes = a->dy_codes;
     uint8_t* product = static_cast<uint8_t*>(a->scratch);
     if (bias) {
@@ -95,8 +98,8 @@ extern "C" int msamp_linear_backward(const msamp_linear_backward_args* a, msamp_
     }
     if (rc != MSAMP_OK) return rc;
     if (a->dx != nullptr) {
-        rc = msamp_fp8_gemm_kmajor(a->w_codes, MSAMP_DT_E4M3, a->w_scale_inv, 1, codes, MSAMP_DT_E5M2, a->g_scale_inv, 0, a->dx, out_dtype,
-                                   d_in, tokens, d_out, 0, nullptr, MSAMP_DT_F32, stream);
+        rc = gemm_kmajor(a->w_codes, MSAMP_DT_E4M3, a->w_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, 0, a->dx, out_dtype, d_in, tokens,
+                         d_out, 0, st);
         if (rc != MSAMP_OK) return rc;
     }
     if (!wgrad) return MSAMP_OK;
@@ -109,8 +112,8 @@ extern "C" int msamp_linear_backward(const msamp_linear_backward_args* a, msamp_
         rc = msamp_fp8_gemm_ksplit(a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, product, out_dtype, d_in,
                                    d_out, tokens, accumulate, reinterpret_cast<float*>(product + s.parts), s.n_parts, stream);
     } else {
-        rc = msamp_fp8_gemm_kmajor(a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, 1, codes, MSAMP_DT_E5M2, a->g_scale_inv, 1, product, out_dtype,
-                                   d_in, d_out, tokens, accumulate, nullptr, MSAMP_DT_F32, stream);
+        rc = gemm_kmajor(a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, 1, product, out_dtype, d_in, d_out,
+                         tokens, accumulate, st);
     }
     if (rc != MSAMP_OK) return rc;
     return msamp_cast_to_fp8_intime(product, out_dtype, n, a->q_scale, a->q_amax, a->q_scale_inv, a->wq, MSAMP_DT_E4M3, 0,

@@ -720,7 +720,13 @@ def gemm_cast_declines(m, n, k):
     """True if fp8_gemm_cast answers None for this problem whatever the types: shapes it has no form for, and those that are
     better off with 128 x 128 tiles and a cast (takes_small_tiles() of the library)."""
     big, limit = ((n + 255) // 256) * ((m + 255) // 256), _small_tile_limit
-    return m % 256 != 0 or n % 256 != 0 or k % 128 != 0 or (k > 384 and (big <= limit // 2 or (big <= limit and k >= 3072)))
+    return m % 256 != 0 or n % 256 != 0 or k % 128 != 0 or k < 256 or (k > 384 and (big <= limit // 2 or (big <= limit and k >= 3072)))
+
+
+def linear_takes_short_k(tokens, d_in, d_out):
+    """True where linear_backward reads its operands in place although K of a product (d_out for dx, tokens for the weight
+    gradient) is a single slice, which gemm_kmajor_supported does not promise."""
+    return min(tokens, d_out) <= 128 and d_in % 16 == 0 and d_out % 16 == 0 and max(tokens * d_out, d_out * d_in, tokens * d_in) < 2**32
 
 
 def linear_forward(x, x_meta, w, w_meta, out_dtype, bias):

@@ -93,6 +93,8 @@ class _FP8GemmFunction(torch.autograd.Function):
         # the float32 sum where the weight gradient is taken in parts of K).
         in_place = (not need_dgrad or Gemm.kmajor_supported(d_in, tokens, d_out, True, False)) and \
             (not need_wgrad or Gemm.kmajor_supported(d_in, d_out, tokens, True, True))
+        if not in_place and (not need_wgrad or _wgrad_in_one_call(ctx, tokens, d_in, d_out)):
+            in_place = _backend.linear_takes_short_k(tokens, d_in, d_out) and _backward_in_one_call(ctx, output_grad, d_in, need_dgrad)
         output_qtype = Dtypes.dtype_to_qtype[ctx.output_dtype]
         words = ctx.weight_words
         input_grad = bias_grad = None

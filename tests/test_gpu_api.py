@@ -1000,12 +1000,15 @@ def test_scratch_that_cannot_be_had_costs_launches_only(monkeypatch):
 
 
 @pytest.mark.parametrize('tokens,d_in,d_out', [(256, 512, 768), (2048, 256, 512), (300, 272, 144), (129, 16, 16), (96, 128, 512),
-                                               (200, 40, 24), (2500, 512, 512)])
+                                               (200, 40, 24), (2500, 512, 512), (16, 64, 48), (128, 256, 256),
+                                               (300, 272, 112), (1, 16, 16)])
 @pytest.mark.parametrize('dtype,bias_dtype', [(torch.bfloat16, None), (torch.float16, torch.float16), (torch.float32, torch.float32),
                                               (torch.bfloat16, torch.float32)])
 def test_a_linear_layer_by_one_call_each_way_has_the_bits_of_the_single_calls(monkeypatch, tokens, d_in, d_out, dtype, bias_dtype):
     """Outputs, gradients and metas over warm-up and delayed scaling, with the weight gradient new and added to an old one, against
-    the same layer with every entry point called from Python.  Shapes that only the single calls take are among them."""
+    the same layer with every entry point called from Python.  Shapes that only the single calls take are among them.  Where a
+    product has a single slice of K the single calls go over transposed copies and take the bias gradient from a sum of its own:
+    two float32 sums of `tokens` numbers each, apart by their roundings (2 * tokens * 2^-24 of the numbers' sum) and the type's."""
     from msamp import _backend
     from msamp.nn import functional
     gen = torch.Generator(device='cuda').manual_seed(tokens + d_in)
@@ -1026,7 +1029,7 @@ def test_a_linear_layer_by_one_call_each_way_has_the_bits_of_the_single_calls(mo
                 lin.bias.copy_(b0)
         model = LinearReplacer.replace(lin, Dtypes.kfloat16)
         opt = LBAdamW(model.parameters(), lr=0.0)
-        out = []
+        out, sums = [], []
         for step in range(18):
             for micro in range(2):
                 x = xs[(step + micro) % 3].clone().requires_grad_(True)
@@ -1035,19 +1038,27 @@ def test_a_linear_layer_by_one_call_each_way_has_the_bits_of_the_single_calls(mo
                 g = model.weight.grad
                 out += [y.detach(), x.grad, g.value, g.meta.scale_inv.clone()]
             if bias_dtype is not None:
-                out.append(model.bias.grad.clone())
+                sums.append(model.bias.grad.clone())
                 model.bias.grad = None
             out += [t.clone() for m in model.scaling_metas.values() for t in (m.scale, m.scale_inv, m.amax)]
             model.weight.grad = None
             opt.step()
-        return out
+        return out, sums
 
-    got = run()
+    got, got_sums = run()
     taken = list(calls)
     for name in ('_forward_in_one_call', '_backward_in_one_call'):
         monkeypatch.setattr(functional, name, lambda *a: False)
     calls.clear()
-    want = run()
+    want, want_sums = run()
     assert not calls and taken.count('linear_forward') == (36 if d_in % 16 == 0 else 0)
     for i, (a, b) in enumerate(zip(got, want)):
         assert torch.equal(a.view(torch.uint8) if a.dim() else a, b.view(torch.uint8) if b.dim() else b), i
+    most = 2 * max(dy.float().abs().sum(0).max().item() for dy in dys)    # two micro-batches
+    for a, b in zip(got_sums, want_sums):
+        if min(tokens, d_out) > 128:
+            assert torch.equal(a, b)
+        else:
+            eps = max(torch.finfo(t).eps for t in (dtype, bias_dtype))
+            assert (a - b).abs().max().item() <= 2 * tokens * 2**-24 * most + 2 * eps * b.abs().max().item()
+

@@ -1022,3 +1022,38 @@ def test_walk_timed_at_first_use_changes_no_bit(be):
     finally:
         be.forget_gemm_walks()
         be.tune_gemm_walks(True)
+
+
+@pytest.mark.parametrize('m,n,k', [(16, 16, 16), (1, 3, 48), (130, 257, 128), (8192, 4100, 112), (1040, 272, 144), (256, 384, 256),
+                                   (272, 144, 272), (304, 640, 384), (2048, 2048, 400), (1008, 1040, 512), (4096, 2048, 640),
+                                   (3072, 2064, 1152), (2304, 2304, 4112)])
+@pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16, torch.float16])
+def test_paired_tiles_agree_with_the_other_kernels_to_the_bit(be, m, n, k, out_dtype):
+    """128 x 128 tiles with two workgroups to a compute unit: one slice of K up to many, whole and ragged, tiles on every kind of
+    edge, one to two tiles a unit, all layouts, bias and sum, against the kernel that takes the product with the paired form off."""
+    layouts = [(False, False)]
+    if k > 128 and m % 16 == 0 and k % 16 == 0:
+        layouts += [(True, False)] + ([(True, True)] if n % 16 == 0 else [])
+    for a_dt, b_dt in ((5, 5), (5, 6), (6, 5)):
+        a, b = _gpu_codes((m, k), a_dt, 3 * m + k + a_dt), _gpu_codes((n, k), b_dt, 7 * n + k + b_dt)
+        sa, sb = torch.tensor(0.25, device='cuda'), torch.tensor(2.0, device='cuda')
+        g = torch.Generator(device='cuda').manual_seed(m + n)
+        bias = torch.randn(m, device='cuda', generator=g).to(out_dtype)
+        prev = torch.randn(n, m, device='cuda', generator=g).to(out_dtype)
+        for a_k, b_k in layouts:
+            x, y = (a.t().contiguous() if a_k else a), (b.t().contiguous() if b_k else b)
+            for extra in ({}, dict(bias=bias), dict(bias=bias, accumulate=True)):
+                outs = []
+                try:
+                    for limit in (128, 0):
+                        be.set_small_tile_limit(limit)
+                        buf = torch.full((n + 2, m), 7.0, dtype=out_dtype, device='cuda')
+                        out = buf[1:n + 1]
+                        out.copy_(prev)
+                        be.fp8_gemm(x, a_dt, sa, y, b_dt, sb, out, a_kmajor=a_k, b_kmajor=b_k, **extra)
+                        assert bool((buf[0] == 7).all()) and bool((buf[n + 1] == 7).all())
+                        outs.append(out.clone())
+                finally:
+                    be.set_small_tile_limit(128)
+                view = torch.int32 if out_dtype == torch.float32 else torch.int16
+                assert torch.equal(outs[0].view(view), outs[1].view(view)), (a_dt, b_dt, a_k, b_k, list(extra))

@@ -316,6 +316,36 @@ def test_direct_to_lds_gemm_kernels_leave_the_accumulator_registers_alone(gemm_a
         assert ours >= (320 if name in small else 512) and compilers == 0 and scratch == 0, (name, ours, compilers, scratch)
 
 
+@pytest.mark.parametrize('pair', GEMM_PAIRS)
+def test_paired_gemm_kernels_leave_their_accumulators_to_the_matrix_instructions(gemm_assembly, pair):
+    """The accumulators of fp8_gemm_pair128_kernel are v192 and up, behind the compiler's back: outside the inline assembly
+    nothing may name those registers, and no vector instruction may write an operand of an MFMA less than two instructions
+    ahead of it (the compiler, which would wait, does not know the MFMA for one)."""
+    registers = lambda text: {n for m in re.finditer(r'\bv(\d+)\b|\bv\[(\d+):(\d+)\]', text)
+                              for n in ([int(m.group(1))] if m.group(1) else range(int(m.group(2)), int(m.group(3)) + 1))}
+    kernel, in_asm, products, recent = None, False, {}, []
+    for line in itertools.chain.from_iterable(open(path) for path in gemm_assembly[pair]):
+        m = re.match(r'^(_Z\w+):', line)
+        if m:
+            kernel, recent = m.group(1), []
+        elif '#ASMSTART' in line:
+            in_asm = True
+        elif '#ASMEND' in line:
+            in_asm = False
+        code = line.split(';')[0].strip()
+        if m or not kernel or 'fp8_gemm_pair128_kernel' not in kernel or not code or code.startswith('.') or code.endswith(':'):
+            continue
+        if not in_asm:
+            assert max(registers(code), default=0) < 192, (kernel, code)
+        op, args = code.split()[0], code[len(code.split()[0]):].split(',')
+        if op.startswith('v_mfma'):
+            products[kernel] = products.get(kernel, 0) + 1
+            assert not (registers(args[1]) | registers(args[2])) & set().union(*recent[-2:]), (kernel, code)
+        recent += [set()] * (int(args[0]) + 1) if op == 's_nop' else [registers(args[0]) if op.startswith('v_') and 'mfma' not in op else set()]
+        recent = recent[-2:]
+    assert len(products) == 18 and min(products.values()) >= 16    # three output types, three layouts, whole and ragged K
+
+
 def test_entry_points_refuse_bad_arguments_before_touching_a_gpu():
     """Argument checks of the entry points run on the host before any HIP call: what they refuse, and the walk registry
     (host data only), can be tried without a GPU."""
