@@ -326,7 +326,10 @@ int msamp_fp8_gemm_cast(const uint8_t* a, int a_type, const float* a_scale_inv, 
  *
  * Forward: msamp_cast_to_fp8_gated (x to E4M3), msamp_cast_scaled_to_fp8 (the scaled 16- or 32-bit weight to E4M3; w_meta
  * receives {scale, scale_inv, update count, amax window} as four-byte words), msamp_fp8_gemm with the bias.  d_in must be a
- * multiple of 16. */
+ * multiple of 16.  With w_codes NULL (nobody needs them; at most MSAMP_FEW_TOKENS tokens, w, x_codes and y 16-byte aligned) the
+ * last two are one launch: the weight is quantized to the same codes on its way into the product, and the float32 sum is taken in
+ * up to eight parts of K; x_codes is scratch of 2048 bytes for every 16 tokens and 128 of d_in begun. */
+#define MSAMP_FEW_TOKENS 64
 typedef struct msamp_linear_forward_args {
     const void* x;             /* [tokens][d_in], x_dtype */
     int64_t x_dtype, tokens, d_in, d_out;
@@ -341,8 +344,8 @@ typedef struct msamp_linear_forward_args {
     const float* w_amax;
     const float* w_scale_inv;
     int64_t w_window;
-    uint8_t* w_codes;          /* out: [d_out][d_in] E4M3 */
-    float* w_meta;             /* out: 3 + w_window words */
+    uint8_t* w_codes;          /* nullable, out: [d_out][d_in] E4M3 */
+    float* w_meta;             /* out: 3 + w_window words (not without w_codes) */
     void* y;                   /* out: [tokens][d_out], y_dtype */
     int64_t y_dtype;
     const void* bias;          /* nullable: [d_out], bias_dtype */

@@ -2029,3 +2029,67 @@ int msamp_scale_update_groups(const msamp_scale_group* groups, int n_groups, int
 }
 
 }    // extern "C"
+
+namespace msamp {
+
+// A workgroup per 128-wide slice of K; a thread takes 16 elements (32 or 64 bytes in, 16 out) at a time.  A few hundred KiB in
+// all: bound by its launch.
+template <typename IT>
+__global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __restrict__ x, uint8_t* __restrict__ out, int tokens, int K,
+                                                                const float* __restrict__ scale_p, float* amax, float* scale_inv,
+                                                                int vec_ok) {
+    constexpr int EPT = In16<IT>::EPT;
+    __shared__ uint32_t red[kCastThreads / kWave];
+    const float s = *scale_p;
+    const int pieces = (tokens + 15) / 16 * 128;
+    float mx = 0.0f;
+    for (int p = threadIdx.x; p < pieces; p += kCastThreads) {
+        const int l = p & 63, token = p / 128 * 16 + (l & 15), k = blockIdx.x * 128 + (p >> 6 & 1) * 64 + (l >> 4) * 16;
+        uint4 q = make_uint4(0, 0, 0, 0);
+        if (token < tokens && k < K) {
+            const IT* src = x + static_cast<size_t>(token) * K + k;
+            float v[16];
+            if (vec_ok) {
+#pragma unroll
+                for (int j = 0; j < 16 / EPT; ++j) In16<IT>::load(src + j * EPT, v + j * EPT);
+            } else {
+                for (int j = 0; j < 16; ++j) v[j] = Elem<IT>::load(src + j);
+            }
+#pragma unroll
+            for (int j = 0; j < 16; ++j) mx = fmaxf(mx, fabsf(v[j]));
+            q.x = quant4<MSAMP_DT_E4M3>(v[0] * s, v[1] * s, v[2] * s, v[3] * s);
+            q.y = quant4<MSAMP_DT_E4M3>(v[4] * s, v[5] * s, v[6] * s, v[7] * s);
+            q.z = quant4<MSAMP_DT_E4M3>(v[8] * s, v[9] * s, v[10] * s, v[11] * s);
+            q.w = quant4<MSAMP_DT_E4M3>(v[12] * s, v[13] * s, v[14] * s, v[15] * s);
+        }
+        *reinterpret_cast<uint4*>(out + (static_cast<size_t>(blockIdx.x) * pieces + p) * 16) = q;
+    }
+    const uint32_t m = block_max_u32(__float_as_uint(mx), red);
+    if (threadIdx.x == 0) {
+        amax_publish(amax, __uint_as_float(m));
+        if (blockIdx.x == 0) *scale_inv = 1.0f / s;
+    }
+}
+
+int few_cast_fragments(const void* x, int in_dtype, int tokens, int K, float* scale, float* amax, float* scale_inv, uint8_t* out,
+                       int flags, const int32_t* counter, int window, void* workspace, hipStream_t st) {
+    MSAMP_REQUIRE(is_hp(in_dtype), MSAMP_ERR_DTYPE, "few_cast_fragments: in_dtype %d", in_dtype);
+    MSAMP_REQUIRE(x && scale && amax && scale_inv && out && counter, MSAMP_ERR_NULL, "few_cast_fragments: null pointer");
+    MSAMP_REQUIRE(workspace != nullptr, MSAMP_ERR_WORKSPACE, "few_cast_fragments: workspace required");
+    // (as the gated cast: while warming up the first kernel sets amax[0] and the scale, afterwards it returns at once)
+    const Gate gate = {counter, window};
+    const Finish fin = {amax, scale, scale_inv, fp8_max(MSAMP_DT_E4M3), 0, flags};
+    const int rc = dispatch_amax(x, in_dtype, static_cast<size_t>(tokens) * K, workspace, scale, st, gate, fin);
+    if (rc != MSAMP_OK) return rc;
+    const dim3 grid((K + 127) / 128);
+    const int vec_ok = aligned(x, 16);
+#define FEW_CAST(IT) hipLaunchKernelGGL((few_cast_kernel<IT>), grid, dim3(kCastThreads), 0, st, static_cast<const IT*>(x), out, tokens, K, scale, amax, scale_inv, vec_ok)
+    if (in_dtype == MSAMP_DT_F32) FEW_CAST(float);
+    else if (in_dtype == MSAMP_DT_F16) FEW_CAST(f16_t);
+    else FEW_CAST(bf16_t);
+#undef FEW_CAST
+    MSAMP_CHECK_LAUNCH("few_cast_kernel");
+    return MSAMP_OK;
+}
+
+}    // namespace msamp

@@ -6,8 +6,169 @@
 #include "common.cuh"
 #include "gemm_call.h"
 
+#include <algorithm>
 
 namespace msamp {
+
+// ---- a few tokens through a layer nobody differentiates ---------------------------------------------------------------
+// y[tokens][d_out] = x . fp8(w)^T, the weight read in its scaled 16- or 32-bit form and quantized on its way to the matrix pipes,
+// with the codes msamp_cast_scaled_to_fp8 gives: it is read once (2 bytes an element), where the cast and the product move 4.
+// Bound by that read and by the loads a compute unit has in flight.  A workgroup takes 16 rows of w and all tokens; its (up to)
+// eight wavefronts take the 128-wide slices of K in turn, the next slice's weights in flight over the present one's arithmetic,
+// and their float32 sums meet in LDS in a fixed order.
+// Inside a slice the k of an MFMA's operand bytes are dealt out anew, alike for both operands: lane group g holds k = 16 g .. +15
+// and 64 + 16 g .. +15, so that w arrives in pairs of loads over whole lines.  x comes in the order of the operand registers from
+// its cast (few_cast_fragments): read row by row, 16 rows a long power of two apart, it
+// cost as much as w (48 tokens 42.6 us, 35.5 so).  Both casts and the product together against the weight cast to memory and
+// the product after it, us for 4096 -> 12288: 16 tokens 48.5 -> 29.6, 48 49.2 -> 35.5, 64 49.8 -> 37.7; 64 x 8192 -> 8192 65.6 ->
+// 48.6, 64 x 16384 -> 4096 84.0 -> 51.4, 64 x 2048 -> 16384 36.6 -> 32.1, 16 x 512 -> 512 20.9 -> 15.3 (launches).
+__device__ __forceinline__ float few_bias(const void* bias, int dt, int i) {
+    if (dt == MSAMP_DT_F32) return static_cast<const float*>(bias)[i];
+    if (dt == MSAMP_DT_F16) return f16_bits_to_float(static_cast<const uint16_t*>(bias)[i]);
+    return bf16_bits_to_float(static_cast<const uint16_t*>(bias)[i]);
+}
+typedef int few_v8i __attribute__((ext_vector_type(8)));
+typedef float few_v4f __attribute__((ext_vector_type(4)));
+
+template <typename WT, typename OT, int MB>
+__global__ __launch_bounds__(512) void few_tokens_kernel(const WT* __restrict__ w, const uint8_t* __restrict__ x, OT* __restrict__ y,
+                                                          int tokens, int d_out, int K, const float* __restrict__ w_amax,
+                                                          const float* __restrict__ w_scale_inv, const float* __restrict__ x_scale_inv,
+                                                          const void* __restrict__ bias, int bias_dt, int stream) {
+    extern __shared__ __attribute__((aligned(16))) float4 few_part[];    // [wavefronts][MB][64]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int l16 = lane & 15, g4 = lane >> 4;
+    const float s_new = scale_rule(*w_amax, 1.0f, 448.0f, 0);
+    const float s = s_new * *w_scale_inv;
+    // (rows past the end are clamped: their products land in outputs that are not stored)
+    const WT* wp = w + static_cast<size_t>(min(static_cast<int>(blockIdx.x) * 16 + l16, d_out - 1)) * K + g4 * 16;
+    const uint8_t* xp = x + lane * 16;
+    const int slices = (K + 127) / 128;
+    few_v4f acc[MB];
+#pragma unroll
+    for (int b = 0; b < MB; ++b) acc[b] = few_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+    constexpr int kPer = 16 / static_cast<int>(sizeof(WT));    // weights of a 16-byte load
+    constexpr int kHalf = 16 / kPer;                           // loads of half a slice
+    struct Weights { uint4 v[2][kHalf]; };
+    // (K is a multiple of 16: the 16 k of a lane group's half slice lie inside together or not at all)
+    auto inside = [&](int kt, int h) __attribute__((always_inline)) { return kt * 128 + h * 64 + g4 * 16 < K; };
+    auto fetch = [&](int kt, Weights& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (!inside(kt, h)) continue;
+#pragma unroll
+            for (int j = 0; j < kHalf; ++j) f.v[h][j] = ld16(wp + kt * 128 + h * 64 + j * kPer, stream != 0);
+        }
+    };
+    // the product of slice kt, whose weights are in `f`, and the loads of the wavefront's next slice into `next`
+    auto work = [&](int kt, const Weights& f, Weights& next) __attribute__((always_inline)) {
+        uint4 xr[MB][2];
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) xr[b][h] = *reinterpret_cast<const uint4*>(xp + ((static_cast<size_t>(kt) * MB + b) * 2 + h) * 1024);
+        if (kt + waves < slices) fetch(kt + waves, next);
+        few_v8i a;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float v[16];
+#pragma unroll
+            for (int j = 0; j < kHalf; ++j) In16<WT>::decode(f.v[h][j], v + j * kPer);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                a[h * 4 + j] = static_cast<int>(quant4<MSAMP_DT_E4M3>(v[4 * j] * s, v[4 * j + 1] * s, v[4 * j + 2] * s, v[4 * j + 3] * s));
+        }
+        if (kt * 128 + 128 > K) {    // the ragged last slice: what was not loaded is zero
+#pragma unroll
+            for (int i = 0; i < 8; ++i) a[i] = inside(kt, i >> 2) ? a[i] : 0;
+        }
+#pragma unroll
+        for (int b = 0; b < MB; ++b) {
+            few_v8i bx;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) bx[h * 4] = xr[b][h].x, bx[h * 4 + 1] = xr[b][h].y, bx[h * 4 + 2] = xr[b][h].z, bx[h * 4 + 3] = xr[b][h].w;
+            acc[b] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, bx, acc[b], 0, 0, 0, 0, 0, 0);
+        }
+    };
+    Weights even = {}, odd = {};
+    int kt = wave;
+    if (kt < slices) fetch(kt, even);
+    while (kt < slices) {
+        work(kt, even, odd);
+        kt += waves;
+        if (kt >= slices) break;
+        work(kt, odd, even);
+        kt += waves;
+    }
+#pragma unroll
+    for (int b = 0; b < MB; ++b) few_part[(wave * MB + b) * 64 + lane] = make_float4(acc[b][0], acc[b][1], acc[b][2], acc[b][3]);
+    __syncthreads();
+
+    // a lane of a block of tokens has four consecutive outputs of one token
+    const float alpha = *x_scale_inv * (1.0f / s_new);
+    const bool whole = d_out % 4 == 0;
+    for (int i = threadIdx.x; i < MB * 64; i += blockDim.x) {
+        float4 t = few_part[i];
+        for (int v = 1; v < waves; ++v) {
+            const float4 u = few_part[v * MB * 64 + i];
+            t.x += u.x, t.y += u.y, t.z += u.z, t.w += u.w;
+        }
+        const int token = i / 64 * 16 + (i & 15), col = blockIdx.x * 16 + ((i & 63) >> 4) * 4;
+        if (token >= tokens) continue;
+        const float f[4] = {t.x, t.y, t.z, t.w};
+        struct __attribute__((aligned(4 * sizeof(OT)))) Four { OT v[4]; };
+        Four o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (bias != nullptr) Elem<OT>::store(&o.v[e], fmaf(f[e], alpha, col + e < d_out ? few_bias(bias, bias_dt, col + e) : 0.0f));
+            else Elem<OT>::store(&o.v[e], f[e] * alpha);
+        }
+        OT* out = y + static_cast<size_t>(token) * d_out + col;
+        if (whole) {
+            if (col < d_out) *reinterpret_cast<Four*>(out) = o;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (col + e < d_out) out[e] = o.v[e];
+        }
+    }
+}
+
+template <typename WT, typename OT, int MB>
+static int launch_few_tokens(const msamp_linear_forward_args& a, hipStream_t st) {
+    const int tokens = static_cast<int>(a.tokens), d_out = static_cast<int>(a.d_out), K = static_cast<int>(a.d_in);
+    const int waves = std::min(8, (K + 127) / 128);    // (four are level with eight, but for one round of few workgroups: 16 x 12288 -> 4096 34.2, 30.5)
+    hipLaunchKernelGGL((few_tokens_kernel<WT, OT, MB>), dim3((d_out + 15) / 16), dim3(64 * waves), waves * MB * 1024, st,
+                       static_cast<const WT*>(a.w), a.x_codes, static_cast<OT*>(a.y), tokens, d_out, K, a.w_amax, a.w_scale_inv,
+                       a.x_scale_inv, a.bias, static_cast<int>(a.bias_dtype),
+                       static_cast<int>(static_cast<size_t>(d_out) * K * sizeof(WT) >= kStreamBytes));
+    MSAMP_CHECK_LAUNCH("few_tokens_kernel");
+    return MSAMP_OK;
+}
+
+template <typename WT, typename OT>
+static int few_tokens_blocks(const msamp_linear_forward_args& a, hipStream_t st) {
+    switch ((a.tokens + 15) / 16) {
+        case 1: return launch_few_tokens<WT, OT, 1>(a, st);
+        case 2: return launch_few_tokens<WT, OT, 2>(a, st);
+        case 3: return launch_few_tokens<WT, OT, 3>(a, st);
+        default: return launch_few_tokens<WT, OT, 4>(a, st);
+    }
+}
+
+template <typename WT>
+static int few_tokens_out(const msamp_linear_forward_args& a, hipStream_t st) {
+    if (a.y_dtype == MSAMP_DT_F32) return few_tokens_blocks<WT, float>(a, st);
+    if (a.y_dtype == MSAMP_DT_F16) return few_tokens_blocks<WT, f16_t>(a, st);
+    return few_tokens_blocks<WT, bf16_t>(a, st);
+}
+
+static int few_tokens(const msamp_linear_forward_args& a, hipStream_t st) {
+    if (a.w_dtype == MSAMP_DT_F32) return few_tokens_out<float>(a, st);
+    if (a.w_dtype == MSAMP_DT_F16) return few_tokens_out<f16_t>(a, st);
+    return few_tokens_out<bf16_t>(a, st);
+}
 
 static size_t round_up(size_t n) { return (n + 255) / 256 * 256; }
 
@@ -45,9 +206,25 @@ extern "C" int msamp_linear_forward(const msamp_linear_forward_args* a, msamp_st
     MSAMP_REQUIRE(a != nullptr, MSAMP_ERR_NULL, "msamp_linear_forward: null arguments");
     MSAMP_REQUIRE(dims_ok(a->tokens, a->d_in, a->d_out), MSAMP_ERR_SHAPE, "msamp_linear_forward: %lld x %lld -> %lld",
                   static_cast<long long>(a->tokens), static_cast<long long>(a->d_in), static_cast<long long>(a->d_out));
-    MSAMP_REQUIRE(a->w_meta, MSAMP_ERR_NULL, "msamp_linear_forward: null w_meta");
+    MSAMP_REQUIRE(a->w_codes == nullptr || a->w_meta, MSAMP_ERR_NULL, "msamp_linear_forward: null w_meta");
     const size_t nx = static_cast<size_t>(a->tokens) * a->d_in, nw = static_cast<size_t>(a->d_out) * a->d_in;
     const int x_dtype = static_cast<int>(a->x_dtype), w_dtype = static_cast<int>(a->w_dtype), y_dtype = static_cast<int>(a->y_dtype);
+    if (a->w_codes == nullptr) {
+        // (refused here and not behind the cast, which changes the input meta)
+        MSAMP_REQUIRE(is_hp(w_dtype) && is_hp(y_dtype) && (a->bias == nullptr || is_hp(static_cast<int>(a->bias_dtype))), MSAMP_ERR_DTYPE,
+                      "msamp_linear_forward: dtypes %d -> %d", w_dtype, y_dtype);
+        MSAMP_REQUIRE(a->tokens <= MSAMP_FEW_TOKENS && a->d_in % 16 == 0, MSAMP_ERR_SHAPE,
+                      "msamp_linear_forward: %lld x %lld without codes of w", static_cast<long long>(a->tokens), static_cast<long long>(a->d_in));
+        MSAMP_REQUIRE(a->w && a->y && a->w_amax && a->w_scale_inv, MSAMP_ERR_NULL, "msamp_linear_forward: null pointer");
+        MSAMP_REQUIRE(aligned(a->w, 16) && aligned(a->x_codes, 16) && aligned(a->y, 16), MSAMP_ERR_ALIGNMENT,
+                      "msamp_linear_forward: w, x_codes and y must be 16-byte aligned");
+    }
+    if (a->w_codes == nullptr) {
+        const int rc = few_cast_fragments(a->x, x_dtype, static_cast<int>(a->tokens), static_cast<int>(a->d_in), a->x_scale, a->x_amax,
+                                          a->x_scale_inv, a->x_codes, static_cast<int>(a->flags), a->x_counter,
+                                          static_cast<int>(a->x_window), a->workspace, static_cast<hipStream_t>(stream));
+        return rc != MSAMP_OK ? rc : few_tokens(*a, static_cast<hipStream_t>(stream));
+    }
     int rc = msamp_cast_to_fp8_gated(a->x, x_dtype, nx, a->x_scale, a->x_amax, a->x_scale_inv, a->x_codes, MSAMP_DT_E4M3, 0,
                                      static_cast<int>(a->flags), a->x_counter, static_cast<int>(a->x_window), a->workspace, stream);
     if (rc != MSAMP_OK) return rc;

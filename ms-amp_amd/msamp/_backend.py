@@ -729,21 +729,28 @@ def linear_takes_short_k(tokens, d_in, d_out):
     return min(tokens, d_out) <= 128 and d_in % 16 == 0 and d_out % 16 == 0 and max(tokens * d_out, d_out * d_in, tokens * d_in) < 2**32
 
 
-def linear_forward(x, x_meta, w, w_meta, out_dtype, bias):
+FEW_TOKENS = 64    # MSAMP_FEW_TOKENS
+
+
+def linear_forward(x, x_meta, w, w_meta, out_dtype, bias, want_codes=True):
     """y = x . w^T (+ bias) through msamp_linear_forward.  x: contiguous [tokens, d_in], cast with x_meta (gated scaling); w: the
-    contiguous scaled payload [d_out, d_in] of a weight with w_meta.  Returns y, the E4M3 codes of x and of w, and the words
-    {scale, scale_inv, update count, amax window} of the codes of w."""
+    contiguous scaled payload [d_out, d_in] of a weight with w_meta.  Returns y and, if want_codes, the E4M3 codes of x
+    and of w and the words {scale, scale_inv, update count, amax window} of the codes of w (else these are not to be used)."""
     lib = load()
     (tokens, d_in), d_out, device, window = x.shape, w.shape[0], x.device, w_meta.window_size
-    x_codes = torch.empty((tokens, d_in), dtype=torch.uint8, device=device)
-    w_codes = torch.empty((d_out, d_in), dtype=torch.uint8, device=device)
-    words = torch.empty(3 + window, dtype=torch.float32, device=device)
+    if want_codes or tokens > FEW_TOKENS or w.data_ptr() % 16:
+        x_codes = torch.empty((tokens, d_in), dtype=torch.uint8, device=device)
+        w_codes = torch.empty((d_out, d_in), dtype=torch.uint8, device=device)
+        words = torch.empty(3 + window, dtype=torch.float32, device=device)
+    else:    # (codes of x in another order, in whole blocks of 16 tokens and 128 wide)
+        x_codes = torch.empty(((tokens + 15) // 16 * ((d_in + 127) // 128) * 2048, ), dtype=torch.uint8, device=device)
+        w_codes = words = None
     y = torch.empty((tokens, d_out), dtype=out_dtype, device=device)
     args = _LINEAR_FORWARD.pack(
         x.data_ptr(), _TORCH_TO_DT[x.dtype], tokens, d_in, d_out, x_meta.scale.data_ptr(), x_meta.amax.data_ptr(),
         x_meta.scale_inv.data_ptr(), x_meta.amax_counter.data_ptr(), x_meta.window_size, x_codes.data_ptr(), w.data_ptr(),
-        _TORCH_TO_DT[w.dtype], w_meta.amax.data_ptr(), w_meta.scale_inv.data_ptr(), window, w_codes.data_ptr(), words.data_ptr(),
-        y.data_ptr(), _TORCH_TO_DT[out_dtype], 0 if bias is None else bias.data_ptr(),
+        _TORCH_TO_DT[w.dtype], w_meta.amax.data_ptr(), w_meta.scale_inv.data_ptr(), window,
+        0 if w_codes is None else w_codes.data_ptr(), 0 if words is None else words.data_ptr(), y.data_ptr(), _TORCH_TO_DT[out_dtype], 0 if bias is None else bias.data_ptr(),
         DT_F32 if bias is None else _TORCH_TO_DT[bias.dtype], FLAG_TWO_PASS if _two_pass_only() else 0, workspace(device).data_ptr()
     )
     _check(lib.msamp_linear_forward(args, _stream()), 'msamp_linear_forward')

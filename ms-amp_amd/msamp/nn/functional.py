@@ -56,7 +56,7 @@ class _FP8GemmFunction(torch.autograd.Function):
     two) and its gradient, the column sums of dy in the output type, is returned from backward as autograd would
     have formed it."""
     @staticmethod
-    def forward(ctx, input, weight, metas, dtype_holder, bias=None):
+    def forward(ctx, input, weight, metas, dtype_holder, bias=None, differentiable=True):
         ctx.metas = metas
         model_state.check_metas_in_flat(metas)
         output_dtype = dtype_holder.dtype
@@ -71,7 +71,7 @@ class _FP8GemmFunction(torch.autograd.Function):
         meta = metas['input']
         if _forward_in_one_call(src, meta, weight, output_dtype, bias):
             out, ctx.input_codes, ctx.weight_codes, ctx.weight_words = _backend.linear_forward(
-                src, meta, weight.value, weight.meta, output_dtype, bias
+                src, meta, weight.value, weight.meta, output_dtype, bias, differentiable
             )
             return out
         input_fp8 = src.cast(Dtypes.kfloat8_e4m3, meta=meta)
@@ -165,7 +165,7 @@ class _FP8GemmFunction(torch.autograd.Function):
 
         if ctx.need_bias_grad and bias_grad is None:
             bias_grad = output_grad.sum(0).to(ctx.bias_dtype)
-        return input_grad, None, None, None, bias_grad
+        return input_grad, None, None, None, bias_grad, None
 
 
 class FunctionalOverider:
@@ -205,7 +205,8 @@ class FunctionalOverider:
                 output_dtype = torch.get_autocast_dtype('cuda')
             else:
                 output_dtype = input.dtype
-            out = _FP8GemmFunction.apply(input, weight, weight._scaling_metas, cls.EMPTY_GRAD_TENSOR.type(output_dtype), bias)
+            out = _FP8GemmFunction.apply(input, weight, weight._scaling_metas, cls.EMPTY_GRAD_TENSOR.type(output_dtype), bias,
+                                         torch.is_grad_enabled())
             if len(shape) != 2:
                 out = out.view(shape[:-1] + (-1, ))
             return out

@@ -1062,3 +1062,57 @@ def test_a_linear_layer_by_one_call_each_way_has_the_bits_of_the_single_calls(mo
             eps = max(torch.finfo(t).eps for t in (dtype, bias_dtype))
             assert (a - b).abs().max().item() <= 2 * tokens * 2**-24 * most + 2 * eps * b.abs().max().item()
 
+
+@pytest.mark.parametrize('tokens,d_in,d_out', [(1, 16, 1), (3, 144, 5), (16, 128, 16), (17, 272, 33), (33, 1040, 132), (48, 64, 4097),
+                                               (64, 2064, 260), (64, 8192, 512)])
+@pytest.mark.parametrize('qtype', [Dtypes.kfloat16, Dtypes.kbfloat16, Dtypes.kfloat32])
+@pytest.mark.parametrize('dtype,bias', [(torch.bfloat16, False), (torch.float16, True), (torch.float32, True)])
+def test_a_few_tokens_without_gradients_have_the_bits_of_the_differentiable_forward(tokens, d_in, d_out, qtype, dtype, bias):
+    """Whole numbers up to 2, whose products sum exactly in float32 in any order (4 * 8192 < 2**24), so that both forwards give the
+    exact result rounded once; the input meta goes through warm-up and delayed scaling alike; and NaN and infinities in x, the
+    weight's codes at saturation, and what lies behind the tensors stays where it is."""
+    gen = torch.Generator(device='cuda').manual_seed(tokens + d_in + d_out)
+    whole = lambda *shape: torch.randint(-2, 3, shape, device='cuda', generator=gen).to(dtype)
+    lin = torch.nn.Linear(d_in, d_out, bias=bias).cuda().to(dtype)
+    with torch.no_grad():
+        lin.weight.copy_(whole(d_out, d_in))
+        lin.weight.view(-1)[0] = 2.0    # (the scales below hold for every draw)
+        if bias:
+            lin.bias.copy_(whole(d_out))
+    model_state.clear()
+    model = LinearReplacer.replace(lin, qtype)
+    metas = model.scaling_metas['input']
+    for step in range(4):
+        x = whole(tokens, d_in)
+        x.view(-1)[-1] = 2.0
+        if step == 2:
+            metas.amax_counter.fill_(16)    # from here on scaling is delayed
+        if step == 3:
+            x.view(-1)[0] = float('nan') if tokens % 2 else float('inf')
+        start = [t.clone() for t in (metas.scale, metas.scale_inv, metas.amax)]
+        want = model(x).detach()
+        after = [t.clone() for t in (metas.scale, metas.scale_inv, metas.amax)]
+        for t, old in zip((metas.scale, metas.scale_inv, metas.amax), start):
+            t.copy_(old)
+        with torch.no_grad():
+            got = model(x)
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(want)), step
+        assert all(same_float(a, b) for a, b in zip((metas.scale, metas.scale_inv, metas.amax), after))
+
+
+def test_a_few_tokens_without_gradients_lose_no_precision():
+    """Real values: against the product of the same codes in 64 bits, the sum in eight parts is as near as the sum in one chain."""
+    from msamp import _backend
+    gen = torch.Generator(device='cuda').manual_seed(4)
+    for tokens, d_in, d_out in ((5, 4096, 512), (48, 2048, 1024), (64, 400, 100)):
+        w = (torch.randn(d_out, d_in, device='cuda', generator=gen) * 0.02).cast(Dtypes.kfloat16)
+        x = torch.randn(tokens, d_in, device='cuda', generator=gen)
+        meta = ScalingMeta(Dtypes.kfloat8_e4m3, window_size=16)
+        meta.amax_counter.fill_(16)
+        meta.scale.fill_(64.0)
+        y, x_codes, w_codes, words = _backend.linear_forward(x, meta, w.value, w.meta, torch.float32, None)
+        exact = _backend.cast_from_fp8(x_codes, meta.scale_inv, 5, torch.float32).double() @ \
+            _backend.cast_from_fp8(w_codes, words[1], 5, torch.float32).double().t()
+        few = _backend.linear_forward(x, meta, w.value, w.meta, torch.float32, None, want_codes=False)[0]
+        assert rel_fro(few.double(), exact) <= 1.1 * rel_fro(y.double(), exact) + 1e-7
