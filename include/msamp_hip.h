@@ -321,8 +321,9 @@ int msamp_fp8_gemm_cast(const uint8_t* a, int a_type, const float* a_scale_inv, 
                         void* workspace, msamp_stream_t stream);
 
 /* One direction of an FP8Linear layer as one call (the reference's sequence of calls: msamp/nn/functional.py:20-123): the
- * entry points named below, one after the other on `stream`, with the arguments a layer in gated scaling gives them.  Every
- * field is eight bytes wide.  Results, metas and error codes are those of the entry points.
+ * entry points named below, one after the other on `stream`, with the arguments a layer in gated scaling gives them, some of
+ * their kernels side by side in one launch.  Every field is eight bytes wide.  Results, metas and error codes are those of the
+ * entry points.
  *
  * Forward: msamp_cast_to_fp8_gated (x to E4M3), msamp_cast_scaled_to_fp8 (the scaled 16- or 32-bit weight to E4M3; w_meta
  * receives {scale, scale_inv, update count, amax window} as four-byte words), msamp_fp8_gemm with the bias.  d_in must be a
@@ -380,7 +381,7 @@ typedef struct msamp_linear_backward_args {
     float* q_scale;            /* the weight gradient's meta */
     float* q_amax;
     float* q_scale_inv;
-    const uint8_t* old_codes;  /* nullable: the weight gradient to add to, [d_out][d_in], old_type (may share q_scale_inv) */
+    const uint8_t* old_codes;  /* nullable: the weight gradient to add to, [d_out][d_in] E4M3 (may share q_scale_inv) */
     const float* old_scale_inv;
     int64_t old_type;
     void* bias_sum;            /* nullable, out: [d_out], bias_sum_dtype */

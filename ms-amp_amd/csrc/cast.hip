@@ -3,7 +3,9 @@
 // wavefront shuffle reductions, one atomic per block.
 #include "common.cuh"
 #include "gemm_call.h"
+#include "linear_call.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -102,12 +104,11 @@ __device__ __forceinline__ float resolve_in_time_scale(const InTimeArgs& a, uint
 // Every workgroup ends with one atomic on the amax cell, and atomics on one address are served one
 // at a time (about 10 ns each): the launch with WITH_AMAX uses few, large workgroups (THREADS = 512,
 // two per CU) so that they stay a small part of the run time.
-template <typename IT, int FMT, bool WITH_AMAX, int INTIME, int THREADS = kCastThreads>
-__global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restrict__ x,
-                                                                    uint8_t* __restrict__ out, size_t n,
-                                                                    const float* __restrict__ scale_p, float* amax,
-                                                                    float* scale_inv, int vec_ok, int reverse,
-                                                                    InTimeArgs it) {
+// (`block` of `blocks`: the whole launch, or the part of one that casts)
+template <typename IT, int FMT, bool WITH_AMAX, int INTIME, int THREADS>
+__device__ __forceinline__ void cast_to_fp8(const IT* __restrict__ x, uint8_t* __restrict__ out, size_t n,
+                                            const float* __restrict__ scale_p, float* amax, float* scale_inv, int vec_ok,
+                                            int reverse, const InTimeArgs& it, unsigned block, unsigned blocks) {
     constexpr int EPT = In16<IT>::EPT;
     constexpr size_t TILE = static_cast<size_t>(THREADS) * EPT * kCastUnroll;
     __shared__ uint32_t red[THREADS / kWave];
@@ -119,12 +120,12 @@ __global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restri
     } else if constexpr (INTIME == kRescale) {
         const float s_new = scale_rule(*it.known_amax, 1.0f, it.fp_max, it.margin);
         s = s_new * *it.old_scale_inv;
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (block == 0 && threadIdx.x == 0) {
             *it.scale_out = s;
             *scale_inv = 1.0f / s_new;
             if (it.counter_out != nullptr) *it.counter_out = 0;
         }
-        if (blockIdx.x == 0 && it.amax_copy != nullptr) {
+        if (block == 0 && it.amax_copy != nullptr) {
             for (int j = threadIdx.x; j < it.window; j += blockDim.x) it.amax_copy[j] = it.known_amax[j];
         }
     } else if constexpr (INTIME == kGivenIfFlagged) {
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restri
     const int tid = threadIdx.x;
     float mx = 0.0f;
     const size_t ntiles = (n + TILE - 1) / TILE;
-    for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    for (size_t t = block; t < ntiles; t += blocks) {
         const size_t tile = reverse ? (ntiles - 1 - t) : t;
         const size_t base = tile * TILE;
         if ((vec_ok & 1) && base + TILE <= n) {
@@ -174,8 +175,17 @@ __global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restri
         if (tid == 0) amax_publish(amax, __uint_as_float(m));
     }
     if constexpr (INTIME == kGivenScale) {
-        if (scale_inv != nullptr && blockIdx.x == 0 && tid == 0) *scale_inv = 1.0f / s;
+        if (scale_inv != nullptr && block == 0 && tid == 0) *scale_inv = 1.0f / s;
     }
+}
+
+template <typename IT, int FMT, bool WITH_AMAX, int INTIME, int THREADS = kCastThreads>
+__global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restrict__ x,
+                                                                    uint8_t* __restrict__ out, size_t n,
+                                                                    const float* __restrict__ scale_p, float* amax,
+                                                                    float* scale_inv, int vec_ok, int reverse,
+                                                                    InTimeArgs it) {
+    cast_to_fp8<IT, FMT, WITH_AMAX, INTIME, THREADS>(x, out, n, scale_p, amax, scale_inv, vec_ok, reverse, it, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -330,26 +340,25 @@ struct Finish {
 };
 constexpr int kWsTicket = 2;
 
-template <typename IT>
-__global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __restrict__ x, size_t n, uint32_t* ws,
-                                                                     const float* scale, int vec_ok, Gate gate,
-                                                                     Finish fin) {
+template <typename IT, int THREADS>
+__device__ __forceinline__ void amax_partial(const IT* __restrict__ x, size_t n, uint32_t* ws, const float* scale, int vec_ok,
+                                             const Gate& gate, const Finish& fin, unsigned block, unsigned blocks) {
     if (gate_closed(gate)) return;
     constexpr int EPT = 16 / sizeof(IT);
     constexpr int UNROLL = 8;
-    constexpr size_t TILE = static_cast<size_t>(kCastThreads) * EPT * UNROLL;
-    __shared__ uint32_t red[kCastThreads / kWave];
+    constexpr size_t TILE = static_cast<size_t>(THREADS) * EPT * UNROLL;
+    __shared__ uint32_t red[THREADS / kWave];
     const int tid = threadIdx.x;
     // running max of the |x| bit pattern; for 2-byte inputs kept in the high half-word
     uint32_t m = 0;
     const size_t ntiles = (n + TILE - 1) / TILE;
-    for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    for (size_t t = block; t < ntiles; t += blocks) {
         const size_t base = t * TILE;
         if (vec_ok && base + TILE <= n) {
             uint4 v[UNROLL];
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u)
-                v[u] = *reinterpret_cast<const uint4*>(x + base + (static_cast<size_t>(u) * kCastThreads + tid) * EPT);
+                v[u] = *reinterpret_cast<const uint4*>(x + base + (static_cast<size_t>(u) * THREADS + tid) * EPT);
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {
                 const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
@@ -364,7 +373,7 @@ __global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __
             }
         } else {
             const size_t end = (base + TILE < n) ? base + TILE : n;
-            for (size_t i = base + tid; i < end; i += kCastThreads) {
+            for (size_t i = base + tid; i < end; i += THREADS) {
                 if constexpr (sizeof(IT) == 4) {
                     m = umax(m, reinterpret_cast<const uint32_t*>(x)[i] & 0x7fffffffu);
                 } else {
@@ -379,10 +388,10 @@ __global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __
         if constexpr (sizeof(IT) == 2 && !__is_same(IT, bf16_t)) {
             m = __float_as_uint(f16_bits_to_float(m >> 16));
         }
-        ws[kWsPartials + blockIdx.x] = m;
-        if (blockIdx.x == 0) {
+        ws[kWsPartials + block] = m;
+        if (block == 0) {
             ws[0] = scale != nullptr ? __float_as_uint(*scale) : __float_as_uint(1.0f);
-            ws[1] = gridDim.x;
+            ws[1] = blocks;
         }
     }
     if (fin.amax == nullptr) return;
@@ -390,14 +399,14 @@ __global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __
     if (tid == 0) {
         __threadfence();    // the partial maximum above is visible before the ticket is taken
         const uint32_t ticket = atomicAdd(ws + kWsTicket, 1u);
-        s_last = ticket == gridDim.x - 1;
+        s_last = ticket == blocks - 1;
         if (s_last) ws[kWsTicket] = 0;    // ready for the next call
     }
     __syncthreads();
     if (!s_last) return;
     __threadfence();    // see every other workgroup's partial maximum
     uint32_t mm = 0;
-    for (int i = tid; i < static_cast<int>(gridDim.x); i += kCastThreads) {
+    for (int i = tid; i < static_cast<int>(blocks); i += THREADS) {
         const uint32_t v = __hip_atomic_load(ws + kWsPartials + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         mm = v > mm ? v : mm;
     }
@@ -410,6 +419,30 @@ __global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __
         *fin.scale = sc;
         *fin.scale_inv = 1.0f / sc;
     }
+}
+
+template <typename IT>
+__global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __restrict__ x, size_t n, uint32_t* ws,
+                                                                     const float* scale, int vec_ok, Gate gate,
+                                                                     Finish fin) {
+    amax_partial<IT, kCastThreads>(x, n, ws, scale, vec_ok, gate, fin, blockIdx.x, gridDim.x);
+}
+
+// The first kernel of a gated cast beside one that does not depend on it.  As a rule the gate is closed and these workgroups
+// return at once: a launch of their own costs the host 3.5 us and the stream 2.5 for nothing.  The first `others` workgroups do the
+// other work.
+constexpr int kBesideThreads = 512;
+
+// ... the rescaling cast of a linear layer's weight
+template <typename IT, typename WT>
+__global__ __launch_bounds__(kBesideThreads) void amax_beside_rescale_kernel(const IT* __restrict__ x, size_t nx, uint32_t* ws,
+                                                                              const float* scale, int x_vec, Gate gate, Finish fin,
+                                                                              const WT* __restrict__ w, uint8_t* __restrict__ out, size_t nw,
+                                                                              float* scale_inv, int w_vec, InTimeArgs it, unsigned others) {
+    if (blockIdx.x < others)
+        cast_to_fp8<WT, MSAMP_DT_E4M3, false, kRescale, kBesideThreads>(w, out, nw, nullptr, nullptr, scale_inv, w_vec, 0, it, blockIdx.x, others);
+    else
+        amax_partial<IT, kBesideThreads>(x, nx, ws, scale, x_vec, gate, fin, blockIdx.x - others, gridDim.x - others);
 }
 
 // First pass of the in-time cast of a tensor too large for the one-pass kernel, with the output written on
@@ -811,24 +844,22 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(4, 
 }
 
 // ---------------------------------------------------------------------------------------------
-template <int FMT, typename OT>
-__global__ __launch_bounds__(kCastThreads) void cast_from_fp8_kernel(const uint8_t* __restrict__ q,
-                                                                      OT* __restrict__ out, size_t n,
-                                                                      const float* __restrict__ scale_inv_p,
-                                                                      int vec_ok) {
+template <int FMT, typename OT, int THREADS>
+__device__ __forceinline__ void cast_from_fp8(const uint8_t* __restrict__ q, OT* __restrict__ out, size_t n,
+                                              const float* __restrict__ scale_inv_p, int vec_ok, unsigned block, unsigned blocks) {
     constexpr int EPT = 16 / sizeof(OT);    // codes per thread per step: 4 (fp32 out) or 8
     constexpr int UNROLL = 4;
-    constexpr size_t TILE = static_cast<size_t>(kCastThreads) * EPT * UNROLL;
+    constexpr size_t TILE = static_cast<size_t>(THREADS) * EPT * UNROLL;
     const float si = *scale_inv_p;
     const int tid = threadIdx.x;
     const size_t ntiles = (n + TILE - 1) / TILE;
-    for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    for (size_t t = block; t < ntiles; t += blocks) {
         const size_t base = t * TILE;
         if (vec_ok && base + TILE <= n) {
             uint32_t w[UNROLL][EPT / 4];
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {
-                const uint8_t* p = q + base + (static_cast<size_t>(u) * kCastThreads + tid) * EPT;
+                const uint8_t* p = q + base + (static_cast<size_t>(u) * THREADS + tid) * EPT;
                 if constexpr (EPT == 4) {
                     w[u][0] = *reinterpret_cast<const uint32_t*>(p);
                 } else {
@@ -845,7 +876,7 @@ __global__ __launch_bounds__(kCastThreads) void cast_from_fp8_kernel(const uint8
                 }
 #pragma unroll
                 for (int j = 0; j < EPT; ++j) f[j] *= si;
-                OT* o = out + base + (static_cast<size_t>(u) * kCastThreads + tid) * EPT;
+                OT* o = out + base + (static_cast<size_t>(u) * THREADS + tid) * EPT;
                 if constexpr (sizeof(OT) == 4) {
                     *reinterpret_cast<float4*>(o) = make_float4(f[0], f[1], f[2], f[3]);
                 } else {
@@ -863,11 +894,30 @@ __global__ __launch_bounds__(kCastThreads) void cast_from_fp8_kernel(const uint8
             }
         } else {
             const size_t end = (base + TILE < n) ? base + TILE : n;
-            for (size_t i = base + tid; i < end; i += kCastThreads) {
+            for (size_t i = base + tid; i < end; i += THREADS) {
                 Elem<OT>::store(out + i, dequant1<FMT>(q[i]) * si);
             }
         }
     }
+}
+
+template <int FMT, typename OT>
+__global__ __launch_bounds__(kCastThreads) void cast_from_fp8_kernel(const uint8_t* __restrict__ q,
+                                                                      OT* __restrict__ out, size_t n,
+                                                                      const float* __restrict__ scale_inv_p,
+                                                                      int vec_ok) {
+    cast_from_fp8<FMT, OT, kCastThreads>(q, out, n, scale_inv_p, vec_ok, blockIdx.x, gridDim.x);
+}
+
+// the first kernel of a gated cast (see amax_beside_rescale_kernel) beside the old weight gradient that the new one is added to
+template <typename IT, typename OT>
+__global__ __launch_bounds__(kBesideThreads) void amax_beside_dequantize_kernel(const IT* __restrict__ x, size_t nx, uint32_t* ws,
+                                                                                 const float* scale, int x_vec, Gate gate, Finish fin,
+                                                                                 const uint8_t* __restrict__ q, OT* __restrict__ out, size_t n,
+                                                                                 const float* __restrict__ scale_inv, int vec_ok,
+                                                                                 unsigned others) {
+    if (blockIdx.x < others) cast_from_fp8<MSAMP_DT_E4M3, OT, kBesideThreads>(q, out, n, scale_inv, vec_ok, blockIdx.x, others);
+    else amax_partial<IT, kBesideThreads>(x, nx, ws, scale, x_vec, gate, fin, blockIdx.x - others, gridDim.x - others);
 }
 
 // out = OT(float(x) * scale), IEEE overflow
@@ -2033,14 +2083,57 @@ int msamp_scale_update_groups(const msamp_scale_group* groups, int n_groups, int
 namespace msamp {
 
 // A workgroup per 128-wide slice of K; a thread takes 16 elements (32 or 64 bytes in, 16 out) at a time.  A few hundred KiB in
-// all: bound by its launch.
+// all: bound by its launch, so while scaling is in time (fin.amax given and the gate open) every workgroup takes the maximum of
+// all of x by itself, out of the L2, instead of waiting for a kernel in front of this one; whichever draws the last ticket, when
+// all have read the old scale, writes the meta.  48 tokens through 4096 -> 12288, the layer call: 35.2 -> GATENOTE us.
 template <typename IT>
 __global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __restrict__ x, uint8_t* __restrict__ out, int tokens, int K,
-                                                                const float* __restrict__ scale_p, float* amax, float* scale_inv,
-                                                                int vec_ok) {
+                                                                const float* scale_p, float* amax, float* scale_inv,
+                                                                int vec_ok, uint32_t* ws, Gate gate, Finish fin) {
     constexpr int EPT = In16<IT>::EPT;
     __shared__ uint32_t red[kCastThreads / kWave];
-    const float s = *scale_p;
+    __shared__ uint32_t s_top;
+    float s = *scale_p;
+    const bool in_time = fin.amax != nullptr && !gate_closed(gate);
+    if (in_time) {
+        uint32_t m = 0;
+        auto fold = [&](uint32_t bits) { m = umax(m, sizeof(IT) == 4 ? bits & 0x7fffffffu : bits << 16 & 0x7fff0000u); };
+        const int n = tokens * K;
+        if (vec_ok) {
+#pragma unroll 4
+            for (int i = threadIdx.x * EPT; i < n; i += kCastThreads * EPT) {
+                const uint4 v = ld16(x + i);
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    fold(w[j]);
+                    if constexpr (sizeof(IT) == 2) fold(w[j] >> 16);
+                }
+            }
+        } else {
+            for (int i = threadIdx.x; i < n; i += kCastThreads) {
+                if constexpr (sizeof(IT) == 4) fold(reinterpret_cast<const uint32_t*>(x)[i]);
+                else fold(reinterpret_cast<const uint16_t*>(x)[i]);
+            }
+        }
+        m = block_max_u32(m, red);
+        if (threadIdx.x == 0) s_top = m;
+        __syncthreads();
+        m = s_top;
+        if constexpr (sizeof(IT) == 2 && !__is_same(IT, bf16_t)) m = __float_as_uint(f16_bits_to_float(m >> 16));
+        float a = __uint_as_float(m);
+        if ((fin.flags & MSAMP_FLAG_NAN_TO_INF) && !(a < __uint_as_float(0x7f800000u))) a = __uint_as_float(0x7f800000u);
+        s = scale_rule(a, s, fin.fp_max, fin.margin);
+        if (threadIdx.x == 0) {
+            const uint32_t ticket = __hip_atomic_fetch_add(ws + kWsTicket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (ticket == gridDim.x - 1) {
+                ws[kWsTicket] = 0;    // ready for the next call
+                *fin.amax = a;
+                *fin.scale = s;
+                *fin.scale_inv = 1.0f / s;
+            }
+        }
+    }
     const int pieces = (tokens + 15) / 16 * 128;
     float mx = 0.0f;
     for (int p = threadIdx.x; p < pieces; p += kCastThreads) {
@@ -2064,6 +2157,7 @@ __global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __rest
         }
         *reinterpret_cast<uint4*>(out + (static_cast<size_t>(blockIdx.x) * pieces + p) * 16) = q;
     }
+    if (in_time) return;
     const uint32_t m = block_max_u32(__float_as_uint(mx), red);
     if (threadIdx.x == 0) {
         amax_publish(amax, __uint_as_float(m));
@@ -2071,25 +2165,127 @@ __global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __rest
     }
 }
 
+// up to this many elements of x (512 KiB of 16-bit ones) in a workgroup's own search for the maximum
+constexpr int kFewOwnMax = 1 << 18;
+
 int few_cast_fragments(const void* x, int in_dtype, int tokens, int K, float* scale, float* amax, float* scale_inv, uint8_t* out,
                        int flags, const int32_t* counter, int window, void* workspace, hipStream_t st) {
     MSAMP_REQUIRE(is_hp(in_dtype), MSAMP_ERR_DTYPE, "few_cast_fragments: in_dtype %d", in_dtype);
     MSAMP_REQUIRE(x && scale && amax && scale_inv && out && counter, MSAMP_ERR_NULL, "few_cast_fragments: null pointer");
     MSAMP_REQUIRE(workspace != nullptr, MSAMP_ERR_WORKSPACE, "few_cast_fragments: workspace required");
-    // (as the gated cast: while warming up the first kernel sets amax[0] and the scale, afterwards it returns at once)
     const Gate gate = {counter, window};
-    const Finish fin = {amax, scale, scale_inv, fp8_max(MSAMP_DT_E4M3), 0, flags};
-    const int rc = dispatch_amax(x, in_dtype, static_cast<size_t>(tokens) * K, workspace, scale, st, gate, fin);
-    if (rc != MSAMP_OK) return rc;
+    Finish fin = {amax, scale, scale_inv, fp8_max(MSAMP_DT_E4M3), 0, flags};
+    const size_t n = static_cast<size_t>(tokens) * K;
+    if (n > kFewOwnMax) {
+        // (as the gated cast: while warming up the first kernel sets amax[0] and the scale, afterwards it returns at once)
+        const int rc = dispatch_amax(x, in_dtype, n, workspace, scale, st, gate, fin);
+        if (rc != MSAMP_OK) return rc;
+        fin.amax = nullptr;
+    }
     const dim3 grid((K + 127) / 128);
     const int vec_ok = aligned(x, 16);
-#define FEW_CAST(IT) hipLaunchKernelGGL((few_cast_kernel<IT>), grid, dim3(kCastThreads), 0, st, static_cast<const IT*>(x), out, tokens, K, scale, amax, scale_inv, vec_ok)
+    uint32_t* ws = static_cast<uint32_t*>(workspace);
+#define FEW_CAST(IT) hipLaunchKernelGGL((few_cast_kernel<IT>), grid, dim3(kCastThreads), 0, st, static_cast<const IT*>(x), out, tokens, K, scale, amax, scale_inv, vec_ok, ws, gate, fin)
     if (in_dtype == MSAMP_DT_F32) FEW_CAST(float);
     else if (in_dtype == MSAMP_DT_F16) FEW_CAST(f16_t);
     else FEW_CAST(bf16_t);
 #undef FEW_CAST
     MSAMP_CHECK_LAUNCH("few_cast_kernel");
     return MSAMP_OK;
+}
+
+// how many workgroups of kBesideThreads the maxima of n elements take
+static unsigned beside_blocks(size_t n, int dtype) {
+    const size_t tile = static_cast<size_t>(kBesideThreads) * (16 / hp_size(dtype)) * 8;
+    const size_t cap = std::min(cu_count() * 2, kMaxPartials);
+    return static_cast<unsigned>(std::min(std::max<size_t>((n + tile - 1) / tile, 1), cap));
+}
+
+template <typename IT, typename WT>
+static void launch_amax_beside_rescale(const msamp_linear_forward_args& a, const Gate& gate, const Finish& fin, hipStream_t st) {
+    const size_t nx = static_cast<size_t>(a.tokens) * a.d_in, nw = static_cast<size_t>(a.d_out) * a.d_in;
+    constexpr int EPT = In16<WT>::EPT;
+    const unsigned others = static_cast<unsigned>(std::min(grid_for(nw, static_cast<size_t>(kBesideThreads) * EPT * kCastUnroll), cu_count() * 2));
+    const int w_vec = (aligned(a.w, 16) && aligned(a.w_codes, EPT) ? 1 : 0) | (nw * sizeof(WT) >= kStreamBytes ? 2 : 0);
+    float* meta = a.w_meta;
+    const InTimeArgs it = {nullptr, meta, nullptr, fp8_max(MSAMP_DT_E4M3), 0, 0, a.w_amax, a.w_scale_inv, meta + 3, static_cast<int>(a.w_window),
+                           reinterpret_cast<int32_t*>(meta + 2), 0};
+    hipLaunchKernelGGL((amax_beside_rescale_kernel<IT, WT>), dim3(others + beside_blocks(nx, static_cast<int>(a.x_dtype))),
+                       dim3(kBesideThreads), 0, st, static_cast<const IT*>(a.x), nx, static_cast<uint32_t*>(a.workspace), a.x_scale,
+                       static_cast<int>(aligned(a.x, 16)), gate, fin, static_cast<const WT*>(a.w), a.w_codes, nw, meta + 1, w_vec, it, others);
+}
+
+int cast_linear_inputs(const msamp_linear_forward_args& a, hipStream_t st) {
+    const int x_dtype = static_cast<int>(a.x_dtype), w_dtype = static_cast<int>(a.w_dtype);
+    MSAMP_REQUIRE(is_hp(x_dtype) && is_hp(w_dtype), MSAMP_ERR_DTYPE, "msamp_linear_forward: dtypes %d, %d", x_dtype, w_dtype);
+    MSAMP_REQUIRE(a.x && a.x_scale && a.x_amax && a.x_scale_inv && a.x_counter && a.x_codes && a.w && a.w_amax && a.w_scale_inv && a.w_codes,
+                  MSAMP_ERR_NULL, "msamp_linear_forward: null pointer");
+    MSAMP_REQUIRE(a.workspace != nullptr, MSAMP_ERR_WORKSPACE, "msamp_linear_forward: workspace required");
+    MSAMP_REQUIRE(a.w_window >= 1, MSAMP_ERR_SHAPE, "msamp_linear_forward: window %lld", static_cast<long long>(a.w_window));
+    const Gate gate = {a.x_counter, static_cast<int>(a.x_window)};
+    const Finish fin = {a.x_amax, a.x_scale, a.x_scale_inv, fp8_max(MSAMP_DT_E4M3), 0, static_cast<int>(a.flags)};
+#define BESIDE(IT)                                                                                     \
+    do {                                                                                               \
+        if (w_dtype == MSAMP_DT_F32) launch_amax_beside_rescale<IT, float>(a, gate, fin, st);          \
+        else if (w_dtype == MSAMP_DT_F16) launch_amax_beside_rescale<IT, f16_t>(a, gate, fin, st);     \
+        else launch_amax_beside_rescale<IT, bf16_t>(a, gate, fin, st);                                 \
+    } while (0)
+    if (x_dtype == MSAMP_DT_F32) BESIDE(float);
+    else if (x_dtype == MSAMP_DT_F16) BESIDE(f16_t);
+    else BESIDE(bf16_t);
+#undef BESIDE
+    MSAMP_CHECK_LAUNCH("amax_beside_rescale_kernel");
+    return dispatch_cast(a.x, x_dtype, static_cast<size_t>(a.tokens) * a.d_in, a.x_scale, a.x_amax, a.x_scale_inv, a.x_codes, MSAMP_DT_E4M3,
+                         nullptr, st);
+}
+
+template <typename IT, typename OT>
+static void launch_amax_beside_dequantize(const msamp_linear_backward_args& a, void* product, const Gate& gate, const Finish& fin,
+                                          hipStream_t st) {
+    const size_t nx = static_cast<size_t>(a.tokens) * a.d_out, n = static_cast<size_t>(a.d_out) * a.d_in;
+    constexpr int EPT = 16 / sizeof(OT);
+    const unsigned others = static_cast<unsigned>(grid_for(n, static_cast<size_t>(kBesideThreads) * EPT * 4));
+    hipLaunchKernelGGL((amax_beside_dequantize_kernel<IT, OT>), dim3(others + beside_blocks(nx, static_cast<int>(a.dy_dtype))),
+                       dim3(kBesideThreads), 0, st, static_cast<const IT*>(a.dy), nx, static_cast<uint32_t*>(a.workspace), a.g_scale,
+                       static_cast<int>(aligned(a.dy, 16)), gate, fin, a.old_codes, static_cast<OT*>(product), n, a.old_scale_inv,
+                       static_cast<int>(aligned(product, 16) && aligned(a.old_codes, EPT)), others);
+}
+
+int cast_output_gradient(const msamp_linear_backward_args& a, void* product, float* sums, hipStream_t st) {
+    const int dy_dtype = static_cast<int>(a.dy_dtype), out_dtype = static_cast<int>(a.out_dtype);
+    const int tokens = static_cast<int>(a.tokens), d_out = static_cast<int>(a.d_out), sum_dtype = static_cast<int>(a.bias_sum_dtype);
+    MSAMP_REQUIRE(is_hp(dy_dtype) && is_hp(out_dtype) && (a.bias_sum == nullptr || is_hp(sum_dtype)), MSAMP_ERR_DTYPE,
+                  "msamp_linear_backward: dtypes %d, %d, %d", dy_dtype, out_dtype, sum_dtype);
+    MSAMP_REQUIRE(a.dy && a.g_scale && a.g_amax && a.g_scale_inv && a.g_counter && a.dy_codes, MSAMP_ERR_NULL,
+                  "msamp_linear_backward: null pointer");
+    MSAMP_REQUIRE(a.workspace != nullptr, MSAMP_ERR_WORKSPACE, "msamp_linear_backward: workspace required");
+    const Gate gate = {a.g_counter, static_cast<int>(a.g_window)};
+    const Finish fin = {a.g_amax, a.g_scale, a.g_scale_inv, fp8_max(MSAMP_DT_E5M2), 0, static_cast<int>(a.flags)};
+    const size_t n = static_cast<size_t>(tokens) * d_out;
+    if (a.wq != nullptr && a.old_codes != nullptr) {
+        MSAMP_REQUIRE(a.old_type == MSAMP_DT_E4M3 && a.old_scale_inv, MSAMP_ERR_DTYPE, "msamp_linear_backward: old gradient of type %lld",
+                      static_cast<long long>(a.old_type));
+#define BESIDE(IT)                                                                                                   \
+    do {                                                                                                             \
+        if (out_dtype == MSAMP_DT_F32) launch_amax_beside_dequantize<IT, float>(a, product, gate, fin, st);          \
+        else if (out_dtype == MSAMP_DT_F16) launch_amax_beside_dequantize<IT, f16_t>(a, product, gate, fin, st);     \
+        else launch_amax_beside_dequantize<IT, bf16_t>(a, product, gate, fin, st);                                   \
+    } while (0)
+        if (dy_dtype == MSAMP_DT_F32) BESIDE(float);
+        else if (dy_dtype == MSAMP_DT_F16) BESIDE(f16_t);
+        else BESIDE(bf16_t);
+#undef BESIDE
+        MSAMP_CHECK_LAUNCH("amax_beside_dequantize_kernel");
+    } else {
+        const int rc = dispatch_amax(a.dy, dy_dtype, n, a.workspace, a.g_scale, st, gate, fin);
+        if (rc != MSAMP_OK) return rc;
+    }
+    if (a.bias_sum == nullptr) return dispatch_cast(a.dy, dy_dtype, n, a.g_scale, a.g_amax, a.g_scale_inv, a.dy_codes, MSAMP_DT_E5M2, nullptr, st);
+#define COLSUM(IT) launch_colsum(static_cast<const IT*>(a.dy), dy_dtype, tokens, d_out, a.g_scale, a.g_amax, a.g_scale_inv, a.dy_codes, MSAMP_DT_E5M2, a.bias_sum, sum_dtype, sums, st)
+    if (dy_dtype == MSAMP_DT_F32) return COLSUM(float);
+    if (dy_dtype == MSAMP_DT_F16) return COLSUM(f16_t);
+    return COLSUM(bf16_t);
+#undef COLSUM
 }
 
 }    // namespace msamp

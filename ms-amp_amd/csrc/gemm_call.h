@@ -115,12 +115,6 @@ inline bool fits_offsets(int NR, int NC, int K) {
 int cast_again_if_flagged(const void* d, int d_dtype, size_t n, const float* scale, uint8_t* q, int q_type, const uint32_t* redo,
                           hipStream_t st);
 
-// x[tokens][K] (K a multiple of 16) to E4M3 as msamp_cast_to_fp8_gated casts it, the codes in the order in which the product of a
-// few tokens reads them: for every 128-wide slice of K, block of 16 tokens and half slice 64 lanes of 16 bytes, lane l those of token
-// l % 16 and k = 16 * (l / 16) .. +15 of the half; zeros past the last token and the last k.
-int few_cast_fragments(const void* x, int in_dtype, int tokens, int K, float* scale, float* amax, float* scale_inv, uint8_t* out,
-                       int flags, const int32_t* counter, int window, void* workspace, hipStream_t st);
-
 extern template int run_gemm_pair<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(const GemmCall&);
 extern template int run_gemm_pair<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_pair<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(const GemmCall&);

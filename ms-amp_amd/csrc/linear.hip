@@ -5,6 +5,7 @@
 // 1522 -> 1137 us.
 #include "common.cuh"
 #include "gemm_call.h"
+#include "linear_call.h"
 
 #include <algorithm>
 
@@ -207,7 +208,6 @@ extern "C" int msamp_linear_forward(const msamp_linear_forward_args* a, msamp_st
     MSAMP_REQUIRE(dims_ok(a->tokens, a->d_in, a->d_out), MSAMP_ERR_SHAPE, "msamp_linear_forward: %lld x %lld -> %lld",
                   static_cast<long long>(a->tokens), static_cast<long long>(a->d_in), static_cast<long long>(a->d_out));
     MSAMP_REQUIRE(a->w_codes == nullptr || a->w_meta, MSAMP_ERR_NULL, "msamp_linear_forward: null w_meta");
-    const size_t nx = static_cast<size_t>(a->tokens) * a->d_in, nw = static_cast<size_t>(a->d_out) * a->d_in;
     const int x_dtype = static_cast<int>(a->x_dtype), w_dtype = static_cast<int>(a->w_dtype), y_dtype = static_cast<int>(a->y_dtype);
     if (a->w_codes == nullptr) {
         // (refused here and not behind the cast, which changes the input meta)
@@ -225,14 +225,9 @@ extern "C" int msamp_linear_forward(const msamp_linear_forward_args* a, msamp_st
                                           static_cast<int>(a->x_window), a->workspace, static_cast<hipStream_t>(stream));
         return rc != MSAMP_OK ? rc : few_tokens(*a, static_cast<hipStream_t>(stream));
     }
-    int rc = msamp_cast_to_fp8_gated(a->x, x_dtype, nx, a->x_scale, a->x_amax, a->x_scale_inv, a->x_codes, MSAMP_DT_E4M3, 0,
-                                     static_cast<int>(a->flags), a->x_counter, static_cast<int>(a->x_window), a->workspace, stream);
+    const int rc = cast_linear_inputs(*a, static_cast<hipStream_t>(stream));
     if (rc != MSAMP_OK) return rc;
-    float* meta = a->w_meta;
-    rc = msamp_cast_scaled_to_fp8(a->w, w_dtype, nw, a->w_amax, a->w_scale_inv, meta, meta + 1, meta + 3, static_cast<int>(a->w_window),
-                                  reinterpret_cast<int32_t*>(meta + 2), a->w_codes, MSAMP_DT_E4M3, 0, stream);
-    if (rc != MSAMP_OK) return rc;
-    return msamp_fp8_gemm(a->w_codes, MSAMP_DT_E4M3, meta + 1, a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, a->y, y_dtype,
+    return msamp_fp8_gemm(a->w_codes, MSAMP_DT_E4M3, a->w_meta + 1, a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, a->y, y_dtype,
                           static_cast<int>(a->d_out), static_cast<int>(a->tokens), static_cast<int>(a->d_in), 0, a->bias,
                           static_cast<int>(a->bias_dtype), stream);
 }
@@ -265,14 +260,7 @@ extern "C" int msamp_linear_backward(const msamp_linear_backward_args* a, msamp_
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint8_t* codes = a->dy_codes;
     uint8_t* product = static_cast<uint8_t*>(a->scratch);
-    if (bias) {
-        rc = msamp_cast_to_fp8_colsum_gated(a->dy, dy_dtype, tokens, d_out, a->g_scale, a->g_amax, a->g_scale_inv, codes, MSAMP_DT_E5M2,
-                                            a->bias_sum, static_cast<int>(a->bias_sum_dtype), reinterpret_cast<float*>(product + s.sums), 0,
-                                            flags, a->g_counter, static_cast<int>(a->g_window), a->workspace, stream);
-    } else {
-        rc = msamp_cast_to_fp8_gated(a->dy, dy_dtype, static_cast<size_t>(tokens) * d_out, a->g_scale, a->g_amax, a->g_scale_inv, codes,
-                                     MSAMP_DT_E5M2, 0, flags, a->g_counter, static_cast<int>(a->g_window), a->workspace, stream);
-    }
+    rc = cast_output_gradient(*a, product, reinterpret_cast<float*>(product + s.sums), st);
     if (rc != MSAMP_OK) return rc;
     if (a->dx != nullptr) {
         rc = gemm_kmajor(a->w_codes, MSAMP_DT_E4M3, a->w_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, 0, a->dx, out_dtype, d_in, tokens,
@@ -281,10 +269,6 @@ extern "C" int msamp_linear_backward(const msamp_linear_backward_args* a, msamp_
     }
     if (!wgrad) return MSAMP_OK;
     const size_t n = static_cast<size_t>(d_out) * d_in;
-    if (accumulate) {
-        rc = msamp_cast_from_fp8(a->old_codes, static_cast<int>(a->old_type), n, a->old_scale_inv, product, out_dtype, stream);
-        if (rc != MSAMP_OK) return rc;
-    }
     if (s.n_parts != 0 && a->scratch_bytes >= static_cast<int64_t>(s.end)) {
         rc = msamp_fp8_gemm_ksplit(a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, product, out_dtype, d_in,
                                    d_out, tokens, accumulate, reinterpret_cast<float*>(product + s.parts), s.n_parts, stream);

@@ -44,7 +44,7 @@ def _wgrad_in_one_call(ctx, tokens, d_in, d_out):
     if old is None:
         return _backend.gemm_walk_settled(d_in, d_out, tokens, True, True)
     # (a product that is added to something is not timed)
-    return type(old) is ScalingTensor and old.value.dtype == torch.uint8 and old.value.shape == (d_out, d_in) and \
+    return type(old) is ScalingTensor and old.meta.qtype == Dtypes.kfloat8_e4m3 and old.value.shape == (d_out, d_in) and \
         old.value.device == ctx.input_codes.device and old.value.is_contiguous()
 
 
