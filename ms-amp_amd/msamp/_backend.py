@@ -288,12 +288,18 @@ class _ScaleGroup(ctypes.Structure):
                 ('fp_max', ctypes.c_float), ('reserved', ctypes.c_int32)]
 
 
+# (array types are made here: one made anew for every call is a cycle that only the garbage collector frees, and its collections
+# cost a small model more than its launches)
+_ScaleTable = _ScaleGroup * MAX_SCALE_GROUPS
+_TwoSizes = ctypes.c_size_t * 2
+
+
 def scale_update_groups(groups, margin):
     """scale_update for several (scales, amaxs, fp_max, counters) groups in one launch (counters may be None)."""
     lib = load()
     for start in range(0, len(groups), MAX_SCALE_GROUPS):
         part = groups[start:start + MAX_SCALE_GROUPS]
-        table = (_ScaleGroup * len(part))()
+        table = _ScaleTable()
         for row, (scales, amaxs, fp_max, counters) in zip(table, part):
             _gpu(scales, 'scales')
             _gpu(amaxs, 'amaxs')
@@ -770,7 +776,7 @@ def linear_backward(dy, g_meta, x_codes, x_scale_inv, w_codes, w_scale_inv_ptr, 
     sums = torch.empty((d_out, ), dtype=bias_dtype, device=device) if bias_dtype is not None else None
     scratch, size = None, 0
     if wq is not None or sums is not None:
-        sizes = (ctypes.c_size_t * 2)()
+        sizes = _TwoSizes()
         where = ctypes.addressof(sizes)
         _check(lib.msamp_linear_backward_scratch(tokens, d_in, d_out, dt, out_dt, wq is not None, sums is not None, where, where + 8),
                'msamp_linear_backward_scratch')
@@ -968,13 +974,16 @@ def adamw_fused(desc, n_tensors, block_map, n_blocks, weight_dt, grad_dt, lr, be
     _gpu(desc, 'descriptor table')
     bpt = None
     if blocks_per_tensor is not None:
-        bpt = (ctypes.c_int32 * n_tensors)(*blocks_per_tensor)
+        bpt = array.array('i', blocks_per_tensor)
+        if len(bpt) > n_tensors:
+            raise IndexError('more counts than tensors')
+        bpt.extend([0] * (n_tensors - len(bpt)))
     gb = ADAMW_GROUP_BLOCKS if group_blocks is None else group_blocks
     _check(
         lib.msamp_adamw_fp8_fused(
             _ptr(desc), n_tensors, _ptr(block_map), n_blocks, weight_dt, grad_dt, lr, beta1, beta2, eps, weight_decay,
             step, 1 if bias_correction else 0, 1 if adam_mode else 0, 1 if maximize else 0, 1 if tensor_scale else 0,
-            ctypes.cast(bpt, ctypes.c_void_p) if bpt is not None else None, gb if bpt is not None else 0, _stream()
+            bpt.buffer_info()[0] if bpt is not None else None, gb if bpt is not None else 0, _stream()
         ), 'msamp_adamw_fp8_fused'
     )
 
@@ -1017,7 +1026,7 @@ def adamw_f32_list(rows, scaled_numels, device, lr, beta1, beta2, eps, weight_de
     words; `scaled_numels`: sizes of the scaled weights among them (they share float32 scratch, that of the largest one if there
     is no memory for more)."""
     flat = [word for row in rows for word in row]
-    table = (ctypes.c_longlong * len(flat))(*flat)
+    table = array.array('q', flat)
     padded = [(n + 3) // 4 * 4 for n in scaled_numels]
     room = max(max(padded), min(sum(padded), F32_SCRATCH)) if padded else 0
     words = torch.empty(F32_WORDS, dtype=torch.int32, device=device)
@@ -1030,7 +1039,7 @@ def adamw_f32_list(rows, scaled_numels, device, lr, beta1, beta2, eps, weight_de
             scratch = torch.empty(room, dtype=torch.float32, device=device)
     _check(
         load().msamp_adamw_f32_list(
-            table, len(rows), _ptr(scratch), room, _ptr(words), lr, beta1, beta2, eps, weight_decay, step,
+            table.buffer_info()[0], len(rows), _ptr(scratch), room, _ptr(words), lr, beta1, beta2, eps, weight_decay, step,
             1 if bias_correction else 0, 1 if adam_mode else 0, 1 if maximize else 0, _stream()
         ), 'msamp_adamw_f32_list'
     )
