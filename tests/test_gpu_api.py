@@ -1116,3 +1116,27 @@ def test_a_few_tokens_without_gradients_lose_no_precision():
             _backend.cast_from_fp8(w_codes, words[1], 5, torch.float32).double().t()
         few = _backend.linear_forward(x, meta, w.value, w.meta, torch.float32, None, want_codes=False)[0]
         assert rel_fro(few.double(), exact) <= 1.1 * rel_fro(y.double(), exact) + 1e-7
+
+
+def test_zero_grad_of_a_mixed_list():
+    """Gradients of several types, strides and layouts, ScalingTensors, shared memory, a missing and an empty one."""
+    dense = lambda *shape, dtype=torch.float32: torch.nn.Parameter(torch.ones(shape, device='cuda', dtype=dtype))
+    params = [dense(5, 3), dense(7, dtype=torch.bfloat16), dense(4, 6), dense(0), dense(2, 2, dtype=torch.float16), dense(3), dense(3), dense(6, 2)]
+    for p in params:
+        p.grad = torch.ones_like(p)
+    params[2].grad = torch.ones(6, 4, device='cuda').t()
+    both = torch.ones(4, device='cuda')
+    params[5].grad, params[6].grad = both[:3], both[1:]
+    params[7].grad = torch.ones(6, 2, device='cuda').to_sparse()
+    quantized = ScalingParameter(torch.ones(16, 16, device='cuda').cast(Dtypes.kfloat16))
+    quantized.grad = torch.ones(16, 16, device='cuda').cast(Dtypes.kfloat8_e4m3)
+    scale_inv = quantized.grad.meta.scale_inv.clone()
+    opt = LBAdamW(params + [quantized, dense(4)])
+    kept = [p.grad for p in params]
+    version = params[0].grad._version
+    opt.zero_grad()
+    assert all(p.grad is g for p, g in zip(params, kept)) and params[0].grad._version > version
+    assert all(not g.to_dense().any() if g.is_sparse else not g.any() for g in kept)
+    assert not quantized.grad.value.any() and torch.equal(quantized.grad.meta.scale_inv, scale_inv)
+    opt.zero_grad(set_to_none=True)
+    assert all(p.grad is None for p in params) and quantized.grad is None
