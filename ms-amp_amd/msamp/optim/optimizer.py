@@ -162,6 +162,7 @@ class LBOptimizer(Optimizer):
         # one launch for all gradients of a type: one by one they were a twentieth of a small model's step
         for grads in fills.values():
             torch._foreach_zero_(grads)
+            torch.autograd.graph.increment_version([g for g in grads if not g.is_inference()])    # (which the launch does not do)
 
     def add_param_group(self, param_group):
         """torch's add_param_group, accepting ScalingTensor entries."""

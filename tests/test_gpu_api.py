@@ -1124,9 +1124,11 @@ def test_zero_grad_of_a_mixed_list():
     params = [dense(5, 3), dense(7, dtype=torch.bfloat16), dense(4, 6), dense(0), dense(2, 2, dtype=torch.float16), dense(3), dense(3), dense(6, 2)]
     for p in params:
         p.grad = torch.ones_like(p)
-    params[2].grad = torch.ones(6, 4, device='cuda').t()
+    # (of a storage, not views: those cannot be detached in place)
+    memory = lambda store, first, size, stride: torch.empty(0, device='cuda').set_(store.untyped_storage(), first, size, stride)
+    params[2].grad = memory(torch.ones(24, device='cuda'), 0, (4, 6), (1, 4))
     both = torch.ones(4, device='cuda')
-    params[5].grad, params[6].grad = both[:3], both[1:]
+    params[5].grad, params[6].grad = memory(both, 0, (3, ), (1, )), memory(both, 1, (3, ), (1, ))
     params[7].grad = torch.ones(6, 2, device='cuda').to_sparse()
     quantized = ScalingParameter(torch.ones(16, 16, device='cuda').cast(Dtypes.kfloat16))
     quantized.grad = torch.ones(16, 16, device='cuda').cast(Dtypes.kfloat8_e4m3)
