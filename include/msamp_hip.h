@@ -326,9 +326,10 @@ int msamp_fp8_gemm_cast(const uint8_t* a, int a_type, const float* a_scale_inv, 
  * entry points.
  *
  * Forward: msamp_cast_to_fp8_gated (x to E4M3), msamp_cast_scaled_to_fp8 (the scaled 16- or 32-bit weight to E4M3; w_meta
- * receives {scale, scale_inv, update count, amax window} as four-byte words), msamp_fp8_gemm with the bias.  d_in must be a
- * multiple of 16.  With w_codes NULL (nobody needs them; at most MSAMP_FEW_TOKENS tokens, w, x_codes and y 16-byte aligned) the
- * last two are one launch: the weight is quantized to the same codes on its way into the product, and the float32 sum is taken in
+ * receives {scale, scale_inv, update count, amax window} as four-byte words), msamp_fp8_gemm with the bias.  Codes lie in rows of
+ * d_in rounded up to a multiple of 16, zeros behind the d_in codes, and w_codes in d_out rounded up likewise, rows of zeros below
+ * (16-byte aligned where there are any).  With w_codes NULL (nobody needs them; at most MSAMP_FEW_TOKENS tokens, d_in a multiple
+ * of 16, w, x_codes and y 16-byte aligned) the last two are one launch: the weight is quantized to the same codes on its way into the product, and the float32 sum is taken in
  * up to eight parts of K; x_codes is scratch of 2048 bytes for every 16 tokens and 128 of d_in begun. */
 #define MSAMP_FEW_TOKENS 64
 typedef struct msamp_linear_forward_args {
@@ -339,13 +340,13 @@ typedef struct msamp_linear_forward_args {
     float* x_scale_inv;
     const int32_t* x_counter;
     int64_t x_window;
-    uint8_t* x_codes;          /* out: [tokens][d_in] E4M3 */
+    uint8_t* x_codes;          /* out: [tokens][d_in, rounded up] E4M3 */
     const void* w;             /* [d_out][d_in], w_dtype, the values times their scale */
     int64_t w_dtype;
     const float* w_amax;
     const float* w_scale_inv;
     int64_t w_window;
-    uint8_t* w_codes;          /* nullable, out: [d_out][d_in] E4M3 */
+    uint8_t* w_codes;          /* nullable, out: [d_out, rounded up][d_in, rounded up] E4M3 */
     float* w_meta;             /* out: 3 + w_window words (not without w_codes) */
     void* y;                   /* out: [tokens][d_out], y_dtype */
     int64_t y_dtype;
@@ -360,7 +361,8 @@ int msamp_linear_forward(const msamp_linear_forward_args* args, msamp_stream_t s
  * msamp_fp8_gemm_kmajor if dx is given; and if wq is given the weight gradient, added to the dequantized old one if there is
  * one: msamp_fp8_gemm_ksplit (if it splits the product and the scratch has room) or msamp_fp8_gemm_kmajor, and
  * msamp_cast_to_fp8_intime with MSAMP_FLAG_NAN_TO_INF.  (A product that msamp_fp8_gemm_cast takes is better left to that: without
- * wq the codes of dy are there for it.)  Shapes as msamp_fp8_gemm_kmajor takes them, but for K, which may be a single slice.
+ * wq the codes of dy are there for it.)  The codes of dy lie in rows of d_out rounded up to a multiple of 16, those of x and w
+ * as the forward call leaves them; shapes otherwise as msamp_fp8_gemm_kmajor takes them, but for K, which may be a single slice.
  * msamp_linear_backward_scratch: the bytes of `scratch` (16-byte aligned) to give, and the least that will do. */
 typedef struct msamp_linear_backward_args {
     const void* dy;            /* [tokens][d_out], dy_dtype */
@@ -370,7 +372,7 @@ typedef struct msamp_linear_backward_args {
     float* g_scale_inv;
     const int32_t* g_counter;
     int64_t g_window;
-    uint8_t* dy_codes;         /* out: [tokens][d_out] E5M2 */
+    uint8_t* dy_codes;         /* out: [tokens][d_out, rounded up] E5M2 */
     const uint8_t* x_codes;    /* from the forward call */
     const float* x_scale_inv;
     const uint8_t* w_codes;

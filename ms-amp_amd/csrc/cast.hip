@@ -68,6 +68,39 @@ struct Gate {
 };
 __device__ __forceinline__ bool gate_closed(const Gate& g) { return g.counter != nullptr && *g.counter >= g.window; }
 
+// A matrix whose codes are written in rows of another length (see PITCHED at cast_to_fp8).
+struct Pitch {
+    unsigned rows, cols, pitch;
+};
+
+// EPT elements at `at` of a matrix whose rows begin anywhere, `valid` of them (maybe none) left in their row, zeros behind those.
+// The 16-byte load is aligned to an element only, and one that runs over the end of its row takes some of the next with it; a lane
+// that may not (the matrix ends there) reads the beginning of x instead and then its elements one by one.  Loads and values apart,
+// so that several loads are in flight.  A matrix of fewer than EPT elements has no load at all.
+template <typename IT>
+struct RowPiece {
+    static constexpr int EPT = In16<IT>::EPT;
+    struct __attribute__((packed, aligned(sizeof(IT)))) Any16 { uint32_t w[4]; };
+    size_t at;
+    int valid;
+    bool whole;
+    Any16 raw;
+    __device__ __forceinline__ void load(const IT* x, size_t n, size_t at_, int valid_) {
+        at = at_, valid = valid_, whole = valid > 0 && at + EPT <= n;
+        if (n >= EPT) raw = *reinterpret_cast<const Any16*>(x + (whole ? at : 0));
+    }
+    __device__ __forceinline__ void values(const IT* x, float* v) const {
+        In16<IT>::decode(make_uint4(raw.w[0], raw.w[1], raw.w[2], raw.w[3]), v);
+#pragma unroll
+        for (int j = 0; j < EPT; ++j) v[j] = whole && j < valid ? v[j] : 0.0f;
+        if (valid > 0 && !whole) {
+#pragma unroll
+            for (int j = 0; j < EPT; ++j)
+                if (j < valid) v[j] = Elem<IT>::load(x + at + j);
+        }
+    }
+};
+
 // where cast_to_fp8_kernel takes its scale from
 // (kGivenIfFlagged: as kGivenScale, but the launch does nothing unless the word it.ws points at is non-zero)
 enum ScaleSource { kGivenScale = 0, kInTime = 1, kRescale = 2, kGivenIfFlagged = 3 };
@@ -105,10 +138,13 @@ __device__ __forceinline__ float resolve_in_time_scale(const InTimeArgs& a, uint
 // at a time (about 10 ns each): the launch with WITH_AMAX uses few, large workgroups (THREADS = 512,
 // two per CU) so that they stay a small part of the run time.
 // (`block` of `blocks`: the whole launch, or the part of one that casts)
-template <typename IT, int FMT, bool WITH_AMAX, int INTIME, int THREADS>
+// PITCHED: x is pt.rows rows of pt.cols, and `out` n codes in rows of pt.pitch, a multiple of 16: zeros behind the columns and
+// below the rows, so that the products read codes of any width 16 bytes at a time where they lie.
+template <typename IT, int FMT, bool WITH_AMAX, int INTIME, int THREADS, bool PITCHED = false>
 __device__ __forceinline__ void cast_to_fp8(const IT* __restrict__ x, uint8_t* __restrict__ out, size_t n,
                                             const float* __restrict__ scale_p, float* amax, float* scale_inv, int vec_ok,
-                                            int reverse, const InTimeArgs& it, unsigned block, unsigned blocks) {
+                                            int reverse, const InTimeArgs& it, unsigned block, unsigned blocks,
+                                            const Pitch& pt = {}) {
     constexpr int EPT = In16<IT>::EPT;
     constexpr size_t TILE = static_cast<size_t>(THREADS) * EPT * kCastUnroll;
     __shared__ uint32_t red[THREADS / kWave];
@@ -140,7 +176,34 @@ __device__ __forceinline__ void cast_to_fp8(const IT* __restrict__ x, uint8_t* _
     for (size_t t = block; t < ntiles; t += blocks) {
         const size_t tile = reverse ? (ntiles - 1 - t) : t;
         const size_t base = tile * TILE;
-        if ((vec_ok & 1) && base + TILE <= n) {
+        if constexpr (PITCHED) {
+            const unsigned groups = pt.pitch / EPT, first = static_cast<unsigned>(base / EPT) + tid;
+            const size_t nx = static_cast<size_t>(pt.rows) * pt.cols;
+            RowPiece<IT> piece[kCastUnroll];
+#pragma unroll
+            for (int u = 0; u < kCastUnroll; ++u) {
+                const unsigned g = first + u * THREADS, row = g / groups, col = (g - row * groups) * EPT;
+                const int valid = row < pt.rows ? static_cast<int>(pt.cols) - static_cast<int>(col) : 0;
+                piece[u].load(x, nx, static_cast<size_t>(row) * pt.cols + col, valid);
+            }
+#pragma unroll
+            for (int u = 0; u < kCastUnroll; ++u) {
+                const size_t o = (static_cast<size_t>(first) + u * THREADS) * EPT;
+                float v[EPT];
+                piece[u].values(x, v);
+                uint32_t w[EPT / 4];
+#pragma unroll
+                for (int j = 0; j < EPT / 4; ++j) {
+                    const float a = v[4 * j], b = v[4 * j + 1], c = v[4 * j + 2], d = v[4 * j + 3];
+                    if (WITH_AMAX) mx = fmaxf(fmaxf(mx, fabsf(a)), fmaxf(fmaxf(fabsf(b), fabsf(c)), fabsf(d)));
+                    w[j] = quant4<FMT>(a * s, b * s, c * s, d * s);
+                }
+                if (o < n) {    // (n is a multiple of 16)
+                    if constexpr (EPT == 4) *reinterpret_cast<uint32_t*>(out + o) = w[0];
+                    else *reinterpret_cast<uint2*>(out + o) = make_uint2(w[0], w[1]);
+                }
+            }
+        } else if ((vec_ok & 1) && base + TILE <= n) {
             float v[kCastUnroll][EPT];
 #pragma unroll
             for (int u = 0; u < kCastUnroll; ++u)
@@ -188,6 +251,15 @@ __global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restri
     cast_to_fp8<IT, FMT, WITH_AMAX, INTIME, THREADS>(x, out, n, scale_p, amax, scale_inv, vec_ok, reverse, it, blockIdx.x, gridDim.x);
 }
 
+constexpr int kBesideThreads = 512;
+template <typename IT, int FMT>
+__global__ __launch_bounds__(kBesideThreads) void cast_pitched_kernel(const IT* __restrict__ x, uint8_t* __restrict__ out, size_t n,
+                                                                      const float* __restrict__ scale_p, float* amax, float* scale_inv,
+                                                                      Pitch pt) {
+    cast_to_fp8<IT, FMT, true, kGivenScale, kBesideThreads, true>(x, out, n, scale_p, amax, scale_inv, 0, 0, InTimeArgs{}, blockIdx.x,
+                                                                  gridDim.x, pt);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Delayed cast of a 2-D tensor that also takes its column sums (a bias gradient beside the cast of dy): bound by memory
 // like the cast alone, and the sums are three more instructions on values that are there anyway.  A wavefront takes
@@ -205,13 +277,18 @@ __global__ __launch_bounds__(THREADS) void cast_to_fp8_kernel(const IT* __restri
 constexpr int kColsumThreads = 256;
 constexpr int kColsumRows = 16;
 
-template <typename IT, int FMT, bool VEC>
+// How a lane takes its columns: every 64th, one by one; EPT in a row by a 16-byte load; or so with codes in rows of `pitch`, a
+// multiple of 16 (see PITCHED above), which takes any columns.
+enum ColumnForm { kColumnsApart = 0, kColumnsWhole = 1, kColumnsPitched = 2 };
+
+template <typename IT, int FMT, int FORM>
 __global__ __launch_bounds__(kColsumThreads) void cast_colsum_kernel(const IT* __restrict__ x, uint8_t* __restrict__ out,
                                                                      int rows, int cols, int rows_per_slab,
                                                                      const float* __restrict__ scale_p, float* scale_inv,
                                                                      float* __restrict__ partial, float* __restrict__ tops,
-                                                                     int stream) {
+                                                                     int stream, int pitch) {
     constexpr int EPT = In16<IT>::EPT;
+    constexpr bool VEC = FORM != kColumnsApart;
     constexpr int W = kWave * EPT, NW = kColsumThreads / kWave, U = 4;
     static_assert(NW * U == kColsumRows, "one round of loads per kColsumRows rows");
     __shared__ float sums[NW - 1][W];
@@ -229,10 +306,22 @@ __global__ __launch_bounds__(kColsumThreads) void cast_colsum_kernel(const IT* _
     float mx = 0.0f;
     for (int r = r0 + wave; r < r1; r += NW * U) {
         float v[U][EPT];
+        if constexpr (FORM == kColumnsPitched) {
+            RowPiece<IT> piece[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int row = r + u * NW;
+                piece[u].load(x, static_cast<size_t>(rows) * cols, static_cast<size_t>(row) * cols + c0, row < r1 ? cols - c0 : 0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) piece[u].values(x, v[u]);
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int row = r + u * NW;
-            if constexpr (VEC) {
+            if constexpr (FORM == kColumnsPitched) {
+                continue;
+            } else if constexpr (VEC) {
                 // (past an end: any row of the slab, any columns; their values do not count)
                 const int row_in = row < r1 ? row : r1 - 1, c_in = c0 < cols ? c0 : cols - EPT;
                 const bool in = row < r1 && c0 < cols;
@@ -250,7 +339,7 @@ __global__ __launch_bounds__(kColsumThreads) void cast_colsum_kernel(const IT* _
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int row = r + u * NW;
-            const size_t at = static_cast<size_t>(row) * cols + c0;
+            const size_t at = static_cast<size_t>(row) * pitch + c0;
             uint32_t w[EPT / 4];
 #pragma unroll
             for (int j = 0; j < EPT / 4; ++j) {
@@ -260,7 +349,7 @@ __global__ __launch_bounds__(kColsumThreads) void cast_colsum_kernel(const IT* _
                 acc[4 * j] += a, acc[4 * j + 1] += b, acc[4 * j + 2] += c, acc[4 * j + 3] += d;
             }
             if constexpr (VEC) {
-                if (row < r1 && c0 < cols) {
+                if (row < r1 && c0 < pitch) {
                     if constexpr (EPT == 4) *reinterpret_cast<uint32_t*>(out + at) = w[0];
                     else *reinterpret_cast<uint2*>(out + at) = make_uint2(w[0], w[1]);
                 }
@@ -431,16 +520,17 @@ __global__ __launch_bounds__(kCastThreads) void amax_partial_kernel(const IT* __
 // The first kernel of a gated cast beside one that does not depend on it.  As a rule the gate is closed and these workgroups
 // return at once: a launch of their own costs the host 3.5 us and the stream 2.5 for nothing.  The first `others` workgroups do the
 // other work.
-constexpr int kBesideThreads = 512;
 
 // ... the rescaling cast of a linear layer's weight
-template <typename IT, typename WT>
+template <typename IT, typename WT, bool PITCHED>
 __global__ __launch_bounds__(kBesideThreads) void amax_beside_rescale_kernel(const IT* __restrict__ x, size_t nx, uint32_t* ws,
                                                                               const float* scale, int x_vec, Gate gate, Finish fin,
                                                                               const WT* __restrict__ w, uint8_t* __restrict__ out, size_t nw,
-                                                                              float* scale_inv, int w_vec, InTimeArgs it, unsigned others) {
+                                                                              float* scale_inv, int w_vec, InTimeArgs it, unsigned others,
+                                                                              Pitch pt) {
     if (blockIdx.x < others)
-        cast_to_fp8<WT, MSAMP_DT_E4M3, false, kRescale, kBesideThreads>(w, out, nw, nullptr, nullptr, scale_inv, w_vec, 0, it, blockIdx.x, others);
+        cast_to_fp8<WT, MSAMP_DT_E4M3, false, kRescale, kBesideThreads, PITCHED>(w, out, nw, nullptr, nullptr, scale_inv, w_vec, 0, it,
+                                                                                 blockIdx.x, others, pt);
     else
         amax_partial<IT, kBesideThreads>(x, nx, ws, scale, x_vec, gate, fin, blockIdx.x - others, gridDim.x - others);
 }
@@ -1518,20 +1608,24 @@ static int colsum_slabs(int rows, int cols, int dtype, int* rows_per_slab) {
 
 template <typename IT>
 static int launch_colsum(const IT* x, int dtype, int rows, int cols, const float* scale, float* amax, float* scale_inv, uint8_t* out,
-                         int fp8_type, void* sum, int sum_dtype, float* partial, hipStream_t st) {
+                         int fp8_type, void* sum, int sum_dtype, float* partial, hipStream_t st, bool pitched = false) {
     constexpr int EPT = In16<IT>::EPT;
+    const int pitch = pitched ? kmajor_pitch(cols) : cols;
     int per = 0;
     const int slabs = colsum_slabs(rows, cols, dtype, &per);
     const dim3 grid((cols + kWave * EPT - 1) / (kWave * EPT), slabs);
     float* tops = partial + static_cast<size_t>(slabs) * cols;
     const bool vec = cols % EPT == 0 && aligned(x, 16) && aligned(out, EPT);
     const int stream = static_cast<size_t>(rows) * cols * sizeof(IT) >= kStreamBytes;
-#define LAUNCH(FMT, VEC) \
-    hipLaunchKernelGGL((cast_colsum_kernel<IT, FMT, VEC>), grid, dim3(kColsumThreads), 0, st, x, out, rows, cols, per, scale, scale_inv, partial, tops, stream)
-    if (fp8_type == MSAMP_DT_E4M3) {
-        if (vec) LAUNCH(MSAMP_DT_E4M3, true); else LAUNCH(MSAMP_DT_E4M3, false);
+#define LAUNCH(FMT, FORM) \
+    hipLaunchKernelGGL((cast_colsum_kernel<IT, FMT, FORM>), grid, dim3(kColsumThreads), 0, st, x, out, rows, cols, per, scale, scale_inv, partial, tops, stream, pitch)
+    if (pitch != cols) {
+        MSAMP_REQUIRE(fp8_type == MSAMP_DT_E5M2 && aligned(out, 16), MSAMP_ERR_ALIGNMENT, "launch_colsum: rows of codes apart: E5M2, 16-byte aligned");
+        LAUNCH(MSAMP_DT_E5M2, kColumnsPitched);
+    } else if (fp8_type == MSAMP_DT_E4M3) {
+        if (vec) LAUNCH(MSAMP_DT_E4M3, kColumnsWhole); else LAUNCH(MSAMP_DT_E4M3, kColumnsApart);
     } else {
-        if (vec) LAUNCH(MSAMP_DT_E5M2, true); else LAUNCH(MSAMP_DT_E5M2, false);
+        if (vec) LAUNCH(MSAMP_DT_E5M2, kColumnsWhole); else LAUNCH(MSAMP_DT_E5M2, kColumnsApart);
     }
 #undef LAUNCH
     MSAMP_CHECK_LAUNCH("cast_colsum_kernel");
@@ -2201,18 +2295,58 @@ static unsigned beside_blocks(size_t n, int dtype) {
     return static_cast<unsigned>(std::min(std::max<size_t>((n + tile - 1) / tile, 1), cap));
 }
 
-template <typename IT, typename WT>
+// how many workgroups of kBesideThreads cast n elements of 16 / EPT bytes each: few, large, long-lived ones
+static unsigned beside_casts(size_t n, int EPT) {
+    return static_cast<unsigned>(std::min(grid_for(n, static_cast<size_t>(kBesideThreads) * EPT * kCastUnroll), cu_count() * 2));
+}
+
+// Delayed cast of x[rows][cols] into codes of rows kmajor_pitch(cols) apart.
+template <typename IT>
+static void launch_cast_pitched(const void* x, const Pitch& pt, const float* scale, float* amax, float* scale_inv, uint8_t* out, bool e4m3,
+                                hipStream_t st) {
+    const size_t n = static_cast<size_t>(pt.rows) * pt.pitch;
+    const dim3 grid(beside_casts(n, In16<IT>::EPT));
+#define PITCHED(FMT) hipLaunchKernelGGL((cast_pitched_kernel<IT, FMT>), grid, dim3(kBesideThreads), 0, st, static_cast<const IT*>(x), out, n, scale, amax, scale_inv, pt)
+    if (e4m3) PITCHED(MSAMP_DT_E4M3);
+    else PITCHED(MSAMP_DT_E5M2);
+#undef PITCHED
+}
+
+// The delayed cast of a matrix of a linear layer, for the products that read it where it lies.
+static int cast_rows(const void* x, int dtype, int rows, int cols, const float* scale, float* amax, float* scale_inv, uint8_t* out,
+                     int fp8_type, hipStream_t st) {
+    if (cols % 16 == 0) return dispatch_cast(x, dtype, static_cast<size_t>(rows) * cols, scale, amax, scale_inv, out, fp8_type, nullptr, st);
+    MSAMP_REQUIRE(aligned(out, 16), MSAMP_ERR_ALIGNMENT, "cast_rows: codes must be 16-byte aligned");
+    const Pitch pt = {static_cast<unsigned>(rows), static_cast<unsigned>(cols), static_cast<unsigned>(kmajor_pitch(cols))};
+    const bool e4m3 = fp8_type == MSAMP_DT_E4M3;
+    if (dtype == MSAMP_DT_F32) launch_cast_pitched<float>(x, pt, scale, amax, scale_inv, out, e4m3, st);
+    else if (dtype == MSAMP_DT_F16) launch_cast_pitched<f16_t>(x, pt, scale, amax, scale_inv, out, e4m3, st);
+    else launch_cast_pitched<bf16_t>(x, pt, scale, amax, scale_inv, out, e4m3, st);
+    MSAMP_CHECK_LAUNCH("cast_pitched_kernel");
+    return MSAMP_OK;
+}
+
+template <typename IT, typename WT, bool PITCHED>
 static void launch_amax_beside_rescale(const msamp_linear_forward_args& a, const Gate& gate, const Finish& fin, hipStream_t st) {
-    const size_t nx = static_cast<size_t>(a.tokens) * a.d_in, nw = static_cast<size_t>(a.d_out) * a.d_in;
+    const int d_in = static_cast<int>(a.d_in), d_out = static_cast<int>(a.d_out);
+    const Pitch pt = {static_cast<unsigned>(d_out), static_cast<unsigned>(d_in), static_cast<unsigned>(kmajor_pitch(d_in))};
+    const size_t nx = static_cast<size_t>(a.tokens) * a.d_in, nw = static_cast<size_t>(kmajor_pitch(d_out)) * pt.pitch;    // (without PITCHED d_out * d_in)
     constexpr int EPT = In16<WT>::EPT;
-    const unsigned others = static_cast<unsigned>(std::min(grid_for(nw, static_cast<size_t>(kBesideThreads) * EPT * kCastUnroll), cu_count() * 2));
+    const unsigned others = beside_casts(nw, EPT);
     const int w_vec = (aligned(a.w, 16) && aligned(a.w_codes, EPT) ? 1 : 0) | (nw * sizeof(WT) >= kStreamBytes ? 2 : 0);
     float* meta = a.w_meta;
     const InTimeArgs it = {nullptr, meta, nullptr, fp8_max(MSAMP_DT_E4M3), 0, 0, a.w_amax, a.w_scale_inv, meta + 3, static_cast<int>(a.w_window),
                            reinterpret_cast<int32_t*>(meta + 2), 0};
-    hipLaunchKernelGGL((amax_beside_rescale_kernel<IT, WT>), dim3(others + beside_blocks(nx, static_cast<int>(a.x_dtype))),
+    hipLaunchKernelGGL((amax_beside_rescale_kernel<IT, WT, PITCHED>), dim3(others + beside_blocks(nx, static_cast<int>(a.x_dtype))),
                        dim3(kBesideThreads), 0, st, static_cast<const IT*>(a.x), nx, static_cast<uint32_t*>(a.workspace), a.x_scale,
-                       static_cast<int>(aligned(a.x, 16)), gate, fin, static_cast<const WT*>(a.w), a.w_codes, nw, meta + 1, w_vec, it, others);
+                       static_cast<int>(aligned(a.x, 16)), gate, fin, static_cast<const WT*>(a.w), a.w_codes, nw, meta + 1, w_vec, it, others,
+                       pt);
+}
+
+template <typename IT, typename WT>
+static void launch_amax_beside_rescale(const msamp_linear_forward_args& a, const Gate& gate, const Finish& fin, hipStream_t st) {
+    if (a.d_in % 16 || a.d_out % 16) launch_amax_beside_rescale<IT, WT, true>(a, gate, fin, st);
+    else launch_amax_beside_rescale<IT, WT, false>(a, gate, fin, st);
 }
 
 int cast_linear_inputs(const msamp_linear_forward_args& a, hipStream_t st) {
@@ -2222,6 +2356,8 @@ int cast_linear_inputs(const msamp_linear_forward_args& a, hipStream_t st) {
                   MSAMP_ERR_NULL, "msamp_linear_forward: null pointer");
     MSAMP_REQUIRE(a.workspace != nullptr, MSAMP_ERR_WORKSPACE, "msamp_linear_forward: workspace required");
     MSAMP_REQUIRE(a.w_window >= 1, MSAMP_ERR_SHAPE, "msamp_linear_forward: window %lld", static_cast<long long>(a.w_window));
+    MSAMP_REQUIRE((a.d_in % 16 == 0 && a.d_out % 16 == 0) || aligned(a.w_codes, 16), MSAMP_ERR_ALIGNMENT,
+                  "msamp_linear_forward: codes must be 16-byte aligned");
     const Gate gate = {a.x_counter, static_cast<int>(a.x_window)};
     const Finish fin = {a.x_amax, a.x_scale, a.x_scale_inv, fp8_max(MSAMP_DT_E4M3), 0, static_cast<int>(a.flags)};
 #define BESIDE(IT)                                                                                     \
@@ -2235,8 +2371,8 @@ int cast_linear_inputs(const msamp_linear_forward_args& a, hipStream_t st) {
     else BESIDE(bf16_t);
 #undef BESIDE
     MSAMP_CHECK_LAUNCH("amax_beside_rescale_kernel");
-    return dispatch_cast(a.x, x_dtype, static_cast<size_t>(a.tokens) * a.d_in, a.x_scale, a.x_amax, a.x_scale_inv, a.x_codes, MSAMP_DT_E4M3,
-                         nullptr, st);
+    return cast_rows(a.x, x_dtype, static_cast<int>(a.tokens), static_cast<int>(a.d_in), a.x_scale, a.x_amax, a.x_scale_inv, a.x_codes,
+                     MSAMP_DT_E4M3, st);
 }
 
 template <typename IT, typename OT>
@@ -2280,8 +2416,8 @@ int cast_output_gradient(const msamp_linear_backward_args& a, void* product, flo
         const int rc = dispatch_amax(a.dy, dy_dtype, n, a.workspace, a.g_scale, st, gate, fin);
         if (rc != MSAMP_OK) return rc;
     }
-    if (a.bias_sum == nullptr) return dispatch_cast(a.dy, dy_dtype, n, a.g_scale, a.g_amax, a.g_scale_inv, a.dy_codes, MSAMP_DT_E5M2, nullptr, st);
-#define COLSUM(IT) launch_colsum(static_cast<const IT*>(a.dy), dy_dtype, tokens, d_out, a.g_scale, a.g_amax, a.g_scale_inv, a.dy_codes, MSAMP_DT_E5M2, a.bias_sum, sum_dtype, sums, st)
+    if (a.bias_sum == nullptr) return cast_rows(a.dy, dy_dtype, tokens, d_out, a.g_scale, a.g_amax, a.g_scale_inv, a.dy_codes, MSAMP_DT_E5M2, st);
+#define COLSUM(IT) launch_colsum(static_cast<const IT*>(a.dy), dy_dtype, tokens, d_out, a.g_scale, a.g_amax, a.g_scale_inv, a.dy_codes, MSAMP_DT_E5M2, a.bias_sum, sum_dtype, sums, st, true)
     if (dy_dtype == MSAMP_DT_F32) return COLSUM(float);
     if (dy_dtype == MSAMP_DT_F16) return COLSUM(f16_t);
     return COLSUM(bf16_t);

@@ -45,7 +45,8 @@ static int dispatch_parts(int x_type, int y_type, const GemmCall& c, const KSpli
 // forward and backward: 335 -> 292.
 static KSplit ksplit_rule(int NR, int NC, int K) {
     KSplit best = {true, 1};
-    if (!takes_small_tiles(NR, NC, K) || !kmajor_shape_ok(NR, NC, K, true, true)) return best;
+    // (the parts are added up four outputs at a time)
+    if (!takes_small_tiles(NR, NC, K) || !fits_offsets(NR, NC, K) || static_cast<size_t>(NR) * NC % 4) return best;
     const int nk = (K + kBK - 1) / kBK, cus = cu_count();
     auto tiles = [&](int edge) { return ((NR + edge - 1) / edge) * ((NC + edge - 1) / edge); };
     const int small = tiles(kDmaTile / 2), large = tiles(kDmaTile);
@@ -275,30 +276,39 @@ extern "C" int msamp_fp8_gemm_kmajor(const uint8_t* a, int a_type, const float* 
 
 int msamp::gemm_kmajor(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv,
                        int b_kmajor, void* d, int d_dtype, int m, int n, int k, int accumulate, hipStream_t st) {
-    if (k > kBK)
-        return msamp_fp8_gemm_kmajor(a, a_type, a_scale_inv, 1, b, b_type, b_scale_inv, b_kmajor, d, d_dtype, m, n, k, accumulate, nullptr,
-                                     MSAMP_DT_F32, st);
     MSAMP_REQUIRE(is_fp8(a_type) && is_fp8(b_type) && is_hp(d_dtype), MSAMP_ERR_DTYPE, "gemm_kmajor: types %d, %d -> %d", a_type, b_type,
                   d_dtype);
-    MSAMP_REQUIRE(m > 0 && n > 0 && k > 0 && kmajor_rows_ok(n, m, k, b_kmajor != 0, true), MSAMP_ERR_SHAPE,
-                  "gemm_kmajor: m=%d n=%d k=%d (leading dimensions must be multiples of 16)", m, n, k);
+    MSAMP_REQUIRE(m > 0 && n > 0 && k > 0 && kmajor_rows_ok(kmajor_pitch(n), kmajor_pitch(m), k, b_kmajor != 0, true), MSAMP_ERR_SHAPE,
+                  "gemm_kmajor: m=%d n=%d k=%d (K of a row-major operand must be a multiple of 16)", m, n, k);
     MSAMP_REQUIRE(a && b && d && a_scale_inv && b_scale_inv, MSAMP_ERR_NULL, "gemm_kmajor: null pointer");
     MSAMP_REQUIRE(aligned(a, 16) && aligned(b, 16), MSAMP_ERR_ALIGNMENT, "gemm_kmajor: operands must be 16-byte aligned");
     const GemmCall c = {b, a, d, d_dtype, n, m, k, b_scale_inv, a_scale_inv, accumulate, nullptr, MSAMP_DT_F32, b_kmajor != 0, true, nullptr, st};
     return dispatch_pair(b_type, a_type, c);
 }
 
+size_t msamp::gemm_ksplit_scratch(int m, int n, int k) {
+    const KSplit split = ksplit_rule(n, m, k);
+    return split.parts > 1 ? static_cast<size_t>(split.parts) * n * m : 0;
+}
+
 extern "C" int msamp_fp8_gemm_ksplit_scratch(int m, int n, int k, size_t* n_floats) {
     MSAMP_REQUIRE(m > 0 && n > 0 && k > 0, MSAMP_ERR_SHAPE, "msamp_fp8_gemm_ksplit_scratch: m=%d n=%d k=%d", m, n, k);
     MSAMP_REQUIRE(n_floats != nullptr, MSAMP_ERR_NULL, "msamp_fp8_gemm_ksplit_scratch: null pointer");
-    const KSplit split = ksplit_rule(n, m, k);
-    *n_floats = split.parts > 1 ? static_cast<size_t>(split.parts) * n * m : 0;
+    *n_floats = kmajor_shape_ok(n, m, k, true, true) ? gemm_ksplit_scratch(m, n, k) : 0;
     return MSAMP_OK;
 }
 
 extern "C" int msamp_fp8_gemm_ksplit(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type,
                                      const float* b_scale_inv, void* d, int d_dtype, int m, int n, int k, int accumulate,
                                      float* scratch, size_t n_floats, msamp_stream_t stream) {
+    MSAMP_REQUIRE(m <= 0 || n <= 0 || k <= 0 || kmajor_shape_ok(n, m, k, true, true), MSAMP_ERR_SHAPE,
+                  "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d is not split", m, n, k);
+    return gemm_ksplit(a, a_type, a_scale_inv, b, b_type, b_scale_inv, d, d_dtype, m, n, k, accumulate, scratch, n_floats,
+                       static_cast<hipStream_t>(stream));
+}
+
+int msamp::gemm_ksplit(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv,
+                       void* d, int d_dtype, int m, int n, int k, int accumulate, float* scratch, size_t n_floats, hipStream_t st) {
     MSAMP_REQUIRE(is_fp8(a_type) && is_fp8(b_type), MSAMP_ERR_DTYPE, "msamp_fp8_gemm_ksplit: operand types %d, %d", a_type, b_type);
     MSAMP_REQUIRE(is_hp(d_dtype), MSAMP_ERR_DTYPE, "msamp_fp8_gemm_ksplit: output dtype %d", d_dtype);
     MSAMP_REQUIRE(m > 0 && n > 0 && k > 0, MSAMP_ERR_SHAPE, "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d", m, n, k);
@@ -310,7 +320,6 @@ extern "C" int msamp_fp8_gemm_ksplit(const uint8_t* a, int a_type, const float* 
     const size_t count = static_cast<size_t>(n) * m;
     MSAMP_REQUIRE(split.parts > 1 && n_floats >= split.parts * count, MSAMP_ERR_SHAPE,
                   "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d is not split, or needs more scratch than %zu floats", m, n, k, n_floats);
-    hipStream_t st = static_cast<hipStream_t>(stream);
     const GemmCall c = {b, a, scratch, MSAMP_DT_F32, n, m, k, b_scale_inv, a_scale_inv, 0, nullptr, 0, true, true, nullptr, st};
     const int rc = dispatch_parts(b_type, a_type, c, split);
     if (rc != MSAMP_OK) return rc;

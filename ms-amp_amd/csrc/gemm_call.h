@@ -24,6 +24,10 @@ struct QuantArgs {
     int walk_plus_one;       // every form of the kernel: 0 = the tile walk the built-in rule picks, 1..4 = walk 0..3 (see registered_walk)
 };
 
+// From one k-row of a K-major operand to the next: its row count, which the entry points want to be a multiple of 16, or in the
+// calls for a linear layer, whose casts write them so, the next one.
+__host__ __device__ inline int kmajor_pitch(int rows) { return (rows + 15) & ~15; }
+
 // One product D[NR][NC] = X[NR][K] . Y[NC][K]^T * *xs * *ys.  xt / yt: that operand is handed over K-major.
 // qa != nullptr: the output is cast on to FP8 in the same launch; D is not written, unless `qspec` asks for the
 // speculative form, which stores D as usual and the codes of D times the scale in force next to it.
@@ -102,9 +106,13 @@ inline bool takes_paired_tiles(int NR, int NC, int K) {
     return K <= kBK || (tiles <= 2L * cu_count() && (tiles > cu_count() || K <= 2048));
 }
 
-// msamp_fp8_gemm_kmajor for any K: a single slice of K is left to the paired tiles.
+// msamp_fp8_gemm_kmajor for any K (a single slice of it is left to the paired tiles) and any m and n, with the operands' k-rows
+// kmajor_pitch() apart; msamp_fp8_gemm_ksplit and its scratch (0: not split) the same way.
 int gemm_kmajor(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv,
                 int b_kmajor, void* d, int d_dtype, int m, int n, int k, int accumulate, hipStream_t st);
+size_t gemm_ksplit_scratch(int m, int n, int k);
+int gemm_ksplit(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv, void* d,
+                int d_dtype, int m, int n, int k, int accumulate, float* scratch, size_t n_floats, hipStream_t st);
 
 // row offsets of the direct-to-LDS kernels are 32 bits
 inline bool fits_offsets(int NR, int NC, int K) {

@@ -437,8 +437,8 @@ __device__ __forceinline__ void k_part(In& X, In& Y, Out& D, int NR, int NC, int
     const int nk = (K + kBK - 1) / kBK, parts = gridDim.y, y = blockIdx.y;
     const int first = static_cast<int>(static_cast<long long>(nk) * y / parts) * kBK;
     const int end = y + 1 == parts ? K : static_cast<int>(static_cast<long long>(nk) * (y + 1) / parts) * kBK;
-    X += static_cast<size_t>(first) * NR;
-    Y += static_cast<size_t>(first) * NC;
+    X += static_cast<size_t>(first) * kmajor_pitch(NR);
+    Y += static_cast<size_t>(first) * kmajor_pitch(NC);
     D += static_cast<size_t>(y) * NR * NC;
     K = end - first;
 }
@@ -538,9 +538,10 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // position l%16, and fetches the logical chunk position ^ (k-row % 8)
     const int chunk_t = (lane & 15) ^ ((wave & 1) * 4 + (lane >> 4));
     // K-major operand, last tile: 16-byte chunks past the end of a k-row are fetched from the tile's first chunk instead
-    // (rows of D that do not exist; the row count is a multiple of 16, so a chunk is in or out as a whole)
+    // (rows of D that do not exist; a k-row's pitch is a multiple of 16, so a chunk is inside it or not as a whole)
     const int xcol = row0 + chunk_t * 16 < NR ? row0 + chunk_t * 16 : row0;
     const int ycol = col0 + chunk_t * 16 < NC ? col0 + chunk_t * 16 : col0;
+    const int ldx = kmajor_pitch(NR), ldy = kmajor_pitch(NC);
     uint32_t xoff[8], yoff[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -549,9 +550,9 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
         gx = gx < NR ? gx : NR - 1;
         gy = gy < NC ? gy : NC - 1;
         const int krow = (i * 4 + wave) * 4 + (lane >> 4);
-        xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NR) + xcol
+        xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(ldx) + xcol
                      : static_cast<uint32_t>(gx) * static_cast<uint32_t>(K) + chunk * 16;
-        yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NC) + ycol
+        yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(ldy) + ycol
                      : static_cast<uint32_t>(gy) * static_cast<uint32_t>(K) + chunk * 16;
     }
     // KTAIL: K is no multiple of 128 and the last slice holds `rem` bytes of K only.  Its loads stay inside the operand (a
@@ -569,7 +570,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
         const int which = SPLIT ? by_need[i] : i;
         const bool is_x = which < 8;
         const size_t slice = static_cast<size_t>(kt) * kBK;
-        const uint8_t* src = is_x ? X + (XT ? slice * NR : slice) : Y + (YT ? slice * NC : slice);
+        const uint8_t* src = is_x ? X + (XT ? slice * ldx : slice) : Y + (YT ? slice * ldy : slice);
         uint32_t off = which < 8 ? xoff[which] : yoff[which - 8];
         if (KTAIL && last) {
             if (is_x ? XT : YT) {
@@ -758,7 +759,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                 const uint8_t* base = is_x ? X : Y;
                 const int n = is_x ? NR : NC, first = is_x ? nr0 : nc0;
                 if (is_x ? XT : YT)
-                    return base + static_cast<size_t>(!KTAIL || r < K ? r : K - 1) * n + (first + hf < n ? first + hf : first);
+                    return base + static_cast<size_t>(!KTAIL || r < K ? r : K - 1) * (is_x ? ldx : ldy) + (first + hf < n ? first + hf : first);
                 const int row = first + r < n ? first + r : n - 1;
                 return base + static_cast<size_t>(row) * K + hf;
             };

@@ -1,6 +1,6 @@
 // The direct-to-LDS FP8 GEMM with 128 x 128 output tiles, for problems that leave most compute units idle with
 // 256 x 256 tiles (a 2048 x 2048 output is 64 of those, a quarter of the chip, and 256 of these).  At least four
-// 128-byte slices of K (the last one may be ragged: KTAIL); operands row-major (K-contiguous) or, with XT / YT, K-major ([K][rows], rows a multiple of 16):
+// 128-byte slices of K (the last one may be ragged: KTAIL); operands row-major (K-contiguous) or, with XT / YT, K-major ([K][rows], kmajor_pitch() apart):
 // the slice then lies in LDS as 128 k-rows of 128 bytes, the 16-byte position XOR-ed with k % 8, and the fragments
 // come from the transposing LDS read, as in the large tile.
 //
@@ -126,6 +126,7 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     // K-major operand, last tile: chunks past the end of a k-row are fetched from the tile's first chunk instead
     const int xcol = row0 + chunk_t * 16 < NR ? row0 + chunk_t * 16 : row0;
     const int ycol = col0 + chunk_t * 16 < NC ? col0 + chunk_t * 16 : col0;
+    const int ldx = kmajor_pitch(NR), ldy = kmajor_pitch(NC);
     uint32_t xoff[4], yoff[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -134,9 +135,9 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
         gx = gx < NR ? gx : NR - 1;
         gy = gy < NC ? gy : NC - 1;
         const int krow = (i * 4 + wave) * 8 + (lane >> 3);
-        xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NR) + xcol
+        xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(ldx) + xcol
                      : static_cast<uint32_t>(gx) * static_cast<uint32_t>(K) + chunk * 16;
-        yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(NC) + ycol
+        yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(ldy) + ycol
                      : static_cast<uint32_t>(gy) * static_cast<uint32_t>(K) + chunk * 16;
     }
     // KTAIL: a ragged last slice of `rem` K bytes, handled as in the large tile (loads kept inside the operand, fragments
@@ -153,7 +154,7 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     auto dma = [&](int kt, int which, bool last = false) __attribute__((always_inline)) {
         const bool is_x = which < 4;
         const size_t slice = static_cast<size_t>(kt) * kBK;
-        const uint8_t* src = is_x ? X + (XT ? slice * NR : slice) : Y + (YT ? slice * NC : slice);
+        const uint8_t* src = is_x ? X + (XT ? slice * ldx : slice) : Y + (YT ? slice * ldy : slice);
         uint32_t off = is_x ? xoff[which] : yoff[which - 4];
         if (KTAIL && last) {
             if (is_x ? XT : YT) {

@@ -735,18 +735,32 @@ def linear_takes_short_k(tokens, d_in, d_out):
     return min(tokens, d_out) <= 128 and d_in % 16 == 0 and d_out % 16 == 0 and max(tokens * d_out, d_out * d_in, tokens * d_in) < 2**32
 
 
+def linear_pitch(n):
+    """From one row of codes to the next where a row has n of them (kmajor_pitch() of the library): the calls for a linear layer
+    write zeros behind them, and as many rows of them below a weight, so that the products read any width in place."""
+    return (n + 15) // 16 * 16
+
+
+def linear_fits(tokens, d_in, d_out):
+    """True where the products of a linear layer read codes of widths that are no multiples of 16 (32-bit offsets)."""
+    d_in, d_out = linear_pitch(d_in), linear_pitch(d_out)
+    return max(tokens * d_out, d_out * d_in, tokens * d_in) < 2**32
+
+
 FEW_TOKENS = 64    # MSAMP_FEW_TOKENS
 
 
 def linear_forward(x, x_meta, w, w_meta, out_dtype, bias, want_codes=True):
     """y = x . w^T (+ bias) through msamp_linear_forward.  x: contiguous [tokens, d_in], cast with x_meta (gated scaling); w: the
     contiguous scaled payload [d_out, d_in] of a weight with w_meta.  Returns y and, if want_codes, the E4M3 codes of x
-    and of w and the words {scale, scale_inv, update count, amax window} of the codes of w (else these are not to be used)."""
+    and of w ([tokens, linear_pitch(d_in)], [linear_pitch(d_out), linear_pitch(d_in)]) and the words {scale, scale_inv, update
+    count, amax window} of the codes of w (else these are not to be used)."""
     lib = load()
     (tokens, d_in), d_out, device, window = x.shape, w.shape[0], x.device, w_meta.window_size
-    if want_codes or tokens > FEW_TOKENS or w.data_ptr() % 16:
-        x_codes = torch.empty((tokens, d_in), dtype=torch.uint8, device=device)
-        w_codes = torch.empty((d_out, d_in), dtype=torch.uint8, device=device)
+    if want_codes or tokens > FEW_TOKENS or w.data_ptr() % 16 or d_in % 16:
+        pitch = linear_pitch(d_in)
+        x_codes = torch.empty((tokens, pitch), dtype=torch.uint8, device=device)
+        w_codes = torch.empty((linear_pitch(d_out), pitch), dtype=torch.uint8, device=device)
         words = torch.empty(3 + window, dtype=torch.float32, device=device)
     else:    # (codes of x in another order, in whole blocks of 16 tokens and 128 wide)
         x_codes = torch.empty(((tokens + 15) // 16 * ((d_in + 127) // 128) * 2048, ), dtype=torch.uint8, device=device)
@@ -763,14 +777,14 @@ def linear_forward(x, x_meta, w, w_meta, out_dtype, bias, want_codes=True):
     return y, x_codes, w_codes, words
 
 
-def linear_backward(dy, g_meta, x_codes, x_scale_inv, w_codes, w_scale_inv_ptr, out_dtype, need_dx, q_meta, old, bias_dtype):
-    """Gradients of linear_forward through msamp_linear_backward: the E5M2 codes of dy, dx in out_dtype (None unless need_dx), the
-    E4M3 codes of the weight gradient (None unless q_meta, its meta, is given; `old`, a ScalingTensor or None, is added to it) and
-    the column sums of dy (None unless bias_dtype is given)."""
+def linear_backward(dy, d_in, g_meta, x_codes, x_scale_inv, w_codes, w_scale_inv_ptr, out_dtype, need_dx, q_meta, old, bias_dtype):
+    """Gradients of linear_forward through msamp_linear_backward: the E5M2 codes of dy ([tokens, linear_pitch(d_out)]), dx in
+    out_dtype (None unless need_dx), the E4M3 codes of the weight gradient (None unless q_meta, its meta, is given; `old`, a
+    ScalingTensor or None, is added to it) and the column sums of dy (None unless bias_dtype is given)."""
     lib = load()
-    (tokens, d_out), d_in, device = dy.shape, x_codes.shape[1], dy.device
+    (tokens, d_out), device = dy.shape, dy.device
     dt, out_dt = _TORCH_TO_DT[dy.dtype], _TORCH_TO_DT[out_dtype]
-    codes = torch.empty((tokens, d_out), dtype=torch.uint8, device=device)
+    codes = torch.empty((tokens, linear_pitch(d_out)), dtype=torch.uint8, device=device)
     dx = torch.empty((tokens, d_in), dtype=out_dtype, device=device) if need_dx else None
     wq = torch.empty((d_out, d_in), dtype=torch.uint8, device=device) if q_meta is not None else None
     sums = torch.empty((d_out, ), dtype=bias_dtype, device=device) if bias_dtype is not None else None

@@ -21,10 +21,11 @@ def _forward_in_one_call(x, meta, weight, output_dtype, bias):
             x.dtype in _FLOATS and output_dtype in _FLOATS and meta.scale.is_cuda):
         return False
     (tokens, d_in), device = x.shape, x.device
-    return w.dim() == 2 and w.numel() > 0 and w.shape[1] == d_in and d_in % 16 == 0 and w.dtype in _FLOATS and w.device == device and \
+    return w.dim() == 2 and w.numel() > 0 and w.shape[1] == d_in and w.dtype in _FLOATS and w.device == device and \
         w.is_contiguous() and w_meta.amax.device == device and 1 <= w_meta.window_size <= w_meta.amax.numel() and \
         (bias is None or (bias.device == device and bias.dtype in _FLOATS and bias.numel() == w.shape[0])) and \
-        _backend.gemm_walk_settled(w.shape[0], tokens, d_in, False, False)
+        (d_in % 16 == 0 and w.shape[0] % 16 == 0 or _backend.linear_fits(tokens, d_in, w.shape[0])) and \
+        _backend.gemm_walk_settled(w.shape[0], tokens, _backend.linear_pitch(d_in), False, False)
 
 
 def _backward_in_one_call(ctx, dy, d_in, need_dgrad):
@@ -61,7 +62,7 @@ class _FP8GemmFunction(torch.autograd.Function):
         model_state.check_metas_in_flat(metas)
         output_dtype = dtype_holder.dtype
         ctx.need_input_grad = input.requires_grad
-        ctx.weight = weight
+        ctx.weight, ctx.d_in = weight, input.shape[1]
         ctx.output_dtype = output_dtype
         ctx.bias_dtype = None if bias is None else bias.dtype
         ctx.need_bias_grad = bias is not None and bias.requires_grad
@@ -85,13 +86,20 @@ class _FP8GemmFunction(torch.autograd.Function):
         output_grad = output_grad.contiguous()
         metas = ctx.metas
         tokens, d_out = output_grad.shape
-        d_in = ctx.input_codes.shape[1]
+        d_in = ctx.d_in
+        input_codes, weight_codes = ctx.input_codes, ctx.weight_codes
         need_dgrad, need_wgrad = ctx.need_input_grad, ctx.weight.requires_grad
         # The reference materializes dy^T, W^T and x^T (fused cast-transpose + two FP8 transposes) because its
         # GEMM reads K-contiguous operands only.  This kernel also reads [K, rows] operands in place, so when
         # the shapes allow, dy is only cast and W, x, dy go to the GEMMs as they are (same results, up to the order of
         # the float32 sum where the weight gradient is taken in parts of K).
-        in_place = (not need_dgrad or Gemm.kmajor_supported(d_in, tokens, d_out, True, False)) and \
+        # Codes of widths that are no multiples of 16 come from the forward call in padded rows, which linear_backward reads.
+        pitched = input_codes.shape[1] != d_in or weight_codes.shape[0] != d_out
+        if pitched and not ((not need_wgrad or _wgrad_in_one_call(ctx, tokens, d_in, d_out)) and
+                            _backward_in_one_call(ctx, output_grad, d_in, need_dgrad)):
+            pitched = False
+            input_codes, weight_codes = input_codes[:, :d_in].contiguous(), weight_codes[:d_out, :d_in].contiguous()
+        in_place = pitched or (not need_dgrad or Gemm.kmajor_supported(d_in, tokens, d_out, True, False)) and \
             (not need_wgrad or Gemm.kmajor_supported(d_in, d_out, tokens, True, True))
         if not in_place and (not need_wgrad or _wgrad_in_one_call(ctx, tokens, d_in, d_out)):
             in_place = _backend.linear_takes_short_k(tokens, d_in, d_out) and _backward_in_one_call(ctx, output_grad, d_in, need_dgrad)
@@ -103,7 +111,7 @@ class _FP8GemmFunction(torch.autograd.Function):
             # (a weight gradient that is cast inside its product keeps a call of its own)
             with_wgrad = need_wgrad and _wgrad_in_one_call(ctx, tokens, d_in, d_out)
             payload, input_grad, wgrad, bias_grad = _backend.linear_backward(
-                output_grad, metas['ograd'], ctx.input_codes, metas['input'].scale_inv, ctx.weight_codes,
+                output_grad, d_in, metas['ograd'], input_codes, metas['input'].scale_inv, weight_codes,
                 words.scale_inv.data_ptr() if isinstance(words, ScalingMeta) else words.data_ptr() + 4, ctx.output_dtype, need_dgrad,
                 metas['wgrad'] if with_wgrad else None, ctx.weight.grad, ctx.bias_dtype if column_sums else None
             )
@@ -122,8 +130,8 @@ class _FP8GemmFunction(torch.autograd.Function):
             ograd_fp8, ograd_fp8_t = output_grad.fused_cast_transpose(Dtypes.kfloat8_e5m2, meta=metas['ograd'])
 
         if need_dgrad or need_wgrad:
-            input_fp8 = ScalingTensor(ctx.input_codes, metas['input'])
-            weight_fp8 = ScalingTensor(ctx.weight_codes, words if isinstance(words, ScalingMeta) else
+            input_fp8 = ScalingTensor(input_codes, metas['input'])
+            weight_fp8 = ScalingTensor(weight_codes, words if isinstance(words, ScalingMeta) else
                                        ScalingMeta._of_words(Dtypes.kfloat8_e4m3, words))
         if need_dgrad:
             if in_place:
