@@ -113,6 +113,21 @@ int registered_walk(int NR, int NC, int K, bool XT, bool YT) {
 static std::atomic<int> g_small_tile_limit{kSmallTileLimit};
 int small_tile_limit() { return g_small_tile_limit.load(std::memory_order_relaxed); }
 
+// 128 x 128 tiles with two workgroups to a compute unit, us against the kernel that would take the product otherwise (row-major,
+// both K-major):
+//   K <= 128 (the generic kernel)                        1024 x 1024  13.8 -> 4.6     8192 x 4096  58.5 -> 17.9
+//   one tile a unit or fewer, K = 256 (large tiles)      2048 x 2048   8.4 -> 5.4,     8.7 -> 5.6
+//     K = 1024 (small tiles, one workgroup a unit)       2048 x 2048   7.5 -> 7.0,     8.3 -> 7.3
+//     K = 2048                                           2048 x 2048   9.9 -> 9.5,    11.4 -> 10.2    K = 4096: 18.1 -> 20.8, 20.1 -> 20.6
+//   up to two tiles a unit, K = 1024 (large tiles)       4096 x 2048  13.9 -> 10.4,   14.2 -> 10.9
+//     K = 4096 (small tiles)                             4096 x 2048  35.5 -> 30.4,   41.0 -> 31.9    K = 12288: 89.0 -> 83.2, 104.5 -> 87.6
+//   more (large tiles)                                   3072 x 4096 x 1024  14.8 -> 13.9, 15.1 -> 15.1;   4096 x 4096 x 1024  16.9 -> 17.7, 17.3 -> 18.8
+bool takes_paired_tiles(int NR, int NC, int K) {
+    if (small_tile_limit() != kSmallTileLimit) return false;
+    const long tiles = static_cast<long>((NR + kDmaTile / 2 - 1) / (kDmaTile / 2)) * ((NC + kDmaTile / 2 - 1) / (kDmaTile / 2));
+    return K <= kBK || (tiles <= 2L * cu_count() && (tiles > cu_count() || K <= 2048));
+}
+
 }    // namespace msamp
 
 using namespace msamp;

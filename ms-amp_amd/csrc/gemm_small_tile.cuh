@@ -94,7 +94,7 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     const int row0 = tr * kSmallTile, col0 = tc * kSmallTile;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = wave >> 1, wc = wave & 1;
-    // the output factor and this lane's bias values are fetched now: in the epilogue they would sit on its critical path
+    // the output factor and the bias are fetched now: in the epilogue they would sit on its critical path
     constexpr int kEsz = static_cast<int>(sizeof(OT));
     constexpr int kElems = 16 / kEsz;              // outputs per 16-byte segment: 8 or 4
     constexpr int kSegs = 64 / kElems;             // segments per 64-column row: 8 or 16
@@ -102,15 +102,13 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     const int gcol = col0 + wc * 64 + seg * kElems;
     float alpha = (*x_scale_inv) * (*y_scale_inv);
     if constexpr (kParts) alpha = gridDim.y > 1 ? 1.0f : alpha;
-    float bv[kElems];
-#pragma unroll
-    for (int e = 0; e < kElems; ++e) bv[e] = 0.0f;
+    // (one column of the wave's 64 a lane, handed out in the epilogue: a load for each of a lane's columns, one behind the other, took
+    // up to 3 us of a tile's time: 4608 x 4096 x 512 with two workgroups to a compute unit 20.5 -> 17.9 us, 8192 x 4096 x 512 29.5 -> 25.4)
+    float bias_lane = 0.0f;
     auto fetch_bias = [&]() __attribute__((always_inline)) {
-        if (bias == nullptr) return;
-#pragma unroll
-        for (int e = 0; e < kElems; ++e) bv[e] = gcol + e < NC ? load_bias(bias, bias_dt, gcol + e) : 0.0f;
-#pragma unroll
-        for (int e = 0; e < kElems; ++e) asm volatile("" : "+v"(bv[e]));
+        const int c = col0 + wc * 64 + lane;
+        if (bias != nullptr) bias_lane = c < NC ? load_bias(bias, bias_dt, c) : 0.0f;
+        asm volatile("" : "+v"(bias_lane));
     };
     if constexpr (!PAIR) fetch_bias();
     asm volatile("" : "+v"(alpha));
@@ -367,7 +365,7 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
             tail4(c0, c1, kt);
         }
     }
-    if constexpr (PAIR) fetch_bias();    // (no registers for them before; the other workgroup works meanwhile)
+    if constexpr (PAIR) fetch_bias();    // (no register for it before; the other workgroup works meanwhile)
     const uint32_t acc_token = PAIR ? vacc_fence() : acc_fence();
     __syncthreads();    // every wave is through with the stages, which the patches below reuse
 
@@ -379,6 +377,9 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
     const bool vec_ok = (NC % kElems == 0) && ((reinterpret_cast<uintptr_t>(D) & 15) == 0);
     const bool plain = !accumulate && bias == nullptr;
     const int prl = lane / kSegs;
+    float bv[kElems];
+#pragma unroll
+    for (int e = 0; e < kElems; ++e) bv[e] = bias != nullptr ? __shfl(bias_lane, seg * kElems + e) : 0.0f;
     static_for<4>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         static_for<4>([&](auto jc) {
