@@ -122,10 +122,19 @@ int small_tile_limit() { return g_small_tile_limit.load(std::memory_order_relaxe
 //   up to two tiles a unit, K = 1024 (large tiles)       4096 x 2048  13.9 -> 10.4,   14.2 -> 10.9
 //     K = 4096 (small tiles)                             4096 x 2048  35.5 -> 30.4,   41.0 -> 31.9    K = 12288: 89.0 -> 83.2, 104.5 -> 87.6
 //   more (large tiles)                                   3072 x 4096 x 1024  14.8 -> 13.9, 15.1 -> 15.1;   4096 x 4096 x 1024  16.9 -> 17.7, 17.3 -> 18.8
+// Large tiles of which a few begin another round cost a whole one, where paired tiles, of half a round's time each, take what is
+// there.  us, row-major with a bias, one operand K-major, both:
+//   1 to 1.5 rounds, K <= 2048     5120 x 4096 x 512   21.5 -> 18.6, 21.2 -> 16.3, 21.8 -> 17.4   K = 2048  46.0 -> 40.0, 45.6 -> 40.1, 46.9 -> 40.9
+//                                  6144 x 4096 x 512   22.4 -> 19.4, 22.2 -> 18.1, 22.0 -> 18.9   K = 2048  46.0 -> 44.8, 45.3 -> 44.8, 47.2 -> 46.6
+//   2 to 2.25                      9216 x 4096 x 512   32.0 -> 30.2, 32.6 -> 26.5, 32.7 -> 27.3   K = 2048  69.8 -> 66.8, 69.1 -> 65.3, 71.8 -> 69.5
+//   elsewhere                      7168 x 4096 x 512   23.1 -> 24.6, 22.6 -> 21.8, 23.0 -> 22.1   K = 2048  47.5 -> 54.2, 48.0 -> 54.7, 49.1 -> 55.2
+//                                  6144 x 4096 x 4096  78.7 -> 80.7, 78.0 -> 81.0   5120 x 4096 x 8192  143.7 -> 131.8, 142.9 -> 140.7, 150.1 -> 172.0
 bool takes_paired_tiles(int NR, int NC, int K) {
     if (small_tile_limit() != kSmallTileLimit) return false;
     const long tiles = static_cast<long>((NR + kDmaTile / 2 - 1) / (kDmaTile / 2)) * ((NC + kDmaTile / 2 - 1) / (kDmaTile / 2));
-    return K <= kBK || (tiles <= 2L * cu_count() && (tiles > cu_count() || K <= 2048));
+    const long large = static_cast<long>((NR + kDmaTile - 1) / kDmaTile) * ((NC + kDmaTile - 1) / kDmaTile), cus = cu_count();
+    if (large > cus && K <= 2048 && (tiles <= 6 * cus || (large > 2 * cus && tiles <= 9 * cus))) return true;
+    return K <= kBK || (tiles <= 2 * cus && (tiles > cus || K <= 2048));
 }
 
 }    // namespace msamp
@@ -166,7 +175,7 @@ extern "C" int msamp_fp8_gemm_tune(const uint8_t* a, int a_type, const float* a_
     const long tiles = (static_cast<long>(n) + kDmaTile - 1) / kDmaTile * ((static_cast<long>(m) + kDmaTile - 1) / kDmaTile);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &capturing) != hipSuccess) capturing = hipStreamCaptureStatusActive, (void)hipGetLastError();
-    const bool candidate = m > 0 && n > 0 && k >= 4 * kBK && k % kBK == 0 && tiles >= 2L * cu_count() && !takes_small_tiles(n, m, k) &&
+    const bool candidate = m > 0 && n > 0 && k >= 4 * kBK && k % kBK == 0 && tiles >= 2L * cu_count() && !takes_small_tiles(n, m, k) && !takes_paired_tiles(n, m, k) &&
                            capturing == hipStreamCaptureStatusNone;
     if (!candidate) return run();
     hipEvent_t e0 = nullptr, e1 = nullptr;
