@@ -330,7 +330,9 @@ int msamp_fp8_gemm_cast(const uint8_t* a, int a_type, const float* a_scale_inv, 
  * d_in rounded up to a multiple of 16, zeros behind the d_in codes, and w_codes in d_out rounded up likewise, rows of zeros below
  * (16-byte aligned where there are any).  With w_codes NULL (nobody needs them; at most MSAMP_FEW_TOKENS tokens, d_in a multiple
  * of 16, w, x_codes and y 16-byte aligned) the last two are one launch: the weight is quantized to the same codes on its way into the product, and the float32 sum is taken in
- * up to eight parts of K; x_codes is scratch of 2048 bytes for every 16 tokens and 128 of d_in begun. */
+ * up to eight parts of K; x_codes is scratch of 2048 bytes for every 16 tokens and 128 of d_in begun.  Otherwise, given the scratch
+ * that msamp_linear_forward_scratch asks for (0 bytes: none needed), a product of a few tiles with a long K is taken in parts of K as
+ * msamp_fp8_gemm_ksplit does; with less it is taken whole. */
 #define MSAMP_FEW_TOKENS 64
 typedef struct msamp_linear_forward_args {
     const void* x;             /* [tokens][d_in], x_dtype */
@@ -354,11 +356,14 @@ typedef struct msamp_linear_forward_args {
     int64_t bias_dtype;
     int64_t flags;             /* MSAMP_FLAG_TWO_PASS */
     void* workspace;
+    void* scratch;             /* nullable, 16-byte aligned: room for a product in parts of K */
+    int64_t scratch_bytes;
 } msamp_linear_forward_args;
+int msamp_linear_forward_scratch(int tokens, int d_in, int d_out, size_t* bytes);
 int msamp_linear_forward(const msamp_linear_forward_args* args, msamp_stream_t stream);
 
 /* Backward: msamp_cast_to_fp8_gated of dy to E5M2 (msamp_cast_to_fp8_colsum_gated if bias_sum is given); dx with
- * msamp_fp8_gemm_kmajor if dx is given; and if wq is given the weight gradient, added to the dequantized old one if there is
+ * msamp_fp8_gemm_kmajor (or in parts of K, where the scratch has room) if dx is given; and if wq is given the weight gradient, added to the dequantized old one if there is
  * one: msamp_fp8_gemm_ksplit (if it splits the product and the scratch has room) or msamp_fp8_gemm_kmajor, and
  * msamp_cast_to_fp8_intime with MSAMP_FLAG_NAN_TO_INF.  (A product that msamp_fp8_gemm_cast takes is better left to that: without
  * wq the codes of dy are there for it.)  The codes of dy lie in rows of d_out rounded up to a multiple of 16, those of x and w
@@ -393,8 +398,8 @@ typedef struct msamp_linear_backward_args {
     int64_t scratch_bytes;
     void* workspace;
 } msamp_linear_backward_args;
-int msamp_linear_backward_scratch(int tokens, int d_in, int d_out, int dy_dtype, int out_dtype, int want_wgrad, int want_bias,
-                                  size_t* bytes, size_t* least);
+int msamp_linear_backward_scratch(int tokens, int d_in, int d_out, int dy_dtype, int out_dtype, int want_dx, int want_wgrad,
+                                  int want_bias, size_t* bytes, size_t* least);
 int msamp_linear_backward(const msamp_linear_backward_args* args, msamp_stream_t stream);
 
 /* Tile walks of the 256 x 256-tile kernel (no counterpart in the reference, whose GEMM is cuBLASLt behind

@@ -43,10 +43,15 @@ static int dispatch_parts(int x_type, int y_type, const GemmCall& c, const KSpli
 // a unit 121.3), 128 x 512 x 16000 54.9 -> 15.2, 256 x 1024 x 8192 29.9 -> 15.6, 1024 x 1024 x 16384 57.6 -> 33.4,
 // 16 x 8192 x 8192 30.3 -> 19.7, 2048 x 1024 x 8192 32.8 -> 27.4, 512 x 512 x 2500 12.7 -> 11.4.  FP8Linear 12605 x 1200 -> 4304,
 // forward and backward: 335 -> 292.
-static KSplit ksplit_rule(int NR, int NC, int K) {
+// Other operands (a forward product, an input gradient) only where the whole product would run 128 x 128 tiles one to a compute unit
+// with a longer K than two to a unit take, and in small tiles: their outputs as a rule are larger.  The layer call,
+// us: forward 468 x 11840 -> 512 58.8 -> 33.9, forward and backward twice over 791 x 15583 -> 1024 453 -> 390.
+static KSplit ksplit_rule(int NR, int NC, int K, bool xt, bool yt) {
     KSplit best = {true, 1};
     // (the parts are added up four outputs at a time)
     if (!takes_small_tiles(NR, NC, K) || !fits_offsets(NR, NC, K) || static_cast<size_t>(NR) * NC % 4) return best;
+    const bool both = xt && yt;
+    if (!both && (K <= 2048 || takes_paired_tiles(NR, NC, K))) return best;
     const int nk = (K + kBK - 1) / kBK, cus = cu_count();
     auto tiles = [&](int edge) { return ((NR + edge - 1) / edge) * ((NC + edge - 1) / edge); };
     const int small = tiles(kDmaTile / 2), large = tiles(kDmaTile);
@@ -62,7 +67,7 @@ static KSplit ksplit_rule(int NR, int NC, int K) {
             const double t = estimate(small, parts, 0.6, 5.0);
             if (t < least) least = t, best = {true, parts};
         }
-        if (static_cast<long>(large) * parts <= 4L * cus) {
+        if (both && static_cast<long>(large) * parts <= 4L * cus) {
             const double t = estimate(large, parts, 1.65, 9.0);
             if (t < least) least = t, best = {false, parts};
         }
@@ -70,11 +75,12 @@ static KSplit ksplit_rule(int NR, int NC, int K) {
     return best;
 }
 
-// D = (sum of the parts, in their order) * alpha (+ D), the expressions of the GEMM's own epilogue, one rounding.  Bound by
+// D = (sum of the parts, in their order) * alpha (+ bias) (+ D), the expressions of the GEMM's own epilogue, one rounding.  Bound by
 // the read of the parts; four elements a lane.
 template <typename OT>
 __global__ __launch_bounds__(256) void ksplit_finish_kernel(const float* __restrict__ part, OT* __restrict__ D, size_t n, int parts,
-                                                            const float* __restrict__ xs, const float* __restrict__ ys, int accumulate) {
+                                                            const float* __restrict__ xs, const float* __restrict__ ys, int accumulate,
+                                                            const void* __restrict__ bias, int bias_dt, unsigned cols) {
     const size_t i = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
     if (i >= n) return;    // (n is a multiple of 4)
     const float alpha = (*xs) * (*ys);
@@ -87,7 +93,17 @@ __global__ __launch_bounds__(256) void ksplit_finish_kernel(const float* __restr
     const float r[4] = {s.x, s.y, s.z, s.w};
     struct __attribute__((aligned(4 * sizeof(OT)))) Four { OT v[4]; };
     Four o;
-    if (accumulate) {
+    if (bias != nullptr) {    // (never with an old output: the callers see to that)
+        unsigned c = static_cast<unsigned>(i) % cols;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float b = bias_dt == MSAMP_DT_F32   ? static_cast<const float*>(bias)[c]
+                            : bias_dt == MSAMP_DT_F16 ? Elem<f16_t>::load(static_cast<const f16_t*>(bias) + c)
+                                                      : Elem<bf16_t>::load(static_cast<const bf16_t*>(bias) + c);
+            Elem<OT>::store(&o.v[e], fmaf(r[e], alpha, b));
+            c = c + 1 == cols ? 0 : c + 1;
+        }
+    } else if (accumulate) {
         const Four old = *reinterpret_cast<const Four*>(D + i);
 #pragma unroll
         for (int e = 0; e < 4; ++e) Elem<OT>::store(&o.v[e], fmaf(r[e], alpha, 0.0f) + Elem<OT>::load(&old.v[e]));
@@ -310,52 +326,51 @@ int msamp::gemm_kmajor(const uint8_t* a, int a_type, const float* a_scale_inv, c
     return dispatch_pair(b_type, a_type, c);
 }
 
-size_t msamp::gemm_ksplit_scratch(int m, int n, int k) {
-    const KSplit split = ksplit_rule(n, m, k);
-    return split.parts > 1 ? static_cast<size_t>(split.parts) * n * m : 0;
+size_t msamp::gemm_parts_scratch(int NR, int NC, int K, bool xt, bool yt) {
+    const KSplit split = ksplit_rule(NR, NC, K, xt, yt);
+    return split.parts > 1 ? static_cast<size_t>(split.parts) * NR * NC : 0;
+}
+
+int msamp::gemm_parts(int x_type, int y_type, const GemmCall& c, float* scratch, size_t n_floats) {
+    const KSplit split = ksplit_rule(c.NR, c.NC, c.K, c.xt, c.yt);
+    const size_t count = static_cast<size_t>(c.NR) * c.NC;
+    MSAMP_REQUIRE(split.parts > 1 && n_floats >= split.parts * count, MSAMP_ERR_SHAPE,
+                  "gemm_parts: m=%d n=%d k=%d is not split, or needs more scratch than %zu floats", c.NC, c.NR, c.K, n_floats);
+    MSAMP_REQUIRE(aligned(c.X, 16) && aligned(c.Y, 16) && aligned(c.D, 16) && aligned(scratch, 16), MSAMP_ERR_ALIGNMENT,
+                  "gemm_parts: operands, output and scratch must be 16-byte aligned");
+    GemmCall part = c;
+    part.D = scratch, part.d_dtype = MSAMP_DT_F32;
+    const int rc = dispatch_parts(x_type, y_type, part, split);
+    if (rc != MSAMP_OK) return rc;
+    const dim3 grid(static_cast<unsigned>((count / 4 + 255) / 256));
+#define FINISH(OT) \
+    hipLaunchKernelGGL((ksplit_finish_kernel<OT>), grid, dim3(256), 0, c.st, static_cast<const float*>(scratch), static_cast<OT*>(c.D), count, split.parts, c.xs, c.ys, c.accumulate, c.bias, c.bias_dt, static_cast<unsigned>(c.NC))
+    if (c.d_dtype == MSAMP_DT_F32) FINISH(float);
+    else if (c.d_dtype == MSAMP_DT_F16) FINISH(f16_t);
+    else FINISH(bf16_t);
+#undef FINISH
+    MSAMP_CHECK_LAUNCH("ksplit_finish_kernel");
+    return MSAMP_OK;
 }
 
 extern "C" int msamp_fp8_gemm_ksplit_scratch(int m, int n, int k, size_t* n_floats) {
     MSAMP_REQUIRE(m > 0 && n > 0 && k > 0, MSAMP_ERR_SHAPE, "msamp_fp8_gemm_ksplit_scratch: m=%d n=%d k=%d", m, n, k);
     MSAMP_REQUIRE(n_floats != nullptr, MSAMP_ERR_NULL, "msamp_fp8_gemm_ksplit_scratch: null pointer");
-    *n_floats = kmajor_shape_ok(n, m, k, true, true) ? gemm_ksplit_scratch(m, n, k) : 0;
+    *n_floats = kmajor_shape_ok(n, m, k, true, true) ? gemm_parts_scratch(n, m, k, true, true) : 0;
     return MSAMP_OK;
 }
 
 extern "C" int msamp_fp8_gemm_ksplit(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type,
                                      const float* b_scale_inv, void* d, int d_dtype, int m, int n, int k, int accumulate,
                                      float* scratch, size_t n_floats, msamp_stream_t stream) {
-    MSAMP_REQUIRE(m <= 0 || n <= 0 || k <= 0 || kmajor_shape_ok(n, m, k, true, true), MSAMP_ERR_SHAPE,
-                  "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d is not split", m, n, k);
-    return gemm_ksplit(a, a_type, a_scale_inv, b, b_type, b_scale_inv, d, d_dtype, m, n, k, accumulate, scratch, n_floats,
-                       static_cast<hipStream_t>(stream));
-}
-
-int msamp::gemm_ksplit(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv,
-                       void* d, int d_dtype, int m, int n, int k, int accumulate, float* scratch, size_t n_floats, hipStream_t st) {
     MSAMP_REQUIRE(is_fp8(a_type) && is_fp8(b_type), MSAMP_ERR_DTYPE, "msamp_fp8_gemm_ksplit: operand types %d, %d", a_type, b_type);
     MSAMP_REQUIRE(is_hp(d_dtype), MSAMP_ERR_DTYPE, "msamp_fp8_gemm_ksplit: output dtype %d", d_dtype);
-    MSAMP_REQUIRE(m > 0 && n > 0 && k > 0, MSAMP_ERR_SHAPE, "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d", m, n, k);
+    MSAMP_REQUIRE(m > 0 && n > 0 && k > 0 && kmajor_shape_ok(n, m, k, true, true), MSAMP_ERR_SHAPE,
+                  "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d", m, n, k);
     MSAMP_REQUIRE(a && b && d && a_scale_inv && b_scale_inv && scratch, MSAMP_ERR_NULL, "msamp_fp8_gemm_ksplit: null pointer");
-    MSAMP_REQUIRE(aligned(a, 16) && aligned(b, 16) && aligned(d, 16) && aligned(scratch, 16), MSAMP_ERR_ALIGNMENT,
-                  "msamp_fp8_gemm_ksplit: operands, output and scratch must be 16-byte aligned");
     // X = b (rows of D), Y = a (columns of D)
-    const KSplit split = ksplit_rule(n, m, k);
-    const size_t count = static_cast<size_t>(n) * m;
-    MSAMP_REQUIRE(split.parts > 1 && n_floats >= split.parts * count, MSAMP_ERR_SHAPE,
-                  "msamp_fp8_gemm_ksplit: m=%d n=%d k=%d is not split, or needs more scratch than %zu floats", m, n, k, n_floats);
-    const GemmCall c = {b, a, scratch, MSAMP_DT_F32, n, m, k, b_scale_inv, a_scale_inv, 0, nullptr, 0, true, true, nullptr, st};
-    const int rc = dispatch_parts(b_type, a_type, c, split);
-    if (rc != MSAMP_OK) return rc;
-    const dim3 grid(static_cast<unsigned>((count / 4 + 255) / 256));
-#define FINISH(OT) \
-    hipLaunchKernelGGL((ksplit_finish_kernel<OT>), grid, dim3(256), 0, st, static_cast<const float*>(scratch), static_cast<OT*>(d), count, split.parts, b_scale_inv, a_scale_inv, accumulate)
-    if (d_dtype == MSAMP_DT_F32) FINISH(float);
-    else if (d_dtype == MSAMP_DT_F16) FINISH(f16_t);
-    else FINISH(bf16_t);
-#undef FINISH
-    MSAMP_CHECK_LAUNCH("ksplit_finish_kernel");
-    return MSAMP_OK;
+    const GemmCall c = {b, a, d, d_dtype, n, m, k, b_scale_inv, a_scale_inv, accumulate, nullptr, 0, true, true, nullptr, static_cast<hipStream_t>(stream)};
+    return gemm_parts(b_type, a_type, c, scratch, n_floats);
 }
 
 extern "C" int msamp_fp8_gemm(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type,

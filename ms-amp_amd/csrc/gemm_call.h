@@ -65,7 +65,7 @@ struct KSplit {
     bool small_tiles;
     int parts;
 };
-// Both operands K-major; c.D is the float32 scratch of `parts` arrays that receives the parts' unscaled sums.
+// (Large tiles: both operands K-major.)  c.D is the float32 scratch of `parts` arrays that receives the parts' unscaled sums.
 template <int XF, int YF>
 int run_gemm_parts(const GemmCall& c, const KSplit& split);
 template <int XF, int YF>
@@ -95,12 +95,13 @@ inline bool takes_small_tiles(int NR, int NC, int K) {
 bool takes_paired_tiles(int NR, int NC, int K);
 
 // msamp_fp8_gemm_kmajor for any K (a single slice of it is left to the paired tiles) and any m and n, with the operands' k-rows
-// kmajor_pitch() apart; msamp_fp8_gemm_ksplit and its scratch (0: not split) the same way.
+// kmajor_pitch() apart.
 int gemm_kmajor(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv,
                 int b_kmajor, void* d, int d_dtype, int m, int n, int k, int accumulate, hipStream_t st);
-size_t gemm_ksplit_scratch(int m, int n, int k);
-int gemm_ksplit(const uint8_t* a, int a_type, const float* a_scale_inv, const uint8_t* b, int b_type, const float* b_scale_inv, void* d,
-                int d_dtype, int m, int n, int k, int accumulate, float* scratch, size_t n_floats, hipStream_t st);
+// A product in parts of K: the floats of scratch that it takes (0: it is better off whole), and the product (all operands and
+// c.D 16-byte aligned).
+size_t gemm_parts_scratch(int NR, int NC, int K, bool xt, bool yt);
+int gemm_parts(int x_type, int y_type, const GemmCall& c, float* scratch, size_t n_floats);
 
 // row offsets of the direct-to-LDS kernels are 32 bits
 inline bool fits_offsets(int NR, int NC, int K) {

@@ -426,19 +426,20 @@ __device__ __forceinline__ v4f acc_quad(uint32_t token) {
     return r;
 }
 
-// A product in gridDim.y parts of K (both operands K-major, so that a part is only another pointer and another K): this
-// workgroup's part.  Its unscaled float32 sum goes to the y-th of gridDim.y arrays of NR x NC; ksplit_finish_kernel adds
+// A product in gridDim.y parts of K: this workgroup's part, which is another pointer and another K (the rows of a row-major operand
+// stay as far apart as they are).  Its unscaled float32 sum goes to the y-th of gridDim.y arrays of NR x NC; ksplit_finish_kernel adds
 // them up.  Every part but the last is whole slices.
+// (large tiles; the 128 x 128 tiles take any operands)
 template <typename OT, bool XT, bool YT>
 constexpr bool kTakesKParts = XT && YT && std::is_same<OT, float>::value;
-template <typename In, typename Out>
+template <bool XT, bool YT, typename In, typename Out>
 __device__ __forceinline__ void k_part(In& X, In& Y, Out& D, int NR, int NC, int& K) {
     if (gridDim.y == 1) return;
     const int nk = (K + kBK - 1) / kBK, parts = gridDim.y, y = blockIdx.y;
     const int first = static_cast<int>(static_cast<long long>(nk) * y / parts) * kBK;
     const int end = y + 1 == parts ? K : static_cast<int>(static_cast<long long>(nk) * (y + 1) / parts) * kBK;
-    X += static_cast<size_t>(first) * kmajor_pitch(NR);
-    Y += static_cast<size_t>(first) * kmajor_pitch(NC);
+    X += XT ? static_cast<size_t>(first) * kmajor_pitch(NR) : first;
+    Y += YT ? static_cast<size_t>(first) * kmajor_pitch(NC) : first;
     D += static_cast<size_t>(y) * NR * NC;
     K = end - first;
 }
@@ -453,7 +454,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                                                                      const void* __restrict__ bias, int bias_dt,
                                                                      QuantArgs qa) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    if constexpr (KTAIL && kTakesKParts<OT, XT, YT>) k_part(X, Y, D, NR, NC, K);
+    if constexpr (KTAIL && kTakesKParts<OT, XT, YT>) k_part<XT, YT>(X, Y, D, NR, NC, K);
     const int tiles_r = (NR + kDmaTile - 1) / kDmaTile, tiles_c = (NC + kDmaTile - 1) / kDmaTile;
     bool by_columns = walk_by_columns(tiles_r, tiles_c, K);
     int tr, tc;
@@ -1458,8 +1459,12 @@ int run_gemm_pair128(const GemmCall& c) {
 }
 template <int XF, int YF>
 int run_gemm_parts(const GemmCall& c, const KSplit& split) {
-    if (split.small_tiles)
-        return launch_gemm_dma128_tail<XF, YF, float, true, true, true>(c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, 0, nullptr, 0, c.st, split.parts);
+#define MSAMP_PARTS_LAUNCH(XT, YT) \
+    return launch_gemm_dma128_tail<XF, YF, float, XT, YT, true>(c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, 0, nullptr, 0, c.st, split.parts)
+    if (!c.yt) MSAMP_PARTS_LAUNCH(false, false);
+    if (!c.xt) MSAMP_PARTS_LAUNCH(false, true);
+    if (split.small_tiles) MSAMP_PARTS_LAUNCH(true, true);
+#undef MSAMP_PARTS_LAUNCH
     return launch_gemm_dma_parity<XF, YF, float, true, true, false, true>(c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, 0, nullptr, 0, c.st, split.parts);
 }
 #endif

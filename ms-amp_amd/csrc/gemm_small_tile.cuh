@@ -86,8 +86,9 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
                                             const float* __restrict__ y_scale_inv, int accumulate, const void* __restrict__ bias,
                                             int bias_dt) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    constexpr bool kParts = KTAIL && !PAIR && kTakesKParts<OT, XT, YT>;
-    if constexpr (kParts) k_part(X, Y, D, NR, NC, K);
+    constexpr bool kParts = KTAIL && !PAIR && std::is_same<OT, float>::value;
+    const int ldk = K;    // from one row of a row-major operand to the next
+    if constexpr (kParts) k_part<XT, YT>(X, Y, D, NR, NC, K);
     const int tiles_r = (NR + kSmallTile - 1) / kSmallTile, tiles_c = (NC + kSmallTile - 1) / kSmallTile;
     int tr, tc;
     tile_of_id(blockIdx.x, tiles_r, tiles_c, false, false, tr, tc);
@@ -134,9 +135,9 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
         gy = gy < NC ? gy : NC - 1;
         const int krow = (i * 4 + wave) * 8 + (lane >> 3);
         xoff[i] = XT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(ldx) + xcol
-                     : static_cast<uint32_t>(gx) * static_cast<uint32_t>(K) + chunk * 16;
+                     : static_cast<uint32_t>(gx) * static_cast<uint32_t>(ldk) + chunk * 16;
         yoff[i] = YT ? static_cast<uint32_t>(krow) * static_cast<uint32_t>(ldy) + ycol
-                     : static_cast<uint32_t>(gy) * static_cast<uint32_t>(K) + chunk * 16;
+                     : static_cast<uint32_t>(gy) * static_cast<uint32_t>(ldk) + chunk * 16;
     }
     // KTAIL: a ragged last slice of `rem` K bytes, handled as in the large tile (loads kept inside the operand, fragments
     // masked)

@@ -178,12 +178,12 @@ static int few_tokens(const msamp_linear_forward_args& a, hipStream_t st) {
 
 static size_t round_up(size_t n) { return (n + 255) / 256 * 256; }
 
-// where a backward call's parts of its scratch begin
+// where a backward call's parts of its scratch begin (the two products take the same room for parts of K one after the other)
 struct BackwardScratch {
-    size_t sums, parts, n_parts, end;
+    size_t sums, parts, n_dx_parts, n_parts, end;
 };
 
-static int backward_scratch(int tokens, int d_in, int d_out, int dy_dtype, int out_dtype, bool wgrad, bool bias, BackwardScratch* s) {
+static int backward_scratch(int tokens, int d_in, int d_out, int dy_dtype, int out_dtype, bool dx, bool wgrad, bool bias, BackwardScratch* s) {
     s->sums = wgrad ? round_up(static_cast<size_t>(d_out) * d_in * hp_size(out_dtype)) : 0;    // (the product comes first)
     size_t words = 0;
     if (bias) {
@@ -191,8 +191,9 @@ static int backward_scratch(int tokens, int d_in, int d_out, int dy_dtype, int o
         if (rc != MSAMP_OK) return rc;
     }
     s->parts = s->sums + round_up(words * sizeof(float));
-    s->n_parts = wgrad ? gemm_ksplit_scratch(d_in, d_out, tokens) : 0;
-    s->end = s->parts + s->n_parts * sizeof(float);
+    s->n_dx_parts = dx ? gemm_parts_scratch(tokens, d_in, kmajor_pitch(d_out), false, true) : 0;
+    s->n_parts = wgrad ? gemm_parts_scratch(d_out, d_in, tokens, true, true) : 0;
+    s->end = s->parts + std::max(s->n_dx_parts, s->n_parts) * sizeof(float);
     return MSAMP_OK;
 }
 
@@ -229,18 +230,33 @@ extern "C" int msamp_linear_forward(const msamp_linear_forward_args* a, msamp_st
     }
     const int rc = cast_linear_inputs(*a, static_cast<hipStream_t>(stream));
     if (rc != MSAMP_OK) return rc;
-    return msamp_fp8_gemm(a->w_codes, MSAMP_DT_E4M3, a->w_meta + 1, a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, a->y, y_dtype,
-                          static_cast<int>(a->d_out), static_cast<int>(a->tokens), kmajor_pitch(static_cast<int>(a->d_in)), 0, a->bias,
-                          static_cast<int>(a->bias_dtype), stream);
+    const int tokens = static_cast<int>(a->tokens), d_out = static_cast<int>(a->d_out), K = kmajor_pitch(static_cast<int>(a->d_in));
+    const int bias_dtype = static_cast<int>(a->bias_dtype);
+    const size_t n_parts = a->scratch_bytes > 0 ? gemm_parts_scratch(tokens, d_out, K, false, false) : 0;
+    if (n_parts == 0 || static_cast<size_t>(a->scratch_bytes) < n_parts * sizeof(float) || !a->scratch || !is_hp(y_dtype) ||
+        (a->bias && !is_hp(bias_dtype)) || !aligned(a->y, 16) || !aligned(a->w_codes, 16) || !aligned(a->x_codes, 16))
+        return msamp_fp8_gemm(a->w_codes, MSAMP_DT_E4M3, a->w_meta + 1, a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, a->y, y_dtype, d_out,
+                              tokens, K, 0, a->bias, bias_dtype, stream);
+    MSAMP_REQUIRE(a->y, MSAMP_ERR_NULL, "msamp_linear_forward: null pointer");
+    const GemmCall c = {a->x_codes, a->w_codes, a->y, y_dtype, tokens, d_out, K, a->x_scale_inv, a->w_meta + 1, 0, a->bias, bias_dtype,
+                        false, false, nullptr, static_cast<hipStream_t>(stream)};
+    return gemm_parts(MSAMP_DT_E4M3, MSAMP_DT_E4M3, c, static_cast<float*>(a->scratch), n_parts);
 }
 
-extern "C" int msamp_linear_backward_scratch(int tokens, int d_in, int d_out, int dy_dtype, int out_dtype, int want_wgrad, int want_bias,
-                                             size_t* bytes, size_t* least) {
+extern "C" int msamp_linear_forward_scratch(int tokens, int d_in, int d_out, size_t* bytes) {
+    MSAMP_REQUIRE(dims_ok(tokens, d_in, d_out), MSAMP_ERR_SHAPE, "msamp_linear_forward_scratch: %d x %d -> %d", tokens, d_in, d_out);
+    MSAMP_REQUIRE(bytes != nullptr, MSAMP_ERR_NULL, "msamp_linear_forward_scratch: null pointer");
+    *bytes = gemm_parts_scratch(tokens, d_out, kmajor_pitch(d_in), false, false) * sizeof(float);
+    return MSAMP_OK;
+}
+
+extern "C" int msamp_linear_backward_scratch(int tokens, int d_in, int d_out, int dy_dtype, int out_dtype, int want_dx, int want_wgrad,
+                                             int want_bias, size_t* bytes, size_t* least) {
     MSAMP_REQUIRE(dims_ok(tokens, d_in, d_out), MSAMP_ERR_SHAPE, "msamp_linear_backward_scratch: %d x %d -> %d", tokens, d_in, d_out);
     MSAMP_REQUIRE(is_hp(dy_dtype) && is_hp(out_dtype), MSAMP_ERR_DTYPE, "msamp_linear_backward_scratch: dtypes %d, %d", dy_dtype, out_dtype);
     MSAMP_REQUIRE(bytes && least, MSAMP_ERR_NULL, "msamp_linear_backward_scratch: null pointer");
     BackwardScratch s;
-    const int rc = backward_scratch(tokens, d_in, d_out, dy_dtype, out_dtype, want_wgrad != 0, want_bias != 0, &s);
+    const int rc = backward_scratch(tokens, d_in, d_out, dy_dtype, out_dtype, want_dx != 0, want_wgrad != 0, want_bias != 0, &s);
     if (rc != MSAMP_OK) return rc;
     *bytes = s.end, *least = s.parts;
     return MSAMP_OK;
@@ -255,7 +271,7 @@ extern "C" int msamp_linear_backward(const msamp_linear_backward_args* a, msamp_
     MSAMP_REQUIRE(is_hp(dy_dtype) && is_hp(out_dtype), MSAMP_ERR_DTYPE, "msamp_linear_backward: dtypes %d, %d", dy_dtype, out_dtype);
     const bool wgrad = a->wq != nullptr, bias = a->bias_sum != nullptr, accumulate = a->old_codes != nullptr;
     BackwardScratch s;
-    int rc = backward_scratch(tokens, d_in, d_out, dy_dtype, out_dtype, wgrad, bias, &s);
+    int rc = backward_scratch(tokens, d_in, d_out, dy_dtype, out_dtype, a->dx != nullptr, wgrad, bias, &s);
     if (rc != MSAMP_OK) return rc;
     MSAMP_REQUIRE(s.parts == 0 || (a->scratch && aligned(a->scratch, 16) && a->scratch_bytes >= static_cast<int64_t>(s.parts)),
                   MSAMP_ERR_WORKSPACE, "msamp_linear_backward: scratch of %lld bytes", static_cast<long long>(a->scratch_bytes));
@@ -264,16 +280,27 @@ extern "C" int msamp_linear_backward(const msamp_linear_backward_args* a, msamp_
     uint8_t* product = static_cast<uint8_t*>(a->scratch);
     rc = cast_output_gradient(*a, product, reinterpret_cast<float*>(product + s.sums), st);
     if (rc != MSAMP_OK) return rc;
+    // (the scratch may be without the room for parts of K)
+    const bool room = a->scratch != nullptr && a->scratch_bytes >= static_cast<int64_t>(s.end);
+    float* parts = reinterpret_cast<float*>(product + s.parts);
     if (a->dx != nullptr) {
-        rc = gemm_kmajor(a->w_codes, MSAMP_DT_E4M3, a->w_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, 0, a->dx, out_dtype, d_in, tokens,
-                         kmajor_pitch(d_out), 0, st);
+        const int K = kmajor_pitch(d_out);
+        if (s.n_dx_parts != 0 && room && a->w_codes && a->w_scale_inv && aligned(a->dx, 16)) {
+            const GemmCall c = {codes, a->w_codes, a->dx, out_dtype, tokens, d_in, K, a->g_scale_inv, a->w_scale_inv, 0, nullptr, MSAMP_DT_F32,
+                                false, true, nullptr, st};
+            rc = gemm_parts(MSAMP_DT_E5M2, MSAMP_DT_E4M3, c, parts, s.n_dx_parts);
+        } else {
+            rc = gemm_kmajor(a->w_codes, MSAMP_DT_E4M3, a->w_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, 0, a->dx, out_dtype, d_in,
+                             tokens, K, 0, st);
+        }
         if (rc != MSAMP_OK) return rc;
     }
     if (!wgrad) return MSAMP_OK;
     const size_t n = static_cast<size_t>(d_out) * d_in;
-    if (s.n_parts != 0 && a->scratch_bytes >= static_cast<int64_t>(s.end)) {
-        rc = gemm_ksplit(a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, product, out_dtype, d_in, d_out,
-                         tokens, accumulate, reinterpret_cast<float*>(product + s.parts), s.n_parts, st);
+    if (s.n_parts != 0 && room && a->x_codes && a->x_scale_inv) {
+        const GemmCall c = {codes, a->x_codes, product, out_dtype, d_out, d_in, tokens, a->g_scale_inv, a->x_scale_inv, accumulate, nullptr,
+                            MSAMP_DT_F32, true, true, nullptr, st};
+        rc = gemm_parts(MSAMP_DT_E5M2, MSAMP_DT_E4M3, c, parts, s.n_parts);
     } else {
         rc = gemm_kmajor(a->x_codes, MSAMP_DT_E4M3, a->x_scale_inv, codes, MSAMP_DT_E5M2, a->g_scale_inv, 1, product, out_dtype, d_in, d_out,
                          tokens, accumulate, st);

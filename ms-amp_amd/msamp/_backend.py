@@ -8,6 +8,7 @@ the GPU, the call raises.
 
 import array
 import ctypes
+import functools
 import os
 import struct
 
@@ -60,7 +61,8 @@ _SIGNATURES = {
     'msamp_fp8_gemm_ksplit': ([_vp, _i, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp, _sz, _vp], _i),
     'msamp_fp8_gemm_cast': ([_vp, _i, _vp, _i, _vp, _i, _vp, _i, _vp, _i, _i, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp], _i),
     'msamp_linear_forward': ([ctypes.c_char_p, _vp], _i),
-    'msamp_linear_backward_scratch': ([_i, _i, _i, _i, _i, _i, _i, _vp, _vp], _i),
+    'msamp_linear_forward_scratch': ([_i, _i, _i, _vp], _i),
+    'msamp_linear_backward_scratch': ([_i, _i, _i, _i, _i, _i, _i, _i, _vp, _vp], _i),
     'msamp_linear_backward': ([ctypes.c_char_p, _vp], _i),
     'msamp_mfma_probe': ([_vp, _vp, _i, _i, _i, _vp, _vp], _i),
     'msamp_set_small_tile_limit': ([_i], None),
@@ -709,7 +711,7 @@ def fp8_gemm_cast(a, a_dt, a_scale_inv, b, b_dt, b_scale_inv, hp_dtype, q_dt, sc
 
 
 # ---- a linear layer's directions, one call each -----------------------------------------------------------------
-_LINEAR_FORWARD = struct.Struct('@24q')     # msamp_linear_forward_args
+_LINEAR_FORWARD = struct.Struct('@26q')     # msamp_linear_forward_args
 _LINEAR_BACKWARD = struct.Struct('@30q')    # msamp_linear_backward_args
 
 
@@ -750,6 +752,14 @@ def linear_fits(tokens, d_in, d_out):
 FEW_TOKENS = 64    # MSAMP_FEW_TOKENS
 
 
+@functools.lru_cache(maxsize=4096)
+def _linear_forward_scratch(tokens, d_in, d_out, device_index):
+    """Bytes of scratch with which a forward product is taken in parts of K (0: it is not)."""
+    sizes = _TwoSizes()
+    _check(load().msamp_linear_forward_scratch(tokens, d_in, d_out, ctypes.addressof(sizes)), 'msamp_linear_forward_scratch')
+    return sizes[0]
+
+
 def linear_forward(x, x_meta, w, w_meta, out_dtype, bias, want_codes=True):
     """y = x . w^T (+ bias) through msamp_linear_forward.  x: contiguous [tokens, d_in], cast with x_meta (gated scaling); w: the
     contiguous scaled payload [d_out, d_in] of a weight with w_meta.  Returns y and, if want_codes, the E4M3 codes of x
@@ -757,7 +767,14 @@ def linear_forward(x, x_meta, w, w_meta, out_dtype, bias, want_codes=True):
     count, amax window} of the codes of w (else these are not to be used)."""
     lib = load()
     (tokens, d_in), d_out, device, window = x.shape, w.shape[0], x.device, w_meta.window_size
+    scratch, size = None, 0
     if want_codes or tokens > FEW_TOKENS or w.data_ptr() % 16 or d_in % 16:
+        size = _linear_forward_scratch(tokens, d_in, d_out, device.index)
+        if size:
+            try:
+                scratch = torch.empty((size, ), dtype=torch.uint8, device=device)
+            except torch.OutOfMemoryError:    # the product is taken whole
+                size = 0
         pitch = linear_pitch(d_in)
         x_codes = torch.empty((tokens, pitch), dtype=torch.uint8, device=device)
         w_codes = torch.empty((linear_pitch(d_out), pitch), dtype=torch.uint8, device=device)
@@ -771,7 +788,8 @@ def linear_forward(x, x_meta, w, w_meta, out_dtype, bias, want_codes=True):
         x_meta.scale_inv.data_ptr(), x_meta.amax_counter.data_ptr(), x_meta.window_size, x_codes.data_ptr(), w.data_ptr(),
         _TORCH_TO_DT[w.dtype], w_meta.amax.data_ptr(), w_meta.scale_inv.data_ptr(), window,
         0 if w_codes is None else w_codes.data_ptr(), 0 if words is None else words.data_ptr(), y.data_ptr(), _TORCH_TO_DT[out_dtype], 0 if bias is None else bias.data_ptr(),
-        DT_F32 if bias is None else _TORCH_TO_DT[bias.dtype], FLAG_TWO_PASS if _two_pass_only() else 0, workspace(device).data_ptr()
+        DT_F32 if bias is None else _TORCH_TO_DT[bias.dtype], FLAG_TWO_PASS if _two_pass_only() else 0, workspace(device).data_ptr(),
+        0 if scratch is None else scratch.data_ptr(), size
     )
     _check(lib.msamp_linear_forward(args, _stream()), 'msamp_linear_forward')
     return y, x_codes, w_codes, words
@@ -789,11 +807,11 @@ def linear_backward(dy, d_in, g_meta, x_codes, x_scale_inv, w_codes, w_scale_inv
     wq = torch.empty((d_out, d_in), dtype=torch.uint8, device=device) if q_meta is not None else None
     sums = torch.empty((d_out, ), dtype=bias_dtype, device=device) if bias_dtype is not None else None
     scratch, size = None, 0
-    if wq is not None or sums is not None:
+    if wq is not None or sums is not None or dx is not None:
         sizes = _TwoSizes()
         where = ctypes.addressof(sizes)
-        _check(lib.msamp_linear_backward_scratch(tokens, d_in, d_out, dt, out_dt, wq is not None, sums is not None, where, where + 8),
-               'msamp_linear_backward_scratch')
+        _check(lib.msamp_linear_backward_scratch(tokens, d_in, d_out, dt, out_dt, dx is not None, wq is not None, sums is not None, where,
+                                                 where + 8), 'msamp_linear_backward_scratch')
         size, least = sizes
         try:
             scratch = torch.empty((size, ), dtype=torch.uint8, device=device)

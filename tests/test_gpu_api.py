@@ -1123,6 +1123,47 @@ def test_a_few_tokens_without_gradients_lose_no_precision():
         assert rel_fro(few.double(), exact) <= 1.1 * rel_fro(y.double(), exact) + 1e-7
 
 
+@pytest.mark.parametrize('tokens,d_in,d_out', [(65, 2064, 132), (300, 8200, 70), (129, 272, 2500), (70, 4096, 4111)])
+@pytest.mark.parametrize('dtype,bias', [(torch.bfloat16, True), (torch.float16, False), (torch.float32, True)])
+def test_products_of_a_few_tiles_in_parts_of_k(monkeypatch, tokens, d_in, d_out, dtype, bias):
+    """A forward product or an input gradient with a long K, over whole numbers up to 2, whose products sum exactly in any order
+    (4 * 8200 < 2**24): the bits of the products taken whole, as they are where there is no memory for the parts."""
+    from msamp import _backend
+    gen = torch.Generator(device='cuda').manual_seed(tokens + d_in + d_out)
+    whole = lambda *shape: torch.randint(-2, 3, shape, device='cuda', generator=gen).to(dtype)
+    w, b, x, dy = whole(d_out, d_in), whole(d_out), whole(tokens, d_in), whole(tokens, d_out)
+    sizes, empty = [], torch.empty
+
+    def run(limit):
+        def scarce(*a, **k):
+            n = a[0][0] if isinstance(a[0], tuple) and len(a[0]) == 1 and k.get('dtype') == torch.uint8 else 0
+            sizes.append(n)
+            if n > limit:
+                raise torch.OutOfMemoryError
+            return empty(*a, **k)
+
+        model_state.clear()
+        lin = torch.nn.Linear(d_in, d_out, bias=bias).cuda().to(dtype)
+        with torch.no_grad():
+            lin.weight.copy_(w)
+            if bias:
+                lin.bias.copy_(b)
+        model = LinearReplacer.replace(lin, Dtypes.kfloat16)
+        xs = x.clone().requires_grad_(True)
+        model.weight.requires_grad = False
+        monkeypatch.setattr(torch, 'empty', scarce)
+        y = model(xs)
+        y.backward(dy)
+        monkeypatch.undo()
+        return y.detach(), xs.grad
+
+    parts = run(1 << 60)
+    most = max(sizes)
+    assert most >= 2 * 4 * tokens * min(d_in, d_out)    # the room for at least two parts was asked for
+    one = run(most - 1)
+    assert all(torch.equal(a, c) for a, c in zip(parts, one))
+
+
 def test_zero_grad_of_a_mixed_list():
     """Gradients of several types, strides and layouts, ScalingTensors, shared memory, a missing and an empty one."""
     dense = lambda *shape, dtype=torch.float32: torch.nn.Parameter(torch.ones(shape, device='cuda', dtype=dtype))
