@@ -1002,7 +1002,7 @@ def test_scratch_that_cannot_be_had_costs_launches_only(monkeypatch):
 @pytest.mark.parametrize('tokens,d_in,d_out', [(256, 512, 768), (2048, 256, 512), (300, 272, 144), (129, 16, 16), (96, 128, 512),
                                                (200, 40, 24), (2500, 512, 512), (16, 64, 48), (128, 256, 256),
                                                (300, 272, 112), (1, 16, 16), (17, 1, 1), (33, 3, 70), (130, 1001, 305), (301, 130, 384),
-                                               (129, 304, 17), (2500, 500, 513)])
+                                               (129, 304, 17), (2500, 500, 513), (8192, 4100, 512), (512, 4100, 8208)])
 @pytest.mark.parametrize('dtype,bias_dtype', [(torch.bfloat16, None), (torch.float16, torch.float16), (torch.float32, torch.float32),
                                               (torch.bfloat16, torch.float32)])
 def test_a_linear_layer_by_one_call_each_way_has_the_bits_of_the_single_calls(monkeypatch, tokens, d_in, d_out, dtype, bias_dtype):
@@ -1010,13 +1010,14 @@ def test_a_linear_layer_by_one_call_each_way_has_the_bits_of_the_single_calls(mo
     the same layer with every entry point called from Python.  Where a product has a single slice of K, or a width is no multiple
     of 16, the single calls go over transposed copies and take the bias gradient from a sum of its own: two float32 sums of
     `tokens` numbers each, apart by their roundings (2 * tokens * 2^-24 of the numbers' sum) and the type's.  They never take a
-    weight gradient of such a width in parts of K: the long one is of whole numbers, whose products sum exactly in any order."""
+    product of such a width in parts of K: the long ones are of whole numbers, whose products sum exactly in any order.  (The
+    last two have a gradient of so many tiles that its walks would be timed, were its rows not padded.)"""
     from msamp import _backend
     from msamp.nn import functional
     gen = torch.Generator(device='cuda').manual_seed(tokens + d_in)
     draw = lambda *shape: torch.randn(shape, device='cuda', generator=gen)
     ragged = d_in % 16 != 0 or d_out % 16 != 0
-    if ragged and tokens == 2500:
+    if ragged and tokens in (512, 2500, 8192):
         draw = lambda *shape: torch.randint(-2, 3, shape, device='cuda', generator=gen).float()
     w0, b0 = draw(d_out, d_in) * 0.05, draw(d_out)
     xs = [draw(tokens, d_in).to(dtype) * f for f in (1.0, 3.0, 0.2)]

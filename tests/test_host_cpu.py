@@ -7,6 +7,7 @@ import json
 import os
 import random
 import re
+import types
 
 import pytest
 import torch
@@ -464,3 +465,28 @@ def test_argument_blocks_of_the_linear_calls_have_the_fields_of_the_header(name)
     fields = sum(len(m.split(',')) for m in members)
     packer = _backend._LINEAR_FORWARD if name == 'forward' else _backend._LINEAR_BACKWARD
     assert packer.size == 8 * fields
+
+
+@pytest.mark.parametrize('tokens,d_in,d_out', [(8192, 4096, 50257), (8192, 4100, 4096), (4096, 11007, 4096), (16384, 9001, 4096), (8192, 768, 50257)])
+def test_a_layer_of_a_ragged_width_does_not_wait_for_walks_that_nobody_times(monkeypatch, tokens, d_in, d_out):
+    """After a pass over single calls, which times row-major products of transposed copies only, the gradients of a layer whose
+    width is no multiple of 16 go by the one call; those of one whose widths are, once its own products have been timed."""
+    from msamp.nn import functional
+    monkeypatch.setattr(_backend, '_tune_walks', True)
+    seen = {(d_out, tokens, _backend.linear_pitch(d_in), False, False), (d_in, tokens, _backend.linear_pitch(d_out), False, False),
+            (d_in, d_out, tokens, False, False)}
+    monkeypatch.setattr(_backend, '_walk_seen', seen)
+    scale = types.SimpleNamespace(is_cuda=True)
+    metas = {'ograd': types.SimpleNamespace(scaling_mode=lambda: 'gated', qtype=Dtypes.kfloat8_e5m2, scale=scale),
+             'wgrad': types.SimpleNamespace(scaling_mode=lambda: 'in_time', qtype=Dtypes.kfloat8_e4m3)}
+
+    def goes_by_one_call(d_in, d_out):
+        dy = torch.empty(tokens, d_out, dtype=torch.bfloat16, device='meta')
+        ctx = types.SimpleNamespace(metas=metas, output_dtype=torch.bfloat16, input_codes=dy, weight=types.SimpleNamespace(grad=None))
+        with torch.no_grad():
+            return functional._backward_in_one_call(ctx, dy, d_in, True), functional._wgrad_in_one_call(ctx, tokens, d_in, d_out)
+
+    assert goes_by_one_call(d_in, d_out) == (True, True)
+    assert not goes_by_one_call(11008, 4096)[0]
+    seen.add((11008, tokens, 4096, True, False))
+    assert goes_by_one_call(11008, 4096)[0]
