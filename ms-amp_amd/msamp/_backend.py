@@ -839,6 +839,7 @@ def set_small_tile_limit(big_tiles):
     global _small_tile_limit
     _small_tile_limit = int(big_tiles)
     load().msamp_set_small_tile_limit(int(big_tiles))
+    _linear_forward_scratch.cache_clear()    # (which products are taken in parts of K depends on the limit)
 
 
 def mfma_probe(seed, sink, iters, workgroups, distinct_operands=False):

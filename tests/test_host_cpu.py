@@ -490,3 +490,24 @@ def test_a_layer_of_a_ragged_width_does_not_wait_for_walks_that_nobody_times(mon
     assert not goes_by_one_call(11008, 4096)[0]
     seen.add((11008, tokens, 4096, True, False))
     assert goes_by_one_call(11008, 4096)[0]
+
+
+def test_the_room_for_parts_of_k_is_asked_for_again_once_the_tile_limit_has_changed(monkeypatch):
+    class Library:
+        limit = 128
+
+        def msamp_set_small_tile_limit(self, limit):
+            self.limit = limit
+
+        def msamp_linear_forward_scratch(self, tokens, d_in, d_out, where):
+            ctypes.c_size_t.from_address(where).value = 4 * tokens * d_out if self.limit else 0
+            return 0
+
+    library = Library()
+    monkeypatch.setattr(_backend, 'load', lambda: library)
+    try:
+        for limit in (128, 0, 128):
+            _backend.set_small_tile_limit(limit)
+            assert _backend._linear_forward_scratch(300, 8192, 64, 0) == (4 * 300 * 64 if limit else 0)
+    finally:
+        _backend.set_small_tile_limit(128)
