@@ -2219,7 +2219,9 @@ __global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __rest
         if ((fin.flags & MSAMP_FLAG_NAN_TO_INF) && !(a < __uint_as_float(0x7f800000u))) a = __uint_as_float(0x7f800000u);
         s = scale_rule(a, s, fin.fp_max, fin.margin);
         if (threadIdx.x == 0) {
-            const uint32_t ticket = __hip_atomic_fetch_add(ws + kWsTicket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // (release: this workgroup has read the old scale; acquire: so has every other before the last one writes the new.
+            // Nothing has been written yet that a release would have to carry out of the L2)
+            const uint32_t ticket = __hip_atomic_fetch_add(ws + kWsTicket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
             if (ticket == gridDim.x - 1) {
                 ws[kWsTicket] = 0;    // ready for the next call
                 *fin.amax = a;

@@ -347,6 +347,32 @@ def test_paired_gemm_kernels_leave_their_accumulators_to_the_matrix_instructions
     assert len(products) == 18 and min(products.values()) >= 16    # three output types, three layouts, whole and ragged K
 
 
+def test_the_last_workgroup_of_a_few_tokens_cast_writes_the_meta_behind_every_read_of_it(tmp_path):
+    """few_cast_kernel: every workgroup reads the old scale and draws a ticket, and the last one overwrites the scale.  The ticket
+    has to release the read and acquire the others' (at agent scope: buffer_wbl2 ahead of it, buffer_inv behind it)."""
+    import shutil
+    import subprocess
+    hipcc = shutil.which('hipcc') or '/opt/rocm/bin/hipcc'
+    if not os.path.exists(hipcc):
+        pytest.skip('no hipcc here')
+    src = os.path.join(os.path.dirname(_backend.__file__), '..', 'csrc')
+    out = str(tmp_path / 'cast.s')
+    subprocess.run([hipcc, '--offload-arch=gfx950', '-O3', '-std=c++17', '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
+                    '-Wno-unused-command-line-argument', '--cuda-device-only', '-S', '-o', out, os.path.join(src, 'cast.hip')],
+                   cwd=src, check=True, capture_output=True)
+    kernel, code = None, {}
+    for line in open(out):
+        m = re.match(r'^(_Z\w+):', line)
+        kernel = m.group(1) if m else kernel
+        op = line.split(';')[0].split()
+        if not m and kernel and 'few_cast_kernel' in kernel and op and not op[0].startswith('.'):
+            code.setdefault(kernel, []).append(op[0])
+    assert len(code) == 3    # float32, float16, bfloat16
+    for ops in code.values():
+        tickets = [i for i, op in enumerate(ops) if op == 'global_atomic_add']
+        assert tickets and all('buffer_wbl2' in ops[i - 2:i] and 'buffer_inv' in ops[i + 1:i + 4] for i in tickets)
+
+
 def test_entry_points_refuse_bad_arguments_before_touching_a_gpu():
     """Argument checks of the entry points run on the host before any HIP call: what they refuse, and the walk registry
     (host data only), can be tried without a GPU."""
