@@ -321,7 +321,8 @@ def test_direct_to_lds_gemm_kernels_leave_the_accumulator_registers_alone(gemm_a
 def test_paired_gemm_kernels_leave_their_accumulators_to_the_matrix_instructions(gemm_assembly, pair):
     """The accumulators of fp8_gemm_pair128_kernel are v192 and up, behind the compiler's back: outside the inline assembly
     nothing may name those registers, and no vector instruction may write an operand of an MFMA less than two instructions
-    ahead of it (the compiler, which would wait, does not know the MFMA for one)."""
+    ahead of it (the compiler, which would wait, does not know the MFMA for one).  Nothing is spilled either: a reload waits for
+    the tile loads in flight, and the counted waits for those would count it."""
     registers = lambda text: {n for m in re.finditer(r'\bv(\d+)\b|\bv\[(\d+):(\d+)\]', text)
                               for n in ([int(m.group(1))] if m.group(1) else range(int(m.group(2)), int(m.group(3)) + 1))}
     kernel, in_asm, products, recent = None, False, {}, []
@@ -339,6 +340,7 @@ def test_paired_gemm_kernels_leave_their_accumulators_to_the_matrix_instructions
         if not in_asm:
             assert max(registers(code), default=0) < 192, (kernel, code)
         op, args = code.split()[0], code[len(code.split()[0]):].split(',')
+        assert not op.startswith('scratch_'), (kernel, code)
         if op.startswith('v_mfma'):
             products[kernel] = products.get(kernel, 0) + 1
             assert not (registers(args[1]) | registers(args[2])) & set().union(*recent[-2:]), (kernel, code)
