@@ -1057,3 +1057,16 @@ def test_paired_tiles_agree_with_the_other_kernels_to_the_bit(be, m, n, k, out_d
                     be.set_small_tile_limit(128)
                 view = torch.int32 if out_dtype == torch.float32 else torch.int16
                 assert torch.equal(outs[0].view(view), outs[1].view(view)), (a_dt, b_dt, a_k, b_k, list(extra))
+
+
+@pytest.mark.parametrize('m,n,k', [(256, 256, 128), (256, 256, 256), (256, 256, 384), (256, 256, 512), (2048, 2048, 384), (2048, 2048, 512),
+                                   (3328, 1280, 512), (3328, 1280, 2944), (3328, 1280, 3072), (4096, 2048, 2944), (4096, 2048, 3072),
+                                   (11008, 768, 3072), (11008, 768, 512), (264, 256, 512), (256, 272, 512), (3328, 1280, 528)])
+def test_what_the_layer_expects_of_the_product_with_its_cast_is_what_the_library_answers(be, m, n, k):
+    """gemm_cast_declines, on both sides of each line of the library's rule (64 and 65, 128 and 129 large tiles, K of 384 / 512, 2944
+    / 3072, sizes that are no whole tiles): a weight gradient goes by the call for the direction only if fp8_gemm_cast would not
+    take it."""
+    a, b = _gpu_codes((k, m), 5, m), _gpu_codes((k, n), 6, n)
+    one, s, si, am = (torch.ones((), device='cuda') for _ in range(4))
+    got = be.fp8_gemm_cast(a, 5, one, b, 6, one, torch.bfloat16, 5, s, am.reshape(1), si, a_kmajor=True, b_kmajor=True)
+    assert (got is None) == be.gemm_cast_declines(m, n, k)
