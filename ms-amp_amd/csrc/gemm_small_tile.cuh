@@ -305,10 +305,11 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
         }
         // four or five slices are left, or there are three or fewer in all
         if constexpr (KTAIL) {
-            // These ways to the end come out one behind the other, each tested for, and what the later ones would start from stayed
-            // in its registers through the earlier ones, where nine others spilled.  Here it is given up at the end of each.
-            // Row-major, one operand K-major, both, us: 2048 x 2048 x 400 7.14, 6.29, 6.95 -> 6.4, 6.3, 6.4; 4096 x 2048 x 1008
-            // 15.4, 13.1, 13.1 -> 14.5, 13.2, 12.1.  (Whole slices spill nothing and are 1 % faster without.)
+            // These ways to the end come out one behind the other, each tested for, and what the others would start from stayed in
+            // its registers through the way of four slices, where nine others spilled.  Here it is given up at the end of that one,
+            // which comes first (at the end of each way the others took 1 to 2 % longer).  Row-major, one operand K-major, both, us:
+            // 2048 x 2048 x 400 7.13, 6.40, 6.98 -> 6.6, 6.4, 6.5; 2048 x 2048 x 912 9.0, 7.7, 8.3 -> 8.4, 7.7, 7.7; five slices, which
+            // spilled nothing, 2048 x 2048 x 528 6.96, 6.7, 6.65 and as before.  (Nor do whole slices, which have it the plain way.)
             int left = nk - kt;
             auto is = [&](int n) __attribute__((always_inline)) {
                 asm volatile("" : "+s"(left));
@@ -319,11 +320,16 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
 #pragma unroll
                 for (int i = 0; i < 32; ++i) asm volatile("" : "=v"(fx[0][i]), "=v"(fy[0][i]), "=v"(fy[1][i]));
             };
-            if (is(5)) turn(c0, kt), turn(c1, kt + 1, true), tail3(c0, c1, kt + 2), give_up();
             if (is(4)) turn(c0, kt, true), tail3(c1, c0, kt + 1), give_up();
-            if (is(3)) tail3(c0, c1, 0), give_up();
-            if (is(2)) tail2(c0, c1, 0), give_up();
-            if (is(1)) step(c0, 0, false, 0, false, false, true);
+            if (is(5)) {
+                turn(c0, kt), turn(c1, kt + 1, true), tail3(c0, c1, kt + 2);
+            } else if (left == 3) {
+                tail3(c0, c1, 0);
+            } else if (left == 2) {
+                tail2(c0, c1, 0);
+            } else if (left == 1) {
+                step(c0, 0, false, 0, false, false, true);
+            }
         } else if (kt + 5 == nk) {
             turn(c0, kt);
             turn(c1, kt + 1, true);
