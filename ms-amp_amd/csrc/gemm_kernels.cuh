@@ -1476,11 +1476,15 @@ int run_gemm_parts(const GemmCall& c, const KSplit& split) {
 // (takes_paired_tiles()) or one (takes_small_tiles()).  The direct-to-LDS kernels need 32-bit row offsets and, but for the paired
 // form, more than one 128-byte slice of K; where they can run they are the faster ones at every size (256 x 256 x 4096: 14 against
 // 80 us with the generic kernel, 8192 x 4096 x 4096: 100 against 555), also with a ragged last slice (12605 x 4304 x 1200 into
-// float16: 94 against 153, 8192 x 4096 x 4080: 121 against 195).  Everything else takes the generic register-staged kernel.
+// float16: 94 against 153, 8192 x 4096 x 4080: 121 against 195).  Everything else takes the generic register-staged kernel.  So does
+// a float32 output of at most 16 columns over less than a slice of K, with a bias or of a few rows, which is a launch and little else
+// (K of 16 to 64, generic against paired, us: with a bias 48 x 16 4.6, 5.2, 2048 x 16 5.2, 6.1; without 16 x 16 3.8, 4.1, 48 x 16 4.5, 4.6,
+// 112 x 16 5.0, 5.0; in bfloat16 it is the paired form that is ahead, 512 x 16 5.7 to 4.7, and with 24 columns everywhere).
 template <int XF, int YF>
 int run_gemm_pair(const GemmCall& c) {
     if (c.qa == nullptr && fits_offsets(c.NR, c.NC, c.K)) {
-        if (takes_paired_tiles(c.NR, c.NC, c.K) || (c.yt && c.K <= kBK)) return run_gemm_pair128<XF, YF>(c);
+        const bool sliver = !c.yt && c.K < kBK && c.NC <= 16 && c.d_dtype == MSAMP_DT_F32 && (c.bias != nullptr || c.NR <= 64);
+        if (!sliver && (takes_paired_tiles(c.NR, c.NC, c.K) || (c.yt && c.K <= kBK))) return run_gemm_pair128<XF, YF>(c);
         if (takes_small_tiles(c.NR, c.NC, c.K)) return run_gemm_small<XF, YF>(c);
         if (c.K > kBK && c.K % kBK && (c.yt || small_tile_limit() >= 0)) return run_gemm_ragged<XF, YF>(c);
     }
