@@ -1026,7 +1026,8 @@ def test_walk_timed_at_first_use_changes_no_bit(be):
 
 @pytest.mark.parametrize('m,n,k', [(16, 16, 16), (1, 3, 48), (130, 257, 128), (8192, 4100, 112), (1040, 272, 144), (256, 384, 256),
                                    (272, 144, 272), (304, 640, 384), (2048, 2048, 400), (1008, 1040, 512), (4096, 2048, 640),
-                                   (3072, 2064, 1152), (2304, 2304, 4112), (4128, 4100, 272), (4096, 8704, 384)])
+                                   (3072, 2064, 1152), (2304, 2304, 4112), (4128, 4100, 272), (4096, 8704, 384), (16, 64, 64),
+                                   (16, 65, 112), (17, 64, 112)])
 @pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16, torch.float16])
 def test_paired_tiles_agree_with_the_other_kernels_to_the_bit(be, m, n, k, out_dtype):
     """128 x 128 tiles with two workgroups to a compute unit: one slice of K up to many, whole and ragged, tiles on every kind of
