@@ -139,17 +139,20 @@ int small_tile_limit() { return g_small_tile_limit.load(std::memory_order_relaxe
 //     K = 4096 (small tiles)                             4096 x 2048  35.5 -> 30.4,   41.0 -> 31.9    K = 12288: 89.0 -> 83.2, 104.5 -> 87.6
 //   more (large tiles)                                   3072 x 4096 x 1024  14.8 -> 13.9, 15.1 -> 15.1;   4096 x 4096 x 1024  16.9 -> 17.7, 17.3 -> 18.8
 // Large tiles of which a few begin another round cost a whole one, where paired tiles, of half a round's time each, take what is
-// there.  us, row-major with a bias, one operand K-major, both:
-//   1 to 1.5 rounds, K <= 2048     5120 x 4096 x 512   21.5 -> 18.6, 21.2 -> 16.3, 21.8 -> 17.4   K = 2048  46.0 -> 40.0, 45.6 -> 40.1, 46.9 -> 40.9
-//                                  6144 x 4096 x 512   22.4 -> 19.4, 22.2 -> 18.1, 22.0 -> 18.9   K = 2048  46.0 -> 44.8, 45.3 -> 44.8, 47.2 -> 46.6
-//   2 to 2.25                      9216 x 4096 x 512   32.0 -> 30.2, 32.6 -> 26.5, 32.7 -> 27.3   K = 2048  69.8 -> 66.8, 69.1 -> 65.3, 71.8 -> 69.5
-//   elsewhere                      7168 x 4096 x 512   23.1 -> 24.6, 22.6 -> 21.8, 23.0 -> 22.1   K = 2048  47.5 -> 54.2, 48.0 -> 54.7, 49.1 -> 55.2
+// there.  us, row-major with a bias, without, one operand K-major, both:
+//   1 to 1.25 rounds, K <= 2048    5120 x 4096 x 512   22.9 -> 19.3, 22.1 -> 17.5, 22.0 -> 16.9, 21.9 -> 16.8   K = 2048  48.4 -> 45.0, 46.9 -> 41.8, 46.8 -> 42.9, 47.8 -> 43.8
+//   1.25 to 1.5, K <= 1024         6144 x 4096 x 512   22.3 -> 19.8, 21.9 -> 18.5, 22.2 -> 19.1, 22.2 -> 19.7   K = 1024  31.0 -> 31.0, 29.9 -> 29.4, 30.3 -> 29.7, 30.2 -> 30.7
+//   2 to 2.25, K <= 1536           9216 x 4096 x 512   34.3 -> 30.4, 32.9 -> 29.1, 33.1 -> 27.4, 33.4 -> 29.8   K = 1536  61.1 -> 59.2, 59.8 -> 58.1, 60.1 -> 58.3, 60.2 -> 59.4
+//   elsewhere                      6144 x 4096 x 2048  47.4 -> 48.9, 46.8 -> 46.9, 47.0 -> 48.9, 47.1 -> 50.0   K = 1536  39.4 -> 40.4, 38.6 -> 39.0, 38.9 -> 39.3, 38.8 -> 40.1
+//                                  9216 x 4096 x 2048  73.4 -> 73.7, 72.3 -> 71.1, 72.8 -> 72.5, 73.4 -> 75.5
+//                                  7168 x 4096 x 512   23.1 -> 24.6, 22.6 -> 21.8, 23.0 -> 22.1                 K = 2048  47.5 -> 54.2, 48.0 -> 54.7, 49.1 -> 55.2 (of these three no row without)
 //                                  6144 x 4096 x 4096  78.7 -> 80.7, 78.0 -> 81.0   5120 x 4096 x 8192  143.7 -> 131.8, 142.9 -> 140.7, 150.1 -> 172.0
 bool takes_paired_tiles(int NR, int NC, int K) {
     if (small_tile_limit() != kSmallTileLimit) return false;
     const long tiles = static_cast<long>((NR + kDmaTile / 2 - 1) / (kDmaTile / 2)) * ((NC + kDmaTile / 2 - 1) / (kDmaTile / 2));
     const long large = static_cast<long>((NR + kDmaTile - 1) / kDmaTile) * ((NC + kDmaTile - 1) / kDmaTile), cus = cu_count();
-    if (large > cus && K <= 2048 && (tiles <= 6 * cus || (large > 2 * cus && tiles <= 9 * cus))) return true;
+    if (large > cus && ((tiles <= 5 * cus && K <= 2048) || (tiles <= 6 * cus && K <= 1024))) return true;
+    if (large > 2 * cus && tiles <= 9 * cus && K <= 1536) return true;
     return K <= kBK || (tiles <= 2 * cus && (tiles > cus || K <= 2048));
 }
 
