@@ -423,11 +423,14 @@ int msamp_fp8_gemm_tune(const uint8_t* a, int a_type, const float* a_scale_inv, 
                         int bias_dtype, int* chosen, msamp_stream_t stream);
 
 /* The GEMM runs 256 x 256 output tiles, one workgroup to a compute unit, where there are enough of them, and 128 x 128 tiles
- * otherwise: two workgroups to a compute unit if the product has at most two such tiles a unit (at most one if K is more than
- * 2048), or a single slice of K; one, with the whole LDS, for longer K.  Same bits whichever.  To compare the kernels, any value
- * but the default, 128, switches the form with two workgroups off: at most `big_tiles` large tiles (at most half that many if K <
- * 3072) with K of more than 384 then run small ones; 0 = the large tile always; negative: every row-major product by the generic
- * kernel that operands of 4 GiB and more take.  Process-wide; no counterpart in the reference. */
+ * otherwise.  Two workgroups of those to a compute unit: K of at most 128 (but for float32 outputs of at most 16 columns with a bias
+ * or of a few rows: the generic kernel); one tile a unit or fewer with K of at most 2048; more than one and up to two tiles a unit,
+ * whatever K; and outputs of 1 to 1.25 (K of at most 2048), 1.25 to 1.5 (1024) or 2 to 2.25 (1536) large tiles a unit.  One, with the whole LDS: the other
+ * products of at most 128 large tiles (64 if K < 3072) with K of more than 384.  Same bits whichever.  To compare the kernels, any
+ * value but the default, 128, switches the form with two workgroups off (but for K-major operands with a single slice of K, which no
+ * other kernel reads): at most `big_tiles` large tiles (at most half that many if K < 3072) with K of more than 384 then run
+ * small ones; 0 = the large tile always; negative: every row-major product by the generic kernel that operands of 4 GiB and
+ * more take.  Process-wide; no counterpart in the reference. */
 void msamp_set_small_tile_limit(int big_tiles);
 
 /* Calibration aid, no counterpart in the reference: `workgroups` workgroups of four wavefronts each issue

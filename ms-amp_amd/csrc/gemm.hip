@@ -45,7 +45,10 @@ static int dispatch_parts(int x_type, int y_type, const GemmCall& c, const KSpli
 // forward and backward: 335 -> 292.
 // Other operands (a forward product, an input gradient) only where the whole product would run 128 x 128 tiles one to a compute unit
 // with a longer K than two to a unit take, and in small tiles: their outputs as a rule are larger.  The layer call,
-// us: forward 468 x 11840 -> 512 58.8 -> 33.9, forward and backward twice over 791 x 15583 -> 1024 453 -> 390.
+// us: forward 468 x 11840 -> 512 61 -> 32, forward and backward twice over 791 x 15583 -> 1024 453 -> 387.
+// The whole product is estimated as small tiles one to a unit; two to a unit take less (takes_paired_tiles), so that the estimate is
+// too high for them.  Over 119 random products that the rule splits (up to 480 small tiles, K from 512 to 40000) the split was the
+// slower choice twice, by 0.7 and 0.9 us (704 x 144 x 2048 10.0 whole, 48 x 320 x 2016 9.4); 4096 x 2048 x 32768 253 -> 182.
 static KSplit ksplit_rule(int NR, int NC, int K, bool xt, bool yt) {
     KSplit best = {true, 1};
     // (the parts are added up four outputs at a time)

@@ -73,8 +73,8 @@ int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int
                    const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st);
 
 // The size up to which 128 x 128 tiles are looked at, in 256 x 256 tiles (msamp_set_small_tile_limit).  Any other value than the
-// default serves to compare the kernels: the paired form is off then, and a negative one sends every row-major product to the
-// generic kernel.
+// default serves to compare the kernels: the paired form is off then (but for K-major operands with a single slice of K), and a
+// negative one sends every row-major product to the generic kernel.
 constexpr int kSmallTileLimit = 128;
 int small_tile_limit();
 // The tile walk registered for this problem of the 256 x 256-tile kernel (msamp_fp8_gemm_set_walk / _tune), or -1: bit 0 =

@@ -1,13 +1,13 @@
 // The two directions of an FP8Linear layer as one call each: the casts and products of the entry points below, enqueued from
 // here.  A small layer is bound by the host, not by these kernels, and most of the host's time went into reaching them one
 // library call at a time (allocation, pointers, stream and argument conversion of each).  Host time by single calls and by
-// these, the same launches: forward of 16 x 512 -> 512 61 -> 33 us, training step of two 1024-wide blocks over 2048 tokens
-// 1522 -> 1137 us.
+// these, with the same launches: forward of 16 x 512 -> 512 61 -> 33 us, training step of two 1024-wide blocks over 2048 tokens
+// 1522 -> 1137 us; by now some of the launches are one (the casts beside the gate, cast.hip), that forward 27 us.
 // Widths that are no multiples of 16: the products read 16 bytes at a time, so the codes were copied into padded rows, and x, dy and
 // the weight transposed (byte by byte where a length is odd) for products that could not read them in place.  The casts here leave
 // their codes in rows a multiple of 16 apart, zeros behind them, which all three products read as they lie; what a product writes is
-// dense.  Forward and backward, bfloat16, us: 145 x 16744 -> 12064 897 -> 597, 861 x 15616 -> 16935 with a bias 1609 -> 1120,
-// 597 x 9654 -> 256 337 -> 172 (host), two of 8949 x 4480 -> 2157 1079 -> 757; forward alone 79 x 936 -> 840 73 -> 28.
+// dense.  Forward and backward, bfloat16, us: 145 x 16744 -> 12064 926 -> 595, 861 x 15616 -> 16935 with a bias 1644 -> 1132,
+// 597 x 9654 -> 256 205 -> 91 (host), two of 8949 x 4480 -> 2157 1129 -> 773; forward alone 79 x 936 -> 840 70 -> 27.
 #include "common.cuh"
 #include "gemm_call.h"
 #include "linear_call.h"
@@ -19,15 +19,19 @@ namespace msamp {
 // ---- a few tokens through a layer nobody differentiates ---------------------------------------------------------------
 // y[tokens][d_out] = x . fp8(w)^T, the weight read in its scaled 16- or 32-bit form and quantized on its way to the matrix pipes,
 // with the codes msamp_cast_scaled_to_fp8 gives: it is read once (2 bytes an element), where the cast and the product move 4.
-// Bound by that read and by the loads a compute unit has in flight.  A workgroup takes 16 rows of w and all tokens; its (up to)
+// Bound by that read and by the codes of x, which every workgroup reads again out of the L2: 48 tokens through 4096 -> 12288 are
+// 2.75 M requests of the L1s to it, 0.86 M of which miss (0.79 M are the weight's lines), and the waves spend 0.38 of their time
+// waiting for loads and 0.46 for their turn to issue.  A workgroup takes 16 rows of w and all tokens; its (up to)
 // eight wavefronts take the 128-wide slices of K in turn, the next slice's weights in flight over the present one's arithmetic,
 // and their float32 sums meet in LDS in a fixed order.
 // Inside a slice the k of an MFMA's operand bytes are dealt out anew, alike for both operands: lane group g holds k = 16 g .. +15
 // and 64 + 16 g .. +15, so that w arrives in pairs of loads over whole lines.  x comes in the order of the operand registers from
 // its cast (few_cast_fragments): read row by row, 16 rows a long power of two apart, it
-// cost as much as w (48 tokens 42.6 us, 35.5 so).  Both casts and the product together against the weight cast to memory and
-// the product after it, us for 4096 -> 12288: 16 tokens 48.5 -> 29.6, 48 49.2 -> 35.5, 64 49.8 -> 37.7; 64 x 8192 -> 8192 65.6 ->
-// 48.6, 64 x 16384 -> 4096 84.0 -> 51.4, 64 x 2048 -> 16384 36.6 -> 32.1, 16 x 512 -> 512 20.9 -> 15.3 (launches).
+// cost as much as w (48 tokens 7 us more).  Both casts and the product together against the weight cast to memory and the product
+// after it, replayed from a graph, us for 4096 -> 12288: 16 tokens 47.1 -> 26.7, 48 47.5 -> 32.0, 64 48.3 -> 34.3; 64 x 8192 -> 8192
+// 64.0 -> 45.4, 64 x 16384 -> 4096 82.1 -> 49.2, 64 x 2048 -> 16384 33.1 -> 23.4, 16 x 512 -> 512 14.3 -> 6.6 (launches).  Where d_out
+// gives a few workgroups and K is long, the product in parts of K that a forward with gradients takes is ahead of it by now:
+// 64 x 16384 -> 256 52.6 before either, 31.0 here, 23.1 in parts.
 __device__ __forceinline__ float few_bias(const void* bias, int dt, int i) {
     if (dt == MSAMP_DT_F32) return static_cast<const float*>(bias)[i];
     if (dt == MSAMP_DT_F16) return f16_bits_to_float(static_cast<const uint16_t*>(bias)[i]);
