@@ -210,14 +210,10 @@ extern "C" int msamp_fp8_gemm_tune(const uint8_t* a, int a_type, const float* a_
     // milliseconds (at least four) between one pair of events
     float best_ms = 0.0f, rule_ms = 0.0f;
     int best = -1, rc = MSAMP_OK;
-    // (row-major operands: the fastest of the four once more with split waits, bit 2)
-    const bool can_split = !a_kmajor && !b_kmajor;
-    float explicit_ms[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int turns = can_split ? 7 : 6;
+    const int turns = 6;
     for (int turn = 0; turn < turns && rc == MSAMP_OK; ++turn) {
         int walk = turn - 1;
         if (turn == turns - 1) walk = -1;    // (the rule's walk once more at the end: a cold start must not cost it the comparison)
-        else if (turn == 5) walk = 4 + static_cast<int>(std::min_element(explicit_ms, explicit_ms + 4) - explicit_ms);
         msamp::t_forced_walk = walk;
         for (int i = 0; i < 2 && rc == MSAMP_OK; ++i) rc = run();
         int reps = 4;
@@ -229,7 +225,6 @@ extern "C" int msamp_fp8_gemm_tune(const uint8_t* a, int a_type, const float* a_
                                hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
             rc = MSAMP_ERR_HIP;
         ms /= reps;
-        if (walk >= 0 && walk < 4) explicit_ms[walk] = ms;
         if (turn == 0) rule_ms = best_ms = ms;
         else if (walk < 0) rule_ms = std::min(rule_ms, ms);
         else if (ms < best_ms) best_ms = ms, best = walk;

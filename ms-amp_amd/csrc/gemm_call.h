@@ -51,9 +51,8 @@ struct GemmCall {
 template <int XF, int YF>
 int run_gemm_pair(const GemmCall& c);
 // The other half of a pair's instantiations lives in a translation unit of its own (gemm_inst.hip built with
-// -DMSAMP_GEMM_SPLIT_UNIT), so that they compile side by side: the 256 x 256-tile kernel for a ragged last slice of K, the
-// 128 x 128-tile kernel (all layouts and output types), and the split-wait form (row-major operands, all three output
-// types, both parities of the slice count).
+// -DMSAMP_GEMM_SPLIT_UNIT), so that they compile side by side: the 256 x 256-tile kernel for a ragged last slice of K and the
+// 128 x 128-tile kernels (all layouts and output types).
 template <int XF, int YF>
 int run_gemm_ragged(const GemmCall& c);
 template <int XF, int YF>
@@ -68,10 +67,6 @@ struct KSplit {
 // (Large tiles: both operands K-major.)  c.D is the float32 scratch of `parts` arrays that receives the parts' unscaled sums.
 template <int XF, int YF>
 int run_gemm_parts(const GemmCall& c, const KSplit& split);
-template <int XF, int YF>
-int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int NR, int NC, int K, const float* xs,
-                   const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st);
-
 // The size up to which 128 x 128 tiles are looked at, in 256 x 256 tiles (msamp_set_small_tile_limit).  Any other value than the
 // default serves to compare the kernels: the paired form is off then (but for K-major operands with a single slice of K), and a
 // negative one sends every row-major product to the generic kernel.
@@ -80,7 +75,7 @@ int small_tile_limit();
 // The tile walk registered for this problem of the 256 x 256-tile kernel (msamp_fp8_gemm_set_walk / _tune), or -1: bit 0 =
 // groups of tile columns walked row by row instead of groups of tile rows, bit 1 = the XCD's patch of 32 tiles turned (4 of
 // the grouped dimension x 8 of the walked one).  Any walk gives the same output bits: it only decides which workgroup
-// takes which tile.  Bit 2 (row-major operands only): the tile loads awaited in two parts, see the kernel.
+// takes which tile.  (Bit 2 is taken and means nothing: it asked for what every product does now.)
 int registered_walk(int NR, int NC, int K, bool XT, bool YT);
 // 128 x 128 tiles with the whole LDS to a workgroup: at least four slices of K; up to half the limit always (one small tile per
 // compute unit with the default limit), up to the limit where K is long enough for the second round of small tiles to
@@ -132,10 +127,5 @@ extern template int run_gemm_ragged<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall
 extern template int run_gemm_small<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_pair128<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&);
 extern template int run_gemm_parts<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(const GemmCall&, const KSplit&);
-#define MSAMP_SPLIT_ARGS const uint8_t*, const uint8_t*, void*, int, int, int, int, const float*, const float*, int, const void*, int, hipStream_t
-extern template int run_gemm_split<MSAMP_DT_E4M3, MSAMP_DT_E4M3>(MSAMP_SPLIT_ARGS);
-extern template int run_gemm_split<MSAMP_DT_E4M3, MSAMP_DT_E5M2>(MSAMP_SPLIT_ARGS);
-extern template int run_gemm_split<MSAMP_DT_E5M2, MSAMP_DT_E4M3>(MSAMP_SPLIT_ARGS);
-extern template int run_gemm_split<MSAMP_DT_E5M2, MSAMP_DT_E5M2>(MSAMP_SPLIT_ARGS);
 
 }    // namespace msamp

@@ -289,17 +289,17 @@ __device__ __forceinline__ uint4 load_out16(const void* p) {
 // quadrant (8 x 8 accumulators of the 16x16x128 FP8 MFMA = 256 accumulation registers per lane).
 //  * Tiles travel global -> LDS with the direct-to-LDS load: no staging registers, no LDS stores.  A
 //    lane group of 8 fetches one whole 128-byte line (full-line requests are what the L2 serves best).
-//  * Two 64 KiB LDS stages.  A slice is computed in four quarters of 16 MFMAs (X half x Y half); the fragment
-//    half the next quarters need is read while the current one executes.
-//  * One workgroup barrier per slice, after the second quarter: by then every wave holds the whole slice
-//    in registers, so the stage is refilled right away with the slice after next (its 16 loads spread over
-//    the last two quarters, which leaves them half a slice to land).
+//  * The LDS is a ring of five blocks of 32 KiB, one operand's part of a slice each.  A slice is computed in four quarters of
+//    16 MFMAs (X half x Y half); the fragment half the next quarters need is read while the current one executes.
+//  * One workgroup barrier per slice, in the third quarter: by then every wave holds the whole slice in registers, so its two
+//    blocks are refilled with Y of the slice after next and X of the one behind it, spread evenly over a slice's time.
 //  * LDS reads and tile loads are interleaved with the MFMAs one at a time, so that neither the LDS nor
 //    the vector-memory queue backs up and stalls the MFMA stream.
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
 
-constexpr int kDmaStage = 2 * kDmaTile * kBK;    // X + Y slice: 64 KiB
+constexpr int kDmaBlock = kDmaTile * kBK;    // one operand's part of a slice: 32 KiB
+constexpr int kDmaBlocks = 5;                // all 160 KiB of the LDS
 
 // s_waitcnt vmcnt(N), leaving the other counters unconstrained (gfx9 encoding: vmcnt = [3:0] and [15:14])
 template <int N>
@@ -309,7 +309,7 @@ __device__ __forceinline__ void wait_vmcnt() {
 
 //  * XT / YT: that operand is handed over K-major, T[K][rows] with the rows contiguous (the transpose of
 //    what the product needs), so that callers need not materialize transposed copies.  Its slice sits in
-//    LDS as 128 k-rows of 256 bytes (same 32 KiB), filled by the same eight 1 KiB loads, and its
+//    LDS as 128 k-rows of 256 bytes (same 32 KiB block), filled by the same eight 1 KiB loads, and its
 //    fragments come from the transposing LDS read: a 16-lane group reads eight k-rows of 16 bytes and
 //    lane i receives byte i of each, i.e. eight consecutive k for its row -- four such reads make the
 //    32-byte operand of the MFMA.  The 16-byte position inside a k-row is XOR-ed with k % 8 (on the global
@@ -444,8 +444,7 @@ __device__ __forceinline__ void k_part(In& X, In& Y, Out& D, int NR, int NC, int
     K = end - first;
 }
 
-template <int XF, int YF, typename OT, bool XT = false, bool YT = false, int QF = 0, bool ODD_NK = false, bool QSPEC = false,
-          bool KTAIL = false, bool SPLIT = false>
+template <int XF, int YF, typename OT, bool XT = false, bool YT = false, int QF = 0, bool QSPEC = false, bool KTAIL = false>
 __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_t* __restrict__ X,
                                                                      const uint8_t* __restrict__ Y, OT* __restrict__ D,
                                                                      int NR, int NC, int K,
@@ -485,21 +484,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
         const int long_n = x_long ? NR : NC, short_n = x_long ? NC : NR;
         if (long_n >= 10240 && long_n % 256 == 0 && short_n <= 8192) by_columns = x_long, wide = true;
     }
-    // Split waits (template flag SPLIT, row-major operands only; the host picks the instantiation: bit 2 of a registered
-    // walk, else by rule).  In the plain form a slice's sixteen tile loads are issued during the second half of a step
-    // (the stage they fill is read until then) and all awaited at the one barrier in the middle of the next step: the
-    // last of them has half a step to arrive.  But a row-major load brings whole rows, and the rows of blocks 0..3 of
-    // every wave's quadrant were already read at the end of the step before.  In the split form the loads go out in the
-    // order of need, four per quarter of the step: X and Y blocks 0..3 of slice kt + 2 during the first half of step kt
-    // (after a barrier of its own at the start of the step: everybody has read those rows of slice kt), Y and X blocks
-    // 4..7 during the second half; the first part is awaited in the middle of step kt + 1, the second at the start of
-    // step kt + 2, each with sixteen younger loads in flight behind it: every load has one to one and a half steps.  That
-    // pays where the loads miss the L2 and the memory-side cache -- the longer K, the more: 16384 x 8192 x K at K = 12288
-    // +1 %, 14336 +5 %, 16384 +2 %, 20480 +5 %, 28672 +8 %, 16384 cubed +5 % -- and is level below (-0.8 to +0.8 % at K
-    // of 4096 .. 11008: the second barrier), hence the host's rule K >= 12288.  (A flag read at run time instead of a
-    // second instantiation cost the plain form 3 to 7 %: the selects between the two orders sat in the K loop.)
-    static_assert(!SPLIT || (!XT && !YT && QF == 0 && !QSPEC), "split waits: plain row-major form only");
-    static_assert(!KTAIL || (!SPLIT && QF == 0), "a ragged last slice: plain and speculative forms only");
+    static_assert(!KTAIL || QF == 0, "a ragged last slice: plain and speculative forms only");
     // a walk registered for this problem (timed on this machine) overrides the rules
     if (qa.walk_plus_one > 0) by_columns = (qa.walk_plus_one - 1) & 1, wide = ((qa.walk_plus_one - 1) >> 1) & 1;
     tile_of_id(blockIdx.x, tiles_r, tiles_c, by_columns, wide, tr, tc);
@@ -528,7 +513,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
         asm volatile("" : "+v"(guess));
     }
 
-    // ---- global -> LDS.  A stage holds 256 X rows then 256 Y rows, 128 bytes per row.  One wave
+    // ---- global -> LDS.  A block of the ring holds 256 X rows or 256 Y rows, 128 bytes per row.  One wave
     // instruction fills 8 rows (1 KiB, lane-contiguous): lane l lands in row l/8, 16-byte position l%8,
     // and therefore fetches the logical chunk position ^ swizzle(row).  Rows past the end of the matrix
     // are clamped to its last row (their results are never stored).
@@ -564,25 +549,28 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     const int nk = KTAIL ? (K + kBK - 1) / kBK : K / kBK;
     const int rem = K - (nk - 1) * kBK;
     const uint32_t tail_back = KTAIL && chunk * 16 >= rem ? chunk * 16 : 0;
-    // one of the 16 loads of a slice (0..7: X rows, 8..15: Y rows), so they can be spread between MFMAs
-    auto dma = [&](int kt, int stage, int i, bool last = false) __attribute__((always_inline)) {
-        // the i-th load of a slice is load i, or in the split form the i-th in order of need
-        constexpr int by_need[16] = {0, 1, 4, 5, 8, 9, 12, 13, 10, 11, 14, 15, 2, 3, 6, 7};
-        const int which = SPLIT ? by_need[i] : i;
-        const bool is_x = which < 8;
+    // The ring: X and Y of a slice side by side, slice after slice.  Where the block lies that is that many on from the one at s0.
+    // (s0, X of the present slice, is handed around as a value: captured by reference it ended up in scratch memory in some forms.)
+    constexpr int kX = 0, kY = 1, kPerSlice = 2;
+    auto place = [](int s0, int blocks_on) __attribute__((always_inline)) {
+        const int p = s0 + blocks_on % kDmaBlocks * kDmaBlock;
+        return p >= kDmaBlocks * kDmaBlock ? p - kDmaBlocks * kDmaBlock : p;
+    };
+    // one of this wave's eight loads for a block of slice kt, which is `ahead` slices on from the present one
+    auto dma = [&](int s0, int block, int kt, int ahead, int w, bool last) __attribute__((always_inline)) {
+        const bool is_x = block == kX;
         const size_t slice = static_cast<size_t>(kt) * kBK;
         const uint8_t* src = is_x ? X + (XT ? slice * ldx : slice) : Y + (YT ? slice * ldy : slice);
-        uint32_t off = which < 8 ? xoff[which] : yoff[which - 8];
+        uint32_t off = is_x ? xoff[w] : yoff[w];
         if (KTAIL && last) {
             if (is_x ? XT : YT) {
-                if (((which & 7) * 4 + wave) * 4 + (lane >> 4) >= rem) off = is_x ? xcol : ycol;
+                if ((w * 4 + wave) * 4 + (lane >> 4) >= rem) off = is_x ? xcol : ycol;
             } else {
                 off -= tail_back;
             }
         }
         // (wave-uniform by construction; the readfirstlane keeps it in a scalar register whatever the compiler makes of it)
-        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + stage * kDmaStage + (which < 8 ? 0 : kDmaTile * kBK) +
-                                                            ((which & 7) * 4 + wave) * 1024);
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + place(s0, ahead * kPerSlice + block) + (w * 4 + wave) * 1024);
         // Written as assembly so that the compiler does not see an LDS write it cannot tell apart from
         // the fragment reads: it would otherwise make every LDS read wait for all loads in flight.
         // Completion is tracked by hand with wait_vmcnt<>() before the barriers below.  M0 holds the
@@ -598,28 +586,26 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     const int fsw = (lane & 7) ^ ((lane >> 3) & 1);
     const int l16 = lane & 15, g4 = lane >> 4;
     const int off_lo = ((2 * g4) ^ fsw) << 4;    // low 16 bytes of this lane's 32; the high ones are at ^ 16
-    const int xrow = (wr * 128 + l16) * kBK;
-    const int yrow = kDmaTile * kBK + (wc * 128 + l16) * kBK;
     const int tj = l16 >> 1;
     const int t_lane = (g4 * 32 + tj) * 256 + (l16 & 1) * 8;    // k-row and 8-byte half of this lane's address
+    // this lane's first read of half 0 in a block; the 16-row blocks of a row-major operand follow 2 KiB apart, of a K-major one
+    // at ^ 16 (its half 1 at ^ 64)
+    const int xlane = XT ? t_lane + wr * 128 + (tj << 4) : (wr * 128 + l16) * kBK + off_lo;
+    const int ylane = YT ? t_lane + wc * 128 + (tj << 4) : (wc * 128 + l16) * kBK + off_lo;
     // The wave's 128 x 128 quadrant is 8 x 8 blocks of 16 x 16.  Fragments are kept by halves: fx[h] / fy[h] hold the
     // four 16-row blocks 4h .. 4h+3 of X / Y (8 registers each).  A half arrives in pieces: two 16-byte reads per
     // block of a row-major operand, four 8-byte transposing reads otherwise.
     constexpr int kPX = XT ? 16 : 8, kPY = YT ? 16 : 8;
-    auto read_piece = [&](int* dst, int stage, bool is_x, int half, int p) __attribute__((always_inline)) {
-        const uint8_t* base = smem + stage * kDmaStage;
+    auto read_piece = [&](int* dst, int at, bool is_x, int half, int p) __attribute__((always_inline)) {
         if ((is_x && !XT) || (!is_x && !YT)) {
             const int b = p >> 1, hf = p & 1;
-            const v4i val = *reinterpret_cast<const v4i*>(base + (is_x ? xrow : yrow) + (half * 4 + b) * 16 * kBK +
-                                                          (off_lo ^ (hf * 16)));
+            const v4i val = *reinterpret_cast<const v4i*>(smem + (at ^ (hf * 16)) + (half * 4 + b) * 16 * kBK);
             int* d = dst + b * 8 + hf * 4;
             d[0] = val[0], d[1] = val[1], d[2] = val[2], d[3] = val[3];
         } else {
             const int b = p >> 2, qq = p & 3;
-            const int wq = is_x ? wr : wc;
-            const int addr = (is_x ? 0 : kDmaTile * kBK) + t_lane + (qq * 8) * 256 + wq * 128 + (((half * 4 + b) ^ tj) << 4);
             const v2i val = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-                (__attribute__((address_space(3))) v2i*)(base + addr));
+                (__attribute__((address_space(3))) v2i*)(smem + (at ^ ((half * 4 + b) * 16)) + qq * 8 * 256));
             int* d = dst + b * 8 + qq * 2;
             d[0] = val[0], d[1] = val[1];
         }
@@ -630,17 +616,21 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
 
     int fx[2][32], fy[2][32];
 
-    // One quarter of a slice: the 16 MFMAs of X half hx against Y half hy, with the reads of one fragment half
-    // (rd_x / rd_half from rd_stage into rd_dst) spread between them and, if asked for, eight of the 16 tile loads
-    // of slice ld_kt (ld_first .. ld_first + 7), one every other MFMA.
+    // One quarter of a slice: the 16 MFMAs of X half hx against Y half hy, with the reads of a fragment half (X or Y half rd_half out
+    // of the block that many on, into rd_dst, if do_read) spread between them, and four loads of slice ld_kt (X, then Y; if do_load),
+    // one every four MFMAs.  With VM >= 0 the waves meet after the second MFMA (by then the fragments read last have come back): what
+    // the quarters before have read nobody needs in the LDS any more, and all but the last VM loads of each wave have landed.
     // srcA = Y rows (columns of D), srcB = X rows (rows of D): a lane then holds, for D row lane % 16 of a block, four
     // consecutive D columns -- the layout the epilogue wants.
-    auto quarter = [&](auto hxc, auto hyc, int* rd_dst, int rd_stage, bool rd_x, int rd_half, bool do_read, int ld_kt,
-                       int ld_stage, int ld_first, bool do_load, bool ld_last = false) __attribute__((always_inline)) {
+    auto quarter = [&](auto hxc, auto hyc, auto vmc, int s0, int* rd_dst, bool rd_x, int rd_lane, int rd_blocks_on, int rd_half, bool do_read,
+                       int ld_kt, int ld_block, int ld_first, bool do_load, bool ld_last) __attribute__((always_inline)) {
         constexpr int cb = (YF == MSAMP_DT_E4M3) ? 0 : 1;
         constexpr int bl = (XF == MSAMP_DT_E4M3) ? 0 : 1;
         const int np = rd_x ? kPX : kPY;
-        constexpr int hx = decltype(hxc)::value, hy = decltype(hyc)::value;
+        constexpr int hx = decltype(hxc)::value, hy = decltype(hyc)::value, vm = decltype(vmc)::value;
+        int block = place(s0, rd_blocks_on);
+        asm volatile("" : "+s"(block));
+        const int at = rd_lane + block;
         static_for<4>([&](auto jc) {    // the Y fragment stays for four MFMAs in a row
             static_for<4>([&](auto ic) {
                 constexpr int i = decltype(ic)::value, j = decltype(jc)::value;
@@ -650,99 +640,79 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                 const v8i vx = {cx[0], cx[1], cx[2], cx[3], cx[4], cx[5], cx[6], cx[7]};
                 const v8i vy = {cy[0], cy[1], cy[2], cy[3], cy[4], cy[5], cy[6], cy[7]};
                 mfma_fixed<(hx * 4 + i) * 8 + hy * 4 + j, cb, bl>(vy, vx);
-                if (do_read) {
+                if constexpr (vm >= 0 && n == 1) {
+                    wait_vmcnt<(vm < 0 ? 0 : vm)>();
+                    __syncthreads();
+                }
+                if (do_read && n >= 2 && n < 14) {
 #pragma unroll
-                    for (int p = n * np / 16; p < (n + 1) * np / 16; ++p) read_piece(rd_dst, rd_stage, rd_x, rd_half, p);
+                    for (int p = (n - 2) * np / 12; p < (n - 1) * np / 12; ++p) read_piece(rd_dst, at, rd_x, rd_half, p);
                 }
-                if constexpr (SPLIT) {    // four loads per quarter, all four quarters
-                    if (do_load && (n & 3) == 3) dma(ld_kt, ld_stage, ld_first + (n >> 2));
-                } else {    // eight per quarter in the second half of the step
-                    if (do_load && (n & 1)) dma(ld_kt, ld_stage, ld_first + (n >> 1), ld_last);
-                }
+                if (do_load && (n & 3) == 3) dma(s0, ld_block, ld_kt, 2, ld_first + (n >> 2), ld_last);
                 // Nothing moves across: one MFMA, then the reads and the load that go with it, so that the LDS reads and
                 // the tile loads stay spread evenly between the MFMAs as written.
                 __builtin_amdgcn_sched_barrier(0);
             });
         });
     };
-    // Slice kt sits in stage st and slice kt + 1 is on its way into the other stage; X half 0 and Y half 0 of slice
-    // kt are in registers.  Quarters 1, 2: X0 x Y0 while Y half 1 arrives, X0 x Y1 while X half 1 arrives -- all of
-    // slice kt is in registers now.  Barrier: slice kt + 1 has landed and nobody needs the LDS copy of slice kt.
-    // Quarters 3, 4: X1 x Y0 while X half 0 of slice kt + 1 arrives, X1 x Y1 while its Y half 0 arrives; the stage of
-    // slice kt is refilled with slice kt + 2 meanwhile.
-    // Split form: at the start of the step the second part of slice kt's loads has landed (behind it in the queue, if the
-    // step before issued loads -- prev_loaded --, the sixteen of slice kt + 1) and everybody is past the reads of the
-    // step before; the first part of slice kt + 2 then goes out during quarters 1 and 2, into the rows of blocks 0..3.
-    // KTAIL: ld_last, the slice being loaded is the last one; masked, the slice being computed is.
-    auto slice = [&](int st, bool has_next, int ld_kt, bool do_load, bool prev_loaded = true, bool ld_last = false,
-                     bool masked = false) __attribute__((always_inline)) {
+    // A step: slice kt, whose X half 0 and Y half 0 are in registers and whose blocks are in the ring, with those of slice kt + 1
+    // there or on their way and the place of X of slice kt + 2 free.  X0 x Y0 while Y half 1 is read, X0 x Y1 while X half 1 is -- all
+    // of slice kt is in registers now -- X1 x Y0 while X half 0 of slice kt + 1 is and X1 x Y1 while its Y half 0 is.  X of slice kt + 2 is
+    // sent for in the first two quarters; the waves meet in the third (slice kt + 1 has landed, and the eight loads of that X may
+    // still be on their way; nobody needs the LDS copy of slice kt); Y of slice kt + 2 follows in the place of X of slice kt.  So
+    // a load has three quarters of a step to one and a half to land, and one goes out every four MFMAs.
+    // What bounds the loop is the way of its loads.  With two stages of a slice each all sixteen went out in the second half of a
+    // step, one every other MFMA, to land by the middle of the next: too late wherever they missed the L2.  us in a loop / each among
+    // other kernels, two stages -> ring, bfloat16:
+    //   row-major      8192 x 2048 x 8192  100 / 109 -> 97 / 101   8192 x 4096 x 4096  103 / 114 -> 103 / 107   8192 x 8192 x 2048  114 / 121 -> 113 / 117
+    //                  12605 x 4304 x 1200  96 / 103 -> 92 / 98    16384 x 11008 x 4096  564 / 567 -> 544 / 541  16384 x 4096 x 11008  528 / 528 -> 495 / 487
+    //   Y K-major      8192 x 2048 x 8192  99 / 105 -> 96 / 99     16384 x 4096 x 11008  541 / 538 -> 497 / 489  16384 x 28672 x 8192  2662 / 2658 -> 2600 / 2595
+    //   both           2048 x 8192 x 8192  95 / 105 -> 92 / 94     11008 x 4096 x 16384  519 / 521 -> 493 / 498  8192 x 28672 x 16384  2602 / 2595 -> 2426 / 2425
+    //   level          8192 x 8192 x 512  51 / 54 -> 50 / 56       4096 x 4096 x 8192, both  91 / 103 -> 91 / 94   8192 x 8192 x 4096, both  190 / 208 -> 192 / 194
+    // (Row-major with K of 12288 and more had a form of its own before, its loads in the order of need over a whole step and two meetings
+    // in it: 16384 x 8192 x 28672 2528 / 2510, here 2560 / 2515.  The ring in units of 16 KiB with two meetings a step, every load two
+    // steps to land, was no faster, and slower with both K-major, whose k-rows it took in pieces of 128 bytes: 8192 x 28672 x 16384 2500.)
+    // `to_go`: slices behind this one, 2 standing for two or more; the last two load nothing.  KTAIL: `last`, the slice that this step
+    // loads is the last one.
+    auto step = [&](auto to_go_c, int s0, int kt, bool last) __attribute__((always_inline)) {
         constexpr std::integral_constant<int, 0> c0{};
         constexpr std::integral_constant<int, 1> c1{};
-        if (KTAIL && masked) mask_fragments(fx[0], g4, rem), mask_fragments(fy[0], g4, rem);
-        if constexpr (SPLIT) {
-            if (prev_loaded) wait_vmcnt<16>();
-            else wait_vmcnt<0>();
-            __syncthreads();
-        }
-        quarter(c0, c0, fy[1], st, false, 1, true, ld_kt, st, 0, SPLIT && do_load);
-        if (KTAIL && masked) mask_fragments(fy[1], g4, rem);
-        quarter(c0, c1, fx[1], st, true, 1, true, ld_kt, st, 4, SPLIT && do_load);
-        if (KTAIL && masked) mask_fragments(fx[1], g4, rem);
-        if (SPLIT && has_next) {
-            // the first part of slice kt + 1; behind it its second part and, if this step loads, the first of slice kt + 2
-            if (do_load) wait_vmcnt<16>();
-            else wait_vmcnt<8>();
-        } else {
-            wait_vmcnt<0>();
-        }
-        __syncthreads();
-        quarter(c1, c0, fx[0], st ^ 1, true, 0, has_next, ld_kt, st, SPLIT ? 8 : 0, do_load, ld_last);
-        quarter(c1, c1, fy[0], st ^ 1, false, 0, has_next, ld_kt, st, SPLIT ? 12 : 8, do_load, ld_last);
+        constexpr std::integral_constant<int, -1> none{};
+        constexpr int to_go = decltype(to_go_c)::value;
+        constexpr bool masked = KTAIL && to_go == 0, loads = to_go >= 2, next = to_go >= 1;
+        constexpr std::integral_constant<int, loads ? 8 : 0> meet{};
+        if (masked) mask_fragments(fx[0], g4, rem), mask_fragments(fy[0], g4, rem);
+        quarter(c0, c0, none, s0, fy[1], false, ylane, kY, 1, true, kt + 2, kX, 0, loads, last);
+        if (masked) mask_fragments(fy[1], g4, rem);
+        quarter(c0, c1, none, s0, fx[1], true, xlane, kX, 1, true, kt + 2, kX, 4, loads, last);
+        if (masked) mask_fragments(fx[1], g4, rem);
+        quarter(c1, c0, meet, s0, fx[0], true, xlane, kPerSlice + kX, 0, next, kt + 2, kY, 0, loads, last);
+        quarter(c1, c1, none, s0, fy[0], false, ylane, kPerSlice + kY, 0, next, kt + 2, kY, 4, loads, last);
+        return place(s0, kPerSlice);
     };
 
     // prologue: slices 0 and 1 (the host sends no problem with fewer than two slices here); wait for slice 0; read
     // its first fragment halves
 #pragma unroll
-    for (int w = 0; w < 16; ++w) dma(0, 0, w);
+    for (int w = 0; w < 16; ++w) dma(0, w < 8 ? kX : kY, 0, 0, w & 7, false);
 #pragma unroll
-    for (int w = 0; w < 16; ++w) dma(1, 1, w, nk == 2);
+    for (int w = 0; w < 16; ++w) dma(0, w < 8 ? kX : kY, 1, 1, w & 7, nk == 2);
     wait_vmcnt<16>();
     __syncthreads();
 #pragma unroll
-    for (int p = 0; p < kPX; ++p) read_piece(fx[0], 0, true, 0, p);
+    for (int p = 0; p < kPX; ++p) read_piece(fx[0], xlane + place(0, kX), true, 0, p);
 #pragma unroll
-    for (int p = 0; p < kPY; ++p) read_piece(fy[0], 0, false, 0, p);
-    // Two slices per turn of the loop (stage 0, stage 1).  What is left afterwards -- two slices when the slice count is
-    // even, three when it is odd (ODD_NK, chosen by the host) -- follows as straight-line code: the last slices load
-    // nothing and the last one reads no fragments for a successor, which the compiler then knows.
-    int kt = 0;
-    // (KTAIL: the load of the last slice is not part of the loop, and both parities are in one kernel)
-    for (; kt + (KTAIL ? 4 : 3) < nk; kt += 2) {
-        slice(0, true, kt + 2, true);
-        slice(1, true, kt + 3, true);
-    }
-    if constexpr (KTAIL) {
-        // two slices left with everything loaded (nk = 2), three with the last one still to load, or four with two to load
-        if (nk - kt == 3) {
-            slice(0, true, kt + 2, true, true, true);
-            slice(1, true, 0, false);
-            slice(0, false, 0, false, false, false, true);
-        } else {
-            if (nk - kt == 4) {
-                slice(0, true, kt + 2, true);
-                slice(1, true, kt + 3, true, true, true);
-            }
-            slice(0, true, 0, false);
-            slice(1, false, 0, false, false, false, true);
-        }
-    } else if constexpr (ODD_NK) {
-        slice(0, true, kt + 2, true);
-        slice(1, true, 0, false);
-        slice(0, false, 0, false, false);
-    } else {
-        slice(0, true, 0, false);
-        slice(1, false, 0, false, false);
-    }
+    for (int p = 0; p < kPY; ++p) read_piece(fy[0], ylane + place(0, kY), false, 0, p);
+    // The last two steps follow the loop as straight-line code (KTAIL: the last three, so that the loop loads whole slices only): they
+    // load nothing and the last one reads no fragments for a successor, which the compiler then knows.
+    constexpr std::integral_constant<int, 2> go2{};
+    constexpr std::integral_constant<int, 1> go1{};
+    constexpr std::integral_constant<int, 0> go0{};
+    int kt = 0, s0 = 0;
+    for (; kt + (KTAIL ? 3 : 2) < nk; ++kt) s0 = step(go2, s0, kt, false);
+    if (KTAIL && kt + 3 == nk) s0 = step(go2, s0, kt, true), ++kt;
+    s0 = step(go1, s0, kt, false);
+    step(go0, s0, kt + 1, false);
     // The workgroup that follows this one on the CU is, as a rule, the one 256 ids on (same XCD).  Touch the first two K
     // slices of its tile now -- one 4-byte load per 128-byte line, dropped into an LDS corner that nothing reads -- so that
     // its prologue finds them in this XCD's L2 instead of waiting for HBM with the MFMA pipe idle.  The loads have no
@@ -765,7 +735,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                 return base + static_cast<size_t>(row) * K + hf;
             };
             const int t = threadIdx.x;
-            const uint32_t dump = __builtin_amdgcn_readfirstlane(lds_base + 2 * kDmaStage - 256);
+            const uint32_t dump = __builtin_amdgcn_readfirstlane(lds_base + kDmaBlocks * kDmaBlock - 256);
             asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off\n\tglobal_load_lds_dword %2, off\n\t"
                          "global_load_lds_dword %3, off\n\tglobal_load_lds_dword %4, off"
                          : : "s"(dump), "v"(line(t, true)), "v"(line(t + 256, true)), "v"(line(t, false)), "v"(line(t + 256, false))
@@ -774,14 +744,15 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     }
     const uint32_t acc_token = acc_fence();
     // No barrier here: the last LDS reads of every wave were issued (and awaited) before the barrier of the last
-    // slice, and no load is in flight, so each wave may start on its patch as soon as its own MFMAs are done.
+    // slice, and no load is in flight but the touches, so each wave may start on its patch as soon as its own MFMAs are done.
+    uint32_t* const red = reinterpret_cast<uint32_t*>(smem + kDmaBlocks * kDmaBlock - 512);    // a few words behind all patches
 
     // The epilogues below handle the quadrant in four units of 32 rows (two 16-row blocks): unit u, half h, column
     // block j -> acc[2u + h][j], patch row h * 16 + lane % 16, patch columns j * 16 + (lane / 16) * 4 .. + 3.
     if constexpr (QF != 0) {
         // ---- fused in-time cast (whole tiles only, no bias, no accumulation: the host sees to that)
-        __shared__ uint32_t q_red[kGemmThreads / kWave];
-        __shared__ uint32_t q_scale, q_amax;
+        uint32_t* const q_red = red;
+        uint32_t &q_scale = red[kGemmThreads / kWave], &q_amax = red[kGemmThreads / kWave + 1];
         const float alpha = alpha_early;
         // max |acc| as an ordered bit pattern: NaN above Inf above everything finite, so a NaN reaches the amax
         // as it does through abs().max()
@@ -1175,8 +1146,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
             if constexpr (__is_same(OT, bf16_t)) m <<= 16;
             else m = __float_as_uint(f16_bits_to_float(m));
         }
-        __shared__ uint32_t spec_red[kGemmThreads / kWave];
-        m = block_max_u32(m, spec_red);    // valid in lane 0 of wave 0
+        m = block_max_u32(m, red);    // valid in lane 0 of wave 0
         if (threadIdx.x == 0) {
             // Fold into the call's one word, then draw a ticket.  Both are atomics of agent scope on neighbouring words,
             // carried out where all XCDs meet; the maximum's old value has come back before the ticket is asked for, so
@@ -1214,14 +1184,12 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     else emit_plain(std::false_type{}, std::false_type{});
 }
 
-// The kernel is built once for an even and once for an odd number of K slices (its last slices are straight-line
-// code); ODD picks the one that fits K.
-template <int XF, int YF, typename OT, bool XT, bool YT, bool ODD, bool KTAIL = false, bool SPLIT = false>
-static int launch_gemm_dma_parity(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
-                                  const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st, int parts = 1) {
-    constexpr int smem = 2 * kDmaStage;
+template <int XF, int YF, typename OT, bool XT, bool YT, bool KTAIL>
+static int launch_gemm_dma_tail(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
+                                const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st, int parts = 1) {
+    constexpr int smem = kDmaBlocks * kDmaBlock;
     static std::atomic<bool> configured{false};    // setting the attribute twice is harmless
-    auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, 0, ODD, false, KTAIL, SPLIT>;
+    auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, 0, false, KTAIL>;
     if (!configured.load(std::memory_order_acquire)) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(fp8_gemm_dma_kernel)");
@@ -1239,25 +1207,16 @@ static int launch_gemm_dma_parity(const uint8_t* X, const uint8_t* Y, void* D, i
 template <int XF, int YF, typename OT, bool XT = false, bool YT = false>
 static int launch_gemm_dma(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
                            const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
-    if constexpr (!XT && !YT) {
-        // split waits: bit 2 of a walk registered for the problem, else from K = 12288 on (see the kernel)
-        const int walk = registered_walk(NR, NC, K, XT, YT);
-        if (walk >= 0 ? (walk & 4) != 0 : K >= 12288) {
-            constexpr int d_dtype = std::is_same<OT, float>::value ? MSAMP_DT_F32 : std::is_same<OT, f16_t>::value ? MSAMP_DT_F16 : MSAMP_DT_BF16;
-            return run_gemm_split<XF, YF>(X, Y, D, d_dtype, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
-        }
-    }
-    if ((K / kBK) & 1) return launch_gemm_dma_parity<XF, YF, OT, XT, YT, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
-    return launch_gemm_dma_parity<XF, YF, OT, XT, YT, false>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
+    return launch_gemm_dma_tail<XF, YF, OT, XT, YT, false>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
 }
 
 // the same kernel with the in-time cast to FP8 fused in (see QF above); the caller has checked the shape
-template <int XF, int YF, typename OT, bool XT, bool YT, int QF, bool ODD>
-static int launch_gemm_dma_quant_parity(const uint8_t* X, const uint8_t* Y, int NR, int NC, int K, const float* xs,
+template <int XF, int YF, typename OT, bool XT, bool YT, int QF>
+static int launch_gemm_dma_quant(const uint8_t* X, const uint8_t* Y, int NR, int NC, int K, const float* xs,
                                         const float* ys, const QuantArgs& qa, hipStream_t st) {
-    constexpr int smem = 2 * kDmaStage;
+    constexpr int smem = kDmaBlocks * kDmaBlock;
     static std::atomic<bool> configured{false};    // setting the attribute twice is harmless
-    auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, QF, ODD>;
+    auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, QF>;
     if (!configured.load(std::memory_order_acquire)) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(fp8_gemm_dma_kernel, fused cast)");
@@ -1282,20 +1241,13 @@ static int launch_gemm_dma_quant_parity(const uint8_t* X, const uint8_t* Y, int 
     return MSAMP_OK;
 }
 
-template <int XF, int YF, typename OT, bool XT, bool YT, int QF>
-static int launch_gemm_dma_quant(const uint8_t* X, const uint8_t* Y, int NR, int NC, int K, const float* xs, const float* ys,
-                                 const QuantArgs& qa, hipStream_t st) {
-    if ((K / kBK) & 1) return launch_gemm_dma_quant_parity<XF, YF, OT, XT, YT, QF, true>(X, Y, NR, NC, K, xs, ys, qa, st);
-    return launch_gemm_dma_quant_parity<XF, YF, OT, XT, YT, QF, false>(X, Y, NR, NC, K, xs, ys, qa, st);
-}
-
 // the same kernel with the cast to FP8 riding along on speculation (see QSPEC above); the caller has checked the shape
-template <int XF, int YF, typename OT, bool XT, bool YT, bool ODD>
-static int launch_gemm_dma_spec_parity(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
+template <int XF, int YF, typename OT, bool XT, bool YT>
+static int launch_gemm_dma_spec(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
                                        const float* ys, int accumulate, const QuantArgs& qa, hipStream_t st) {
-    constexpr int smem = 2 * kDmaStage;
+    constexpr int smem = kDmaBlocks * kDmaBlock;
     static std::atomic<bool> configured{false};    // setting the attribute twice is harmless
-    auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, 0, ODD, true>;
+    auto kern = fp8_gemm_dma_kernel<XF, YF, OT, XT, YT, 0, true>;
     if (!configured.load(std::memory_order_acquire)) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(fp8_gemm_dma_kernel, speculative cast)");
@@ -1308,13 +1260,6 @@ static int launch_gemm_dma_spec_parity(const uint8_t* X, const uint8_t* Y, void*
                        static_cast<const void*>(nullptr), 0, qw);
     MSAMP_CHECK_LAUNCH("fp8_gemm_dma_kernel (speculative cast)");
     return MSAMP_OK;
-}
-
-template <int XF, int YF, typename OT, bool XT, bool YT>
-static int launch_gemm_dma_spec(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
-                                const float* ys, int accumulate, const QuantArgs& qa, hipStream_t st) {
-    if ((K / kBK) & 1) return launch_gemm_dma_spec_parity<XF, YF, OT, XT, YT, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, qa, st);
-    return launch_gemm_dma_spec_parity<XF, YF, OT, XT, YT, false>(X, Y, D, NR, NC, K, xs, ys, accumulate, qa, st);
 }
 
 template <int BR, int BC, int XF, int YF, typename OT, bool KGUARD>
@@ -1410,21 +1355,6 @@ static int pick_out_spec(const uint8_t* X, const uint8_t* Y, void* D, int d_dtyp
 }
 
 #ifdef MSAMP_GEMM_SPLIT_UNIT
-template <int XF, int YF>
-int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int NR, int NC, int K, const float* xs,
-                   const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
-    const bool odd = (K / kBK) & 1;
-#define MSAMP_SPLIT_LAUNCH(OT)                                                                                                         \
-    return odd ? launch_gemm_dma_parity<XF, YF, OT, false, false, true, false, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st) \
-               : launch_gemm_dma_parity<XF, YF, OT, false, false, false, false, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st)
-    switch (d_dtype) {
-        case MSAMP_DT_F32: MSAMP_SPLIT_LAUNCH(float);
-        case MSAMP_DT_F16: MSAMP_SPLIT_LAUNCH(f16_t);
-        default: MSAMP_SPLIT_LAUNCH(bf16_t);
-    }
-#undef MSAMP_SPLIT_LAUNCH
-}
-
 // output type and operand layout of a call -> one instantiation of LAUNCH<XF, YF, output type, XT, YT>
 #define MSAMP_LAYOUT_LAUNCH(LAUNCH, OT)                                                                                              \
     do {                                                                                                                             \
@@ -1443,7 +1373,7 @@ int run_gemm_split(const uint8_t* X, const uint8_t* Y, void* D, int d_dtype, int
 template <int XF, int YF, typename OT, bool XT, bool YT>
 static int launch_gemm_ragged(const uint8_t* X, const uint8_t* Y, void* D, int NR, int NC, int K, const float* xs,
                               const float* ys, int accumulate, const void* bias, int bias_dt, hipStream_t st) {
-    return launch_gemm_dma_parity<XF, YF, OT, XT, YT, false, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
+    return launch_gemm_dma_tail<XF, YF, OT, XT, YT, true>(X, Y, D, NR, NC, K, xs, ys, accumulate, bias, bias_dt, st);
 }
 template <int XF, int YF>
 int run_gemm_ragged(const GemmCall& c) {
@@ -1465,7 +1395,7 @@ int run_gemm_parts(const GemmCall& c, const KSplit& split) {
     if (!c.xt) MSAMP_PARTS_LAUNCH(false, true);
     if (split.small_tiles) MSAMP_PARTS_LAUNCH(true, true);
 #undef MSAMP_PARTS_LAUNCH
-    return launch_gemm_dma_parity<XF, YF, float, true, true, false, true>(c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, 0, nullptr, 0, c.st, split.parts);
+    return launch_gemm_dma_tail<XF, YF, float, true, true, true>(c.X, c.Y, c.D, c.NR, c.NC, c.K, c.xs, c.ys, 0, nullptr, 0, c.st, split.parts);
 }
 #endif
 
