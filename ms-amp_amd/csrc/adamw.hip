@@ -129,29 +129,78 @@ __global__ __launch_bounds__(kAdamThreads) void stage2_kernel(const float* __res
 }
 
 // ---- fused multi-tensor step -------------------------------------------------------------------
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 constexpr int kEPT = 16;                                   // elements per thread per step
 // tensors of more chunks than these look at their maxima's words before they raise them (raise_max.cuh)
 constexpr size_t kAmaxLookChunks = 320, kSpecLookChunks = 384;
+// Chunks (of 80 KiB) that the first pass reads last, with ordinary loads, because the second one, which goes back to front, finds them in
+// the memory-side cache; it reads the others past the caches.
+constexpr unsigned kAmaxKept = 3072;
 constexpr int kSteps = MSAMP_ADAMW_CHUNK / (kAdamThreads * kEPT);    // 4
 
-template <int WDT>
-__device__ __forceinline__ void load_w16(const void* base, size_t i, float* f) {
-    if constexpr (WDT == MSAMP_DT_F16) {
-        const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(base) + i);
-        uint4 a = p[0], b = p[1];
-        const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+// 16 elements of one tensor as they lie in memory
+template <int DT>
+struct Raw16 {
+    static constexpr int kWords = DT == MSAMP_DT_F16 ? 8 : 4;
+    uint32_t w[kWords];
+    __device__ __forceinline__ void load(const void* base, size_t i, bool stream = false) {
+        const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(base) + i * (kWords / 4));
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            f[2 * j] = f16_bits_to_float(w[j] & 0xffffu);
-            f[2 * j + 1] = f16_bits_to_float(w[j] >> 16);
+        for (int q = 0; q < kWords / 4; ++q) {
+            const uint4 a = ld16(p + q, stream);
+            w[4 * q] = a.x, w[4 * q + 1] = a.y, w[4 * q + 2] = a.z, w[4 * q + 3] = a.w;
         }
-    } else {
-        uint4 a = *reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(base) + i);
-        dequant4<WDT>(a.x, f[0], f[1], f[2], f[3]);
-        dequant4<WDT>(a.y, f[4], f[5], f[6], f[7]);
-        dequant4<WDT>(a.z, f[8], f[9], f[10], f[11]);
-        dequant4<WDT>(a.w, f[12], f[13], f[14], f[15]);
     }
+    __device__ __forceinline__ void launder() {
+#pragma unroll
+        for (int q = 0; q < kWords; ++q) asm volatile("" : "+v"(w[q]));
+    }
+    // elements 4q .. 4q + 3
+    __device__ __forceinline__ void quad(int q, float* f) const {
+        if constexpr (DT == MSAMP_DT_F16) {
+            f[0] = f16_bits_to_float(w[2 * q] & 0xffffu), f[1] = f16_bits_to_float(w[2 * q] >> 16);
+            f[2] = f16_bits_to_float(w[2 * q + 1] & 0xffffu), f[3] = f16_bits_to_float(w[2 * q + 1] >> 16);
+        } else {
+            dequant4<DT>(w[q], f[0], f[1], f[2], f[3]);
+        }
+    }
+    __device__ __forceinline__ void widen(float* f) const {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) quad(q, f + 4 * q);
+    }
+    // largest magnitude; a NaN comes through
+    __device__ __forceinline__ float max_abs() const {
+        if constexpr (DT == MSAMP_DT_F16) {
+            f16x2_t m = __builtin_bit_cast(f16x2_t, w[0] & 0x7fff7fffu);
+#pragma unroll
+            for (int j = 1; j < 8; ++j) m = __builtin_elementwise_maximum(m, __builtin_bit_cast(f16x2_t, w[j] & 0x7fff7fffu));
+            return __builtin_elementwise_maximum(static_cast<float>(m[0]), static_cast<float>(m[1]));
+        } else {
+            float f[16];
+            widen(f);
+            float m = fabsf(f[0]);
+#pragma unroll
+            for (int j = 1; j < 16; ++j) m = __builtin_elementwise_maximum(m, fabsf(f[j]));
+            return m;
+        }
+    }
+    // (float16) largest and smallest value; NaNs come through
+    __device__ __forceinline__ void range(float& hi, float& lo) const {
+        f16x2_t h = __builtin_bit_cast(f16x2_t, w[0]), l = h;
+#pragma unroll
+        for (int j = 1; j < 8; ++j) {
+            h = __builtin_elementwise_maximum(h, __builtin_bit_cast(f16x2_t, w[j]));
+            l = __builtin_elementwise_minimum(l, __builtin_bit_cast(f16x2_t, w[j]));
+        }
+        hi = __builtin_elementwise_maximum(static_cast<float>(h[0]), static_cast<float>(h[1]));
+        lo = __builtin_elementwise_minimum(static_cast<float>(l[0]), static_cast<float>(l[1]));
+    }
+};
+template <int DT>
+__device__ __forceinline__ void load_w16(const void* base, size_t i, float* f) {
+    Raw16<DT> r;
+    r.load(base, i);
+    r.widen(f);
 }
 
 template <int WDT>
@@ -211,48 +260,136 @@ __device__ __forceinline__ void load16(const msamp_adamw_tensor& d, size_t i, fl
     load_w16<MSAMP_DT_F16>(d.exp_avg_sq, i, v);
 }
 
-// One lane's 16 elements of the first pass (p, g, m, v hold the dequantized stored values on entry).
+// What a lane needs of 16 elements, as it lies in memory.
+template <int WDT, int GDT>
+struct RawState {
+    Raw16<WDT> w;
+    Raw16<GDT> g;
+    Raw16<MSAMP_DT_E4M3> m;
+    Raw16<MSAMP_DT_F16> v;
+    __device__ __forceinline__ void load(const msamp_adamw_tensor& d, size_t i, bool stream) {
+        w.load(d.weight, i, stream), g.load(d.grad, i, stream), m.load(d.exp_avg, i, stream), v.load(d.exp_avg_sq, i, stream);
+    }
+    // Makes the compiler forget what it has worked out from the words (the widened values of all 16 elements, kept for later).
+    __device__ __forceinline__ void launder() { w.launder(), g.launder(), m.launder(), v.launder(); }
+};
+
+// One lane's 16 elements of the first pass, from i on.
 // Only bounds on |p'| are needed here: |p| - D <= |p'| <= |p| + D with D >= |step * m' / (sqrt(v') / sbc2 + eps)|,
 // and since eps >= 0 the quotient is at most sbc2 / sqrt(v') and at most 1 / eps.  k.bound_rsq and k.bound_eps hold
 // |step| times those two factors, widened by 4e-6 for the roundings of both chains (the exact one has six, the
 // hardware reciprocal square root is good to one ulp).  A NaN or negative v' keeps its NaN through the selection.
-template <bool L2>
-__device__ __forceinline__ void amax_step(float* p, const float* g, float* m, float* v, float w_si, float g_si, float inv_m,
-                                          float inv_v, const AdamConsts& k, float& floor_p, uint32_t& mxp, float& mxm,
+// (The few elements next to the maximum take the exact chain from the words in registers: fetched again, they held up a step that
+// evaluates by as much as all the rest of it.)
+template <int WDT, int GDT, bool L2>
+__device__ __forceinline__ void amax_step(const RawState<WDT, GDT>& r, float w_si, float g_si,
+                                          float inv_m, float inv_v, const AdamConsts& k, float& floor_p, uint32_t& mxp, float& mxm,
                                           float& mxv) {
     float hi[kEPT];
     float lo_max = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kEPT; ++j) {
-        float pj, g_plain, m_new, v_new;
-        prepare<L2>(p[j], g[j], m[j], v[j], w_si, g_si, inv_m, inv_v, k, pj, g_plain, m_new, v_new);
-        const float t = k.bound_rsq * __builtin_amdgcn_rsqf(v_new);
-        const float lim = k.bound_eps < t ? k.bound_eps : t;
-        const float dmax = fabsf(m_new) * lim;
-        mxm = fmaxf(mxm, fabsf(m_new));
-        mxv = fmaxf(mxv, fabsf(v_new));
-        p[j] = pj, m[j] = m_new, v[j] = v_new;
-        hi[j] = fabsf(pj) + dmax;
-        lo_max = fmaxf(lo_max, fabsf(pj) - dmax);    // NaN bounds are skipped here, caught below
+    for (int q = 0; q < 4; ++q) {
+        float p[4], g[4], m[4], v[4];
+        r.w.quad(q, p), r.g.quad(q, g), r.m.quad(q, m), r.v.quad(q, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float pj, g_plain, m_new, v_new;
+            prepare<L2>(p[e], g[e], m[e], v[e], w_si, g_si, inv_m, inv_v, k, pj, g_plain, m_new, v_new);
+            const float t = k.bound_rsq * __builtin_amdgcn_rsqf(v_new);
+            const float lim = k.bound_eps < t ? k.bound_eps : t;
+            const float dmax = fabsf(m_new) * lim;
+            mxm = fmaxf(mxm, fabsf(m_new));
+            mxv = fmaxf(mxv, fabsf(v_new));
+            hi[4 * q + e] = fabsf(pj) + dmax;
+            lo_max = fmaxf(lo_max, fabsf(pj) - dmax);    // NaN bounds are skipped here, caught below
+        }
     }
     floor_p = fmaxf(floor_p, __uint_as_float(wave_max_u32(__float_as_uint(lo_max))));
     // the additions above and the last subtraction of the exact chain round once each: leave room for them
     const float skip_below = floor_p * 0.999999f;
+    uint32_t near = 0;
+#pragma unroll
+    for (int j = 0; j < kEPT; ++j) near |= !(hi[j] < skip_below) ? 1u << j : 0u;
+    if (near == 0u) return;
 #pragma unroll
     for (int j = 0; j < kEPT; ++j) {
-        if (!(hi[j] < skip_below)) {
-            const uint32_t ab = __float_as_uint(param_update(p[j], m[j], v[j], k)) & 0x7fffffffu;
+        if (near & (1u << j)) {
+            float p[4], g[4], m[4], v[4];
+            r.w.quad(j / 4, p), r.g.quad(j / 4, g), r.m.quad(j / 4, m), r.v.quad(j / 4, v);
+            const int e = j & 3;
+            float pj, g_plain, m_new, v_new;
+            prepare<L2>(p[e], g[e], m[e], v[e], w_si, g_si, inv_m, inv_v, k, pj, g_plain, m_new, v_new);
+            const uint32_t ab = __float_as_uint(param_update(pj, m_new, v_new, k)) & 0x7fffffffu;
             mxp = ab > mxp ? ab : mxp;
         }
     }
 }
 
-// First pass: exact max |m'| and |v'| (they are cheap), and the exact max |p'| found by bounding:
-// every element gets cheap bounds; only elements whose upper bound reaches the best lower bound
-// seen so far (by this wavefront, or already published for the tensor) are evaluated exactly.  The
-// element that attains the true maximum always passes that test, so the result is the exact maximum.
+// Factors of bounds16(), the same for all elements of a tensor.
+struct RatioBound {
+    float m, g;    // |m'| / sqrt(v') <= m * max(|m_raw| / sqrt(v_raw)) + g
+};
+// m' = beta1 m + omb1 g and v' = beta2 v + omb2 g^2, where neither part of v' is negative, so |m'| / sqrt(v') is at most
+// beta1 |m| / sqrt(beta2 v) + omb1 |g| / sqrt(omb2 g^2).  The factors are widened for the roundings of the chain.
+__device__ __forceinline__ RatioBound ratio_bound(float inv_m, float inv_v, const AdamConsts& k) {
+    return {1.00001f * k.beta1 * inv_m / sqrtf(k.beta2 * inv_v), 1.00001f * k.omb1 / sqrtf(k.omb2)};
+}
+// Do bounds16()'s bounds hold: factors without surprises, and no g^2 of a code but zero underflows.
+__device__ __forceinline__ bool bounds_hold(float g_si, float inv_m, float inv_v, const AdamConsts& k) {
+    auto fine = [](float x) { return x >= 0x1.0p-60f && x <= 0x1.0p60f; };
+    return fine(inv_m) && fine(inv_v) && fine(fabsf(g_si) * 0x1.0p20f) && k.beta1 >= 0.0f && k.omb1 >= 0.0f && fine(k.beta2) && fine(k.omb2);
+}
+// Upper bounds of |p'|, |m'| and |v'| over 16 elements, without evaluating them (decoupled decay only).  |m'| and |v'|: every operation
+// of prepare() is monotonic in the magnitudes, rounding included, so the chain of the largest magnitudes is a bound without any slack.
+// |p'|: amax_step()'s |p| + D with D from the ratio above, where max(m^2 / v) comes from the codes as they are: an E4M3 code c is at
+// most 2^(c/8 - 7 + 0.0861), a float16 pattern b > 0 at least 2^((b + 10 min(b, 1024)) / 1024 - 25) (b/1024 - 15 for normal ones; below,
+// 11 b/1024 - 25 <= log2(b) - 24, the logarithm being concave and no smaller at 1 and at 1024), so that e = 256 c - b - 10 min(b, 1024), which
+// takes packed 16-bit operations, gives m^2 / v <= 2^(e/1024 + 11.1722); 24576 is added to stay above zero wherever it matters.  (The
+// largest |m'| over the smallest v' of 16 would be far too wide: one element in a thousand has hardly any v, and then all 1024 are
+// evaluated.)  Where a v is zero that is what is left.  NaN where anything is NaN.
+template <int WDT, int GDT>
+__device__ __forceinline__ void bounds16(const Raw16<WDT>& rw, const Raw16<GDT>& rg, const Raw16<MSAMP_DT_E4M3>& rm,
+                                         const Raw16<MSAMP_DT_F16>& rv, float w_si, float g_si, float inv_m, float inv_v,
+                                         const RatioBound& rb, const AdamConsts& k, float& up, float& um, float& uv) {
+#pragma clang fp contract(off)
+    typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+    float v_hi, v_lo;
+    rv.range(v_hi, v_lo);
+    u16x2_t most = {0, 0};
+    auto ratio = [&](uint32_t m, uint32_t v) __attribute__((always_inline)) {
+        const u16x2_t b = __builtin_bit_cast(u16x2_t, v), ten = {10, 10}, normal = {1024, 1024};
+        most = __builtin_elementwise_max(most, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2_t, m + 0x60006000u),
+                                                                           static_cast<u16x2_t>(b + ten * __builtin_elementwise_min(b, normal))));
+    };
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        // elements 1 and 3, 0 and 2 of four
+        ratio(rm.w[q] & 0x7f007f00u, __builtin_amdgcn_perm(rv.w[2 * q + 1], rv.w[2 * q], 0x07060302u));
+        ratio((rm.w[q] << 8) & 0x7f007f00u, __builtin_amdgcn_perm(rv.w[2 * q + 1], rv.w[2 * q], 0x05040100u));
+    }
+    const float root = __builtin_amdgcn_exp2f(static_cast<float>(most[0] > most[1] ? most[0] : most[1]) * (0.5f / 1024.0f) - 6.41f);    // sqrt
+    const float p = rw.max_abs() * fabsf(w_si) * fabsf(k.decay), g = rg.max_abs() * fabsf(g_si);
+    um = (k.beta1 * rm.max_abs()) * inv_m + k.omb1 * g;
+    const float gg = g * g;
+    uv = (k.beta2 * v_hi) * inv_v + k.omb2 * gg;
+    const float t = k.bound_rsq * __builtin_amdgcn_rsqf((k.beta2 * v_lo) * inv_v);
+    float d = um * (k.bound_eps < t ? k.bound_eps : t);
+    if (v_lo > 0.0f) d = fminf(d, k.bound_rsq * (rb.m * root + rb.g));
+    up = p + d;
+}
+
+// First pass: the exact maxima of |p'|, |m'| and |v'| by bounding.  A wavefront's 1024 elements are evaluated (amax_step) only if the
+// bounds over some lane's 16 of them reach above the maxima found so far, by this wavefront or, as published when its workgroup began,
+// by others; the elements that attain the true maxima always do.  The workgroups that run first in a tensor have nothing to compare
+// with and evaluate everything: all of a tensor of up to about a thousand chunks, a third of one of three thousand.
+// The evaluation takes 28 vector instructions an element, with a reciprocal square root, the bounds 10: evaluating everything bound the pass
+// to 4.3 TB/s, now it is bound by its read of 5 bytes an element.  405 M parameters in ten tensors, E4M3 weights, the step: 1070 -> 1001 us
+// repeated, 1084 -> 1023 where other data has passed the caches in between; one tensor of 50 M 139 -> 123; float16 weights 1287 -> 1214.
+// Tried: several chunks to a workgroup, to compare with more (fewer and longer workgroups read more slowly: 550 us); chunks of sixteen tensors
+// side by side (3 % evaluated, and slower by 20 us: the order of the reads); a few workgroups publishing early, or looking again while
+// there is nothing (slower by 30 to 80 us: every look and atomic of a tensor meets at one line).
 template <int WDT, int GDT, bool L2>
-__global__ __launch_bounds__(kAdamThreads) void fused_amax_kernel(msamp_adamw_tensor* __restrict__ tensors,
+__global__ __launch_bounds__(kAdamThreads, 4) void fused_amax_kernel(msamp_adamw_tensor* __restrict__ tensors,
                                                                    const int32_t* __restrict__ block_map,
                                                                    AdamConsts k) {
     __shared__ uint32_t red[kAdamThreads / kWave];
@@ -264,18 +401,38 @@ __global__ __launch_bounds__(kAdamThreads) void fused_amax_kernel(msamp_adamw_te
     const float inv_m = 1.0f / *d.m_scale, inv_v = 1.0f / *d.v_scale;
     uint32_t mxp = 0;    // exact |p'| bit patterns of the candidates (NaN patterns compare highest)
     float mxm = 0.0f, mxv = 0.0f;
-    // lower bound on the tensor's max |p'|: what other workgroups have published so far
-    float floor_p = __uint_as_float(__hip_atomic_load(&d.acc[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    // lower bounds on the tensor's maxima: what other workgroups have published so far
+    float floor_p = __uint_as_float(seen_word(&d.acc[0])), floor_m = __uint_as_float(seen_word(&d.acc[1])), floor_v = __uint_as_float(seen_word(&d.acc[2]));
     if (!(floor_p >= 0.0f)) floor_p = 0.0f;    // a NaN already published: everything is exact from here on
+    bool evaluated = false;
+    const bool stream = blockIdx.x + kAmaxKept < gridDim.x;
     if (base + MSAMP_ADAMW_CHUNK <= n) {
+        const bool usable = !L2 && bounds_hold(g_si, inv_m, inv_v, k);
+        const RatioBound rb = ratio_bound(inv_m, inv_v, k);
 #pragma unroll 1
         for (int s = 0; s < kSteps; ++s) {
             const size_t i = base + (static_cast<size_t>(s) * kAdamThreads + threadIdx.x) * kEPT;
-            float p[kEPT], g[kEPT], m[kEPT], v[kEPT];
-            load16<WDT, GDT>(d, i, p, g, m, v);
-            amax_step<L2>(p, g, m, v, w_si, g_si, inv_m, inv_v, k, floor_p, mxp, mxm, mxv);
+            RawState<WDT, GDT> r;
+            if (stream) {
+                r.load(d, i, true);
+                asm volatile("" : : : "memory");    // (or the two become one, without the mark)
+            } else {
+                r.load(d, i, false);
+            }
+            if (!L2 && usable && floor_v > 0.0f) {
+                float up, um, uv;
+                bounds16<WDT, GDT>(r.w, r.g, r.m, r.v, w_si, g_si, inv_m, inv_v, rb, k, up, um, uv);
+                // (0.999999: as in amax_step)
+                if (__all(up < floor_p * 0.999999f && um <= floor_m && uv <= floor_v)) continue;
+            }
+            evaluated = true;
+            r.launder();
+            amax_step<WDT, GDT, L2>(r, w_si, g_si, inv_m, inv_v, k, floor_p, mxp, mxm, mxv);
+            floor_m = fmaxf(floor_m, __uint_as_float(wave_max_u32(__float_as_uint(mxm))));
+            floor_v = fmaxf(floor_v, __uint_as_float(wave_max_u32(__float_as_uint(mxv))));
         }
     } else {
+        evaluated = true;
         for (size_t i = base + threadIdx.x; i < n; i += kAdamThreads) {
             float pj, g_plain, m_new, v_new;
             prepare<L2>(load_w1<WDT>(d.weight, i), load_w1<GDT>(d.grad, i), load_w1<MSAMP_DT_E4M3>(d.exp_avg, i),
@@ -286,6 +443,7 @@ __global__ __launch_bounds__(kAdamThreads) void fused_amax_kernel(msamp_adamw_te
             mxv = fmaxf(mxv, fabsf(v_new));
         }
     }
+    if (!__syncthreads_or(evaluated)) return;
     const uint32_t a = block_max_u32(mxp, red);
     const uint32_t b = block_max_u32(__float_as_uint(mxm), red);
     const uint32_t c = block_max_u32(__float_as_uint(mxv), red);

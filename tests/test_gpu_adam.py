@@ -235,6 +235,38 @@ def test_maxima_of_tensors_around_the_looking_lines(be, chunks):
             assert all(same_float(x, y) for k in ('wm', 'mm', 'vm') for x, y in zip(d[k], first[k])), n
 
 
+@pytest.mark.parametrize('w_fmt,w_dt,g_fmt,g_dt', [(fp8.E4M3, 5, fp8.E5M2, 6), ('f16', 3, fp8.E4M3, 5), (fp8.E5M2, 6, fp8.E5M2, 6)])
+@pytest.mark.parametrize('plant', ['nothing', 'weight', 'hardly any v', 'no v', 'moment', 'gradient', 'second moment', 'negative v', 'nan'])
+def test_first_pass_evaluates_whatever_may_hold_a_maximum(be, w_fmt, w_dt, g_fmt, g_dt, plant):
+    """The first pass skips elements whose bounds stay below what other workgroups have published.  A tensor of 1700 chunks, of
+    which the last third runs behind the first, with one element there that decides a maximum by each way a bound knows; against the
+    one-pass step, which looks at every element."""
+    n = 1700 * be.ADAMW_CHUNK + 77
+    t = _inputs(1 << 18, 60, w_fmt, g_fmt)
+    for key in 'wgmv':
+        t[key] = t[key].repeat((n >> 18) + 1)[:n].clone()
+    # as after some steps: v about g^2, with a few elements that have hardly any
+    t['v'][5::1009], t['m'][5::1009] = 3.0 * 2.0**-24, 1
+    at = n - 40 * be.ADAMW_CHUNK + 4321
+    if plant == 'weight':
+        t['w'][at] = t['w'].max() if w_fmt == 'f16' else 0x7e if w_fmt == fp8.E4M3 else 0x7b
+    elif plant in ('hardly any v', 'no v'):
+        t['m'][at], t['v'][at], t['g'][at] = 0x30, 2.0**-24 if plant == 'hardly any v' else 0.0, 0
+    elif plant == 'moment':
+        t['m'][at] = 0xfe
+    elif plant == 'gradient':
+        t['g'][at] = 0xfe if g_fmt == fp8.E4M3 else 0xfb
+    elif plant == 'second moment':
+        t['v'][at] = 65504.0
+    elif plant == 'negative v':
+        t['v'][at] = -1.0
+    elif plant == 'nan':
+        t['m'][at] = 0x7f
+    two = _fused(be, [t], w_dt, g_dt, 7)[0]
+    one = _fused(be, [t], w_dt, g_dt, 7, speculative=True)[0]
+    assert _same_state(two, one)
+
+
 def _same_state(a, b):
     bits = lambda t: t.view(torch.int32) if t.dtype == torch.float32 else (t.view(torch.int16) if t.dtype == torch.float16 else t)
     return all(torch.equal(bits(x), bits(y)) for x, y in zip([a['w'], a['m'], a['v']] + a['wm'] + a['mm'] + a['vm'],
