@@ -20,38 +20,58 @@ namespace msamp {
 // y[tokens][d_out] = x . fp8(w)^T, the weight read in its scaled 16- or 32-bit form and quantized on its way to the matrix pipes,
 // with the codes msamp_cast_scaled_to_fp8 gives: it is read once (2 bytes an element), where the cast and the product move 4.
 // Bound by that read and by the codes of x, which every workgroup reads again out of the L2: 48 tokens through 4096 -> 12288 are
-// 2.75 M requests of the L1s to it, 0.86 M of which miss (0.79 M are the weight's lines), and the waves spend 0.38 of their time
-// waiting for loads and 0.46 for their turn to issue.  A workgroup takes 16 rows of w and all tokens; its (up to)
-// eight wavefronts take the 128-wide slices of K in turn, the next slice's weights in flight over the present one's arithmetic,
-// and their float32 sums meet in LDS in a fixed order.
-// Inside a slice the k of an MFMA's operand bytes are dealt out anew, alike for both operands: lane group g holds k = 16 g .. +15
-// and 64 + 16 g .. +15, so that w arrives in pairs of loads over whole lines.  x comes in the order of the operand registers from
-// its cast (few_cast_fragments): read row by row, 16 rows a long power of two apart, it
-// cost as much as w (48 tokens 7 us more).  Both casts and the product together against the weight cast to memory and the product
-// after it, replayed from a graph, us for 4096 -> 12288: 16 tokens 47.1 -> 26.7, 48 47.5 -> 32.0, 64 48.3 -> 34.3; 64 x 8192 -> 8192
-// 64.0 -> 45.4, 64 x 16384 -> 4096 82.1 -> 49.2, 64 x 2048 -> 16384 33.1 -> 23.4, 16 x 512 -> 512 14.3 -> 6.6 (launches).  Where d_out
-// gives a few workgroups and K is long, the product in parts of K that a forward with gradients takes is ahead of it by now:
-// 64 x 16384 -> 256 52.6 before either, 31.0 here, 23.1 in parts.
+// 2.75 M requests of the L1s to it, 0.86 M of which miss (0.79 M are the weight's lines).  A workgroup takes 16 rows of w and all
+// tokens; its wavefronts take the 128-wide slices of K in turn, and their float32 sums meet in LDS in a fixed order.
+// A load of w covers whole rows of the slice (16-bit: four of 256 bytes): it is read as it would be for a matrix instruction, 16 rows
+// to a load, at 0.85 of that speed (100 MB by nothing but such loads: 19.0 us, 16.2).  The codes go through 2 KiB of LDS that is the
+// wavefront's own, where the operand's registers find them, and the loads of the next slice are on their way as soon as the codes
+// are made: into the same registers, which leaves room for another workgroup.  Inside a slice the k of an MFMA's operand bytes are
+// dealt out anew, alike for both operands: lane group g holds k = 16 g .. +15 and 64 + 16 g .. +15.  x comes in the order of the
+// operand registers from its cast (few_cast_fragments): read row by row, 16 rows a long power of two apart, it cost as much as w
+// (48 tokens 7 us more).  Both casts and the product together, replayed from a graph, us, with the weight cast to memory and the
+// product after it | with the weight read in the operand's order and quantized one by one | now, for 4096 -> 12288: 16 tokens
+// 47.1 | 29.4 | 23.0, 48 47.5 | 34.4 | 28.5, 64 48.3 | 37.8 | 31.8; 64 x 8192 -> 8192 64.0 | 48.5 | 40.3, 64 x 16384 -> 4096 82.1 | 52.3 | 43.8,
+// 64 x 2048 -> 16384 33.1 | 25.9 | 21.5, 16 x 512 -> 512 14.3 | 6.9 | 6.7 (launches).  Where d_out gives a few workgroups and K is long,
+// the product in parts of K that a forward with gradients takes was ahead by a little: 64 x 16384 -> 256 32.9 | 25.0, 23.1 in parts.
 __device__ __forceinline__ float few_bias(const void* bias, int dt, int i) {
     if (dt == MSAMP_DT_F32) return static_cast<const float*>(bias)[i];
     if (dt == MSAMP_DT_F16) return f16_bits_to_float(static_cast<const uint16_t*>(bias)[i]);
     return bf16_bits_to_float(static_cast<const uint16_t*>(bias)[i]);
 }
 typedef int few_v8i __attribute__((ext_vector_type(8)));
+typedef short few_v2s __attribute__((ext_vector_type(2)));
+// Four 16-bit weights times a power of two to E4M3 codes, by one instruction a pair where quant4 takes ten with the widening: the same
+// codes, but 0x7f (NaN) for whatever lies beyond the format, which quant4 saturates (all patterns of both types at 61 scales).  A slice
+// with such a code is quantized again by quant4, and so is every slice whose factor is no power of two.  Alone it gave 1 us of 30.
+template <typename WT>
+__device__ __forceinline__ uint32_t few_codes4(uint32_t lo, uint32_t hi, float inv_scale) {
+    few_v2s q = {0, 0};
+    if constexpr (__is_same(WT, bf16_t)) {
+        typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(q, __builtin_bit_cast(v2b, lo), inv_scale, false);
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(q, __builtin_bit_cast(v2b, hi), inv_scale, true);
+    } else {
+        typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(q, __builtin_bit_cast(v2h, lo), inv_scale, false);
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(q, __builtin_bit_cast(v2h, hi), inv_scale, true);
+    }
+    return __builtin_bit_cast(uint32_t, q);
+}
 typedef float few_v4f __attribute__((ext_vector_type(4)));
 
-template <typename WT, typename OT, int MB>
+template <typename WT, typename OT, int MB, bool STREAM>
 __global__ __launch_bounds__(512) void few_tokens_kernel(const WT* __restrict__ w, const uint8_t* __restrict__ x, OT* __restrict__ y,
                                                           int tokens, int d_out, int K, const float* __restrict__ w_amax,
                                                           const float* __restrict__ w_scale_inv, const float* __restrict__ x_scale_inv,
-                                                          const void* __restrict__ bias, int bias_dt, int stream) {
+                                                          const void* __restrict__ bias, int bias_dt) {
     extern __shared__ __attribute__((aligned(16))) float4 few_part[];    // [wavefronts][MB][64]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int l16 = lane & 15, g4 = lane >> 4;
     const float s_new = scale_rule(*w_amax, 1.0f, 448.0f, 0);
     const float s = s_new * *w_scale_inv;
-    // (rows past the end are clamped: their products land in outputs that are not stored)
-    const WT* wp = w + static_cast<size_t>(min(static_cast<int>(blockIdx.x) * 16 + l16, d_out - 1)) * K + g4 * 16;
+    const uint32_t s_exp = __float_as_uint(s) >> 23;
+    const bool pow2 = sizeof(WT) == 2 && (__float_as_uint(s) & 0x7fffffu) == 0u && s_exp >= 127u - 30u && s_exp <= 127u + 30u;
+    const float s_inv = 1.0f / s;
     const uint8_t* xp = x + lane * 16;
     const int slices = (K + 127) / 128;
     few_v4f acc[MB];
@@ -59,40 +79,75 @@ __global__ __launch_bounds__(512) void few_tokens_kernel(const WT* __restrict__ 
     for (int b = 0; b < MB; ++b) acc[b] = few_v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
     constexpr int kPer = 16 / static_cast<int>(sizeof(WT));    // weights of a 16-byte load
-    constexpr int kHalf = 16 / kPer;                           // loads of half a slice
-    struct Weights { uint4 v[2][kHalf]; };
-    // (K is a multiple of 16: the 16 k of a lane group's half slice lie inside together or not at all)
-    auto inside = [&](int kt, int h) __attribute__((always_inline)) { return kt * 128 + h * 64 + g4 * 16 < K; };
+    constexpr int kAcross = 128 / kPer;                        // lanes to a row of a slice
+    constexpr int kRows = 64 / kAcross, kLoads = 16 / kRows;   // rows of a load, loads of a slice
+    const int k_lane = lane % kAcross * kPer, r_lane = lane / kAcross;
+    struct Weights { uint4 v[kLoads]; };
+    // (rows past the end are clamped: their products land in outputs that are not stored)
+    const WT* wp[kLoads];
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) wp[j] = w + static_cast<size_t>(min(static_cast<int>(blockIdx.x) * 16 + j * kRows + r_lane, d_out - 1)) * K;
+    // (K is a multiple of 16: the k of a load lie inside together or not at all.  A load past the end reads the row's last 16 bytes
+    // instead: loads that may or may not be made can't be counted, and the product then waits for the next slice's weights)
     auto fetch = [&](int kt, Weights& f) __attribute__((always_inline)) {
+        const int k = min(kt * 128 + k_lane, K - kPer);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (!inside(kt, h)) continue;
-#pragma unroll
-            for (int j = 0; j < kHalf; ++j) f.v[h][j] = ld16(wp + kt * 128 + h * 64 + j * kPer, stream != 0);
-        }
+        for (int j = 0; j < kLoads; ++j) f.v[j] = ld16(wp[j] + k, STREAM);
     };
-    // the product of slice kt, whose weights are in `f`, and the loads of the wavefront's next slice into `next`
-    auto work = [&](int kt, const Weights& f, Weights& next) __attribute__((always_inline)) {
+    uint8_t* const codes = reinterpret_cast<uint8_t*>(few_part + waves * MB * 64) + wave * 2048;    // of a slice, 128 bytes a row
+    // where the codes of load j go: 16-byte chunk c of row r lies at c ^ (r % 8)
+    auto code_at = [&](int j) __attribute__((always_inline)) {
+        const int r = j * kRows + r_lane;
+        return codes + r * 128 + (((k_lane >> 4) ^ (r & 7)) << 4) + (k_lane & 15);
+    };
+    Weights f = {};
+    if (wave < slices) fetch(wave, f);
+    for (int kt = wave; kt < slices; kt += waves) {
         uint4 xr[MB][2];
 #pragma unroll
         for (int b = 0; b < MB; ++b)
 #pragma unroll
             for (int h = 0; h < 2; ++h) xr[b][h] = *reinterpret_cast<const uint4*>(xp + ((static_cast<size_t>(kt) * MB + b) * 2 + h) * 1024);
-        if (kt + waves < slices) fetch(kt + waves, next);
+        const bool in = kt * 128 + k_lane < K;    // (the ragged last slice: what was not loaded is zero)
+        bool done = false;
+        if constexpr (sizeof(WT) == 2) {
+            if (pow2) {
+                uint2 c[kLoads];
+                uint32_t odd = 0u;    // high bits: a code of all ones below its sign
+#pragma unroll
+                for (int j = 0; j < kLoads; ++j) {
+                    c[j] = make_uint2(few_codes4<WT>(f.v[j].x, f.v[j].y, s_inv), few_codes4<WT>(f.v[j].z, f.v[j].w, s_inv));
+                    if (!in) c[j] = make_uint2(0u, 0u);
+                    odd |= ((c[j].x & 0x7f7f7f7fu) + 0x01010101u) | ((c[j].y & 0x7f7f7f7fu) + 0x01010101u);
+                    *reinterpret_cast<uint2*>(code_at(j)) = c[j];
+                }
+                done = !__any((odd & 0x80808080u) != 0u);
+            }
+        }
+        if (!done) {
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j) {
+                float v[kPer];
+                In16<WT>::decode(f.v[j], v);
+#pragma unroll
+                for (int e = 0; e < kPer / 4; ++e) {
+                    const uint32_t c = quant4<MSAMP_DT_E4M3>(v[4 * e] * s, v[4 * e + 1] * s, v[4 * e + 2] * s, v[4 * e + 3] * s);
+                    *reinterpret_cast<uint32_t*>(code_at(j) + 4 * e) = in ? c : 0u;
+                }
+            }
+        }
+        fetch(kt + waves, f);
+        // (the rows are this wavefront's own and the LDS serves its requests in order: only the compiler has to keep them so)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
         few_v8i a;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            float v[16];
-#pragma unroll
-            for (int j = 0; j < kHalf; ++j) In16<WT>::decode(f.v[h][j], v + j * kPer);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                a[h * 4 + j] = static_cast<int>(quant4<MSAMP_DT_E4M3>(v[4 * j] * s, v[4 * j + 1] * s, v[4 * j + 2] * s, v[4 * j + 3] * s));
+            const uint4 c = *reinterpret_cast<const uint4*>(codes + l16 * 128 + (((g4 + 4 * h) ^ (l16 & 7)) << 4));
+            a[h * 4] = c.x, a[h * 4 + 1] = c.y, a[h * 4 + 2] = c.z, a[h * 4 + 3] = c.w;
         }
-        if (kt * 128 + 128 > K) {    // the ragged last slice: what was not loaded is zero
-#pragma unroll
-            for (int i = 0; i < 8; ++i) a[i] = inside(kt, i >> 2) ? a[i] : 0;
-        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");    // (and the next slice's codes behind these reads)
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int b = 0; b < MB; ++b) {
             few_v8i bx;
@@ -100,16 +155,6 @@ __global__ __launch_bounds__(512) void few_tokens_kernel(const WT* __restrict__ 
             for (int h = 0; h < 2; ++h) bx[h * 4] = xr[b][h].x, bx[h * 4 + 1] = xr[b][h].y, bx[h * 4 + 2] = xr[b][h].z, bx[h * 4 + 3] = xr[b][h].w;
             acc[b] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, bx, acc[b], 0, 0, 0, 0, 0, 0);
         }
-    };
-    Weights even = {}, odd = {};
-    int kt = wave;
-    if (kt < slices) fetch(kt, even);
-    while (kt < slices) {
-        work(kt, even, odd);
-        kt += waves;
-        if (kt >= slices) break;
-        work(kt, odd, even);
-        kt += waves;
     }
 #pragma unroll
     for (int b = 0; b < MB; ++b) few_part[(wave * MB + b) * 64 + lane] = make_float4(acc[b][0], acc[b][1], acc[b][2], acc[b][3]);
@@ -148,11 +193,16 @@ __global__ __launch_bounds__(512) void few_tokens_kernel(const WT* __restrict__ 
 template <typename WT, typename OT, int MB>
 static int launch_few_tokens(const msamp_linear_forward_args& a, hipStream_t st) {
     const int tokens = static_cast<int>(a.tokens), d_out = static_cast<int>(a.d_out), K = static_cast<int>(a.d_in);
-    const int waves = std::min(8, (K + 127) / 128);    // (four are level with eight, but for one round of few workgroups: 16 x 12288 -> 4096 34.2, 30.5)
-    hipLaunchKernelGGL((few_tokens_kernel<WT, OT, MB>), dim3((d_out + 15) / 16), dim3(64 * waves), waves * MB * 1024, st,
+    // Up to two workgroups of eight wavefronts fit a CU, and what no longer fits at once begins a round of its own: beyond 512
+    // workgroups they are of four, five a CU.  us with eight and four: 48 x 4096 -> 12288 33.3, 28.5, 64 x 4096 -> 11008 33.1, 28.0,
+    // 64 x 2048 -> 16384 23.0, 21.5, 48 x 4096 -> 32000 66.4, 64.3; up to 512, 48 x 1040 -> 6000 11.1, 10.9, 64 x 4096 -> 8192 20.9, 21.0,
+    // 16 x 8192 -> 8192 30.1, 32.6, 32 x 11008 -> 4096 24.9, 27.1.
+    const int waves = std::min(d_out > 512 * 16 ? 4 : 8, (K + 127) / 128);
+    const bool stream = static_cast<size_t>(d_out) * K * sizeof(WT) >= kStreamBytes;
+    const auto kernel = stream ? few_tokens_kernel<WT, OT, MB, true> : few_tokens_kernel<WT, OT, MB, false>;
+    hipLaunchKernelGGL(kernel, dim3((d_out + 15) / 16), dim3(64 * waves), waves * (MB * 1024 + 2048), st,
                        static_cast<const WT*>(a.w), a.x_codes, static_cast<OT*>(a.y), tokens, d_out, K, a.w_amax, a.w_scale_inv,
-                       a.x_scale_inv, a.bias, static_cast<int>(a.bias_dtype),
-                       static_cast<int>(static_cast<size_t>(d_out) * K * sizeof(WT) >= kStreamBytes));
+                       a.x_scale_inv, a.bias, static_cast<int>(a.bias_dtype));
     MSAMP_CHECK_LAUNCH("few_tokens_kernel");
     return MSAMP_OK;
 }

@@ -1126,6 +1126,33 @@ def test_a_few_tokens_without_gradients_lose_no_precision():
         assert rel_fro(few.double(), exact) <= 1.1 * rel_fro(y.double(), exact) + 1e-7
 
 
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('exponent', [0, 6, -5, 29, 30, 31, -30, -31, None])
+def test_a_few_tokens_quantize_every_weight_as_the_cast_does(dtype, exponent):
+    """x is the identity, so that the outputs are the codes of w themselves: all 65536 patterns of a 16-bit type in rows of 64 (whole
+    rows in and beyond the format's range, and both in one), times powers of two that one instruction takes, that it doesn't, and
+    a factor that is none."""
+    from msamp import _backend
+    w = torch.arange(65536, dtype=torch.int32, device='cuda').to(torch.int16).view(dtype).view(1024, 64)
+    x = torch.eye(64, device='cuda', dtype=torch.bfloat16)
+    x_meta, w_meta = (ScalingMeta(Dtypes.kfloat8_e4m3, window_size=16) for _ in range(2))
+    x_meta.amax_counter.fill_(16)
+    w_meta.amax.fill_(448.0)    # (the rule's scale is 1: the factor is scale_inv)
+    w_meta.scale_inv.fill_(3.0 if exponent is None else 2.0**exponent)
+    want = _backend.linear_forward(x, x_meta, w, w_meta, torch.float32, None)[0]
+    got = _backend.linear_forward(x, x_meta, w, w_meta, torch.float32, None, want_codes=False)[0]
+    nan = w.isnan().any(1)    # (0 times NaN: such a row of w is NaN in every token)
+    assert got[:, nan].isnan().all() and not got[:, ~nan].isnan().any()
+    assert torch.equal(got[:, ~nan].view(torch.int32), want[:, ~nan].view(torch.int32))
+    # the same patterns shuffled over the rows: a wavefront's slice has lanes of both kinds
+    finite = w.view(-1)[~w.view(-1).isnan()]
+    order = torch.randperm(finite.numel(), device='cuda', generator=torch.Generator(device='cuda').manual_seed(3))
+    w = finite[order][:finite.numel() // 64 * 64].view(-1, 64).contiguous()
+    want = _backend.linear_forward(x, x_meta, w, w_meta, torch.float32, None)[0]
+    got = _backend.linear_forward(x, x_meta, w, w_meta, torch.float32, None, want_codes=False)[0]
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
 @pytest.mark.parametrize('tokens,d_in,d_out', [(65, 2064, 132), (300, 8200, 70), (129, 272, 2500), (70, 4096, 4111)])
 @pytest.mark.parametrize('dtype,bias', [(torch.bfloat16, True), (torch.float16, False), (torch.float32, True)])
 def test_products_of_a_few_tiles_in_parts_of_k(monkeypatch, tokens, d_in, d_out, dtype, bias):
