@@ -34,8 +34,15 @@ constexpr int kMaxPartials = 1024;
 // run when the rule gives another scale
 constexpr int kWsSpecDone = 9;
 constexpr int kWsGuess = 13;
-// word kWsMissed: non-zero when that pass met a value too large for its guess and wrote no further output
+// word kWsMissed: non-zero when a pass with a guess from a sample met a value too large for it: the bits of infinity less those of
+// the scale it went on with (so that the smallest scale is the largest word; those of infinity themselves: none)
 constexpr int kWsMissed = 14;
+// behind the partial maxima of such a pass, a word per workgroup: the exponent of the scale it ended with in the top eight bits,
+// below it the first of its turns that was written with that scale by all of its wavefronts (kNoTurn in all bits: redo them all)
+constexpr int kMaxSpecBlocks = kMaxPartials / 2;
+constexpr int kWsTurns = kWsPartials + kMaxSpecBlocks;
+constexpr uint32_t kNoTurn = 0xffffffffu;
+constexpr int kSpecThreads = 512;
 static_assert(kWsMissed < kWsPartials, "the words in front of the partial maxima");
 // a sample of partial maxima from which a fresh meta's scale is guessed: kSampleBlocks words behind the meeting slots
 constexpr int kWsSampleBytes = 12544;
@@ -148,11 +155,24 @@ __device__ __forceinline__ void cast_to_fp8(const IT* __restrict__ x, uint8_t* _
     constexpr int EPT = In16<IT>::EPT;
     constexpr size_t TILE = static_cast<size_t>(THREADS) * EPT * kCastUnroll;
     __shared__ uint32_t red[THREADS / kWave];
+    __shared__ uint32_t first_turn[INTIME == kInTime ? kMaxSpecBlocks : 1];
+    unsigned spec_blocks = 0;    // of the first pass, where its turns decide what is redone
     float s;
     if constexpr (INTIME == kInTime) {
         s = resolve_in_time_scale(it, red, scale_inv);
-        // the first pass quantized all of x with its guess, and the rule confirms that scale: done
-        if (it.speculative && it.ws[kWsSpecDone] != 0u && it.ws[kWsMissed] == 0u && __float_as_uint(s) == it.ws[kWsGuess]) return;
+        if (it.speculative && it.ws[kWsSpecDone] != 0u) {
+            // the first pass quantized all of x with its guess, and the rule confirms that scale: done
+            if (it.ws[kWsMissed] == 0u && __float_as_uint(s) == it.ws[kWsGuess]) return;
+            // or it went on with another one from some turn of each of its workgroups
+            if (it.ws[kWsMissed] != 0u) {
+                spec_blocks = __builtin_amdgcn_readfirstlane(it.ws[1]);
+                for (int b = threadIdx.x; b < kMaxSpecBlocks; b += THREADS) {
+                    const uint32_t w = it.ws[kWsTurns + b];
+                    first_turn[b] = w != kNoTurn && (w >> 24) << 23 == __float_as_uint(s) ? w & 0xffffffu : kNoTurn;
+                }
+                __syncthreads();
+            }
+        }
     } else if constexpr (INTIME == kRescale) {
         const float s_new = scale_rule(*it.known_amax, 1.0f, it.fp_max, it.margin);
         s = s_new * *it.old_scale_inv;
@@ -176,6 +196,14 @@ __device__ __forceinline__ void cast_to_fp8(const IT* __restrict__ x, uint8_t* _
     for (size_t t = block; t < ntiles; t += blocks) {
         const size_t tile = reverse ? (ntiles - 1 - t) : t;
         const size_t base = tile * TILE;
+        if constexpr (INTIME == kInTime) {
+            constexpr size_t kSpecTile = static_cast<size_t>(kSpecThreads) * EPT * kCastUnroll;
+            static_assert(kSpecTile % TILE == 0, "a tile of this pass lies in one of the first");
+            if (spec_blocks != 0u) {
+                const unsigned t1 = static_cast<unsigned>(base / kSpecTile);
+                if (t1 / spec_blocks >= first_turn[t1 % spec_blocks]) continue;    // (kNoTurn: no turn is as late)
+            }
+        }
         if constexpr (PITCHED) {
             const unsigned groups = pt.pitch / EPT, first = static_cast<unsigned>(base / EPT) + tid;
             const size_t nx = static_cast<size_t>(pt.rows) * pt.cols;
@@ -551,13 +579,15 @@ __global__ __launch_bounds__(kBesideThreads) void amax_beside_rescale_kernel(con
 // 64-piece maxima) is continued to the size of x.  What counts is only whether guess and maximum lie in the same binade of
 // fp_max / amax.  235 M bfloat16 elements with a fresh meta: 203 us in two passes (maxima, then the cast; 213 with the fills
 // that made the meta), 122 us when the guess holds, and 257 us when it does not, if all of x is quantized with it all the
-// same.  So a wavefront that meets a value beyond what the guess can stand for raises kWsMissed, and from where a workgroup
-// learns of it, it only takes maxima: 221 to 254 us, the later the few values beyond the guess lie in x (a guess too small a
-// scale is not found out: 257).  Over eight scales in an octave, us on average with the guess, and in two passes with the
-// fills: normal values 138, 213; with rare outliers 123, 216; exponential tails 169, 214; Cauchy 122, 214; log-normal 217,
-// 213 (seven of eight missed; 241 before the pass looked at what it met).
+// same.  So a wavefront that meets a value beyond what its scale can stand for publishes one for it (kWsMissed),
+// from where a workgroup learns of it, it goes on with that one, and the second pass redoes what was written before (kWsTurns): 160 to
+// 170 us where large values are met at once, up to 245 where the first of a few is met late (221 to 254 as long as the pass then only
+// took maxima; a guess of too small a scale is not found out: 257).  Over eight scales in an octave, us on average in two passes with
+// the fills | with maxima only behind a miss | now: normal values 213 | 130 | 130; with rare outliers 216 | 145 | 144; exponential
+// tails 214 | 142 | 135; Cauchy 214 | 166 | 143; log-normal 213 | 209 | 178.  24 draws with one element in a thousand 50 times larger,
+// whose maxima lie about the edge of a binade: 181 | 177.  There a guess of 0.95, 0.9, 0.85 of the maximum gave 186, 195, 199: values
+// beyond it are too few to be met early.
 // A meta that was used before but holds amax 0 and scale 1 is not speculated on: the pass then only takes the maxima.
-constexpr int kSpecThreads = 512;
 
 // The scale for the maximum that the 512 sampled ones (one per lane, as bit patterns) suggest; 0 = no guess.  `growth` =
 // log2(elements of x / elements of 64 pieces) / 6.  The same in every workgroup.
@@ -631,7 +661,8 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
     constexpr int EPT = In16<IT>::EPT;
     constexpr size_t TILE = static_cast<size_t>(kSpecThreads) * EPT * kCastUnroll;
     __shared__ uint32_t red[kSpecThreads / kWave];
-    __shared__ uint32_t s_missed;    // (raised by any wavefront at any time, read whenever it suits: no barrier in the loop)
+    __shared__ uint32_t s_missed;    // (kWsMissed as far as known here: raised by any wavefront at any time, read whenever it suits)
+    __shared__ uint32_t s_wave[kSpecThreads / kWave][2];
     const int tid = threadIdx.x;
     float guess = 1.0f, in_force = 1.0f;
     bool spec = false;
@@ -645,22 +676,30 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
         spec = !(*amax == 0.0f && guess == 1.0f);
     }
     const bool guessed = spec;
-    const float limit = fp_max / guess;    // of a value that the guess can stand for
-    uint32_t m = 0, turn = 0;
+    constexpr uint32_t kInf = 0x7f800000u;
+    const float room = ldexpf(fp_max, -margin);
+    float limit = room / guess;      // of a value that the guess can stand for
+    float cur = guess;               // this wavefront's scale, from its turn `since` on, and the word that says so
+    uint32_t m = 0, turn = 0, missed = 0, since = 0;
     const size_t ntiles = (n + TILE - 1) / TILE;
-    for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x, ++turn) {
         const size_t base = t * TILE;
         if ((vec_ok & 1) && base + TILE <= n) {
             uint4 raw[kCastUnroll];
 #pragma unroll
             for (int u = 0; u < kCastUnroll; ++u)
                 raw[u] = ld16(x + base + (static_cast<size_t>(u) * kSpecThreads + tid) * EPT, (vec_ok & 2) != 0);
-            // One wavefront looks whether another workgroup has found the guess too small, every fourth tile and behind the
-            // tile's loads: the look takes longer than they do (in front of them, every tile: 122 -> 127 us when the guess holds).
+            // One wavefront looks whether another workgroup has met more, every other tile and behind the tile's loads: the look takes
+            // longer than they do (in front of them, every tile: 122 -> 127 us when the guess holds).
             uint32_t elsewhere = 0;
             if (spec && sample != nullptr) {
-                if (tid < kWave && (++turn & 3) == 0) elsewhere = __hip_atomic_load(ws + kWsMissed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                spec = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&s_missed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) == 0u;
+                if (tid < kWave && (turn & 1) != 0) elsewhere = __hip_atomic_load(ws + kWsMissed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t now = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&s_missed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+                if (now != missed) {
+                    missed = now, since = turn;
+                    cur = __uint_as_float(kInf - now), limit = room / cur;
+                    spec = cur > 0.0f;
+                }
             }
 #pragma unroll
             for (int u = 0; u < kCastUnroll; ++u) {
@@ -676,7 +715,7 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
                     uint32_t q[EPT / 4];
 #pragma unroll
                     for (int j = 0; j < EPT / 4; ++j)
-                        q[j] = quant4<FMT>(f[4 * j] * guess, f[4 * j + 1] * guess, f[4 * j + 2] * guess, f[4 * j + 3] * guess);
+                        q[j] = quant4<FMT>(f[4 * j] * cur, f[4 * j + 1] * cur, f[4 * j + 2] * cur, f[4 * j + 3] * cur);
                     uint8_t* o = out + base + (static_cast<size_t>(u) * kSpecThreads + tid) * EPT;
                     if constexpr (EPT == 4) *reinterpret_cast<uint32_t*>(o) = q[0];
                     else *reinterpret_cast<uint2*>(o) = make_uint2(q[0], q[1]);
@@ -684,9 +723,15 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
             }
             if (spec && sample != nullptr) {
                 const float top = sizeof(IT) == 2 && !__is_same(IT, bf16_t) ? f16_bits_to_float(m >> 16) : __uint_as_float(m);
-                const bool here = !(top <= limit);
-                if (here) __hip_atomic_store(ws + kWsMissed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (here || elsewhere != 0u) __hip_atomic_store(&s_missed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (!(top <= limit)) {
+                    // (by halves, as the rule's code in this loop cost 1 us of 130; zero, which ends it, for what has no scale)
+                    float to = top < __uint_as_float(kInf) ? cur : 0.0f;
+                    do to *= 0.5f;
+                    while (to > 0.0f && top > room / to);
+                    elsewhere = kInf - __float_as_uint(to);
+                    __hip_atomic_fetch_max(ws + kWsMissed, elsewhere, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                if (elsewhere > missed) __hip_atomic_fetch_max(&s_missed, elsewhere, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
         } else {
             const size_t end = (base + TILE < n) ? base + TILE : n;
@@ -696,14 +741,23 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
                 } else {
                     m = umax(m, (static_cast<uint32_t>(reinterpret_cast<const uint16_t*>(x)[i]) << 16) & 0x7fff0000u);
                 }
-                if (spec) out[i] = static_cast<uint8_t>(quant1<FMT>(Elem<IT>::load(x + i) * guess));
+                if (spec) out[i] = static_cast<uint8_t>(quant1<FMT>(Elem<IT>::load(x + i) * cur));
             }
         }
     }
+    if ((tid & (kWave - 1)) == 0) s_wave[tid / kWave][0] = missed, s_wave[tid / kWave][1] = since;
     m = block_max_u32(m, red);
     if (tid == 0) {
         if constexpr (sizeof(IT) == 2 && !__is_same(IT, bf16_t)) m = __float_as_uint(f16_bits_to_float(m >> 16));
         ws[kWsPartials + blockIdx.x] = m;
+        if (sample != nullptr) {
+            bool alike = spec && (__float_as_uint(cur) & 0x7fffffu) == 0u;
+            for (int w = 1; w < kSpecThreads / kWave; ++w) {
+                alike = alike && s_wave[w][0] == missed;
+                since = umax(since, s_wave[w][1]);
+            }
+            ws[kWsTurns + blockIdx.x] = alike && since < 0xffffffu ? ((__float_as_uint(cur) << 1) & 0xff000000u) | since : kNoTurn;
+        }
         if (blockIdx.x == 0) {
             ws[0] = __float_as_uint(in_force);
             ws[1] = gridDim.x;
@@ -1540,7 +1594,7 @@ static int launch_speculative(const IT* x, size_t n, const float* scale, const f
     // bit 1: stream the input (this pass reads it once; measured faster at 64 MiB as well as at 470 MiB)
     const int vec_ok = (aligned(x, 16) && aligned(out, EPT) ? 1 : 0) | 2;
     int grid = grid_for(n, static_cast<size_t>(kSpecThreads) * EPT * kCastUnroll);
-    const int cap = cu_count() * 2 < kMaxPartials ? cu_count() * 2 : kMaxPartials;
+    const int cap = cu_count() * 2 < kMaxSpecBlocks ? cu_count() * 2 : kMaxSpecBlocks;
     grid = grid < cap ? grid : cap;
     // a fresh meta (scale == nullptr): guess from a sample, if x is large enough for one to be a small part of it
     uint32_t* sample = nullptr;

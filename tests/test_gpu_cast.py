@@ -580,6 +580,34 @@ def test_fresh_meta_cast_guesses_from_a_sample(be, dtype, what):
     assert torch.equal(got, want) and same_float(fs, s) and same_float(fsi, si) and same_float(fam, am) and count.item() == 0
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('where', ['first', 'middle', 'last', 'steps', 'ragged end', 'steps, then nan', 'steps, then inf'])
+def test_fresh_meta_cast_goes_on_with_a_smaller_scale(be, dtype, where):
+    """Values beyond the sample's guess, met early and late in the pass, once and in several steps of a power of two, on
+    their own and below a value without a scale: every code is the two plain passes'."""
+    esz = torch.finfo(dtype).bits // 8
+    n = (160 << 20) // esz + 1021
+    piece, gen = 16384 // esz, torch.Generator(device='cuda').manual_seed(5)
+    x = torch.empty(n, device='cuda').uniform_(-0.5, 0.5, generator=gen).to(dtype)
+    pieces = n // piece
+    taken = {pieces * b // 512 for b in range(512)}
+    free = [p * piece for p in range(pieces) if p not in taken]
+    at = {'first': 0, 'middle': len(free) // 2, 'last': len(free) - 1}.get(where)
+    if at is not None:
+        x[free[at] + 7] = -40.0
+    elif where == 'ragged end':
+        x[-1] = 3.0
+    else:
+        for i, value in enumerate((0.9, 1.9, 30.0, 7.0, 500.0, 20000.0)):
+            x[free[(i + 1) * len(free) // 8] + i] = value
+        if 'then' in where:
+            x[free[7 * len(free) // 8]] = float(where[-3:])
+    s, si, am = make_meta()
+    want = be.cast_to_fp8_intime(x, s, am[0:1], si, 5, two_pass=True, speculate=False)
+    got, fs, fsi, count, fam = _fresh(be, x, 5)
+    assert torch.equal(got, want) and same_float(fs, s) and same_float(fsi, si) and same_float(fam, am) and count.item() == 0
+
+
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('rows,cols', [(1, 1), (3, 8), (16, 512), (17, 520), (96, 1001), (1000, 260), (4099, 384), (33, 4304),
                                        (12605, 4304), (70001, 264), (40001, 1001)])    # (slabs of several rounds of 16 rows)
