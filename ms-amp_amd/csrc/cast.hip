@@ -2230,17 +2230,32 @@ int msamp_scale_update_groups(const msamp_scale_group* groups, int n_groups, int
 
 namespace msamp {
 
-// A workgroup per 128-wide slice of K; a thread takes 16 elements (32 or 64 bytes in, 16 out) at a time.  A few hundred KiB in
+// A workgroup per 128-wide slice of K; a thread takes 16 elements (32 or 64 bytes in, 16 out).  A few hundred KiB in
 // all: bound by its launch, so while scaling is in time (fin.amax given and the gate open) every workgroup takes the maximum of
 // all of x by itself, out of the L2, instead of waiting for a kernel in front of this one; whichever draws the last ticket, when
 // all have read the old scale, writes the meta.  48 tokens through 4096 -> 12288, the layer call: 35.1 -> 33.8 us.
+// What is left of it is its chain of round trips to memory, so the loads of x, the gate, the scale and the look at amax go out
+// together, where each waited for the one before (and 256 threads took up to 512 pieces in two turns): with the product, from a graph,
+// us, 48 x 4096 -> 12288 28.1 -> 27.5, 64 x 4096 -> 8192 20.8 -> 20.0, 48 x 1040 -> 6000 10.9 -> 9.9, 64 x 64 -> 64 9.4 -> 8.9.
+constexpr int kFewThreads = MSAMP_FEW_TOKENS / 16 * 128;
 template <typename IT>
-__global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __restrict__ x, uint8_t* __restrict__ out, int tokens, int K,
+__global__ __launch_bounds__(kFewThreads) void few_cast_kernel(const IT* __restrict__ x, uint8_t* __restrict__ out, int tokens, int K,
                                                                 const float* scale_p, float* amax, float* scale_inv,
                                                                 int vec_ok, uint32_t* ws, Gate gate, Finish fin) {
     constexpr int EPT = In16<IT>::EPT;
-    __shared__ uint32_t red[kCastThreads / kWave];
+    __shared__ uint32_t red[kFewThreads / kWave];
     __shared__ uint32_t s_top;
+    // this lane's 16 values, on their way before the gate and the scale are known
+    const int p = threadIdx.x, l = p & 63, token = p / 128 * 16 + (l & 15), k = blockIdx.x * 128 + (p >> 6 & 1) * 64 + (l >> 4) * 16;
+    const bool in = token < tokens && k < K;
+    const IT* src = x + (in ? static_cast<size_t>(token) * K + k : 0);
+    uint4 raw[16 / EPT];
+    if (vec_ok) {
+#pragma unroll
+        for (int j = 0; j < 16 / EPT; ++j) raw[j] = ld16(src + j * EPT);
+    }
+    // (the look of amax_publish, here where it costs nothing; a few workgroups more then raise it)
+    const int seen = __hip_atomic_load(reinterpret_cast<int*>(amax), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     float s = *scale_p;
     const bool in_time = fin.amax != nullptr && !gate_closed(gate);
     if (in_time) {
@@ -2249,7 +2264,7 @@ __global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __rest
         const int n = tokens * K;
         if (vec_ok) {
 #pragma unroll 4
-            for (int i = threadIdx.x * EPT; i < n; i += kCastThreads * EPT) {
+            for (int i = threadIdx.x * EPT; i < n; i += blockDim.x * EPT) {
                 const uint4 v = ld16(x + i);
                 const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -2259,7 +2274,7 @@ __global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __rest
                 }
             }
         } else {
-            for (int i = threadIdx.x; i < n; i += kCastThreads) {
+            for (int i = threadIdx.x; i < n; i += blockDim.x) {
                 if constexpr (sizeof(IT) == 4) fold(reinterpret_cast<const uint32_t*>(x)[i]);
                 else fold(reinterpret_cast<const uint16_t*>(x)[i]);
             }
@@ -2284,33 +2299,29 @@ __global__ __launch_bounds__(kCastThreads) void few_cast_kernel(const IT* __rest
             }
         }
     }
-    const int pieces = (tokens + 15) / 16 * 128;
     float mx = 0.0f;
-    for (int p = threadIdx.x; p < pieces; p += kCastThreads) {
-        const int l = p & 63, token = p / 128 * 16 + (l & 15), k = blockIdx.x * 128 + (p >> 6 & 1) * 64 + (l >> 4) * 16;
-        uint4 q = make_uint4(0, 0, 0, 0);
-        if (token < tokens && k < K) {
-            const IT* src = x + static_cast<size_t>(token) * K + k;
-            float v[16];
-            if (vec_ok) {
+    uint4 q = make_uint4(0, 0, 0, 0);
+    if (in) {
+        float v[16];
+        if (vec_ok) {
 #pragma unroll
-                for (int j = 0; j < 16 / EPT; ++j) In16<IT>::load(src + j * EPT, v + j * EPT);
-            } else {
-                for (int j = 0; j < 16; ++j) v[j] = Elem<IT>::load(src + j);
-            }
-#pragma unroll
-            for (int j = 0; j < 16; ++j) mx = fmaxf(mx, fabsf(v[j]));
-            q.x = quant4<MSAMP_DT_E4M3>(v[0] * s, v[1] * s, v[2] * s, v[3] * s);
-            q.y = quant4<MSAMP_DT_E4M3>(v[4] * s, v[5] * s, v[6] * s, v[7] * s);
-            q.z = quant4<MSAMP_DT_E4M3>(v[8] * s, v[9] * s, v[10] * s, v[11] * s);
-            q.w = quant4<MSAMP_DT_E4M3>(v[12] * s, v[13] * s, v[14] * s, v[15] * s);
+            for (int j = 0; j < 16 / EPT; ++j) In16<IT>::decode(raw[j], v + j * EPT);
+        } else {
+            for (int j = 0; j < 16; ++j) v[j] = Elem<IT>::load(src + j);
         }
-        *reinterpret_cast<uint4*>(out + (static_cast<size_t>(blockIdx.x) * pieces + p) * 16) = q;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, fabsf(v[j]));
+        q.x = quant4<MSAMP_DT_E4M3>(v[0] * s, v[1] * s, v[2] * s, v[3] * s);
+        q.y = quant4<MSAMP_DT_E4M3>(v[4] * s, v[5] * s, v[6] * s, v[7] * s);
+        q.z = quant4<MSAMP_DT_E4M3>(v[8] * s, v[9] * s, v[10] * s, v[11] * s);
+        q.w = quant4<MSAMP_DT_E4M3>(v[12] * s, v[13] * s, v[14] * s, v[15] * s);
     }
+    const int pieces = (tokens + 15) / 16 * 128;
+    if (p < pieces) *reinterpret_cast<uint4*>(out + (static_cast<size_t>(blockIdx.x) * pieces + p) * 16) = q;
     if (in_time) return;
     const uint32_t m = block_max_u32(__float_as_uint(mx), red);
     if (threadIdx.x == 0) {
-        amax_publish(amax, __uint_as_float(m));
+        if (static_cast<int>(m) > seen) atomicMax(reinterpret_cast<int*>(amax), static_cast<int>(m));
         if (blockIdx.x == 0) *scale_inv = 1.0f / s;
     }
 }
@@ -2333,9 +2344,9 @@ int few_cast_fragments(const void* x, int in_dtype, int tokens, int K, float* sc
         fin.amax = nullptr;
     }
     const dim3 grid((K + 127) / 128);
-    const int vec_ok = aligned(x, 16);
+    const int vec_ok = aligned(x, 16), threads = std::max(kCastThreads, (tokens + 15) / 16 * 128);
     uint32_t* ws = static_cast<uint32_t*>(workspace);
-#define FEW_CAST(IT) hipLaunchKernelGGL((few_cast_kernel<IT>), grid, dim3(kCastThreads), 0, st, static_cast<const IT*>(x), out, tokens, K, scale, amax, scale_inv, vec_ok, ws, gate, fin)
+#define FEW_CAST(IT) hipLaunchKernelGGL((few_cast_kernel<IT>), grid, dim3(threads), 0, st, static_cast<const IT*>(x), out, tokens, K, scale, amax, scale_inv, vec_ok, ws, gate, fin)
     if (in_dtype == MSAMP_DT_F32) FEW_CAST(float);
     else if (in_dtype == MSAMP_DT_F16) FEW_CAST(f16_t);
     else FEW_CAST(bf16_t);
