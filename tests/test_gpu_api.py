@@ -1109,6 +1109,24 @@ def test_a_few_tokens_without_gradients_have_the_bits_of_the_differentiable_forw
         assert all(same_float(a, b) for a, b in zip((metas.scale, metas.scale_inv, metas.amax), after))
 
 
+@pytest.mark.parametrize('tokens,d_in,d_out', [(5, 1040, 8192), (64, 1040, 8193), (33, 2064, 8300), (17, 144, 12320)])
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16, torch.float32])
+def test_a_few_tokens_through_many_outputs(dtype, tokens, d_in, d_out):
+    """Beyond 8192 outputs a workgroup has four wavefronts, each with more slices of K (a ragged last one among them): whole numbers,
+    whose sums are exact in any order, against the product of the weight's codes."""
+    from msamp import _backend
+    gen = torch.Generator(device='cuda').manual_seed(d_out)
+    w = torch.randint(-8, 9, (d_out, d_in), device='cuda', generator=gen).to(dtype)
+    x = torch.randint(-8, 9, (tokens, d_in), device='cuda', generator=gen).to(torch.bfloat16)
+    x_meta, w_meta = (ScalingMeta(Dtypes.kfloat8_e4m3, window_size=16) for _ in range(2))
+    x_meta.amax_counter.fill_(16)
+    w_meta.amax.fill_(8.0)
+    want = _backend.linear_forward(x, x_meta, w, w_meta, torch.float32, None)[0]
+    got = _backend.linear_forward(x, x_meta, w, w_meta, torch.float32, None, want_codes=False)[0]
+    assert torch.equal(got, want)
+    assert torch.equal(got, (x.double() @ w.double().t()).float())
+
+
 def test_a_few_tokens_without_gradients_lose_no_precision():
     """Real values: against the product of the same codes in 64 bits, the sum in eight parts is as near as the sum in one chain."""
     from msamp import _backend
