@@ -136,6 +136,11 @@ constexpr size_t kAmaxLookChunks = 320, kSpecLookChunks = 384;
 // Chunks (of 80 KiB) that the first pass reads last, with ordinary loads, because the second one, which goes back to front, finds them in
 // the memory-side cache; it reads the others past the caches.
 constexpr unsigned kAmaxKept = 3072;
+// Tensors of more chunks than these are bounded before they are evaluated; in a smaller one hardly anything is published in time, and the
+// bounds and the wavefront's own maxima after every step, which only they need, are left out.  1.0e9 parameters, the step, us, everything
+// evaluated as before | bounds in all | bounds beyond 320: tensors of 256 chunks 3080 | 3105 | 3060, 300 3120 | 3020 | 3001; bounds beyond 800
+// | 320: 384 3018 | 2994, 512 2959 | 2943, 640 2938 | 2925, 768 2897 | 2895.
+constexpr size_t kBoundsChunks = 320;
 constexpr int kSteps = MSAMP_ADAMW_CHUNK / (kAdamThreads * kEPT);    // 4
 
 // 16 elements of one tensor as they lie in memory
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(kAdamThreads, 4) void fused_amax_kernel(msamp_adamw
     bool evaluated = false;
     const bool stream = blockIdx.x + kAmaxKept < gridDim.x;
     if (base + MSAMP_ADAMW_CHUNK <= n) {
-        const bool usable = !L2 && bounds_hold(g_si, inv_m, inv_v, k);
+        const bool usable = !L2 && n > kBoundsChunks * MSAMP_ADAMW_CHUNK && bounds_hold(g_si, inv_m, inv_v, k);
         const RatioBound rb = ratio_bound(inv_m, inv_v, k);
 #pragma unroll 1
         for (int s = 0; s < kSteps; ++s) {
@@ -428,6 +433,7 @@ __global__ __launch_bounds__(kAdamThreads, 4) void fused_amax_kernel(msamp_adamw
             evaluated = true;
             r.launder();
             amax_step<WDT, GDT, L2>(r, w_si, g_si, inv_m, inv_v, k, floor_p, mxp, mxm, mxv);
+            if (!usable) continue;
             floor_m = fmaxf(floor_m, __uint_as_float(wave_max_u32(__float_as_uint(mxm))));
             floor_v = fmaxf(floor_v, __uint_as_float(wave_max_u32(__float_as_uint(mxv))));
         }

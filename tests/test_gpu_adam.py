@@ -267,6 +267,17 @@ def test_first_pass_evaluates_whatever_may_hold_a_maximum(be, w_fmt, w_dt, g_fmt
     assert _same_state(two, one)
 
 
+@pytest.mark.parametrize('extra', [-1, 0, 1, 77, 16384])
+def test_first_pass_where_bounds_begin(be, extra):
+    """Tensors of up to 320 chunks are evaluated without bounds, longer ones with them."""
+    n = 320 * be.ADAMW_CHUNK + extra
+    t = _inputs(1 << 18, 61, fp8.E4M3, fp8.E5M2)
+    for key in 'wgmv':
+        t[key] = t[key].repeat((n >> 18) + 1)[:n].clone()
+    t['m'][n - 4321] = 0xfe
+    assert _same_state(_fused(be, [t], 5, 6, 7)[0], _fused(be, [t], 5, 6, 7, speculative=True)[0])
+
+
 def _same_state(a, b):
     bits = lambda t: t.view(torch.int32) if t.dtype == torch.float32 else (t.view(torch.int16) if t.dtype == torch.float16 else t)
     return all(torch.equal(bits(x), bits(y)) for x, y in zip([a['w'], a['m'], a['v']] + a['wm'] + a['mm'] + a['vm'],
