@@ -377,7 +377,8 @@ __device__ __forceinline__ void bounds16(const Raw16<WDT>& rw, const Raw16<GDT>&
     um = (k.beta1 * rm.max_abs()) * inv_m + k.omb1 * g;
     const float gg = g * g;
     uv = (k.beta2 * v_hi) * inv_v + k.omb2 * gg;
-    const float t = k.bound_rsq * __builtin_amdgcn_rsqf((k.beta2 * v_lo) * inv_v);
+    // (+ 0.0f: as in prepare(), where g^2 is added, a stored -0 counts as zero; its own reciprocal root is -inf, a bound below everything)
+    const float t = k.bound_rsq * __builtin_amdgcn_rsqf((k.beta2 * v_lo) * inv_v + 0.0f);
     float d = um * (k.bound_eps < t ? k.bound_eps : t);
     if (v_lo > 0.0f) d = fminf(d, k.bound_rsq * (rb.m * root + rb.g));
     up = p + d;

@@ -236,7 +236,8 @@ def test_maxima_of_tensors_around_the_looking_lines(be, chunks):
 
 
 @pytest.mark.parametrize('w_fmt,w_dt,g_fmt,g_dt', [(fp8.E4M3, 5, fp8.E5M2, 6), ('f16', 3, fp8.E4M3, 5), (fp8.E5M2, 6, fp8.E5M2, 6)])
-@pytest.mark.parametrize('plant', ['nothing', 'weight', 'hardly any v', 'no v', 'moment', 'gradient', 'second moment', 'negative v', 'nan'])
+@pytest.mark.parametrize('plant', ['nothing', 'weight', 'hardly any v', 'no v', 'moment', 'gradient', 'second moment', 'negative v', 'negative zero v',
+                                   'nan'])
 def test_first_pass_evaluates_whatever_may_hold_a_maximum(be, w_fmt, w_dt, g_fmt, g_dt, plant):
     """The first pass skips elements whose bounds stay below what other workgroups have published.  A tensor of 1700 chunks, of
     which the last third runs behind the first, with one element there that decides a maximum by each way a bound knows; against the
@@ -260,6 +261,8 @@ def test_first_pass_evaluates_whatever_may_hold_a_maximum(be, w_fmt, w_dt, g_fmt
         t['v'][at] = 65504.0
     elif plant == 'negative v':
         t['v'][at] = -1.0
+    elif plant == 'negative zero v':    # among the sixteen of a lane, one of which has the largest weight
+        t['v'][at - 1], t['w'][at] = -0.0, 65504.0 if w_fmt == 'f16' else 0x7e if w_fmt == fp8.E4M3 else 0x7b
     elif plant == 'nan':
         t['m'][at] = 0x7f
     two = _fused(be, [t], w_dt, g_dt, 7)[0]
