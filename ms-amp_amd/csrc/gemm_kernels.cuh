@@ -372,6 +372,28 @@ __device__ __forceinline__ void mfma_fixed(const v8i& a, const v8i& b) {
                  :
                  : "v"(a), "v"(b), "n"(N * 4), "n"(N * 4 + 3), "n"(CB), "n"(BL));
 }
+// A wave's load of 1 KiB, 16 bytes a lane, from `src` (scalar: operand + slice) + `off` (the lane's, 32 bits: no vector instruction is
+// spent on addresses) to LDS at `dst`.  Written as assembly so that the compiler does not see an LDS write it cannot tell apart from
+// the fragment reads: it would otherwise make every LDS read wait for all loads in flight.  Completion is tracked by hand with
+// wait_vmcnt<>() before the barriers of the kernels.
+struct LdsLoad {
+    uint32_t dst, off;
+    const uint8_t* src;
+};
+// The destination goes through M0, and between its write and the load there has to be another instruction, which the compiler sees to
+// only for loads of its own.  In front of the K loop that is an s_nop, in it the MFMA that the load goes with.  us with nothing between
+// them | an s_nop | the MFMA: 16384 x 8192 x 28672 row-major 2348 | 2357 | 2340, both K-major 2373 | 2391 | 2358, 16384 x 16384 x 16384 2783 | 2797 |
+// 2769; 128 x 128 tiles, 1024 x 1024 x 8192 both K-major 32.1 | 32.2 | 31.4, the others level.
+__device__ __forceinline__ void load_to_lds(const LdsLoad& l) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(l.dst), "v"(l.off), "s"(l.src) : "memory", "m0");
+}
+template <int N, int CB, int BL>
+__device__ __forceinline__ void mfma_fixed_and_load(const v8i& a, const v8i& b, const LdsLoad& l) {
+    asm volatile("s_mov_b32 m0, %6\n\tv_mfma_f32_16x16x128_f8f6f4 a[%2:%3], %0, %1, a[%2:%3] cbsz:%4 blgp:%5\n\tglobal_load_lds_dwordx4 %7, %8"
+                 :
+                 : "v"(a), "v"(b), "n"(N * 4), "n"(N * 4 + 3), "n"(CB), "n"(BL), "s"(l.dst), "v"(l.off), "s"(l.src)
+                 : "memory", "m0");
+}
 __device__ __forceinline__ void acc_clear() {
     static_for<64>([&](auto nc) {
         constexpr int n = decltype(nc)::value;
@@ -557,7 +579,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
         return p >= kDmaBlocks * kDmaBlock ? p - kDmaBlocks * kDmaBlock : p;
     };
     // one of this wave's eight loads for a block of slice kt, which is `ahead` slices on from the present one
-    auto dma = [&](int s0, int block, int kt, int ahead, int w, bool last) __attribute__((always_inline)) {
+    auto load_of = [&](int s0, int block, int kt, int ahead, int w, bool last) __attribute__((always_inline)) {
         const bool is_x = block == kX;
         const size_t slice = static_cast<size_t>(kt) * kBK;
         const uint8_t* src = is_x ? X + (XT ? slice * ldx : slice) : Y + (YT ? slice * ldy : slice);
@@ -571,12 +593,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
         }
         // (wave-uniform by construction; the readfirstlane keeps it in a scalar register whatever the compiler makes of it)
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + place(s0, ahead * kPerSlice + block) + (w * 4 + wave) * 1024);
-        // Written as assembly so that the compiler does not see an LDS write it cannot tell apart from
-        // the fragment reads: it would otherwise make every LDS read wait for all loads in flight.
-        // Completion is tracked by hand with wait_vmcnt<>() before the barriers below.  M0 holds the
-        // wave's LDS destination.  The address is a scalar base (operand + slice) plus the lane's 32-bit
-        // offset, so no vector instruction is spent on it.
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(off), "s"(src) : "memory", "m0");
+        return LdsLoad{dst, off, src};
     };
 
     // ---- LDS -> fragments of the 16x16x128 MFMA: a lane holds, for row lane % 16 of a 16-row block, the 32 K-bytes
@@ -639,7 +656,10 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                 const int* cy = fy[hy] + j * 8;
                 const v8i vx = {cx[0], cx[1], cx[2], cx[3], cx[4], cx[5], cx[6], cx[7]};
                 const v8i vy = {cy[0], cy[1], cy[2], cy[3], cy[4], cy[5], cy[6], cy[7]};
-                mfma_fixed<(hx * 4 + i) * 8 + hy * 4 + j, cb, bl>(vy, vx);
+                if (do_load && (n & 3) == 3)
+                    mfma_fixed_and_load<(hx * 4 + i) * 8 + hy * 4 + j, cb, bl>(vy, vx, load_of(s0, ld_block, ld_kt, 2, ld_first + (n >> 2), ld_last));
+                else
+                    mfma_fixed<(hx * 4 + i) * 8 + hy * 4 + j, cb, bl>(vy, vx);
                 if constexpr (vm >= 0 && n == 1) {
                     wait_vmcnt<(vm < 0 ? 0 : vm)>();
                     __syncthreads();
@@ -648,8 +668,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
 #pragma unroll
                     for (int p = (n - 2) * np / 12; p < (n - 1) * np / 12; ++p) read_piece(rd_dst, at, rd_x, rd_half, p);
                 }
-                if (do_load && (n & 3) == 3) dma(s0, ld_block, ld_kt, 2, ld_first + (n >> 2), ld_last);
-                // Nothing moves across: one MFMA, then the reads and the load that go with it, so that the LDS reads and
+                // Nothing moves across: one MFMA, with it the load and then the reads that go with it, so that the LDS reads and
                 // the tile loads stay spread evenly between the MFMAs as written.
                 __builtin_amdgcn_sched_barrier(0);
             });
@@ -670,8 +689,11 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     //   both           2048 x 8192 x 8192  95 / 105 -> 92 / 94     11008 x 4096 x 16384  519 / 521 -> 493 / 498  8192 x 28672 x 16384  2602 / 2595 -> 2426 / 2425
     //   level          8192 x 8192 x 512  51 / 54 -> 50 / 56       4096 x 4096 x 8192, both  91 / 103 -> 91 / 94   8192 x 8192 x 4096, both  190 / 208 -> 192 / 194
     // (Row-major with K of 12288 and more had a form of its own before, its loads in the order of need over a whole step and two meetings
-    // in it: 16384 x 8192 x 28672 2528 / 2510, here 2560 / 2515.  The ring in units of 16 KiB with two meetings a step, every load two
-    // steps to land, was no faster, and slower with both K-major, whose k-rows it took in pieces of 128 bytes: 8192 x 28672 x 16384 2500.)
+    // in it.  16384 x 8192 x K with that form | here: K = 12288 1007 / 1011 | 1005 / 1004, 16384 1335 / 1329 | 1330 / 1321, 20480 1660 / 1657 |
+    // 1659 / 1652, 28672 2349 / 2345 | 2346 / 2344.  Behind kernels that have passed other data through the caches four slices and their
+    // outputs vary by a quarter in either form, here to the slow side more often: 8192 x 8192 x 512 49 to 64, 4096 x 8192 x 512 28 to 36, medians
+    // with the two stages | here 52 | 61 and 29 to 35 | 35; behind small kernels 52 | 52 and 27 | 27.)
+    // (The ring in units of 16 KiB with two meetings a step, every load two steps to land, was no faster, and slower with both K-major, whose k-rows it took in pieces of 128 bytes: 8192 x 28672 x 16384 2500.)
     // `to_go`: slices behind this one, 2 standing for two or more; the last two load nothing.  KTAIL: `last`, the slice that this step
     // loads is the last one.
     auto step = [&](auto to_go_c, int s0, int kt, bool last) __attribute__((always_inline)) {
@@ -694,9 +716,9 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // prologue: slices 0 and 1 (the host sends no problem with fewer than two slices here); wait for slice 0; read
     // its first fragment halves
 #pragma unroll
-    for (int w = 0; w < 16; ++w) dma(0, w < 8 ? kX : kY, 0, 0, w & 7, false);
+    for (int w = 0; w < 16; ++w) load_to_lds(load_of(0, w < 8 ? kX : kY, 0, 0, w & 7, false));
 #pragma unroll
-    for (int w = 0; w < 16; ++w) dma(0, w < 8 ? kX : kY, 1, 1, w & 7, nk == 2);
+    for (int w = 0; w < 16; ++w) load_to_lds(load_of(0, w < 8 ? kX : kY, 1, 1, w & 7, nk == 2));
     wait_vmcnt<16>();
     __syncthreads();
 #pragma unroll
@@ -736,7 +758,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
             };
             const int t = threadIdx.x;
             const uint32_t dump = __builtin_amdgcn_readfirstlane(lds_base + kDmaBlocks * kDmaBlock - 256);
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off\n\tglobal_load_lds_dword %2, off\n\t"
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\tglobal_load_lds_dword %2, off\n\t"
                          "global_load_lds_dword %3, off\n\tglobal_load_lds_dword %4, off"
                          : : "s"(dump), "v"(line(t, true)), "v"(line(t + 256, true)), "v"(line(t, false)), "v"(line(t + 256, false))
                          : "memory", "m0");

@@ -54,6 +54,13 @@ __device__ __forceinline__ void vmfma_fixed(const v8i& a, const v8i& b) {
                  :
                  : "v"(a), "v"(b), "n"(kVacc + N * 4), "n"(kVacc + N * 4 + 3), "n"(CB), "n"(BL));
 }
+template <int N, int CB, int BL>
+__device__ __forceinline__ void vmfma_fixed_and_load(const v8i& a, const v8i& b, const LdsLoad& l) {
+    asm volatile("s_mov_b32 m0, %6\n\tv_mfma_f32_16x16x128_f8f6f4 v[%2:%3], %0, %1, v[%2:%3] cbsz:%4 blgp:%5\n\tglobal_load_lds_dwordx4 %7, %8"
+                 :
+                 : "v"(a), "v"(b), "n"(kVacc + N * 4), "n"(kVacc + N * 4 + 3), "n"(CB), "n"(BL), "s"(l.dst), "v"(l.off), "s"(l.src)
+                 : "memory", "m0");
+}
 __device__ __forceinline__ void vacc_clear() {
     static_for<16>([&](auto nc) {
         constexpr int n = decltype(nc)::value;
@@ -153,8 +160,8 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
         return PAIR ? (2 * kt + (is_x ? 0 : 1)) % kPairUnits * kPairUnit
                     : kt % kSmallStages * kSmallStage + (is_x ? 0 : kSmallTile * kBK);
     };
-    // one of the 8 loads of a slice (0..3: X rows, 4..7: Y rows); assembly for the reason given at the large tile
-    auto dma = [&](int kt, int which, bool last = false) __attribute__((always_inline)) {
+    // one of the 8 loads of a slice (0..3: X rows, 4..7: Y rows); where it comes from and goes to
+    auto load_of = [&](int kt, int which, bool last = false) __attribute__((always_inline)) {
         const bool is_x = which < 4;
         const size_t slice = static_cast<size_t>(kt) * kBK;
         const uint8_t* src = is_x ? X + (XT ? slice * ldx : slice) : Y + (YT ? slice * ldy : slice);
@@ -167,8 +174,9 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
             }
         }
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + place(kt, is_x) + ((which & 3) * 4 + wave) * 1024);
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(off), "s"(src) : "memory", "m0");
+        return LdsLoad{dst, off, src};
     };
+    auto dma = [&](int kt, int which, bool last = false) __attribute__((always_inline)) { load_to_lds(load_of(kt, which, last)); };
     auto dma_slice = [&](int kt, bool last = false) __attribute__((always_inline)) {
 #pragma unroll
         for (int w = 0; w < 8; ++w) dma(kt, w, last);
@@ -232,7 +240,14 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
             const v8i vx = {cx[0], cx[1], cx[2], cx[3], cx[4], cx[5], cx[6], cx[7]};
             const v8i vy = {cy[0], cy[1], cy[2], cy[3], cy[4], cy[5], cy[6], cy[7]};
             if constexpr (PAIR) {
-                vmfma_fixed<i * 4 + j, cb, bl>(vy, vx);
+                const bool load_y = do_load && (n & 1) && n < 8, load_x = next_x && (n & 1) && n >= 8, tail = KTAIL && ld_last;
+                auto load = [&]() __attribute__((always_inline)) {
+                    return load_y ? load_of(ld_kt, 4 + (n >> 1), ld_last && !next_x) : load_of(ld_kt + 1, (n >> 1) - 4, ld_last);
+                };
+                // (the loads of a ragged last slice have offsets of their own, for which there is no register beside the operands)
+                if ((load_y || load_x) && !tail) vmfma_fixed_and_load<i * 4 + j, cb, bl>(vy, vx, load());
+                else vmfma_fixed<i * 4 + j, cb, bl>(vy, vx);
+                if ((load_y || load_x) && tail) load_to_lds(load());
                 // the Y fragments of the next slice with the first eight MFMAs, an X block in place of this slice's behind
                 // its last MFMA
                 if (do_read && n < 8) {
@@ -243,19 +258,17 @@ __device__ __forceinline__ void gemm_dma128(const uint8_t* __restrict__ X, const
 #pragma unroll
                     for (int p = i * kPX / 4; p < (i + 1) * kPX / 4; ++p) read_piece(fx[0], fy[cur ^ 1], px, py, p);
                 }
-                if (do_load && (n & 1) && n < 8) dma(ld_kt, 4 + (n >> 1), ld_last && !next_x);
-                if (next_x && (n & 1) && n >= 8) dma(ld_kt + 1, (n >> 1) - 4, ld_last);
             } else {
-                mfma_fixed<i * 4 + j, cb, bl>(vy, vx);
+                // the eight tile loads of slice ld_kt, one every other MFMA: issued in one go they hold the wave, and with
+                // it its MFMAs, for as long as the memory pipe takes to accept them
+                if (do_load && (n & 1)) mfma_fixed_and_load<i * 4 + j, cb, bl>(vy, vx, load_of(ld_kt, n >> 1, ld_last));
+                else mfma_fixed<i * 4 + j, cb, bl>(vy, vx);
                 // the fragment reads go with the first eight MFMAs (two to four each) and have come back by the barrier that
                 // follows the last one; nothing moves across, so they stay spread as written
                 if (do_read && n < 8) {
 #pragma unroll
                     for (int p = n * kPieces / 8; p < (n + 1) * kPieces / 8; ++p) read_piece(fx[cur ^ 1], fy[cur ^ 1], px, py, p);
                 }
-                // the eight tile loads of slice ld_kt, one every other MFMA: issued in one go they hold the wave, and with
-                // it its MFMAs, for as long as the memory pipe takes to accept them
-                if (do_load && (n & 1)) dma(ld_kt, n >> 1, ld_last);
             }
             __builtin_amdgcn_sched_barrier(0);
         });

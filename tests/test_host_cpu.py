@@ -350,6 +350,35 @@ def test_paired_gemm_kernels_leave_their_accumulators_to_the_matrix_instructions
     assert len(products) == 18 and min(products.values()) >= 16    # three output types, three layouts, whole and ragged K
 
 
+@pytest.mark.parametrize('pair', GEMM_PAIRS)
+def test_loads_to_lds_wait_for_their_address(gemm_assembly, pair):
+    """A load to LDS takes its destination from M0 and needs a wait state behind the instruction that writes it; its scalar base
+    needs five behind a vector instruction that writes that.  The compiler keeps both only for loads of its own, not for those
+    written as assembly."""
+    registers = lambda text: {n for m in re.finditer(r'\bs(\d+)\b|\bs\[(\d+):(\d+)\]', text)
+                              for n in ([int(m.group(1))] if m.group(1) else range(int(m.group(2)), int(m.group(3)) + 1))}
+    loads, m0, vector, kernel = {}, 0, {}, None    # instructions since M0, and since each scalar register, was written
+    for line in itertools.chain.from_iterable(open(path) for path in gemm_assembly[pair]):
+        m = re.match(r'^(_Z\w+):', line)
+        code = line.split(';')[0].strip()
+        if m:
+            kernel, m0, vector = m.group(1), 9, {}
+        if m or not code or code.startswith('.') or code.endswith(':'):
+            continue
+        op, args = code.split()[0], code[len(code.split()[0]):].split(',')
+        if '_load_lds_' in op:
+            loads[kernel] = loads.get(kernel, 0) + 1
+            assert m0 >= 1, (kernel, code)
+            assert all(vector.get(r, 9) >= 5 for r in registers(args[-1])), (kernel, code)
+        states = int(args[0], 0) + 1 if op == 's_nop' else 1
+        m0, vector = m0 + states, {r: n + states for r, n in vector.items() if n < 9}
+        if args[0].strip() == 'm0':
+            m0 = 0
+        elif op.startswith('v_'):
+            vector.update((r, 0) for r in registers(args[0]))
+    assert len(loads) >= 64 and min(loads.values()) >= 16    # 28 with 256 x 256 tiles, 18 with 128 x 128 and as many in pairs
+
+
 def test_the_last_workgroup_of_a_few_tokens_cast_writes_the_meta_behind_every_read_of_it(tmp_path):
     """few_cast_kernel: every workgroup reads the old scale and draws a ticket, and the last one overwrites the scale.  The ticket
     has to release the read and acquire the others' (at agent scope: buffer_wbl2 ahead of it, buffer_inv behind it)."""
