@@ -919,7 +919,7 @@ def test_every_tile_is_written_whatever_the_walk(be, nr, nc, k, a_kmajor, b_kmaj
     # the walk the rules pick, then each of the four registered by hand (what the timing at first use may choose)
     be.tune_gemm_walks(False)
     try:
-        for walk in (-1, 0, 1, 2, 3, 4, 7):    # (4..7: the split waits too; they apply to row-major operands only)
+        for walk in (-1, 0, 1, 2, 3, 4, 7):    # (the third bit is taken and changes nothing)
             assert lib.msamp_fp8_gemm_set_walk(nc, nr, k, int(a_kmajor), int(b_kmajor), walk) == 0
             assert lib.msamp_fp8_gemm_get_walk(nc, nr, k, int(a_kmajor), int(b_kmajor)) == walk
             out.fill_(float('nan'))
@@ -933,35 +933,58 @@ def test_every_tile_is_written_whatever_the_walk(be, nr, nc, k, a_kmajor, b_kmaj
 
 @pytest.mark.parametrize('n, m, k', [(1024, 768, 256), (2048, 1280, 384), (1536, 2048, 1152), (4096, 2048, 4096), (2304, 1792, 640),
                                      (8192, 4096, 24576 + 128)])
-def test_split_waits_change_no_bit(be, large_tiles_only, n, m, k):
-    """With both operands row-major the K loop can await a slice's tile loads in two parts (bit 2 of a registered walk; by
-    rule from K = 24576 on): random codes, even and odd slice counts down to two and three, ragged edges, bias and sum
-    -- the same bits as the plain form and as the generic kernel."""
-    g = torch.Generator(device='cuda').manual_seed(n + m + k)
-    a = torch.randint(0, 0x7f, (m, k), device='cuda', dtype=torch.uint8, generator=g)
-    b = torch.randint(0, 0x7f, (n - 3, k), device='cuda', dtype=torch.uint8, generator=g)    # a ragged last tile row
+def test_large_tiles_change_no_bit_whatever_the_walk(be, large_tiles_only, n, m, k):
+    """Both operands row-major, random finite codes, even and odd slice counts down to two and three, ragged edges, bias and sum:
+    with every walk the bits of the generic kernel, which has no walk, no ring of blocks in LDS and another tile."""
+    a = _gpu_codes((m, k), 5, n + m + k)
+    b = _gpu_codes((n - 3, k), 6, n + m + k + 1)    # a ragged last tile row
     a_si = torch.tensor(0.37, device='cuda')
-    b_si = torch.tensor(1.9, device='cuda')
-    bias = torch.randn(m, device='cuda', generator=g).bfloat16()
+    b_si = torch.tensor(1.9e-4, device='cuda')
+    bias = torch.randn(m, device='cuda', generator=torch.Generator(device='cuda').manual_seed(n + m + k)).bfloat16()
     lib = be.load()
     be.tune_gemm_walks(False)
+
+    def products():
+        plain = be.fp8_gemm(a, 5, a_si, b, 6, b_si, torch.full((n - 3, m), float('nan'), dtype=torch.bfloat16, device='cuda'))
+        return plain, be.fp8_gemm(a, 5, a_si, b, 6, b_si, plain.clone(), accumulate=True, bias=bias)
+
     outs = {}
     try:
-        for walk in (0, 4, 1, 5, 6, 7, -1):
+        for walk in (0, 1, 2, 3, 4, 7, -1):
             assert lib.msamp_fp8_gemm_set_walk(m, n - 3, k, 0, 0, walk) == 0
-            plain = be.fp8_gemm(a, 5, a_si, b, 6, b_si, torch.full((n - 3, m), float('nan'), dtype=torch.bfloat16, device='cuda'))
-            summed = be.fp8_gemm(a, 5, a_si, b, 6, b_si, plain.clone(), accumulate=True, bias=bias)
-            outs[walk] = (plain, summed)
+            outs[walk] = products()
     finally:
         lib.msamp_fp8_gemm_set_walk(m, n - 3, k, 0, 0, -1)
         be.tune_gemm_walks(True)
+    be.set_small_tile_limit(-1)    # (the fixture puts the default back)
+    generic = products()
+    assert all(t.isfinite().all() for t in generic)
     for walk, (plain, summed) in outs.items():
-        assert torch.equal(plain.view(torch.int16), outs[0][0].view(torch.int16)), walk
-        assert torch.equal(summed.view(torch.int16), outs[0][1].view(torch.int16)), walk
-    if k <= 4096:
-        be.set_small_tile_limit(-1)    # (the fixture puts the default back)
-        generic = be.fp8_gemm(a, 5, a_si, b, 6, b_si, torch.empty(n - 3, m, dtype=torch.bfloat16, device='cuda'))
-        assert torch.equal(generic.view(torch.int16), outs[0][0].view(torch.int16))
+        assert torch.equal(plain.view(torch.int16), generic[0].view(torch.int16)), walk
+        assert torch.equal(summed.view(torch.int16), generic[1].view(torch.int16)), walk
+
+
+@pytest.mark.parametrize('k', [256, 384, 512, 640, 768, 896, 1408, 24704, 144, 272, 400, 528, 656, 784, 1008, 24704 + 112])
+@pytest.mark.parametrize('a_kmajor,b_kmajor', [(False, False), (True, False), (True, True)])
+def test_large_tiles_over_any_number_of_slices(be, large_tiles_only, k, a_kmajor, b_kmajor):
+    """The large tile's operands pass through a ring of five blocks of LDS, two to a slice of K: two to seven slices begin and end at
+    each of its places, whole and with a ragged last one, and long K goes around it many times.  Whole numbers up to 2: every sum
+    is a whole number below 2**24, exact in float32, so the product is the exact one."""
+    n, m = 1008, 784    # ragged last tiles
+    g = torch.Generator(device='cuda').manual_seed(k)
+
+    def operand(rows, dt, kmajor):
+        values = torch.randint(-2, 3, (rows, k), device='cuda', generator=g)
+        codes = torch.tensor([0xC0, 0xB8 if dt == 5 else 0xBC, 0, 0x38 if dt == 5 else 0x3C, 0x40], device='cuda', dtype=torch.uint8)
+        t = codes[values + 2]
+        return (t.t() if kmajor else t).contiguous(), values.double()
+
+    a, av = operand(m, 5, a_kmajor)
+    b, bv = operand(n, 6, b_kmajor)
+    one = torch.ones((), device='cuda')
+    out = torch.full((n, m), float('nan'), device='cuda')
+    be.fp8_gemm(a, 5, one, b, 6, one, out, a_kmajor=a_kmajor, b_kmajor=b_kmajor)
+    assert torch.equal(out.double(), bv @ av.t().contiguous())
 
 
 def test_walk_timed_at_first_use_changes_no_bit(be):
