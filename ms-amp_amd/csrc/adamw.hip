@@ -339,10 +339,12 @@ struct RatioBound {
 __device__ __forceinline__ RatioBound ratio_bound(float inv_m, float inv_v, const AdamConsts& k) {
     return {1.00001f * k.beta1 * inv_m / sqrtf(k.beta2 * inv_v), 1.00001f * k.omb1 / sqrtf(k.omb2)};
 }
-// Do bounds16()'s bounds hold: factors without surprises, and no g^2 of a code but zero underflows.
+// Do bounds16()'s bounds hold: factors without surprises.  beta2 v of a v above zero (2^-24 and more) is a normal number then, 2^-124 and
+// more.  omb2 g^2 need not be one: where it is less than 2^-126 and comes out with few bits or none, |g| is below 2^-63 / sqrt(omb2), and its
+// part of the ratio, at most omb1 |g| / sqrt(beta2 v), half of what ratio_bound() has for it.  Nor may g^2 overflow.
 __device__ __forceinline__ bool bounds_hold(float g_si, float inv_m, float inv_v, const AdamConsts& k) {
     auto fine = [](float x) { return x >= 0x1.0p-60f && x <= 0x1.0p60f; };
-    return fine(inv_m) && fine(inv_v) && fine(fabsf(g_si) * 0x1.0p20f) && k.beta1 >= 0.0f && k.omb1 >= 0.0f && fine(k.beta2) && fine(k.omb2);
+    return fine(inv_m) && fine(inv_v) && fabsf(g_si) <= 0x1.0p40f && k.beta1 >= 0.0f && k.omb1 >= 0.0f && k.beta2 >= 0x1.0p-40f && fine(k.omb2);
 }
 // Upper bounds of |p'|, |m'| and |v'| over 16 elements, without evaluating them (decoupled decay only).  |m'| and |v'|: every operation
 // of prepare() is monotonic in the magnitudes, rounding included, so the chain of the largest magnitudes is a bound without any slack.

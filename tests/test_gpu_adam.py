@@ -270,6 +270,27 @@ def test_first_pass_evaluates_whatever_may_hold_a_maximum(be, w_fmt, w_dt, g_fmt
     assert _same_state(two, one)
 
 
+@pytest.mark.parametrize('g_exp', [-110, -80, -66, -56, -48, 40, 41])
+@pytest.mark.parametrize('v_exp', [-59, 0])
+def test_first_pass_bounds_gradients_of_any_size(be, g_exp, v_exp):
+    """Gradients whose squares are too small for a float32, or nearly so, beside second moments down to the smallest that the bounds
+    take, and gradients up to the largest whose squares are finite and beyond: with eps far below both the update is the ratio of the
+    moments, which the first pass bounds; against the one-pass step, which looks at every element."""
+    n = 700 * be.ADAMW_CHUNK
+    t = _inputs(1 << 18, 62, fp8.E4M3, fp8.E5M2)
+    g = torch.Generator().manual_seed(63)
+    t['g'] = torch.randint(0, 0x7c, t['g'].shape, generator=g, dtype=torch.uint8) | torch.randint(0, 2, t['g'].shape, generator=g, dtype=torch.uint8) << 7
+    t['v'] = torch.randint(1, 2048, t['v'].shape, generator=g, dtype=torch.int16).view(torch.float16)
+    t['v'][torch.rand(t['v'].shape, generator=g) < 0.01] = 0.0
+    for key in 'wgmv':
+        t[key] = t[key].repeat(n >> 18 if n % (1 << 18) == 0 else (n >> 18) + 1)[:n].clone()
+    t['m'][n - 50 * be.ADAMW_CHUNK + 5] = 0x7e
+    t['gm']['scale_inv'], t['gm']['scale'] = torch.tensor(2.0**g_exp), torch.tensor(2.0**-g_exp)
+    t['vm']['scale_inv'], t['vm']['scale'] = torch.tensor(2.0**v_exp), torch.tensor(2.0**-v_exp)
+    for eps in (1e-8, 1e-36):
+        assert _same_state(_fused(be, [t], 5, 6, 7, eps=eps)[0], _fused(be, [t], 5, 6, 7, eps=eps, speculative=True)[0]), eps
+
+
 @pytest.mark.parametrize('extra', [-1, 0, 1, 77, 16384])
 def test_first_pass_where_bounds_begin(be, extra):
     """Tensors of up to 320 chunks are evaluated without bounds, longer ones with them."""
