@@ -133,9 +133,10 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 constexpr int kEPT = 16;                                   // elements per thread per step
 // tensors of more chunks than these look at their maxima's words before they raise them (raise_max.cuh)
 constexpr size_t kAmaxLookChunks = 320, kSpecLookChunks = 384;
-// Chunks (of 80 KiB) that the first pass reads last, with ordinary loads, because the second one, which goes back to front, finds them in
-// the memory-side cache; it reads the others past the caches.
-constexpr unsigned kAmaxKept = 3072;
+// What the first pass reads last of its inputs it reads with ordinary loads, because the second one, which goes back to front, finds it in
+// the memory-side cache (256 MiB); the rest it reads past the caches.  (Float16 weights, the step, us repeated / behind other data, with 3072
+// chunks kept, 288 MiB of theirs | with 240 MiB: 49 M parameters 146 / 193 | 140 / 193, 74 M 211 / 261 | 209 / 257, 400 M level.)
+constexpr size_t kAmaxKeptBytes = size_t(240) << 20;
 // Tensors of more chunks than these are bounded before they are evaluated; in a smaller one hardly anything is published in time, and the
 // bounds and the wavefront's own maxima after every step, which only they need, are left out.  1.0e9 parameters, the step, us, everything
 // evaluated as before | bounds in all | bounds beyond 320: tensors of 256 chunks 3080 | 3105 | 3060, 300 3120 | 3020 | 3001; bounds beyond 800
@@ -413,7 +414,8 @@ __global__ __launch_bounds__(kAdamThreads, 4) void fused_amax_kernel(msamp_adamw
     float floor_p = __uint_as_float(seen_word(&d.acc[0])), floor_m = __uint_as_float(seen_word(&d.acc[1])), floor_v = __uint_as_float(seen_word(&d.acc[2]));
     if (!(floor_p >= 0.0f)) floor_p = 0.0f;    // a NaN already published: everything is exact from here on
     bool evaluated = false;
-    const bool stream = blockIdx.x + kAmaxKept < gridDim.x;
+    constexpr unsigned kKept = kAmaxKeptBytes / (MSAMP_ADAMW_CHUNK * (Raw16<WDT>::kWords + Raw16<GDT>::kWords + 4 + 8) / 4);    // chunks
+    const bool stream = blockIdx.x + kKept < gridDim.x;
     if (base + MSAMP_ADAMW_CHUNK <= n) {
         const bool usable = !L2 && n > kBoundsChunks * MSAMP_ADAMW_CHUNK && bounds_hold(g_si, inv_m, inv_v, k);
         const RatioBound rb = ratio_bound(inv_m, inv_v, k);

@@ -250,7 +250,7 @@ def test_first_pass_evaluates_whatever_may_hold_a_maximum(be, w_fmt, w_dt, g_fmt
     t['v'][5::1009], t['m'][5::1009] = 3.0 * 2.0**-24, 1
     at = n - 40 * be.ADAMW_CHUNK + 4321
     if plant == 'weight':
-        t['w'][at] = t['w'].max() if w_fmt == 'f16' else 0x7e if w_fmt == fp8.E4M3 else 0x7b
+        t['w'][at] = 65504.0 if w_fmt == 'f16' else 0x7e if w_fmt == fp8.E4M3 else 0x7b
     elif plant in ('hardly any v', 'no v'):
         t['m'][at], t['v'][at], t['g'][at] = 0x30, 2.0**-24 if plant == 'hardly any v' else 0.0, 0
     elif plant == 'moment':
@@ -289,6 +289,21 @@ def test_first_pass_bounds_gradients_of_any_size(be, g_exp, v_exp):
     t['vm']['scale_inv'], t['vm']['scale'] = torch.tensor(2.0**v_exp), torch.tensor(2.0**-v_exp)
     for eps in (1e-8, 1e-36):
         assert _same_state(_fused(be, [t], 5, 6, 7, eps=eps)[0], _fused(be, [t], 5, 6, 7, eps=eps, speculative=True)[0]), eps
+
+
+@pytest.mark.parametrize('w_fmt,w_dt,g_fmt,g_dt', [(fp8.E4M3, 5, fp8.E5M2, 6), ('f16', 3, fp8.E4M3, 5)])
+@pytest.mark.parametrize('chunk', [3, 1250, 4300])
+def test_first_pass_of_more_than_the_memory_side_cache_holds(be, w_fmt, w_dt, g_fmt, g_dt, chunk):
+    """4400 chunks are 344 MiB and more: the first 1328 are read past the caches, those behind by ordinary loads.  What decides the
+    three maxima lies among the first of all, among those read past the caches behind them, or among the last; against the one-pass step."""
+    n = 4400 * be.ADAMW_CHUNK
+    t = _inputs(1 << 18, 64, w_fmt, g_fmt)
+    for key in 'wgmv':
+        t[key] = t[key].repeat(n >> 18)[:n].clone()
+    at = chunk * be.ADAMW_CHUNK + 4321
+    t['w'][at] = 65504.0 if w_fmt == 'f16' else 0x7e
+    t['m'][at + 2048], t['v'][at + 4096] = 0xfe, 65504.0
+    assert _same_state(_fused(be, [t], w_dt, g_dt, 7)[0], _fused(be, [t], w_dt, g_dt, 7, speculative=True)[0])
 
 
 @pytest.mark.parametrize('extra', [-1, 0, 1, 77, 16384])
