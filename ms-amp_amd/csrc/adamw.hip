@@ -138,9 +138,9 @@ constexpr size_t kAmaxLookChunks = 320, kSpecLookChunks = 384;
 // chunks kept, 288 MiB of theirs | with 240 MiB: 49 M parameters 146 / 193 | 140 / 193, 74 M 211 / 261 | 209 / 257, 400 M level.)
 constexpr size_t kAmaxKeptBytes = size_t(240) << 20;
 // Tensors of more chunks than these are bounded before they are evaluated; in a smaller one hardly anything is published in time, and the
-// bounds and the wavefront's own maxima after every step, which only they need, are left out.  1.0e9 parameters, the step, us, everything
-// evaluated as before | bounds in all | bounds beyond 320: tensors of 256 chunks 3080 | 3105 | 3060, 300 3120 | 3020 | 3001; bounds beyond 800
-// | 320: 384 3018 | 2994, 512 2959 | 2943, 640 2938 | 2925, 768 2897 | 2895.
+// bounds and the wavefront's own maxima after every step, which only they need, are left out.  5.0e8 parameters, the step, us, nothing
+// bounded | everything: tensors of 256 chunks 1312 | 1337, 300 1318 | 1335, 340 1366 | 1336 (the words are looked at beyond 320, too), 384 1351 |
+// 1336, 512 1338 | 1328, 1024 1325 | 1322, 3000 1268 | 1199.
 constexpr size_t kBoundsChunks = 320;
 constexpr int kSteps = MSAMP_ADAMW_CHUNK / (kAdamThreads * kEPT);    // 4
 
@@ -390,7 +390,8 @@ __device__ __forceinline__ void bounds16(const Raw16<WDT>& rw, const Raw16<GDT>&
 // First pass: the exact maxima of |p'|, |m'| and |v'| by bounding.  A wavefront's 1024 elements are evaluated (amax_step) only if the
 // bounds over some lane's 16 of them reach above the maxima found so far, by this wavefront or, as published when its workgroup began,
 // by others; the elements that attain the true maxima always do.  The workgroups that run first in a tensor have nothing to compare
-// with and evaluate everything: all of a tensor of up to about a thousand chunks, a third of one of three thousand.
+// with but what they have found themselves, which holds off a sixth: a tensor of up to a thousand chunks, which run all at once, has 0.84 of
+// it evaluated, one of 1500 0.56, of 2000 0.43, of 3000 0.28.
 // The evaluation takes 28 vector instructions an element, with a reciprocal square root, the bounds 10: evaluating everything bound the pass
 // to 4.3 TB/s, now it is bound by its read of 5 bytes an element.  405 M parameters in ten tensors, E4M3 weights, the step: 1070 -> 1001 us
 // repeated, 1084 -> 1023 where other data has passed the caches in between; one tensor of 50 M 139 -> 123; float16 weights 1287 -> 1214.
