@@ -193,14 +193,15 @@ __global__ __launch_bounds__(512) void few_tokens_kernel(const WT* __restrict__ 
 template <typename WT, typename OT, int MB>
 static int launch_few_tokens(const msamp_linear_forward_args& a, hipStream_t st) {
     const int tokens = static_cast<int>(a.tokens), d_out = static_cast<int>(a.d_out), K = static_cast<int>(a.d_in);
-    // Up to two workgroups of eight wavefronts fit a CU, and what no longer fits at once begins a round of its own: beyond 512
-    // workgroups they are of four, five a CU.  us with eight and four: 48 x 4096 -> 12288 33.3, 28.5, 64 x 4096 -> 11008 33.1, 28.0,
+    // Up to two workgroups of eight wavefronts fit a CU, and what no longer fits at once begins a round of its own: beyond two a CU
+    // (here 512) they are of four wavefronts, five a CU.  us with eight and four: 48 x 4096 -> 12288 33.3, 28.5, 64 x 4096 -> 11008 33.1, 28.0,
     // 64 x 2048 -> 16384 23.0, 21.5, 48 x 4096 -> 32000 66.4, 64.3; up to 512, 48 x 1040 -> 6000 11.1, 10.9, 64 x 4096 -> 8192 20.9, 21.0,
-    // 16 x 8192 -> 8192 30.1, 32.6, 32 x 11008 -> 4096 24.9, 27.1.
-    const int waves = std::min(d_out > 512 * 16 ? 4 : 8, (K + 127) / 128);
+    // 16 x 8192 -> 8192 30.1, 32.6, 32 x 11008 -> 4096 24.9, 27.1.  Just beyond the line either is ahead somewhere: 16 x 4096 -> 8208 18.1, 16.7,
+    // 48 tokens 19.5, 20.8, 16 x 8192 -> 8208 32.0, 34.9, 16 x 16384 -> 8208 67.6, 61.6.
+    const int workgroups = (d_out + 15) / 16, waves = std::min(workgroups > 2 * cu_count() ? 4 : 8, (K + 127) / 128);
     const bool stream = static_cast<size_t>(d_out) * K * sizeof(WT) >= kStreamBytes;
     const auto kernel = stream ? few_tokens_kernel<WT, OT, MB, true> : few_tokens_kernel<WT, OT, MB, false>;
-    hipLaunchKernelGGL(kernel, dim3((d_out + 15) / 16), dim3(64 * waves), waves * (MB * 1024 + 2048), st,
+    hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(64 * waves), waves * (MB * 1024 + 2048), st,
                        static_cast<const WT*>(a.w), a.x_codes, static_cast<OT*>(a.y), tokens, d_out, K, a.w_amax, a.w_scale_inv,
                        a.x_scale_inv, a.bias, static_cast<int>(a.bias_dtype));
     MSAMP_CHECK_LAUNCH("few_tokens_kernel");
