@@ -51,7 +51,7 @@ struct GemmCall {
 template <int XF, int YF>
 int run_gemm_pair(const GemmCall& c);
 // The other half of a pair's instantiations lives in a translation unit of its own (gemm_inst.hip built with
-// -DMSAMP_GEMM_SPLIT_UNIT), so that they compile side by side: the 256 x 256-tile kernel for a ragged last slice of K and the
+// -DMSAMP_GEMM_SECOND_UNIT), so that they compile side by side: the 256 x 256-tile kernel for a ragged last slice of K and the
 // 128 x 128-tile kernels (all layouts and output types).
 template <int XF, int YF>
 int run_gemm_ragged(const GemmCall& c);

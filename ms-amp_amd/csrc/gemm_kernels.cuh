@@ -854,7 +854,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
                 q_scale = posted ? static_cast<uint32_t>(ps) : 0x7fc00000u;
             }
         }
-        __syncthreads();    // also: every wave is through with the stages, which the patches below reuse
+        __syncthreads();    // also: every wave is through with the ring, which the patches below reuse
         const float sc = __uint_as_float(q_scale);
         const uint32_t acc_token2 = acc_refence(acc_token);    // a second round of reads, not the first one kept alive
         // with a positive finite amax and the scale derived from it nothing leaves the format and nothing is NaN:
@@ -1376,7 +1376,7 @@ static int pick_out_spec(const uint8_t* X, const uint8_t* Y, void* D, int d_dtyp
     }
 }
 
-#ifdef MSAMP_GEMM_SPLIT_UNIT
+#ifdef MSAMP_GEMM_SECOND_UNIT
 // output type and operand layout of a call -> one instantiation of LAUNCH<XF, YF, output type, XT, YT>
 #define MSAMP_LAYOUT_LAUNCH(LAUNCH, OT)                                                                                              \
     do {                                                                                                                             \

@@ -273,7 +273,7 @@ def gemm_assembly(tmp_path_factory):
     procs = []
     for xf, yf in GEMM_PAIRS:
         # (each pair is two translation units: large tiles over whole slices of K, and the ragged ones and small tiles)
-        for unit, extra in (('inst', []), ('split', ['-DMSAMP_GEMM_SPLIT_UNIT'])):
+        for unit, extra in (('inst', []), ('second', ['-DMSAMP_GEMM_SECOND_UNIT'])):
             out = str(tmp / f'gemm_{unit}_{xf}{yf}.s')
             cmd = [hipcc, '--offload-arch=gfx950', '-O3', '-std=c++17', '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
                    '-Wno-unused-command-line-argument', '-Wno-inline-asm', f'-DMSAMP_XF={xf}', f'-DMSAMP_YF={yf}', *extra,
