@@ -9,7 +9,9 @@ update.  A step is one such pass over the five layers; `value` is the fifteen GE
 the whole step time, inputs resident in HBM.
 
 `roofline` is the GEMM kernel alone: the flops of the GEMM launches bracketed by HIP events inside the timed
-region (every fourth step), divided by their summed duration, against the dense-FP8 MFMA peak.
+region (every fourth step), divided by their summed duration, against the dense-FP8 MFMA peak.  Those are the weight
+gradients with their casts; the other products are launched by library calls for a whole direction, between whose kernels no
+event can be recorded from here.
 
 Beside it: the same step at config 2 (one FP8Linear 8192 x 4096 x 4096), a per-shape GEMM sweep over the
 Llama-7B (config 4) and Llama-70B (config 5) projections x {forward, dgrad, wgrad}, the cast+amax and fused
@@ -923,7 +925,8 @@ def main():
                                'scaling (history 16) after %d untimed scaling warm-up steps, outputs bf16, dW -> E4M3'
                                % SCALING_WARMUP_STEPS},
         'roofline': {
-            'kernel': 'fp8_gemm_dma_kernel (flop-weighted over the 15 GEMM launches of the config-4 step)',
+            'kernel': 'fp8_gemm_dma_kernel (flop-weighted over the GEMM launches of the config-4 step that events can bracket: '
+                      'the 5 weight gradients of 15; traffic: per launch over all 15)',
             'bound': 'mfma', 'achieved': lin['gemm_tflops'], 'peak': FP8_PEAK_TFLOPS, 'unit': 'TFLOP/s',
             'frac': lin['gemm_tflops'] / FP8_PEAK_TFLOPS, 'traffic': traffic, 'traffic_source': traffic_source,
             'avg_launch_ms': lin['gemm_avg_launch_ms'], 'avg_launch_flops': lin['gemm_avg_launch_flops'],
