@@ -42,6 +42,7 @@ constexpr int kWsMissed = 14;
 constexpr int kMaxSpecBlocks = kMaxPartials / 2;
 constexpr int kWsTurns = kWsPartials + kMaxSpecBlocks;
 constexpr uint32_t kNoTurn = 0xffffffffu;
+constexpr size_t kGoOnBytes = size_t(144) << 20;    // (measured at cast_speculative_kernel)
 constexpr int kSpecThreads = 512;
 static_assert(kWsMissed < kWsPartials, "the words in front of the partial maxima");
 // a sample of partial maxima from which a fresh meta's scale is guessed: kSampleBlocks words behind the meeting slots
@@ -164,7 +165,7 @@ __device__ __forceinline__ void cast_to_fp8(const IT* __restrict__ x, uint8_t* _
             // the first pass quantized all of x with its guess, and the rule confirms that scale: done
             if (it.ws[kWsMissed] == 0u && __float_as_uint(s) == it.ws[kWsGuess]) return;
             // or it went on with another one from some turn of each of its workgroups
-            if (it.ws[kWsMissed] != 0u) {
+            if (it.ws[kWsMissed] != 0u && it.ws[kWsMissed] != 0x7f800000u) {
                 spec_blocks = __builtin_amdgcn_readfirstlane(it.ws[1]);
                 for (int b = threadIdx.x; b < kMaxSpecBlocks; b += THREADS) {
                     const uint32_t w = it.ws[kWsTurns + b];
@@ -581,12 +582,21 @@ __global__ __launch_bounds__(kBesideThreads) void amax_beside_rescale_kernel(con
 // that made the meta), 122 us when the guess holds, and 257 us when it does not, if all of x is quantized with it all the
 // same.  So a wavefront that meets a value beyond what its scale can stand for publishes one for it (kWsMissed),
 // from where a workgroup learns of it, it goes on with that one, and the second pass redoes what was written before (kWsTurns): 160 to
-// 170 us where large values are met at once, up to 245 where the first of a few is met late (221 to 254 as long as the pass then only
-// took maxima; a guess of too small a scale is not found out: 257).  Over eight scales in an octave, us on average in two passes with
-// the fills | with maxima only behind a miss | now: normal values 213 | 130 | 130; with rare outliers 216 | 145 | 144; exponential
-// tails 214 | 142 | 135; Cauchy 214 | 166 | 143; log-normal 213 | 209 | 178.  24 draws with one element in a thousand 50 times larger,
-// whose maxima lie about the edge of a binade: 181 | 177.  There a guess of 0.95, 0.9, 0.85 of the maximum gave 186, 195, 199: values
-// beyond it are too few to be met early.
+// 170 us where large values are met at once, up to 245 to 290 where the largest is met late, where what was written with the scales before it
+// was written for nothing (221 to 254 if the pass then only takes maxima; a guess of too small a scale is not found out: 257).  So the fewer
+// the values beyond the guess, the less there is to gain, and as long as x and its codes stay in the memory-side cache, where reading
+// them again costs little, there is something to lose: up to 144 MiB of x (kGoOnBytes) the pass only takes maxima behind a miss.
+// us, means of 16 to 60 draws at scales all over an octave, only maxima | going on:
+//   float32, MiB   72       112      144      160      180      208      360        940        1600
+//   log-normal  37 | 40   50 | 52  62 | 63  69 | 69  77 | 75  89 | 83  157 | 137  404 | 338  674 | 599
+//   t(3)        37 | 39   53 | 55  62 | 63  70 | 69  78 | 76  88 | 81  157 | 146  379 | 321  679 | 612
+//   Cauchy      34 | 36   46 | 46  53 | 52  60 | 57  64 | 61  74 | 67  131 | 105  318 | 258  552 | 429
+//   bfloat16, MiB  80       112      144      160      180      220        470        800
+//   log-normal  45 | 47   59 | 60  70 | 70  84 | 80  94 | 90  112 | 104  244 | 232  394..399 | 352..417
+//   t(3)        45 | 47   57 | 59  72 | 71  80 | 78  92 | 88  111 | 106  237 | 225  397..401 | 381..393
+// Where the guess holds, to be ready for a miss costs 0 to 1 %: 470 MiB of normal bfloat16 148 | 149.  24 draws with one element in a
+// thousand 50 times larger, whose maxima lie about the edge of a binade: 181 | 177.  There a guess of 0.95, 0.9, 0.85 of the maximum gave
+// 186, 195, 199: values beyond it are too few to be met early.
 // A meta that was used before but holds amax 0 and scale 1 is not speculated on: the pass then only takes the maxima.
 
 // The scale for the maximum that the 512 sampled ones (one per lane, as bit patterns) suggest; 0 = no guess.  `growth` =
@@ -724,8 +734,9 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
             if (spec && sample != nullptr) {
                 const float top = sizeof(IT) == 2 && !__is_same(IT, bf16_t) ? f16_bits_to_float(m >> 16) : __uint_as_float(m);
                 if (!(top <= limit)) {
-                    // (by halves, as the rule's code in this loop cost 1 us of 130; zero, which ends it, for what has no scale)
-                    float to = top < __uint_as_float(kInf) ? cur : 0.0f;
+                    // (by halves, as the rule's code in this loop cost 1 us of 130; zero, which ends it, for what has no scale and for
+                    // tensors of which only the maxima are taken from here on)
+                    float to = (vec_ok & 4) != 0 && top < __uint_as_float(kInf) ? cur : 0.0f;
                     do to *= 0.5f;
                     while (to > 0.0f && top > room / to);
                     elsewhere = kInf - __float_as_uint(to);
@@ -750,10 +761,11 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
     if (tid == 0) {
         if constexpr (sizeof(IT) == 2 && !__is_same(IT, bf16_t)) m = __float_as_uint(f16_bits_to_float(m >> 16));
         ws[kWsPartials + blockIdx.x] = m;
-        if (sample != nullptr) {
+        if (sample != nullptr && (vec_ok & 4) != 0) {
             bool alike = spec && (__float_as_uint(cur) & 0x7fffffu) == 0u;
+#pragma unroll
             for (int w = 1; w < kSpecThreads / kWave; ++w) {
-                alike = alike && s_wave[w][0] == missed;
+                alike &= s_wave[w][0] == missed;
                 since = umax(since, s_wave[w][1]);
             }
             ws[kWsTurns + blockIdx.x] = alike && since < 0xffffffu ? ((__float_as_uint(cur) << 1) & 0xff000000u) | since : kNoTurn;
@@ -1592,7 +1604,8 @@ static int launch_speculative(const IT* x, size_t n, const float* scale, const f
                               int margin, uint32_t* ws, hipStream_t st) {
     constexpr int EPT = In16<IT>::EPT;
     // bit 1: stream the input (this pass reads it once; measured faster at 64 MiB as well as at 470 MiB)
-    const int vec_ok = (aligned(x, 16) && aligned(out, EPT) ? 1 : 0) | 2;
+    // bit 2: behind a miss go on with the next scale
+    const int vec_ok = (aligned(x, 16) && aligned(out, EPT) ? 1 : 0) | 2 | (n * sizeof(IT) > kGoOnBytes ? 4 : 0);
     int grid = grid_for(n, static_cast<size_t>(kSpecThreads) * EPT * kCastUnroll);
     const int cap = cu_count() * 2 < kMaxSpecBlocks ? cu_count() * 2 : kMaxSpecBlocks;
     grid = grid < cap ? grid : cap;

@@ -582,11 +582,13 @@ def test_fresh_meta_cast_guesses_from_a_sample(be, dtype, what):
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize('where', ['first', 'middle', 'last', 'steps', 'ragged end', 'steps, then nan', 'steps, then inf'])
-def test_fresh_meta_cast_goes_on_with_a_smaller_scale(be, dtype, where):
+@pytest.mark.parametrize('mib', [100, 160])
+def test_fresh_meta_cast_goes_on_with_a_smaller_scale(be, dtype, where, mib):
     """Values beyond the sample's guess, met early and late in the pass, once and in several steps of a power of two, on
-    their own and below a value without a scale: every code is the two plain passes'."""
+    their own and below a value without a scale: every code is the two plain passes'.  Up to 144 MiB the pass only takes the maxima
+    behind such a value, beyond it goes on with the next scale."""
     esz = torch.finfo(dtype).bits // 8
-    n = (160 << 20) // esz + 1021
+    n = (mib << 20) // esz + 1021
     piece, gen = 16384 // esz, torch.Generator(device='cuda').manual_seed(5)
     x = torch.empty(n, device='cuda').uniform_(-0.5, 0.5, generator=gen).to(dtype)
     pieces = n // piece
