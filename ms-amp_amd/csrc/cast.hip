@@ -594,7 +594,8 @@ __global__ __launch_bounds__(kBesideThreads) void amax_beside_rescale_kernel(con
 //   bfloat16, MiB  80       112      144      160      180      220        470        800
 //   log-normal  45 | 47   59 | 60  70 | 70  84 | 80  94 | 90  112 | 104  244 | 232  394..399 | 352..417
 //   t(3)        45 | 47   57 | 59  72 | 71  80 | 78  92 | 88  111 | 106  237 | 225  397..401 | 381..393
-// Where the guess holds, to be ready for a miss costs 0 to 1 %: 470 MiB of normal bfloat16 148 | 149.  24 draws with one element in a
+// (Only maxima by a word that is stored: raised by an atomic maximum of each wavefront, as it has to be for going on, 72 MiB took 38.2 where it
+// takes 37.0.)  Where the guess holds, to be ready for a miss costs 0 to 1 %: 470 MiB of normal bfloat16 148 | 149.  24 draws with one element in a
 // thousand 50 times larger, whose maxima lie about the edge of a binade: 181 | 177.  There a guess of 0.95, 0.9, 0.85 of the maximum gave
 // 186, 195, 199: values beyond it are too few to be met early.
 // A meta that was used before but holds amax 0 and scale 1 is not speculated on: the pass then only takes the maxima.
@@ -733,16 +734,20 @@ __global__ __launch_bounds__(kSpecThreads) void cast_speculative_kernel(const IT
             }
             if (spec && sample != nullptr) {
                 const float top = sizeof(IT) == 2 && !__is_same(IT, bf16_t) ? f16_bits_to_float(m >> 16) : __uint_as_float(m);
-                if (!(top <= limit)) {
-                    // (by halves, as the rule's code in this loop cost 1 us of 130; zero, which ends it, for what has no scale and for
-                    // tensors of which only the maxima are taken from here on)
-                    float to = (vec_ok & 4) != 0 && top < __uint_as_float(kInf) ? cur : 0.0f;
-                    do to *= 0.5f;
-                    while (to > 0.0f && top > room / to);
-                    elsewhere = kInf - __float_as_uint(to);
-                    __hip_atomic_fetch_max(ws + kWsMissed, elsewhere, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((vec_ok & 4) == 0) {    // only the maxima from here on: one word, which may be stored by all
+                    if (!(top <= limit)) __hip_atomic_store(ws + kWsMissed, elsewhere = kInf, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (elsewhere != 0u) __hip_atomic_store(&s_missed, kInf, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                } else {
+                    if (!(top <= limit)) {
+                        // (by halves, as the rule's code in this loop cost 1 us of 130; zero, which ends it, for what has no scale)
+                        float to = top < __uint_as_float(kInf) ? cur : 0.0f;
+                        do to *= 0.5f;
+                        while (to > 0.0f && top > room / to);
+                        elsewhere = kInf - __float_as_uint(to);
+                        __hip_atomic_fetch_max(ws + kWsMissed, elsewhere, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                    if (elsewhere > missed) __hip_atomic_fetch_max(&s_missed, elsewhere, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
-                if (elsewhere > missed) __hip_atomic_fetch_max(&s_missed, elsewhere, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
         } else {
             const size_t end = (base + TILE < n) ? base + TILE : n;
