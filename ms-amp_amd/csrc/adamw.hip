@@ -2060,29 +2060,44 @@ static int fused_args_ok(const char* who, const void* tensors, int n_tensors, co
     return MSAMP_OK;
 }
 
-// launch KERNEL<weight type, gradient type, l2> for the runtime types
-#define FUSED_LAUNCH_WG(KERNEL, NB, W, G, ...)                                                                        \
+// launch KERNEL<weight type, gradient type, l2> for the runtime types, with LDS bytes of dynamic LDS
+#define FUSED_LAUNCH_WG(KERNEL, NB, LDS, W, G, ...)                                                                   \
     do {                                                                                                              \
         if (l2)                                                                                                       \
-            hipLaunchKernelGGL((KERNEL<W, G, true>), dim3(NB), dim3(kAdamThreads), 0, st, __VA_ARGS__);               \
+            hipLaunchKernelGGL((KERNEL<W, G, true>), dim3(NB), dim3(kAdamThreads), LDS, st, __VA_ARGS__);             \
         else                                                                                                          \
-            hipLaunchKernelGGL((KERNEL<W, G, false>), dim3(NB), dim3(kAdamThreads), 0, st, __VA_ARGS__);              \
+            hipLaunchKernelGGL((KERNEL<W, G, false>), dim3(NB), dim3(kAdamThreads), LDS, st, __VA_ARGS__);            \
     } while (0)
-#define FUSED_LAUNCH(KERNEL, NB, ...)                                                                                 \
+#define FUSED_LAUNCH_LDS(KERNEL, NB, LDS, ...)                                                                        \
     do {                                                                                                              \
         if (weight_dtype == MSAMP_DT_E4M3 && grad_dtype == MSAMP_DT_E4M3)                                             \
-            FUSED_LAUNCH_WG(KERNEL, NB, MSAMP_DT_E4M3, MSAMP_DT_E4M3, __VA_ARGS__);                                   \
+            FUSED_LAUNCH_WG(KERNEL, NB, LDS, MSAMP_DT_E4M3, MSAMP_DT_E4M3, __VA_ARGS__);                              \
         else if (weight_dtype == MSAMP_DT_E4M3)                                                                       \
-            FUSED_LAUNCH_WG(KERNEL, NB, MSAMP_DT_E4M3, MSAMP_DT_E5M2, __VA_ARGS__);                                   \
+            FUSED_LAUNCH_WG(KERNEL, NB, LDS, MSAMP_DT_E4M3, MSAMP_DT_E5M2, __VA_ARGS__);                              \
         else if (weight_dtype == MSAMP_DT_E5M2 && grad_dtype == MSAMP_DT_E4M3)                                        \
-            FUSED_LAUNCH_WG(KERNEL, NB, MSAMP_DT_E5M2, MSAMP_DT_E4M3, __VA_ARGS__);                                   \
+            FUSED_LAUNCH_WG(KERNEL, NB, LDS, MSAMP_DT_E5M2, MSAMP_DT_E4M3, __VA_ARGS__);                              \
         else if (weight_dtype == MSAMP_DT_E5M2)                                                                       \
-            FUSED_LAUNCH_WG(KERNEL, NB, MSAMP_DT_E5M2, MSAMP_DT_E5M2, __VA_ARGS__);                                   \
+            FUSED_LAUNCH_WG(KERNEL, NB, LDS, MSAMP_DT_E5M2, MSAMP_DT_E5M2, __VA_ARGS__);                              \
         else if (grad_dtype == MSAMP_DT_E4M3)                                                                         \
-            FUSED_LAUNCH_WG(KERNEL, NB, MSAMP_DT_F16, MSAMP_DT_E4M3, __VA_ARGS__);                                    \
+            FUSED_LAUNCH_WG(KERNEL, NB, LDS, MSAMP_DT_F16, MSAMP_DT_E4M3, __VA_ARGS__);                               \
         else                                                                                                          \
-            FUSED_LAUNCH_WG(KERNEL, NB, MSAMP_DT_F16, MSAMP_DT_E5M2, __VA_ARGS__);                                    \
+            FUSED_LAUNCH_WG(KERNEL, NB, LDS, MSAMP_DT_F16, MSAMP_DT_E5M2, __VA_ARGS__);                               \
     } while (0)
+
+#define FUSED_LAUNCH(KERNEL, NB, ...) FUSED_LAUNCH_LDS(KERNEL, NB, 0, __VA_ARGS__)
+
+// Dynamic LDS that the first pass asks for and does not use, so that four of its workgroups run on a compute unit and not five (as
+// the registers have it for FP8 weights; with float16 ones it is four anyway): where five leave a second round of a few workgroups
+// that run by themselves, or one with little to compare with.  E4M3 weights, the step, us repeated / behind other data, five | four:
+//   one tensor of 1290 chunks  69.9 / 102.4 | 66.0 / 90.4     1400  71.4 / 102.7 | 66.9 / 95.3     1900  80.7 / 118.0 | 79.4 / 112.4
+//   4 of 330  74.2 / 104.6 | 74.9 / 99.0     2 of 700  74.8 / 103.0 | 74.3 / 96.3     2 of 800  81.5 / 113.8 | 81.8 / 106.7
+//   in one round  4 of 310  72.1 / 89.3 | 74.7 / 93.4     in more than two  3 of 800  110.2 / 147.7 | 111.9 / 143.6     6 of 400  110.2 / 148.9 |
+//   112.3 / 145.6     8 of 400  145.8 / 193.3 | 148.7 / 192.1     20 of 1000  853 / 884 | 874 / 903
+// Where every tensor is evaluated whole five are the better (8 of 200  83.8 / 106.8 | 85.4 / 107.0).
+static unsigned amax_lds(int blocks, const int32_t* blocks_per_tensor, int n_tensors) {
+    if (blocks <= 5 * cu_count() || blocks > 8 * cu_count() || blocks_per_tensor == nullptr) return 0;
+    return *std::max_element(blocks_per_tensor, blocks_per_tensor + n_tensors) > static_cast<int32_t>(kBoundsChunks) ? 36 * 1024 : 0;
+}
 
 int msamp_adamw_fp8_fused(msamp_adamw_tensor* tensors, int n_tensors, const int32_t* block_map, int n_blocks,
                           int weight_dtype, int grad_dtype, double lr, double beta1, double beta2, double eps,
@@ -2113,7 +2128,7 @@ int msamp_adamw_fp8_fused(msamp_adamw_tensor* tensors, int n_tensors, const int3
         MSAMP_REQUIRE(b1 <= n_blocks, MSAMP_ERR_SHAPE, "msamp_adamw_fp8_fused: blocks_per_tensor exceeds n_blocks");
         const int nb = b1 - b0, nt = t1 - t0;
         if (nb > 0) {
-            FUSED_LAUNCH(fused_amax_kernel, nb, tensors, block_map + 2 * b0, k);
+            FUSED_LAUNCH_LDS(fused_amax_kernel, nb, amax_lds(nb, blocks_per_tensor == nullptr ? nullptr : blocks_per_tensor + t0, nt), tensors, block_map + 2 * b0, k);
             MSAMP_CHECK_LAUNCH("fused_amax_kernel");
         }
         hipLaunchKernelGGL(fused_scales_kernel, dim3((nt + 63) / 64), dim3(64), 0, st, tensors + t0, nt, w_fp_max,
