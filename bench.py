@@ -443,7 +443,7 @@ def bench_cast(iters=20):
     n_layer = sum(wt.numel() for wt in weights)
     row('c5_intime_bf16_e4m3_layer_856M', _time_gpu(layer_cast, 5, warm=2), n_layer * 3)
     del w, weights
-    # what a plain copy reaches on this box (the practical ceiling of the streaming kernels above): 256 MiB of
+    # what a plain copy reaches on this card (the practical ceiling of the streaming kernels above): 256 MiB of
     # fp32 through the library's scale_cast at scale 1, read once, written once
     src = torch.ones(64 * 1024 * 1024, device='cuda')
     one = torch.ones((), device='cuda')
@@ -631,7 +631,7 @@ def cpu_baseline():
     [28672,8192] weight, and the GEMM definition (fp32 matmul of dequantized operands) on a slice of config 2."""
     import torch
     from oracle import adamw as oadam, cast as ocast, fp8
-    # the box sets OMP_NUM_THREADS to its CPU share; never spread over more threads than that
+    # OMP_NUM_THREADS may be set to a share of the CPUs; never spread over more threads than that
     cores = min(os.cpu_count() or 1, int(os.environ.get('OMP_NUM_THREADS', '16') or 16))
     torch.set_num_threads(cores)
 

@@ -691,7 +691,7 @@ __global__ __launch_bounds__(kGemmThreads) void fp8_gemm_dma_kernel(const uint8_
     // (Row-major with K of 12288 and more had a form of its own before, its loads in the order of need over a whole step and two meetings
     // in it.  16384 x 8192 x K with that form | here: K = 12288 1007 / 1011 | 1005 / 1004, 16384 1335 / 1329 | 1330 / 1321, 20480 1660 / 1657 |
     // 1659 / 1652, 28672 2349 / 2345 | 2346 / 2344.  Four slices behind kernels that have passed other data
-    // through the caches: with the two stages | here 8192 x 8192 x 512 50 | 49, 4096 x 8192 x 512 29 | 28; on one box of four either form varied, by
+    // through the caches: with the two stages | here 8192 x 8192 x 512 50 | 49, 4096 x 8192 x 512 29 | 28; on one card of four either form varied, by
     // a quarter, and this one was more often at the slow end, 49 to 64 and 28 to 36, medians 52 | 61 and 29 to 35 | 35.)
     // (The ring in units of 16 KiB with two meetings a step, every load two steps to land, was no faster, and slower with both K-major, whose k-rows it took in pieces of 128 bytes: 8192 x 28672 x 16384 2500.)
     // `to_go`: slices behind this one, 2 standing for two or more; the last two load nothing.  KTAIL: `last`, the slice that this step
