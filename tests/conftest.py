@@ -10,4 +10,4 @@ for p in (ROOT, os.path.join(ROOT, 'ms-amp_amd')):
 
 
 def pytest_configure(config):
-    config.addinivalue_line('markers', 'gpu: needs a real MI355X (run with -m gpu on the GPU box)')
+    config.addinivalue_line('markers', 'gpu: needs a real MI355X (run with -m gpu where there is one)')
